@@ -120,8 +120,8 @@ int omni_attn_fwd_gfx950(const void* q, const void* k, const void* v, void* o,
  * D in 1..256 -- the generality of the reference's scalar kernel omni_attn_simple_kernel
  * (omni-attn-mma/mma/attn_naive.cu:21-302; D <= 256 from its `float out[256]`, :189-190; its
  * launcher :305-408 has no block-size or head-dim whitelist).  Same arguments, semantics and
- * status codes as omni_attn_fwd_gfx950 (pointers need only their natural alignment); two-pass
- * fp32 softmax per query row like the reference's kernel.  A correctness path, not a fast one.
+ * status codes as omni_attn_fwd_gfx950 (pointers need only their natural alignment).  The weights are
+ * not rounded to 16 bits before the second product, as in the reference's kernel.
  */
 int omni_attn_fwd_generic_gfx950(const void* q, const void* k, const void* v, void* o,
                                  float* lse_or_null,

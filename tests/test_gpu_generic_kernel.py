@@ -70,3 +70,26 @@ def test_simple_wrapper_takes_shapes_the_other_wrappers_refuse(gpu_device):
     assert (out.float().cpu() - ref).abs().max().item() <= 2e-3
     with pytest.raises(ValueError, match="head_dim"):
         oat.omni_attention_shared_kv_swizzle(q, k, v, mask)
+
+
+@pytest.mark.parametrize("QB,KB,D", [(16, 16, 5), (48, 48, 8), (33, 7, 13), (32, 32, 31), (40, 40, 33), (64, 48, 100),
+                                     (16, 32, 129), (128, 128, 161), (32, 64, 224), (48, 16, 250)])
+def test_generic_kernel_edges_of_tiles_and_chunks(QB, KB, D, gpu_device):
+    """Head dimensions around the 8-column chunks and 32-column tiles, key blocks that do not fill or
+    that straddle a 32-key step, query blocks of a fraction of a 32-row tile.  Tighter than the bars:
+    the weights are not rounded before the second product, so the error is the rounding of the
+    result (half an ulp of |o| < 4: 2^-10) and fp32 sums of at most 600 terms."""
+    gen = torch.Generator().manual_seed(QB * 1000 + KB * 10 + D)
+    B, H = 2, 1
+    S = 2 * QB * KB if QB * KB < 300 else 3 * max(QB, KB)
+    S = -(-S // QB) * QB
+    q, k, v = (torch.randn(B, H, S, D, generator=gen).to(torch.float16) for _ in range(3))
+    Tk = -(-S // KB)
+    nb, idx, tys, pidx, pm = random_block_metadata(gen, B, H, S // QB, Tk, QB, KB, p_empty=0.2, shuffle=True)
+    for seqlen in (S, S - 5):
+        o, lse = run_generic(q, k, v, nb, idx, tys, QB, KB, seqlen, pidx, pm, gpu_device)
+        wo, wl = attention_block_walk(q, k, v, nb, idx, tys, QB, KB, seqlen, pidx, pm)
+        assert torch.equal(torch.isinf(lse.cpu()), torch.isinf(wl))
+        assert (o.float().cpu() - wo).abs().max().item() <= 2.0 ** -10, (QB, KB, D, seqlen)
+        live = ~torch.isinf(wl)
+        assert (lse.cpu()[live] - wl[live]).abs().max().item() <= 2e-5

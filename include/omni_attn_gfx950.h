@@ -145,6 +145,36 @@ int omni_attn_pack_partial_masks_gfx950(const uint8_t* partial_masks, uint32_t* 
                                         int num_partial, int QB, int KB, void* stream);
 
 /*
+ * Block mask of a prefix rule: row i of batch element b attends the keys below R[b, i].  R comes
+ * either from `prefix` ([B, q_len] int64) or from `spans` ([B, M, 3] int64 rows of (type, offset,
+ * length)) by the rule of transfusion_pytorch/transfusion.py:496-515: R = max(i + 1, offset + length
+ * of every span of positive length with offset <= i).  R is cut at kv_len; rows >= q_len of the
+ * last query block attend nothing.  A key block is not listed when no row attends any of it, FULL
+ * when all rows attend all of it, CAUSAL when the rows attend exactly the keys <= their own index,
+ * else PARTIAL.  The tiles are numbered in (b, query block, slot) order and shared by the heads.
+ *
+ * omni_attn_mask_lists_gfx950 writes kv_num_blocks [B, H, Tq] and kv_indices, block_mask_types,
+ * partial_idx [B, H, Tq, Tk] (Tq = ceil(q_len / QB), Tk = ceil(kv_len / KB); zeros, and -1 in
+ * partial_idx, behind the lists), and the number of PARTIAL tiles to host_total[0] -- host
+ * memory that the device can write (hipHostMalloc) -- and then `ticket` to host_total[1]: the caller
+ * waits for the ticket (or for the stream), allocates the tiles and calls
+ * omni_attn_mask_tiles_gfx950 with the same arguments and the same workspace
+ * (omni_attn_mask_workspace_bytes), which writes partial_masks [P, QB, KB] bytes (16-byte
+ * aligned) and, where asked for (KB a multiple of 32), the packed words of
+ * omni_attn_pack_partial_masks_gfx950.  QB up to OMNI_ATTN_MASK_MAX_QB.
+ */
+#define OMNI_ATTN_MASK_MAX_QB 8192
+size_t omni_attn_mask_workspace_bytes(int B, int q_len, int kv_len, int QB, int KB);
+int omni_attn_mask_lists_gfx950(const int64_t* spans_or_null, const int64_t* prefix_or_null,
+                                int32_t* kv_num_blocks, int32_t* kv_indices, int32_t* block_mask_types,
+                                int32_t* partial_idx, void* workspace, int32_t* host_total, int ticket,
+                                int B, int M, int H, int q_len, int kv_len, int QB, int KB, void* stream);
+int omni_attn_mask_tiles_gfx950(const int64_t* spans_or_null, const int64_t* prefix_or_null,
+                                void* workspace, uint8_t* partial_masks, uint32_t* partial_bits_or_null,
+                                int num_partial, int B, int M, int H, int q_len, int kv_len, int QB, int KB,
+                                void* stream);
+
+/*
  * omni_attn_fwd_gfx950 with the PARTIAL tiles already packed by
  * omni_attn_pack_partial_masks_gfx950 (same semantics and results bit for bit; the byte
  * tiles of the reference's signature, omni-attn-mma/pybind/omni_attn.cc:10-68, are

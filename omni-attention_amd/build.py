@@ -138,7 +138,7 @@ def build_capi(jobs):
         cmds.append([HIPCC] + DEVICE_FLAGS + [
             "-DOMNI_INST_BF16=%d" % bf, "-DOMNI_INST_D=%d" % d,
             "-c", os.path.join(CSRC, "omni_attn_bwd_inst.hip"), "-o", obj])
-    for src in ("omni_attn_capi", "omni_attn_probe", "omni_attn_mask_pack", "omni_attn_fwd_generic"):
+    for src in ("omni_attn_capi", "omni_attn_probe", "omni_attn_mask_pack", "omni_attn_mask_build", "omni_attn_fwd_generic"):
         obj = os.path.join(OBJ, src + ".o")
         objs.append(obj)
         cmds.append([HIPCC] + DEVICE_FLAGS + ["-c", os.path.join(CSRC, src + ".hip"), "-o", obj])

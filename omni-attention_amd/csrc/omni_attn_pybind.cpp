@@ -10,8 +10,10 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
+#include <mutex>
 #include <stdexcept>
 #include <string>
+#include <vector>
 
 #include "omni_attn_gfx950.h"
 
@@ -295,6 +297,122 @@ void omni_attn_backward(torch::Tensor Q, torch::Tensor K, torch::Tensor V, torch
   }
 }
 
+// Where a kernel writes one number that the host waits for: pinned host memory, handed out per
+// call (so calls of several threads and streams do not meet) and taken back; at most kKeep of
+// them are kept between calls.
+class HostNumber {
+ public:
+  HostNumber() {
+    std::lock_guard<std::mutex> lock(mutex());
+    if (!spare().empty()) {
+      slot_ = spare().back();
+      spare().pop_back();
+      return;
+    }
+    void* mem = nullptr;
+    const hipError_t e = hipHostMalloc(&mem, 64, hipHostMallocDefault);
+    if (e != hipSuccess) throw std::runtime_error(std::string("omni_attn: hipHostMalloc: ") + hipGetErrorString(e));
+    slot_ = static_cast<int32_t*>(mem);
+    slot_[0] = slot_[1] = slot_[2] = 0;
+  }
+  ~HostNumber() {
+    if (!idle_) return;  // a kernel may still write it: the memory stays allocated
+    std::lock_guard<std::mutex> lock(mutex());
+    if (spare().size() < kKeep) {
+      spare().push_back(slot_);
+    } else {
+      (void)hipHostFree(slot_);
+    }
+  }
+  HostNumber(const HostNumber&) = delete;
+  HostNumber& operator=(const HostNumber&) = delete;
+
+  int32_t* memory() { return slot_; }
+  int next_ticket() {
+    idle_ = false;
+    return ++slot_[2];
+  }
+  // The number, once the kernel that writes it has run.  Ends as well when the stream has
+  // nothing left to run or reports an error.
+  int wait(int ticket, hipStream_t stream) {
+    for (unsigned spins = 1;; ++spins) {
+      if (__atomic_load_n(slot_ + 1, __ATOMIC_ACQUIRE) == ticket) break;
+      if (spins % 8192 == 0) {
+        const hipError_t e = hipStreamQuery(stream);
+        if (e == hipErrorNotReady) continue;
+        if (e == hipSuccess && __atomic_load_n(slot_ + 1, __ATOMIC_ACQUIRE) == ticket) break;
+        throw std::runtime_error(std::string("omni_attn: the mask was not built: ") + hipGetErrorString(e));
+      }
+    }
+    idle_ = true;
+    return slot_[0];
+  }
+
+ private:
+  static constexpr size_t kKeep = 16;
+  static std::mutex& mutex() {
+    static std::mutex* m = new std::mutex;
+    return *m;
+  }
+  static std::vector<int32_t*>& spare() {
+    static std::vector<int32_t*>* v = new std::vector<int32_t*>;
+    return *v;
+  }
+  int32_t* slot_ = nullptr;
+  bool idle_ = true;
+};
+
+// The block mask of a prefix rule: `source` is [B, M, 3] spans or [B, q_len] prefix lengths, int64 on
+// the GPU.  Returns (kv_num_blocks, kv_indices, block_mask_types, partial_block_mask_indices,
+// partial_block_masks, partial_block_bits); the last three None where no block is PARTIAL, the
+// last one also without `pack`.
+pybind11::tuple omni_attn_build_prefix_mask(torch::Tensor source, bool spans, int64_t H, int64_t q_len, int64_t kv_len,
+                                            int64_t QB, int64_t KB, bool pack) {
+  namespace py = pybind11;
+  if (!source.is_cuda() || source.scalar_type() != torch::kInt64 || !source.is_contiguous() ||
+      source.dim() != (spans ? 3 : 2) || source.size(1) > 0x7fffffff || (spans && source.size(2) != 3) ||
+      (!spans && source.size(1) != q_len))
+    throw std::runtime_error("the mask source must be a contiguous int64 GPU tensor: spans [B, M, 3] or prefix lengths [B, q_len]");
+  const int64_t B = source.size(0);
+  const int64_t M = spans ? source.size(1) : 0;
+  c10::DeviceGuard guard(source.device());
+  const hipStream_t stream = c10::hip::getCurrentHIPStream(source.device().index()).stream();
+  const size_t ws_bytes = omni_attn_mask_workspace_bytes(int(B), int(q_len), int(kv_len), int(QB), int(KB));
+  if (ws_bytes == 0) throw std::runtime_error("omni_attn: the block mask's sizes are not positive or too large");
+  const int64_t Tq = (q_len + QB - 1) / QB, Tk = (kv_len + KB - 1) / KB;
+  const auto i32 = source.options().dtype(torch::kInt32);
+  torch::Tensor nb = torch::empty({B, H, Tq}, i32), idx = torch::empty({B, H, Tq, Tk}, i32),
+                types = torch::empty({B, H, Tq, Tk}, i32), pidx = torch::empty({B, H, Tq, Tk}, i32),
+                workspace = torch::empty({int64_t(ws_bytes / 4)}, i32);
+  // (a span pointer of an empty [B, 0, 3] tensor may be null: any address, nothing is read through it)
+  const int64_t* src = source.numel() > 0 ? source.data_ptr<int64_t>()
+                                          : reinterpret_cast<const int64_t*>(workspace.data_ptr<int32_t>());
+  const int64_t* sp = spans ? src : nullptr;
+  const int64_t* prefix = spans ? nullptr : src;
+  int P = 0;
+  {
+    py::gil_scoped_release release;
+    HostNumber total;
+    const int ticket = total.next_ticket();
+    const int rc = omni_attn_mask_lists_gfx950(
+        sp, prefix, nb.data_ptr<int32_t>(), idx.data_ptr<int32_t>(), types.data_ptr<int32_t>(),
+        pidx.data_ptr<int32_t>(), workspace.data_ptr<int32_t>(), total.memory(), ticket, int(B), int(M), int(H),
+        int(q_len), int(kv_len), int(QB), int(KB), static_cast<void*>(stream));
+    if (rc != OMNI_ATTN_OK) throw std::runtime_error(std::string("omni_attn: ") + omni_attn_status_string(rc));
+    P = total.wait(ticket, stream);
+  }
+  if (P == 0) return py::make_tuple(nb, idx, types, py::none(), py::none(), py::none());
+  torch::Tensor tiles = torch::empty({P, QB, KB}, source.options().dtype(torch::kBool));
+  torch::Tensor bits;
+  if (pack) bits = torch::empty({P, QB, KB / 32}, i32);
+  const int rc = omni_attn_mask_tiles_gfx950(
+      sp, prefix, workspace.data_ptr<int32_t>(), static_cast<uint8_t*>(tiles.data_ptr()),
+      pack ? reinterpret_cast<uint32_t*>(bits.data_ptr<int32_t>()) : nullptr, P, int(B), int(M), int(H), int(q_len),
+      int(kv_len), int(QB), int(KB), static_cast<void*>(stream));
+  if (rc != OMNI_ATTN_OK) throw std::runtime_error(std::string("omni_attn: ") + omni_attn_status_string(rc));
+  return py::make_tuple(nb, idx, types, pidx, tiles, pack ? py::cast(bits) : py::object(py::none()));
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -326,5 +444,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("Q_BLOCK_SIZE"), py::arg("KV_BLOCK_SIZE"), py::arg("seqlen_orig"),
         py::arg("partial_block_mask_indices"), py::arg("partial_tiles"), py::arg("has_partial"), py::arg("packed"),
         py::arg("softcap") = 0.0);
+  m.def("omni_attn_build_prefix_mask", &omni_attn_build_prefix_mask,
+        "omni_attn_build_prefix_mask (block mask of spans or prefix lengths)");
   m.def("abi_version", []() { return omni_attn_abi_version(); });
 }

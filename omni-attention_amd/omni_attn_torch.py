@@ -399,6 +399,25 @@ def naive_attn_mask(seq_len: int, modalities: Tensor, device=None) -> Tensor:
     return j < R.unsqueeze(-1)
 
 
+# the largest query block the native builder takes (include/omni_attn_gfx950.h)
+_NATIVE_MASK_MAX_QB = 8192
+
+
+def _native_prefix_mask(source: Tensor, spans: bool, nheads: int, q_len: int, kv_len: int, QB: int, KB: int,
+                        pack: bool) -> Optional[OmniBlockMask]:
+    """Block mask of ``source`` ([B, M, 3] spans or [B, q_len] prefix lengths, on a GPU), built there by
+    three kernels; None for sizes outside their range (the tensor algebra below takes those)."""
+    B, Tq, Tk = source.shape[0], -(-q_len // QB), -(-kv_len // KB)
+    if min(B, nheads, q_len, kv_len) <= 0 or QB > _NATIVE_MASK_MAX_QB or B * Tq * Tk > 0x7fffffff:
+        return None
+    if source.dim() != (3 if spans else 2) or (source.shape[2] != 3 if spans else source.shape[1] != q_len):
+        return None
+    pack = pack and QB in _SUPPORTED_BLOCKS and KB in _SUPPORTED_BLOCKS
+    nb, idx, tys, pidx, pm, bits = _load_extension().omni_attn_build_prefix_mask(
+        source.to(torch.int64).contiguous(), spans, nheads, q_len, kv_len, QB, KB, pack)
+    return OmniBlockMask(nb, idx, tys, Tq * QB, Tk * KB, QB, KB, pidx, pm, bits, pm is not None)
+
+
 def create_omni_block_mask_from_prefix_lengths(
     prefix_len: Tensor, nheads: int, q_len: int, kv_len: int,
     Q_BLOCK_SIZE: int = 128, KV_BLOCK_SIZE: int = 128,
@@ -414,6 +433,10 @@ def create_omni_block_mask_from_prefix_lengths(
     QB, KB = Q_BLOCK_SIZE, KV_BLOCK_SIZE
     B = prefix_len.shape[0]
     dev = prefix_len.device
+    if prefix_len.is_cuda:
+        mask = _native_prefix_mask(prefix_len[:, :q_len], False, nheads, q_len, kv_len, QB, KB, False)
+        if mask is not None:
+            return mask
     q_pad, kv_pad = _round_up(q_len, QB), _round_up(kv_len, KB)
     Tq, Tk = q_pad // QB, kv_pad // KB
     R = torch.zeros(B, q_pad, dtype=torch.long, device=dev)
@@ -463,12 +486,21 @@ def create_omni_block_mask_from_modality_positions(
     individual labels can differ from the heuristic's where that one is conservative
     (e.g. PARTIAL for a tile that is in fact all True).
     """
+    return _modality_block_mask(modality_positions, batch, nheads, q_len, kv_len, Q_BLOCK_SIZE, KV_BLOCK_SIZE,
+                                device, False)
+
+
+def _modality_block_mask(modality_positions, batch, nheads, q_len, kv_len, QB, KB, device, pack) -> OmniBlockMask:
     assert modality_positions.shape[0] == batch, "modality_positions must be [batch, M, 3]"
     assert q_len == kv_len, "Q and KV sequence lengths must match"
     mp = modality_positions.to(device)
-    R = modality_prefix_lengths(mp, q_len)
-    return create_omni_block_mask_from_prefix_lengths(R, nheads, q_len, kv_len,
-                                                      Q_BLOCK_SIZE, KV_BLOCK_SIZE)
+    mask = _native_prefix_mask(mp, True, nheads, q_len, kv_len, QB, KB, pack) if mp.is_cuda else None
+    if mask is None:
+        R = modality_prefix_lengths(mp, q_len)
+        mask = create_omni_block_mask_from_prefix_lengths(R, nheads, q_len, kv_len, QB, KB)
+    if pack and mp.is_cuda and mask.partial_block_bits is None:
+        mask.pack_partial_masks()
+    return mask
 
 
 # ----------------------------------------------------------------------------

@@ -25,8 +25,8 @@ from typing import Optional, Union
 import torch
 from torch import Tensor
 
-from omni_attn_torch import (OmniBlockMask, create_causal_omni_block_mask,
-                             create_omni_block_mask_from_modality_positions, omni_attention)
+from omni_attn_torch import (OmniBlockMask, _modality_block_mask, create_causal_omni_block_mask,
+                             omni_attention)
 
 
 class SoftcapScoreMod:
@@ -66,18 +66,14 @@ def create_transfusion_block_mask(modality_positions: Tensor, heads: int, seq_le
                                   pack: bool = True) -> OmniBlockMask:
     """Block mask of the Transfusion rule -- text causal, a modality span bidirectional within
     itself and visible to everything after it (transfusion_attn_mask, transfusion.py:343-356) --
-    for ``modality_positions`` [batch, M, 3] rows of (type, offset, length).  Built with tensor
-    algebra on ``device`` (default: where modality_positions live); with ``pack`` the PARTIAL tiles
-    are packed to bits once, for the many launches (layers, steps) that reuse the mask."""
+    for ``modality_positions`` [batch, M, 3] rows of (type, offset, length).  Built on ``device``
+    (default: where modality_positions live); with ``pack`` the PARTIAL tiles are packed to bits
+    once, for the many launches (layers, steps) that reuse the mask."""
     device = modality_positions.device if device is None else torch.device(device)
     block = max(Q_BLOCK_SIZE, KV_BLOCK_SIZE)
     n = _round_up(seq_len, block)
-    mask = create_omni_block_mask_from_modality_positions(
-        modality_positions.long(), modality_positions.shape[0], heads, n, n, Q_BLOCK_SIZE, KV_BLOCK_SIZE,
-        device=device)
-    if pack and torch.device(device).type == "cuda":
-        mask.pack_partial_masks()
-    return mask
+    return _modality_block_mask(modality_positions.long(), modality_positions.shape[0], heads, n, n, Q_BLOCK_SIZE,
+                                KV_BLOCK_SIZE, device, pack)
 
 
 def omni_flex_attention(query: Tensor, key: Tensor, value: Tensor, block_mask: Optional[OmniBlockMask] = None,

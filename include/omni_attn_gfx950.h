@@ -144,6 +144,33 @@ int omni_attn_fwd_generic_gfx950(const void* q, const void* k, const void* v, vo
 int omni_attn_pack_partial_masks_gfx950(const uint8_t* partial_masks, uint32_t* partial_bits,
                                         int num_partial, int QB, int KB, void* stream);
 
+/* Strides of a [B, H, rows, D] operand in elements; the last dimension is contiguous. */
+typedef struct omni_attn_strides {
+  int64_t batch, head, row;
+} omni_attn_strides;
+
+/*
+ * The forward on operands that are not laid out as contiguous padded slabs: q, k and v are read at
+ * their strides (a projection's [B, rows, H, D] result as it is) and need only seqlen_orig rows; o and
+ * lse are contiguous [B, H, S_out, D] and [B, H, S_out] with seqlen_orig <= S_out <= S_pad, so a
+ * ragged length needs no padded copies.  S_pad is the length the mask was made for.  Otherwise as
+ * omni_attn_fwd_gfx950 (omni_attn_fwd_generic_gfx950 with `generic`), with the tiles as bytes or (not
+ * generic) packed, one of them or neither.  Not generic: strides are multiples of 8 elements and k
+ * and v have one row stride, else OMNI_ATTN_ERR_MISALIGNED; (S_pad + KB) rows of an operand lie within
+ * 4 GiB, else OMNI_ATTN_ERR_TOO_LARGE.
+ */
+int omni_attn_fwd_strided_gfx950(const void* q, const void* k, const void* v, omni_attn_strides q_at,
+                                 omni_attn_strides k_at, omni_attn_strides v_at, void* o, float* lse_or_null,
+                                 const int32_t* kv_num_blocks,
+                                 const int32_t* kv_indices,
+                                 const int32_t* block_mask_types,
+                                 const int32_t* partial_idx_or_null,
+                                 const uint8_t* partial_masks_or_null,
+                                 const uint32_t* partial_bits_or_null,
+                                 int B, int H, int S_pad, int S_out, int D,
+                                 int Tq, int max_blocks, int QB, int KB, int num_partial,
+                                 int seqlen_orig, int dtype, float softcap, int generic, void* stream);
+
 /*
  * Block mask of a prefix rule: row i of batch element b attends the keys below R[b, i].  R comes
  * either from `prefix` ([B, q_len] int64) or from `spans` ([B, M, 3] int64 rows of (type, offset,
@@ -229,6 +256,27 @@ int omni_attn_bwd_gfx950(const void* q, const void* k, const void* v, const void
                          int B, int H, int S_pad, int D,
                          int Tq, int max_blocks, int QB, int KB, int num_partial,
                          int seqlen_orig, int dtype, float softcap, void* stream);
+
+/*
+ * The backward on such operands: q, k, v and dout are read at their strides; o, lse, dq, dk and dv are
+ * contiguous with S_out rows per slab; the workspace is that of S_out rows
+ * (omni_attn_bwd_workspace_bytes(B, H, S_out)).  The conditions are those of
+ * omni_attn_fwd_strided_gfx950; k and v, and q and dout, need not share a row stride.
+ */
+int omni_attn_bwd_strided_gfx950(const void* q, const void* k, const void* v, const void* dout,
+                                 omni_attn_strides q_at, omni_attn_strides k_at, omni_attn_strides v_at,
+                                 omni_attn_strides dout_at, const void* o, const float* lse,
+                                 void* dq, void* dk, void* dv,
+                                 const int32_t* kv_num_blocks,
+                                 const int32_t* kv_indices,
+                                 const int32_t* block_mask_types,
+                                 const int32_t* partial_idx_or_null,
+                                 const uint8_t* partial_masks_or_null,
+                                 const uint32_t* partial_bits_or_null,
+                                 void* workspace, size_t workspace_bytes,
+                                 int B, int H, int S_pad, int S_out, int D,
+                                 int Tq, int max_blocks, int QB, int KB, int num_partial,
+                                 int seqlen_orig, int dtype, float softcap, void* stream);
 
 /*
  * omni_attn_bwd_gfx950 for callers that cannot allocate device memory for the workspace: code

@@ -49,6 +49,7 @@ struct BwdParams {
   const uint16_t* v;
   const uint16_t* o;
   const uint16_t* dout;
+  RowStrides q_at, k_at, v_at, dout_at;  // (o, dq, dk, dv are contiguous)
   const float* lse;  // [B,H,S] natural-log logsumexp written by the forward
   uint16_t* dq;
   uint16_t* dk;
@@ -65,7 +66,7 @@ struct BwdParams {
   const uint8_t* partial_masks;
   const uint32_t* partial_bits;
   int num_partial;
-  int S, Tq, Tk, max_blocks, seqlen, n_slabs;
+  int S, Tq, Tk, max_blocks, seqlen, H, n_slabs;
   int n_xcd;      // XCDs (L2 domains) of the device; workgroup ids go round-robin over them
   float sl2;      // log2(e) / sqrt(D)
   float scale;    // 1 / sqrt(D)
@@ -151,7 +152,8 @@ __device__ __forceinline__ uint32_t bwd_tr_lane(int g, int c, int upper) {
 // [ROWS][D] tile from a slab into LDS in that layout.  Rows at or beyond the end of the slab
 // read as zeros.
 template <int D, int NT, int ROWS>
-__device__ __forceinline__ void bwd_load_tile(i32x4_t rsrc, int row0, uint32_t lds_tile, int tid, int w) {
+__device__ __forceinline__ void bwd_load_tile(i32x4_t rsrc, uint32_t pitch, int row0, uint32_t lds_tile, int tid,
+                                              int w) {
   constexpr int CPR = D / 8;
   constexpr int TOTAL = ROWS * CPR;  // 16-byte chunks of the tile
   constexpr int NCH = TOTAL >= NT ? TOTAL / NT : 1;
@@ -167,11 +169,11 @@ __device__ __forceinline__ void bwd_load_tile(i32x4_t rsrc, int row0, uint32_t l
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     const int row = ld_row + i * ROW_STRIDE;
-    lane_off[i] = uint32_t(row * D + (ld_pch ^ bwd_swizzle<D>(row)) * 8) * 2u - uint32_t(i * ROW_STRIDE * D * 2);
+    lane_off[i] = uint32_t(ld_row) * pitch + uint32_t(ld_pch ^ bwd_swizzle<D>(row)) * 16u;
   }
 #pragma unroll
   for (int i = 0; i < NCH; ++i)
-    buffer_to_lds_b128(rsrc, lane_off[i % PER], uint32_t(row0 + i * ROW_STRIDE) * uint32_t(D * 2),
+    buffer_to_lds_b128(rsrc, lane_off[i % PER], uint32_t(row0 + i * ROW_STRIDE) * pitch,
                        lds_tile + uint32_t(w) * 1024u + uint32_t(i) * (NT * 16u));
 }
 
@@ -274,10 +276,10 @@ __global__ void __launch_bounds__(QB * 2, 2) bwd_dq_kernel(const BwdParams p) {
   // Rows at or beyond the sequence are never used: the resources of K and V end there (those
   // rows arrive as zeros) and the query rows beyond it are replaced by zeros below, whatever the
   // caller left in the padding.
-  const size_t slab = size_t(bh) * size_t(p.S) * D;
-  const uint32_t live_bytes = uint32_t(p.seqlen) * uint32_t(D * 2);
-  const i32x4_t rK = make_buffer_resource(p.k + slab, live_bytes);
-  const i32x4_t rV = make_buffer_resource(p.v + slab, live_bytes);
+  const size_t slab = size_t(bh) * size_t(p.S) * D;  // of the contiguous ones
+  const uint32_t k_pitch = p.k_at.row * 2u, v_pitch = p.v_at.row * 2u;  // bytes from row to row
+  const i32x4_t rK = row_resource<D>(p.k, p.k_at, bh, p.H, p.seqlen);
+  const i32x4_t rV = row_resource<D>(p.v, p.v_at, bh, p.H, p.seqlen);
   const int q_row = qb * QB + 32 * w + c;
   const int q_wave_min = qb * QB + 32 * w;
   const int qr = q_row < p.S ? q_row : p.S - 1;
@@ -305,8 +307,9 @@ __global__ void __launch_bounds__(QB * 2, 2) bwd_dq_kernel(const BwdParams p) {
   u32x4_t qf[KS], dof[KS];
   float dsum = 0.f;
   {
-    const uint16_t* qp = p.q + slab + size_t(qr) * D + 8 * g;
-    const uint16_t* dop = p.dout + slab + size_t(qr) * D + 8 * g;
+    const int ql = q_row < p.seqlen ? q_row : 0;
+    const uint16_t* qp = row_base(p.q, p.q_at, bh, p.H) + size_t(ql) * p.q_at.row + 8 * g;
+    const uint16_t* dop = row_base(p.dout, p.dout_at, bh, p.H) + size_t(ql) * p.dout_at.row + 8 * g;
     const uint16_t* op = p.o + slab + size_t(qr) * D + 8 * g;
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
@@ -398,8 +401,8 @@ __global__ void __launch_bounds__(QB * 2, 2) bwd_dq_kernel(const BwdParams p) {
   const uint32_t lds_tiles = lds_offset_of(lds16);
   auto issue_loads = [&](const BwdStepInfo& st, int set) {
     const uint32_t base = lds_tiles + uint32_t(set) * (2u * TILE * 2u);
-    bwd_load_tile<D, NT, STEP>(rK, st.row0, base, tid, w);
-    bwd_load_tile<D, NT, STEP>(rV, st.row0, base + TILE * 2u, tid, w);
+    bwd_load_tile<D, NT, STEP>(rK, k_pitch, st.row0, base, tid, w);
+    bwd_load_tile<D, NT, STEP>(rV, v_pitch, st.row0, base + TILE * 2u, tid, w);
   };
   const uint32_t row_lane = bwd_row_lane<D>(g, c);
   const uint32_t tr_lo = bwd_tr_lane<D>(g, c, 0);
@@ -672,14 +675,13 @@ __global__ void __launch_bounds__(KB * 4, D == 128 ? 2 : 4) bwd_dkdv_kernel(cons
   // Rows at or beyond the sequence are never read: the resources of Q and dO end there, so
   // those rows arrive as zeros whatever the caller left in them.
   const size_t slab = size_t(bh) * size_t(p.S) * D;
-  const uint32_t live_bytes = uint32_t(p.seqlen) * uint32_t(D * 2);
-  const i32x4_t rQ = make_buffer_resource(p.q + slab, live_bytes);
-  const i32x4_t rD = make_buffer_resource(p.dout + slab, live_bytes);
+  const uint32_t q_pitch = p.q_at.row * 2u, do_pitch = p.dout_at.row * 2u;  // bytes from row to row
+  const i32x4_t rQ = row_resource<D>(p.q, p.q_at, bh, p.H, p.seqlen);
+  const i32x4_t rD = row_resource<D>(p.dout, p.dout_at, bh, p.H, p.seqlen);
   const i32x4_t rNd = make_buffer_resource(p.ws + size_t(bh) * p.S, uint32_t(p.S) * 4u);
   const i32x4_t rL2 = make_buffer_resource(p.ws + size_t(p.n_slabs) * p.S + size_t(bh) * p.S, uint32_t(p.S) * 4u);
   const int key_wave_min = kvb * KB + 32 * kg;
   const int key = key_wave_min + c;  // this lane's key row inside the slab
-  const int kr = key < p.S ? key : p.S - 1;
   const bool key_live = key < p.seqlen;
   const bool has_partial = p.partial_idx != nullptr && (p.partial_masks != nullptr || p.partial_bits != nullptr);
   const size_t meta_slab = size_t(bh) * p.Tq;
@@ -693,11 +695,11 @@ __global__ void __launch_bounds__(KB * 4, D == 128 ? 2 : 4) bwd_dkdv_kernel(cons
   // beyond the sequence).
   u32x4_t bop[KS];
   {
-    const uint16_t* src = (grad_role ? p.v : p.k) + slab + size_t(kr) * D + 8 * g;
+    const uint16_t* src = (grad_role ? row_base(p.v, p.v_at, bh, p.H) + size_t(key_live ? key : 0) * p.v_at.row
+                                     : row_base(p.k, p.k_at, bh, p.H) + size_t(key_live ? key : 0) * p.k_at.row) + 8 * g;
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
-      const u32x4_t val = *reinterpret_cast<const u32x4_t*>(src + 16 * s);
-      bop[s] = key_live ? val : u32x4_t{0u, 0u, 0u, 0u};
+      bop[s] = key_live ? *reinterpret_cast<const u32x4_t*>(src + 16 * s) : u32x4_t{0u, 0u, 0u, 0u};
     }
   }
 
@@ -823,12 +825,12 @@ __global__ void __launch_bounds__(KB * 4, D == 128 ? 2 : 4) bwd_dkdv_kernel(cons
   // The rows of step j + 1 are loaded during iteration j: Q and the exponent offsets by the
   // weight waves, dO and -delta by the gradient waves.
   auto load_q = [&](const BwdStepInfo& st, int set) {
-    bwd_load_tile<D, RT, STEP>(rQ, st.row0, tile_at(set, 0), rtid, kg);
+    bwd_load_tile<D, RT, STEP>(rQ, q_pitch, st.row0, tile_at(set, 0), rtid, kg);
     if (rtid < STEP)
       buffer_to_lds_b32(rL2, uint32_t(rtid) * 4u, uint32_t(st.row0) * 4u, lds_l2 + uint32_t(set * STEP) * 4u);
   };
   auto load_do = [&](const BwdStepInfo& st, int set) {
-    bwd_load_tile<D, RT, STEP>(rD, st.row0, tile_at(set, 1), rtid, kg);
+    bwd_load_tile<D, RT, STEP>(rD, do_pitch, st.row0, tile_at(set, 1), rtid, kg);
     if (rtid < STEP)
       buffer_to_lds_b32(rNd, uint32_t(rtid) * 4u, uint32_t(st.row0) * 4u, lds_nd + uint32_t(set * STEP) * 4u);
   };

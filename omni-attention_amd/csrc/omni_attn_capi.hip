@@ -29,6 +29,16 @@ template <> int launch_bwd_blocks<true, 64>(const BwdParams&, int, int, hipStrea
 template <> int launch_bwd_blocks<true, 128>(const BwdParams&, int, int, hipStream_t);
 }  // namespace omni_attn
 
+namespace omni_attn {
+// The forward for shapes without an instance (omni_attn_fwd_generic.hip).
+int forward_generic(const void* q, const void* k, const void* v, const omni_attn_strides& q_at,
+                    const omni_attn_strides& k_at, const omni_attn_strides& v_at, int S_out, void* o,
+                    float* lse_or_null, const int32_t* kv_num_blocks, const int32_t* kv_indices,
+                    const int32_t* block_mask_types, const int32_t* partial_idx_or_null,
+                    const uint8_t* partial_masks_or_null, int B, int H, int S_pad, int D, int Tq, int max_blocks,
+                    int QB, int KB, int num_partial, int seqlen_orig, int dtype, float softcap, void* stream);
+}  // namespace omni_attn
+
 namespace {
 thread_local int g_last_hip_error = 0;
 }  // namespace
@@ -76,8 +86,22 @@ int query_topology(DeviceTopology* out) {
 }  // namespace
 
 namespace {
-// Both forward entry points: PARTIAL tiles as bytes (partial_masks) or packed (partial_bits).
-int forward(const void* q, const void* k, const void* v, void* o, float* lse_or_null,
+// [B, H, S, D] contiguous.
+omni_attn_strides contiguous(int H, int S, int D) {
+  return {int64_t(H) * S * D, int64_t(S) * D, D};
+}
+// Can the kernels read an operand there?  16-byte loads, and 32-bit byte offsets inside a slab.
+int check_strides(const omni_attn_strides& at, int S_pad, int KB, int D) {
+  if (at.batch < 0 || at.head < 0 || at.row < D || at.batch % 8 != 0 || at.head % 8 != 0 || at.row % 8 != 0)
+    return OMNI_ATTN_ERR_MISALIGNED;
+  if (at.row > 0x7fffffffLL || ((long long)S_pad + KB) * at.row * 2 > 0xffffffffLL) return OMNI_ATTN_ERR_TOO_LARGE;
+  return OMNI_ATTN_OK;
+}
+omni_attn::RowStrides row_strides(const omni_attn_strides& at) { return {at.batch, at.head, uint32_t(at.row)}; }
+
+// All forward entry points: PARTIAL tiles as bytes (partial_masks) or packed (partial_bits).
+int forward(const void* q, const void* k, const void* v, const omni_attn_strides& q_at,
+            const omni_attn_strides& k_at, const omni_attn_strides& v_at, int S_out, void* o, float* lse_or_null,
             const int32_t* kv_num_blocks, const int32_t* kv_indices, const int32_t* block_mask_types,
             const int32_t* partial_idx_or_null, const uint8_t* partial_masks_or_null,
             const uint32_t* partial_bits_or_null, int B, int H, int S_pad, int D, int Tq,
@@ -111,6 +135,9 @@ int forward(const void* q, const void* k, const void* v, void* o, float* lse_or_
   p.k = static_cast<const uint16_t*>(k);
   p.v = static_cast<const uint16_t*>(v);
   p.o = static_cast<uint16_t*>(o);
+  p.q_at = row_strides(q_at);
+  p.k_at = row_strides(k_at);
+  p.v_at = row_strides(v_at);
   p.lse = lse_or_null;
   p.kv_num_blocks = kv_num_blocks;
   p.kv_indices = kv_indices;
@@ -122,11 +149,12 @@ int forward(const void* q, const void* k, const void* v, void* o, float* lse_or_
   p.partial_masks = has_partial ? partial_masks_or_null : nullptr;
   p.partial_bits = has_partial ? partial_bits_or_null : nullptr;
   p.num_partial = has_partial ? num_partial : 0;
-  p.S = S_pad;
+  p.S = S_out;
   p.Tq = Tq;
   p.Tk = (S_pad + KB - 1) / KB;
   p.max_blocks = max_blocks;
   p.seqlen = seqlen_orig < S_pad ? seqlen_orig : S_pad;
+  p.H = H;
   p.n_slabs = B * H;
   DeviceTopology topo;
   if (const int e = query_topology(&topo)) {
@@ -181,8 +209,9 @@ extern "C" int omni_attn_fwd_gfx950(const void* q, const void* k, const void* v,
                                     const uint8_t* partial_masks_or_null, int B, int H, int S_pad,
                                     int D, int Tq, int max_blocks, int QB, int KB, int num_partial,
                                     int seqlen_orig, int dtype, float softcap, void* stream) {
-  return forward(q, k, v, o, lse_or_null, kv_num_blocks, kv_indices, block_mask_types, partial_idx_or_null,
-                 partial_masks_or_null, nullptr, B, H, S_pad, D, Tq, max_blocks, QB, KB, num_partial,
+  const omni_attn_strides at = contiguous(H, S_pad, D);
+  return forward(q, k, v, at, at, at, S_pad, o, lse_or_null, kv_num_blocks, kv_indices, block_mask_types,
+                 partial_idx_or_null, partial_masks_or_null, nullptr, B, H, S_pad, D, Tq, max_blocks, QB, KB, num_partial,
                  seqlen_orig, dtype, softcap, stream);
 }
 
@@ -193,9 +222,35 @@ extern "C" int omni_attn_fwd_packed_gfx950(const void* q, const void* k, const v
                                            const uint32_t* partial_bits_or_null, int B, int H, int S_pad,
                                            int D, int Tq, int max_blocks, int QB, int KB, int num_partial,
                                            int seqlen_orig, int dtype, float softcap, void* stream) {
-  return forward(q, k, v, o, lse_or_null, kv_num_blocks, kv_indices, block_mask_types, partial_idx_or_null,
-                 nullptr, partial_bits_or_null, B, H, S_pad, D, Tq, max_blocks, QB, KB, num_partial,
-                 seqlen_orig, dtype, softcap, stream);
+  const omni_attn_strides at = contiguous(H, S_pad, D);
+  return forward(q, k, v, at, at, at, S_pad, o, lse_or_null, kv_num_blocks, kv_indices, block_mask_types,
+                 partial_idx_or_null, nullptr, partial_bits_or_null, B, H, S_pad, D, Tq, max_blocks, QB, KB,
+                 num_partial, seqlen_orig, dtype, softcap, stream);
+}
+
+extern "C" int omni_attn_fwd_strided_gfx950(const void* q, const void* k, const void* v, omni_attn_strides q_at,
+                                            omni_attn_strides k_at, omni_attn_strides v_at, void* o,
+                                            float* lse_or_null, const int32_t* kv_num_blocks,
+                                            const int32_t* kv_indices, const int32_t* block_mask_types,
+                                            const int32_t* partial_idx_or_null,
+                                            const uint8_t* partial_masks_or_null,
+                                            const uint32_t* partial_bits_or_null, int B, int H, int S_pad, int S_out,
+                                            int D, int Tq, int max_blocks, int QB, int KB, int num_partial,
+                                            int seqlen_orig, int dtype, float softcap, int generic, void* stream) {
+  if (S_out <= 0 || S_out > S_pad || S_out < seqlen_orig || (partial_masks_or_null && partial_bits_or_null))
+    return OMNI_ATTN_ERR_BAD_SHAPE;
+  if (generic) {
+    if (partial_bits_or_null) return OMNI_ATTN_ERR_BAD_SHAPE;
+    return omni_attn::forward_generic(q, k, v, q_at, k_at, v_at, S_out, o, lse_or_null, kv_num_blocks, kv_indices,
+                                      block_mask_types, partial_idx_or_null, partial_masks_or_null, B, H, S_pad, D, Tq,
+                                      max_blocks, QB, KB, num_partial, seqlen_orig, dtype, softcap, stream);
+  }
+  for (const omni_attn_strides* at : {&q_at, &k_at, &v_at})
+    if (const int rc = check_strides(*at, S_pad, KB, D)) return rc;
+  if (k_at.row != v_at.row) return OMNI_ATTN_ERR_MISALIGNED;
+  return forward(q, k, v, q_at, k_at, v_at, S_out, o, lse_or_null, kv_num_blocks, kv_indices, block_mask_types,
+                 partial_idx_or_null, partial_masks_or_null, partial_bits_or_null, B, H, S_pad, D, Tq, max_blocks, QB,
+                 KB, num_partial, seqlen_orig, dtype, softcap, stream);
 }
 
 extern "C" size_t omni_attn_bwd_workspace_bytes(int B, int H, int S_pad) {
@@ -206,8 +261,11 @@ extern "C" size_t omni_attn_bwd_workspace_bytes(int B, int H, int S_pad) {
 
 namespace {
 // The backward with the workspace already chosen (caller's, or the library's static one).
+struct BwdStrides {
+  omni_attn_strides q, k, v, dout;
+};
 int backward(const void* q, const void* k, const void* v, const void* o, const void* dout,
-             const float* lse, void* dq, void* dk, void* dv, const int32_t* kv_num_blocks,
+             const BwdStrides& at, int S_out, const float* lse, void* dq, void* dk, void* dv, const int32_t* kv_num_blocks,
              const int32_t* kv_indices, const int32_t* block_mask_types,
              const int32_t* partial_idx_or_null, const uint8_t* partial_masks_or_null,
              const uint32_t* partial_bits_or_null, float* delta_workspace, int B, int H, int S_pad,
@@ -245,6 +303,10 @@ int backward(const void* q, const void* k, const void* v, const void* o, const v
   p.v = static_cast<const uint16_t*>(v);
   p.o = static_cast<const uint16_t*>(o);
   p.dout = static_cast<const uint16_t*>(dout);
+  p.q_at = row_strides(at.q);
+  p.k_at = row_strides(at.k);
+  p.v_at = row_strides(at.v);
+  p.dout_at = row_strides(at.dout);
   p.lse = lse;
   p.dq = static_cast<uint16_t*>(dq);
   p.dk = static_cast<uint16_t*>(dk);
@@ -259,11 +321,12 @@ int backward(const void* q, const void* k, const void* v, const void* o, const v
   p.partial_masks = has_partial && partial_bits_or_null == nullptr ? partial_masks_or_null : nullptr;
   p.partial_bits = has_partial ? partial_bits_or_null : nullptr;
   p.num_partial = has_partial ? num_partial : 0;
-  p.S = S_pad;
+  p.S = S_out;
   p.Tq = Tq;
   p.Tk = Tk;
   p.max_blocks = max_blocks;
   p.seqlen = seqlen_orig < S_pad ? seqlen_orig : S_pad;
+  p.H = H;
   p.n_slabs = B * H;
   DeviceTopology topo;
   if (const int e = query_topology(&topo)) {
@@ -303,10 +366,32 @@ extern "C" int omni_attn_bwd_gfx950(const void* q, const void* k, const void* v,
                                     int dtype, float softcap, void* stream) {
   if (B > 0 && H > 0 && S_pad > 0 && workspace_bytes < omni_attn_bwd_workspace_bytes(B, H, S_pad))
     return OMNI_ATTN_ERR_WORKSPACE;
-  return backward(q, k, v, o, dout, lse, dq, dk, dv, kv_num_blocks, kv_indices, block_mask_types,
-                  partial_idx_or_null, partial_masks_or_null, partial_bits_or_null,
+  const omni_attn_strides at = contiguous(H, S_pad, D);
+  return backward(q, k, v, o, dout, {at, at, at, at}, S_pad, lse, dq, dk, dv, kv_num_blocks, kv_indices,
+                  block_mask_types, partial_idx_or_null, partial_masks_or_null, partial_bits_or_null,
                   static_cast<float*>(workspace), B, H, S_pad, D, Tq, max_blocks, QB, KB, num_partial,
                   seqlen_orig, dtype, softcap, stream);
+}
+
+extern "C" int omni_attn_bwd_strided_gfx950(const void* q, const void* k, const void* v, const void* dout,
+                                            omni_attn_strides q_at, omni_attn_strides k_at, omni_attn_strides v_at,
+                                            omni_attn_strides dout_at, const void* o, const float* lse, void* dq,
+                                            void* dk, void* dv, const int32_t* kv_num_blocks,
+                                            const int32_t* kv_indices, const int32_t* block_mask_types,
+                                            const int32_t* partial_idx_or_null,
+                                            const uint8_t* partial_masks_or_null,
+                                            const uint32_t* partial_bits_or_null, void* workspace,
+                                            size_t workspace_bytes, int B, int H, int S_pad, int S_out, int D, int Tq,
+                                            int max_blocks, int QB, int KB, int num_partial, int seqlen_orig,
+                                            int dtype, float softcap, void* stream) {
+  if (S_out <= 0 || S_out > S_pad || S_out < seqlen_orig) return OMNI_ATTN_ERR_BAD_SHAPE;
+  for (const omni_attn_strides* at : {&q_at, &k_at, &v_at, &dout_at})
+    if (const int rc = check_strides(*at, S_pad, KB > QB ? KB : QB, D)) return rc;
+  if (B > 0 && H > 0 && workspace_bytes < omni_attn_bwd_workspace_bytes(B, H, S_out)) return OMNI_ATTN_ERR_WORKSPACE;
+  return backward(q, k, v, o, dout, {q_at, k_at, v_at, dout_at}, S_out, lse, dq, dk, dv, kv_num_blocks, kv_indices,
+                  block_mask_types, partial_idx_or_null, partial_masks_or_null, partial_bits_or_null,
+                  static_cast<float*>(workspace), B, H, S_pad, D, Tq, max_blocks, QB, KB, num_partial, seqlen_orig,
+                  dtype, softcap, stream);
 }
 
 // ---- the backward for callers that cannot allocate -------------------------------------------
@@ -361,9 +446,10 @@ extern "C" int omni_attn_bwd_noalloc_gfx950(const void* q, const void* k, const 
   }
   // Nothing in the array has to start at zero: the dQ kernel writes both floats of every row of
   // every slab before the dK/dV kernel, which runs after it on the same stream, reads any of them.
-  return backward(q, k, v, o, dout, lse, dq, dk, dv, kv_num_blocks, kv_indices, block_mask_types,
-                  partial_idx_or_null, partial_masks_or_null, partial_bits_or_null, delta, B, H, S_pad, D,
-                  Tq, max_blocks, QB, KB, num_partial, seqlen_orig, dtype, softcap, stream);
+  const omni_attn_strides at = contiguous(H, S_pad, D);
+  return backward(q, k, v, o, dout, {at, at, at, at}, S_pad, lse, dq, dk, dv, kv_num_blocks, kv_indices,
+                  block_mask_types, partial_idx_or_null, partial_masks_or_null, partial_bits_or_null, delta, B, H,
+                  S_pad, D, Tq, max_blocks, QB, KB, num_partial, seqlen_orig, dtype, softcap, stream);
 }
 
 extern "C" const char* omni_attn_status_string(int status) {

@@ -58,6 +58,7 @@ struct GenericParams {
   const uint16_t* q;
   const uint16_t* k;
   const uint16_t* v;
+  omni_attn_strides q_at, k_at, v_at;  // (o is contiguous, S rows per slab)
   uint16_t* o;
   float* lse;
   const int32_t* kv_num_blocks;
@@ -66,7 +67,7 @@ struct GenericParams {
   const int32_t* partial_idx;
   const uint8_t* partial_masks;
   int num_partial;
-  int S, D, Tq, Tk, max_blocks, QB, KB, seqlen;
+  int S, D, H, Tq, Tk, max_blocks, QB, KB, seqlen;
   int kb_eff;         // keys of a block that can be inside the sequence: min(KB, S)
   int adv_slot, adv_off;  // 32 kWaves positions = adv_slot blocks of kb_eff keys + adv_off keys
   int q_tiles;        // 32-row tiles per query block
@@ -189,7 +190,10 @@ __global__ void __launch_bounds__(64 * kWaves, DT <= 4 ? 2 : 1) fwd_generic_kern
   int32_t* const sPid = sKey + 64;
   float* const sStat = reinterpret_cast<float*>(lds + Traits::kTiles + Traits::kQBytes + kWaves * 384);  // [2][kWaves][32]
 
-  const size_t slab = bh * size_t(p.S) * p.D;
+  const int64_t b = int64_t(bh) / p.H, h = int64_t(bh) - b * p.H;
+  const uint16_t* const q_slab = p.q + b * p.q_at.batch + h * p.q_at.head;
+  const uint16_t* const k_slab = p.k + b * p.k_at.batch + h * p.k_at.head;
+  const uint16_t* const v_slab = p.v + b * p.v_at.batch + h * p.v_at.head;
   const size_t mrow = bh * p.Tq + qb;
   const size_t moff = mrow * p.max_blocks;
   int nb = p.kv_num_blocks[mrow];
@@ -202,7 +206,7 @@ __global__ void __launch_bounds__(64 * kWaves, DT <= 4 ? 2 : 1) fwd_generic_kern
   // Q as B operand: lane holds Q[row][16 s + 8 g .. +7]
   u32x4_t qf[Traits::kQInLds ? 1 : KS];
   {
-    const uint16_t* qrow = p.q + slab + size_t(q_live ? q_idx : 0) * p.D;
+    const uint16_t* qrow = q_slab + int64_t(q_live ? q_idx : 0) * p.q_at.row;
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
       if (Traits::kQInLds && s % kWaves != w) continue;
@@ -278,8 +282,8 @@ __global__ void __launch_bounds__(64 * kWaves, DT <= 4 ? 2 : 1) fwd_generic_kern
 
   constexpr bool kPrefetchV = DT < 8;  // (at 256 columns the registers do not hold a step's V rows as well)
   u32x4_t kf[KS], vf[KS];
-  auto load_rows = [&](const uint16_t* base, const Key& k, u32x4_t (&dst)[KS]) {
-    const uint16_t* row = base + slab + size_t(k.row) * p.D;
+  auto load_rows = [&](const uint16_t* base, int64_t pitch, const Key& k, u32x4_t (&dst)[KS]) {
+    const uint16_t* row = base + int64_t(k.row) * pitch;
 #pragma unroll
     for (int s = 0; s < KS; ++s) dst[s] = load8<SMALL>(row, 16 * s + 8 * g, p.D);
   };
@@ -297,13 +301,13 @@ __global__ void __launch_bounds__(64 * kWaves, DT <= 4 ? 2 : 1) fwd_generic_kern
   if (go) {
     load_meta();
     cur = resolve();
-    load_rows(p.k, cur, kf);
-    if (kPrefetchV) load_rows(p.v, cur, vf);
+    load_rows(k_slab, p.k_at.row, cur, kf);
+    if (kPrefetchV) load_rows(v_slab, p.v_at.row, cur, vf);
     advance();
     load_meta();
   }
   while (go) {
-    if (!kPrefetchV) load_rows(p.v, cur, vf);
+    if (!kPrefetchV) load_rows(v_slab, p.v_at.row, cur, vf);
     // what the softmax needs to know about the 32 keys, by key
     if (g == 0) {
       sKey[c] = cur.cmp;
@@ -323,8 +327,8 @@ __global__ void __launch_bounds__(64 * kWaves, DT <= 4 ? 2 : 1) fwd_generic_kern
     Key nxt = cur;
     if (go) {
       nxt = resolve();
-      load_rows(p.k, nxt, kf);
-      if (kPrefetchV) load_rows(p.v, nxt, vf);
+      load_rows(k_slab, p.k_at.row, nxt, kf);
+      if (kPrefetchV) load_rows(v_slab, p.v_at.row, nxt, vf);
       advance();
       load_meta();
     }
@@ -447,7 +451,7 @@ __global__ void __launch_bounds__(64 * kWaves, DT <= 4 ? 2 : 1) fwd_generic_kern
     }
     __syncthreads();
     if (w < G && d0 + w < DT) {
-      uint16_t* orow = p.o + slab + size_t(q_idx) * p.D;
+      uint16_t* orow = p.o + (bh * p.S + q_idx) * p.D;
 #pragma unroll
       for (int r4 = 0; r4 < 4; ++r4) {
         f32x4_t x = {0.f, 0.f, 0.f, 0.f};
@@ -512,13 +516,13 @@ int launch_tiles(const GenericParams& p, unsigned grid, hipStream_t s, std::inte
 
 }  // namespace
 
-extern "C" int omni_attn_fwd_generic_gfx950(const void* q, const void* k, const void* v, void* o,
-                                            float* lse_or_null, const int32_t* kv_num_blocks,
-                                            const int32_t* kv_indices, const int32_t* block_mask_types,
-                                            const int32_t* partial_idx_or_null,
-                                            const uint8_t* partial_masks_or_null, int B, int H, int S_pad,
-                                            int D, int Tq, int max_blocks, int QB, int KB, int num_partial,
-                                            int seqlen_orig, int dtype, float softcap, void* stream) {
+namespace omni_attn {
+int forward_generic(const void* q, const void* k, const void* v, const omni_attn_strides& q_at,
+                    const omni_attn_strides& k_at, const omni_attn_strides& v_at, int S_out, void* o,
+                    float* lse_or_null, const int32_t* kv_num_blocks, const int32_t* kv_indices,
+                    const int32_t* block_mask_types, const int32_t* partial_idx_or_null,
+                    const uint8_t* partial_masks_or_null, int B, int H, int S_pad, int D, int Tq, int max_blocks,
+                    int QB, int KB, int num_partial, int seqlen_orig, int dtype, float softcap, void* stream) {
   if (!q || !k || !v || !o || !kv_num_blocks || !kv_indices || !block_mask_types)
     return OMNI_ATTN_ERR_NULL_POINTER;
   const auto misaligned = [](const void* ptr, uintptr_t a) { return (reinterpret_cast<uintptr_t>(ptr) & (a - 1)) != 0; };
@@ -541,6 +545,9 @@ extern "C" int omni_attn_fwd_generic_gfx950(const void* q, const void* k, const 
   p.k = static_cast<const uint16_t*>(k);
   p.v = static_cast<const uint16_t*>(v);
   p.o = static_cast<uint16_t*>(o);
+  p.q_at = q_at;
+  p.k_at = k_at;
+  p.v_at = v_at;
   p.lse = lse_or_null;
   p.kv_num_blocks = kv_num_blocks;
   p.kv_indices = kv_indices;
@@ -549,8 +556,9 @@ extern "C" int omni_attn_fwd_generic_gfx950(const void* q, const void* k, const 
   p.partial_idx = has_partial ? partial_idx_or_null : nullptr;
   p.partial_masks = has_partial ? partial_masks_or_null : nullptr;
   p.num_partial = has_partial ? num_partial : 0;
-  p.S = S_pad;
+  p.S = S_out;
   p.D = D;
+  p.H = H;
   p.Tq = Tq;
   p.Tk = (S_pad + KB - 1) / KB;
   p.max_blocks = max_blocks;
@@ -579,4 +587,18 @@ extern "C" int omni_attn_fwd_generic_gfx950(const void* q, const void* k, const 
     return OMNI_ATTN_ERR_LAUNCH;
   }
   return OMNI_ATTN_OK;
+}
+}  // namespace omni_attn
+
+extern "C" int omni_attn_fwd_generic_gfx950(const void* q, const void* k, const void* v, void* o,
+                                            float* lse_or_null, const int32_t* kv_num_blocks,
+                                            const int32_t* kv_indices, const int32_t* block_mask_types,
+                                            const int32_t* partial_idx_or_null,
+                                            const uint8_t* partial_masks_or_null, int B, int H, int S_pad,
+                                            int D, int Tq, int max_blocks, int QB, int KB, int num_partial,
+                                            int seqlen_orig, int dtype, float softcap, void* stream) {
+  const omni_attn_strides at = {int64_t(H) * S_pad * D, int64_t(S_pad) * D, D};
+  return omni_attn::forward_generic(q, k, v, at, at, at, S_pad, o, lse_or_null, kv_num_blocks, kv_indices,
+                                    block_mask_types, partial_idx_or_null, partial_masks_or_null, B, H, S_pad, D, Tq,
+                                    max_blocks, QB, KB, num_partial, seqlen_orig, dtype, softcap, stream);
 }

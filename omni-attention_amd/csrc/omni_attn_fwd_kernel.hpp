@@ -56,10 +56,18 @@ enum : int { kMasked = 0, kCausal = 1, kFull = 2, kPartial = 3 };
 // OMNI_ATTN_ERR_LAUNCH (read back through omni_attn_last_hip_error()); defined beside that function.
 void record_hip_error(int hip_error);
 
+// Where the rows of a [B, H, rows, D] operand lie, in elements (multiples of 8; the last dimension is
+// contiguous): a projection's [B, rows, H, D] result is read as it is.
+struct RowStrides {
+  int64_t b, h;
+  uint32_t row;
+};
+
 struct FwdParams {
   const uint16_t* q;
   const uint16_t* k;
   const uint16_t* v;
+  RowStrides q_at, k_at, v_at;  // (o is contiguous; K and V have one row stride)
   uint16_t* o;
   float* lse;                    // may be null
   const int32_t* kv_num_blocks;  // [B,H,Tq]
@@ -75,6 +83,7 @@ struct FwdParams {
   int Tk;          // ceil(S / KB)
   int max_blocks;  // slots per query block
   int seqlen;      // min(seqlen_orig, S): rows/keys at or beyond it are padding
+  int H;
   int n_slabs;     // B*H
   int n_xcd;       // XCDs (L2 domains) of the device; workgroup ids go round-robin over them
   int slab_group;  // slabs of one XCD that are walked together (>= 1)
@@ -204,6 +213,17 @@ __device__ __forceinline__ i32x4_t make_buffer_resource(const void* base, uint32
   r[3] = 0x00020000;
   return r;
 }
+// First row of slab bh of an operand, and a buffer resource that ends with its last live row (so rows
+// at or beyond the sequence read as zeros).
+__device__ __forceinline__ const uint16_t* row_base(const uint16_t* base, const RowStrides& at, int bh, int H) {
+  const int b = bh / H;
+  return base + int64_t(b) * at.b + int64_t(bh - b * H) * at.h;
+}
+template <int D>
+__device__ __forceinline__ i32x4_t row_resource(const uint16_t* base, const RowStrides& at, int bh, int H, int live) {
+  const uint32_t bytes = live > 0 ? uint32_t(live - 1) * at.row * 2u + uint32_t(D * 2) : 0u;
+  return make_buffer_resource(row_base(base, at, bh, H), bytes);
+}
 // 16 bytes per lane from a buffer straight into LDS: the wave's 64 chunks land at
 // lds_base + 16 * lane.  The source offset is a wave-uniform part plus a per-lane part.
 // Written as inline asm so that the compiler does not order later LDS reads of *other*
@@ -331,10 +351,10 @@ __global__ void __launch_bounds__(QB * 2, 2) fwd_kernel(const FwdParams p) {
   // Rows at or beyond the sequence are never used: the resources of K and V end there (those
   // rows arrive as zeros) and the query rows beyond it are replaced by zeros, whatever the caller
   // left in the padding.
-  const size_t slab = size_t(bh) * size_t(p.S) * D;
-  const uint32_t live_bytes = uint32_t(p.seqlen) * uint32_t(D * 2);
-  const i32x4_t rK = make_buffer_resource(p.k + slab, live_bytes);
-  const i32x4_t rV = make_buffer_resource(p.v + slab, live_bytes);
+  const size_t slab = size_t(bh) * size_t(p.S) * D;  // of o
+  const uint32_t pitch = p.k_at.row * 2u;  // bytes from row to row of K, and of V
+  const i32x4_t rK = row_resource<D>(p.k, p.k_at, bh, p.H, p.seqlen);
+  const i32x4_t rV = row_resource<D>(p.v, p.v_at, bh, p.H, p.seqlen);
 
   const int q_row = qb * QB + 32 * w + c;  // this lane's query row inside the slab
   const int q_wave_min = qb * QB + 32 * w;
@@ -372,8 +392,7 @@ __global__ void __launch_bounds__(QB * 2, 2) fwd_kernel(const FwdParams p) {
   // Q as the B operand of S^T = K.Q^T: lane holds Q[q_row][16s + 8g .. +7].
   u32x4_t qf[KS];
   {
-    const int qr = q_row < p.S ? q_row : p.S - 1;
-    const uint16_t* qp = p.q + slab + size_t(qr) * D + 8 * g;
+    const uint16_t* qp = row_base(p.q, p.q_at, bh, p.H) + size_t(q_row < p.seqlen ? q_row : 0) * p.q_at.row + 8 * g;
 #pragma unroll
     for (int s = 0; s < KS; ++s)
       qf[s] = q_row < p.seqlen ? *reinterpret_cast<const u32x4_t*>(qp + 16 * s) : u32x4_t{0u, 0u, 0u, 0u};
@@ -406,14 +425,14 @@ __global__ void __launch_bounds__(QB * 2, 2) fwd_kernel(const FwdParams p) {
   static_assert(ROW_STRIDE % 8 == 0, "V swizzle must be the same for all loads of a thread");
   const int ld_row = tid / CPR;  // row of this thread's first load
   const int ld_pch = tid % CPR;
-  auto k_off = [&](int row) { return uint32_t(row * D + (ld_pch ^ k_swizzle<D>(row)) * 8) * 2u; };
+  auto k_off = [&](int row) { return uint32_t(row) * pitch + uint32_t(ld_pch ^ k_swizzle<D>(row)) * 16u; };
   auto v_off = [&](int row) {
-    return uint32_t(row * D + ((((ld_pch >> 1) ^ v_swizzle<D>(row)) << 1) | (ld_pch & 1)) * 8) * 2u;
+    return uint32_t(row) * pitch + uint32_t((((ld_pch >> 1) ^ v_swizzle<D>(row)) << 1) | (ld_pch & 1)) * 16u;
   };
   uint32_t koff[KPER];
 #pragma unroll
   for (int i = 0; i < KPER; ++i)
-    koff[i] = k_off(ld_row + i * ROW_STRIDE) - uint32_t(i * ROW_STRIDE * D * 2);
+    koff[i] = k_off(ld_row + i * ROW_STRIDE) - uint32_t(i * ROW_STRIDE) * pitch;
   const uint32_t voff = v_off(ld_row);
   const uint32_t lds_k0 = lds_offset_of(sK) + uint32_t(w) * 1024u;
   const uint32_t lds_v0 = lds_offset_of(sV) + uint32_t(w) * 1024u;
@@ -423,7 +442,7 @@ __global__ void __launch_bounds__(QB * 2, 2) fwd_kernel(const FwdParams p) {
     const int i = is_v ? n : n - NCH;
     const uint32_t dst = (is_v ? lds_v0 : lds_k0) + uint32_t(buf) * (TILE * 2u) + uint32_t(i) * (NT * 16u);
     const uint32_t row = uint32_t(is_v ? v_row0 : k_row0) + uint32_t(i * ROW_STRIDE);
-    buffer_to_lds_b128(is_v ? rV : rK, is_v ? voff : koff[i % KPER], row * uint32_t(D * 2), dst);
+    buffer_to_lds_b128(is_v ? rV : rK, is_v ? voff : koff[i % KPER], row * pitch, dst);
   };
 
   // PARTIAL blocks, in two stages so that no load latency is exposed.  One iteration ahead

@@ -362,6 +362,230 @@ class HostNumber {
   bool idle_ = true;
 };
 
+// ---- the operator as one call -----------------------------------------------------------------
+// What the wrappers of omni_attn_torch.py do per call, in one native call: look the operands and the
+// mask over, allocate the results, launch.  Operands are read at their strides and at their own
+// length.  The functions return None for anything out of the ordinary (a mask on another device or
+// of other types, sizes that do not fit, an unsupported shape): the wrapper's general path then
+// converts, pads or raises.
+
+struct MaskArgs {
+  torch::Tensor nb, idx, types, pidx, tiles;  // pidx, tiles: undefined when there are none
+  int64_t q_len, kv_len, QB, KB;
+  bool packed;
+};
+
+int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
+
+bool has_instance(int64_t D, int64_t QB, int64_t KB) {
+  return (D == 32 || D == 64 || D == 128) && (QB == 64 || QB == 128) && (KB == 64 || KB == 128);
+}
+
+bool plain_meta(const torch::Tensor& t, const torch::Tensor& q) {
+  return t.scalar_type() == torch::kInt32 && t.device() == q.device() && t.is_contiguous();
+}
+
+// Operands and mask as the kernels take them?
+bool ordinary(const torch::Tensor& q, const torch::Tensor& k, const torch::Tensor& v, const MaskArgs& m, bool generic) {
+  if (!q.is_cuda() || q.dim() != 4 || (q.scalar_type() != torch::kHalf && q.scalar_type() != torch::kBFloat16)) return false;
+  if (k.scalar_type() != q.scalar_type() || v.scalar_type() != q.scalar_type() || k.device() != q.device() ||
+      v.device() != q.device() || k.sizes() != q.sizes() || v.sizes() != q.sizes() || q.numel() == 0)
+    return false;
+  const int64_t B = q.size(0), H = q.size(1), S = q.size(2), D = q.size(3);
+  if (m.QB <= 0 || m.KB <= 0 || S > 0x3fffffff || round_up(S, m.QB) != m.q_len || round_up(S, m.KB) != m.kv_len ||
+      m.kv_len > m.q_len)
+    return false;
+  if (!has_instance(D, m.QB, m.KB) && !(generic && D <= 256 && !m.packed && m.QB < 0x3fffffff && m.KB < 0x3fffffff))
+    return false;
+  const int64_t Tq = m.q_len / m.QB;
+  if (!plain_meta(m.nb, q) || !plain_meta(m.idx, q) || !plain_meta(m.types, q) || m.nb.dim() != 3 ||
+      m.nb.size(0) != B || m.nb.size(1) != H || m.nb.size(2) != Tq || m.idx.dim() != 4 || m.idx.size(0) != B ||
+      m.idx.size(1) != H || m.idx.size(2) != Tq || m.types.sizes() != m.idx.sizes())
+    return false;
+  if (m.tiles.defined()) {
+    if (!plain_meta(m.pidx, q) || m.pidx.sizes() != m.idx.sizes() || m.tiles.dim() != 3 ||
+        m.tiles.scalar_type() != (m.packed ? torch::kInt32 : torch::kBool) || m.tiles.device() != q.device() ||
+        !m.tiles.is_contiguous() || m.tiles.size(1) != m.QB || m.tiles.size(2) != (m.packed ? m.KB / 32 : m.KB))
+      return false;
+  }
+  return true;
+}
+
+omni_attn_strides strides_of(const torch::Tensor& t) { return {t.stride(0), t.stride(1), t.stride(2)}; }
+
+// Rows the matrix-core kernels can read in place (16-byte loads, 32-bit byte offsets in a slab)?
+bool readable(const torch::Tensor& t, int64_t rows) {
+  return t.stride(3) == 1 && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 && t.stride(2) % 8 == 0 &&
+         t.stride(2) >= t.size(3) && rows * t.stride(2) * 2 <= 0xffffffffLL &&
+         (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
+}
+torch::Tensor in_rows(const torch::Tensor& t, int64_t rows, bool generic) {
+  if (generic ? t.stride(3) == 1 : readable(t, rows)) return t;
+  // (clone: contiguous() would return a contiguous but misaligned tensor as it is)
+  return t.clone(at::MemoryFormat::Contiguous);
+}
+
+[[noreturn]] void fail(int rc) {
+  std::string msg = std::string("omni_attn: ") + omni_attn_status_string(rc);
+  if (rc == OMNI_ATTN_ERR_LAUNCH) msg += " (hipError " + std::to_string(omni_attn_last_hip_error()) + ")";
+  throw std::runtime_error(msg);
+}
+
+struct Tiles {
+  const int32_t* pidx = nullptr;
+  const uint8_t* bytes = nullptr;
+  const uint32_t* bits = nullptr;
+  int n = 0;
+  explicit Tiles(const MaskArgs& m) {
+    if (!m.tiles.defined() || m.tiles.size(0) == 0) return;
+    pidx = m.pidx.data_ptr<int32_t>();
+    n = int(m.tiles.size(0));
+    if (m.packed) {
+      bits = reinterpret_cast<const uint32_t*>(m.tiles.data_ptr<int32_t>());
+    } else {
+      bytes = static_cast<const uint8_t*>(m.tiles.data_ptr());
+    }
+  }
+};
+
+int dtype_of(const torch::Tensor& q) {
+  return q.scalar_type() == torch::kBFloat16 ? OMNI_ATTN_DTYPE_BF16 : OMNI_ATTN_DTYPE_F16;
+}
+void* stream_of(const torch::Tensor& q) {
+  return static_cast<void*>(c10::hip::getCurrentHIPStream(q.device().index()).stream());
+}
+
+// q, k and v become the tensors the kernel has read (copies where it could not read them in place).
+torch::Tensor launch_forward(torch::Tensor& q, torch::Tensor& k, torch::Tensor& v, const MaskArgs& m, double softcap,
+                             torch::Tensor* lse) {
+  const int64_t B = q.size(0), H = q.size(1), S = q.size(2), D = q.size(3);
+  const bool generic = !has_instance(D, m.QB, m.KB);
+  q = in_rows(q, m.q_len + m.KB, generic);
+  k = in_rows(k, m.q_len + m.KB, generic);
+  v = in_rows(v, m.q_len + m.KB, generic);
+  if (!generic && k.stride(2) != v.stride(2)) {  // one row stride for both
+    k = k.contiguous();
+    v = v.contiguous();
+  }
+  torch::Tensor out = torch::empty({B, H, S, D}, q.options());
+  if (lse) *lse = torch::empty({B, H, S}, q.options().dtype(torch::kFloat32));
+  const Tiles t(m);
+  const int rc = omni_attn_fwd_strided_gfx950(
+      q.data_ptr(), k.data_ptr(), v.data_ptr(), strides_of(q), strides_of(k), strides_of(v), out.data_ptr(),
+      lse ? lse->data_ptr<float>() : nullptr, m.nb.data_ptr<int32_t>(), m.idx.data_ptr<int32_t>(),
+      m.types.data_ptr<int32_t>(), t.pidx, t.bytes, t.bits, int(B), int(H), int(m.q_len), int(S), int(D),
+      int(m.q_len / m.QB), int(m.idx.size(3)), int(m.QB), int(m.KB), t.n, int(S), dtype_of(q), float(softcap), generic,
+      stream_of(q));
+  if (rc != OMNI_ATTN_OK) fail(rc);
+  return out;
+}
+
+MaskArgs mask_args(torch::Tensor nb, torch::Tensor idx, torch::Tensor types, int64_t q_len, int64_t kv_len, int64_t QB,
+                   int64_t KB, c10::optional<torch::Tensor> pidx, c10::optional<torch::Tensor> tiles, bool packed) {
+  MaskArgs m;
+  m.nb = std::move(nb);
+  m.idx = std::move(idx);
+  m.types = std::move(types);
+  m.q_len = q_len;
+  m.kv_len = kv_len;
+  m.QB = QB;
+  m.KB = KB;
+  m.packed = packed;
+  if (pidx && tiles) {
+    m.pidx = std::move(*pidx);
+    m.tiles = std::move(*tiles);
+  }
+  return m;
+}
+
+// The output, or (output, logsumexp) with `want_lse`.  `any_shape`: the entry point takes any block
+// size and head_dim <= 256.
+pybind11::object omni_attn_attend(torch::Tensor q, torch::Tensor k, torch::Tensor v, torch::Tensor nb,
+                                  torch::Tensor idx, torch::Tensor types, int64_t q_len, int64_t kv_len, int64_t QB,
+                                  int64_t KB, c10::optional<torch::Tensor> pidx, c10::optional<torch::Tensor> tiles,
+                                  bool packed, bool want_lse, double softcap, bool any_shape) {
+  const MaskArgs m = mask_args(std::move(nb), std::move(idx), std::move(types), q_len, kv_len, QB, KB, std::move(pidx),
+                               std::move(tiles), packed);
+  if (!ordinary(q, k, v, m, any_shape)) return pybind11::none();
+  c10::DeviceGuard guard(q.device());
+  at::NoGradGuard no_grad;
+  torch::Tensor lse;
+  torch::Tensor out = launch_forward(q, k, v, m, softcap, want_lse ? &lse : nullptr);
+  if (want_lse) return pybind11::make_tuple(std::move(out), std::move(lse));
+  return pybind11::cast(std::move(out));
+}
+
+// Forward and backward kernels as one differentiable operator.
+class AttendFunction : public torch::autograd::Function<AttendFunction> {
+ public:
+  static torch::Tensor forward(torch::autograd::AutogradContext* ctx, torch::Tensor q, torch::Tensor k,
+                               torch::Tensor v, const MaskArgs& m, double softcap) {
+    torch::Tensor lse;
+    torch::Tensor out = launch_forward(q, k, v, m, softcap, &lse);
+    ctx->save_for_backward({q, k, v, out, lse});
+    std::vector<torch::Tensor> meta = {m.nb, m.idx, m.types};
+    if (m.tiles.defined()) {
+      meta.push_back(m.pidx);
+      meta.push_back(m.tiles);
+    }
+    ctx->saved_data["mask"] = std::move(meta);
+    ctx->saved_data["sizes"] = std::vector<int64_t>{m.q_len, m.kv_len, m.QB, m.KB, int64_t(m.packed)};
+    ctx->saved_data["softcap"] = softcap;
+    return out;
+  }
+
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                 torch::autograd::variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const torch::Tensor &q = saved[0], &k = saved[1], &v = saved[2], &out = saved[3], &lse = saved[4];
+    const std::vector<torch::Tensor> meta = ctx->saved_data["mask"].toTensorVector();
+    const std::vector<int64_t> sizes = ctx->saved_data["sizes"].toIntVector();
+    MaskArgs m;
+    m.nb = meta[0];
+    m.idx = meta[1];
+    m.types = meta[2];
+    if (meta.size() > 3) {
+      m.pidx = meta[3];
+      m.tiles = meta[4];
+    }
+    m.q_len = sizes[0];
+    m.kv_len = sizes[1];
+    m.QB = sizes[2];
+    m.KB = sizes[3];
+    m.packed = sizes[4] != 0;
+    const int64_t B = q.size(0), H = q.size(1), S = q.size(2), D = q.size(3);
+    c10::DeviceGuard guard(q.device());
+    torch::Tensor dout = grads[0];
+    if (dout.scalar_type() != q.scalar_type()) dout = dout.to(q.scalar_type());
+    dout = in_rows(dout, m.q_len + std::max(m.QB, m.KB), false);
+    torch::Tensor dq = torch::empty({B, H, S, D}, q.options()), dk = torch::empty({B, H, S, D}, q.options()),
+                  dv = torch::empty({B, H, S, D}, q.options());
+    const size_t ws_bytes = omni_attn_bwd_workspace_bytes(int(B), int(H), int(S));
+    torch::Tensor workspace = torch::empty({int64_t(ws_bytes / 4)}, lse.options());
+    const Tiles t(m);
+    const int rc = omni_attn_bwd_strided_gfx950(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(), strides_of(q), strides_of(k), strides_of(v),
+        strides_of(dout), out.data_ptr(), lse.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+        m.nb.data_ptr<int32_t>(), m.idx.data_ptr<int32_t>(), m.types.data_ptr<int32_t>(), t.pidx, t.bytes, t.bits,
+        workspace.data_ptr<float>(), ws_bytes, int(B), int(H), int(m.q_len), int(S), int(D), int(m.q_len / m.QB),
+        int(m.idx.size(3)), int(m.QB), int(m.KB), t.n, int(S), dtype_of(q),
+        float(ctx->saved_data["softcap"].toDouble()), stream_of(q));
+    if (rc != OMNI_ATTN_OK) fail(rc);
+    return {dq, dk, dv, torch::Tensor(), torch::Tensor()};
+  }
+};
+
+pybind11::object omni_attn_attend_autograd(torch::Tensor q, torch::Tensor k, torch::Tensor v, torch::Tensor nb,
+                                           torch::Tensor idx, torch::Tensor types, int64_t q_len, int64_t kv_len,
+                                           int64_t QB, int64_t KB, c10::optional<torch::Tensor> pidx,
+                                           c10::optional<torch::Tensor> tiles, bool packed, double softcap) {
+  const MaskArgs m = mask_args(std::move(nb), std::move(idx), std::move(types), q_len, kv_len, QB, KB, std::move(pidx),
+                               std::move(tiles), packed);
+  if (!ordinary(q, k, v, m, false)) return pybind11::none();
+  c10::DeviceGuard guard(q.device());
+  return pybind11::cast(AttendFunction::apply(q, k, v, m, softcap));
+}
+
 // The block mask of a prefix rule: `source` is [B, M, 3] spans or [B, q_len] prefix lengths, int64 on
 // the GPU.  Returns (kv_num_blocks, kv_indices, block_mask_types, partial_block_mask_indices,
 // partial_block_masks, partial_block_bits); the last three None where no block is PARTIAL, the
@@ -444,6 +668,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("Q_BLOCK_SIZE"), py::arg("KV_BLOCK_SIZE"), py::arg("seqlen_orig"),
         py::arg("partial_block_mask_indices"), py::arg("partial_tiles"), py::arg("has_partial"), py::arg("packed"),
         py::arg("softcap") = 0.0);
+  m.def("omni_attn_attend", &omni_attn_attend, "omni_attn_attend (the operator as one call)");
+  m.def("omni_attn_attend_autograd", &omni_attn_attend_autograd, "omni_attn_attend_autograd (differentiable)");
   m.def("omni_attn_build_prefix_mask", &omni_attn_build_prefix_mask,
         "omni_attn_build_prefix_mask (block mask of spans or prefix lengths)");
   m.def("abi_version", []() { return omni_attn_abi_version(); });

@@ -21,11 +21,13 @@ EXPORTED_SYMBOLS = (
     "omni_attn_fwd_gfx950",
     "omni_attn_fwd_packed_gfx950",
     "omni_attn_fwd_generic_gfx950",
+    "omni_attn_fwd_strided_gfx950",
     "omni_attn_pack_partial_masks_gfx950",
     "omni_attn_mask_workspace_bytes",
     "omni_attn_mask_lists_gfx950",
     "omni_attn_mask_tiles_gfx950",
     "omni_attn_bwd_gfx950",
+    "omni_attn_bwd_strided_gfx950",
     "omni_attn_bwd_workspace_bytes",
     "omni_attn_bwd_noalloc_gfx950",
     "omni_attn_bwd_noalloc_max_rows",

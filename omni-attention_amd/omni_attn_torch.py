@@ -535,6 +535,9 @@ def naive_attention(query: Tensor, key: Tensor, value: Tensor,
 def _load_extension():
     """``from omni_attn import ...`` with the directory of this file on the path, the
     place build.py puts the module (the reference looks there too, :548-552)."""
+    module = sys.modules.get("omni_attn")
+    if module is not None:
+        return module
     try:
         return importlib.import_module("omni_attn")
     except ImportError:
@@ -564,10 +567,28 @@ _SUPPORTED_HEAD_DIMS = (32, 64, 128)
 _SUPPORTED_BLOCKS = (64, 128)
 
 
+def _native_mask(block_mask: OmniBlockMask, partial_needs_partial_types: bool):
+    """The mask as the arguments of the native calls."""
+    m = block_mask
+    pidx, tiles, packed = m.partial_block_mask_indices, m.partial_block_masks, False
+    if pidx is None or tiles is None or (partial_needs_partial_types and not m.has_partial_slots()):
+        pidx = tiles = None
+    elif m.partial_block_bits is not None and m.partial_block_bits.device == pidx.device:
+        tiles, packed = m.partial_block_bits, True
+    return (m.kv_num_blocks, m.kv_indices, m.block_mask_types, m.q_len, m.kv_len, m.Q_BLOCK_SIZE, m.KV_BLOCK_SIZE,
+            pidx, tiles, packed)
+
+
 def _omni_attention(op_name: str, query: Tensor, key: Tensor, value: Tensor,
                     block_mask: OmniBlockMask, partial_needs_partial_types: bool,
                     return_lse: bool = False, keep_padded: bool = False, softcap: float = 0.0):
     ext = _load_extension()
+    if query.is_cuda and not keep_padded:
+        # operands and mask of the usual types and sizes: one native call, no padded copies
+        out = ext.omni_attn_attend(query, key, value, *_native_mask(block_mask, partial_needs_partial_types),
+                                   return_lse, float(softcap), op_name == "omni_attn_simple_kernel")
+        if out is not None:
+            return out
     B, H, Q, D = query.shape
     KV = key.shape[2]
     assert key.shape == (B, H, KV, D), f"Key shape mismatch: {key.shape} vs expected {(B, H, KV, D)}"
@@ -758,6 +779,11 @@ def omni_attention(query: Tensor, key: Tensor, value: Tensor, block_mask: OmniBl
     behind ``.backward()`` (gradients with respect to query, key and value).  ``softcap`` > 0
     replaces the scaled score x by softcap * tanh(x / softcap) before mask and softmax
     (transfusion_pytorch/transfusion.py:358-364)."""
+    if query.is_cuda:
+        out = _load_extension().omni_attn_attend_autograd(query, key, value, *_native_mask(block_mask, False),
+                                                          float(softcap))
+        if out is not None:
+            return out
     return _OmniAttentionFunction.apply(query, key, value, block_mask, float(softcap))
 
 

@@ -124,3 +124,47 @@ def test_mask_builders_run_on_the_gpu_and_agree_with_the_cpu(gpu_device):
     o = oat.omni_attention_shared_kv(q, k, v, small)
     ref = torch.nan_to_num(oat.naive_attention(q.float(), k.float(), v.float(), small), nan=0.0)
     assert (o.float() - ref).abs().max().item() <= 2e-3
+
+
+@pytest.mark.parametrize("S,QB,KB,D", [(1, 64, 64, 32), (127, 128, 64, 64), (129, 128, 128, 128), (500, 64, 64, 128)])
+@pytest.mark.parametrize("layout", ["bhsd", "bshd", "odd offset", "other pitch"])
+def test_operands_are_read_where_they_lie(S, QB, KB, D, layout, gpu_device):
+    """Ragged lengths and strided operands against contiguous ones padded by hand (which the C ABI
+    takes): the same kernels on the same values, so the results are equal bit for bit.  The rows
+    behind the operands' own are NaN: none may be read."""
+    gen = torch.Generator().manual_seed(S + D)
+    B, H = 2, 3
+    spans = torch.tensor([[[1, S // 3, max(1, S // 4)]], [[1, S // 2, S // 3]]])
+    n = -(-S // QB) * QB
+    mask = create_omni_block_mask_from_modality_positions(spans, B, H, n, n, QB, KB, device=gpu_device)
+    raw = [torch.randn(B, S, H, D, generator=gen).to(torch.bfloat16).to(gpu_device) for _ in range(4)]
+
+    def place(x, i):
+        if layout == "bhsd":
+            return x.transpose(1, 2).contiguous()
+        if layout == "bshd":
+            big = torch.full((B, S + 2, H, D), float("nan"), dtype=x.dtype, device=x.device)
+            big[:, :S] = x
+            return big[:, :S].transpose(1, 2)
+        pad = 3 if layout == "odd offset" else 8 * (i + 1)  # rows at any alignment; K and V of unlike pitch
+        big = torch.full((B, H, S, D + pad), float("nan"), dtype=x.dtype, device=x.device)
+        big[..., pad:] = x.transpose(1, 2)
+        return big[..., pad:]
+
+    q, k, v, dout = (place(x, i) for i, x in enumerate(raw))
+    pads = [torch.nn.functional.pad(x.transpose(1, 2), (0, 0, 0, n - S)).contiguous() for x in raw]
+    import omni_attn_capi
+    meta = (mask.kv_num_blocks, mask.kv_indices, mask.block_mask_types, QB, KB, S, mask.partial_block_mask_indices,
+            mask.partial_block_masks)
+    ro, dq, dk, dv = (torch.empty_like(pads[0]) for _ in range(4))
+    rl = torch.empty(B, H, n, dtype=torch.float32, device=gpu_device)
+    omni_attn_capi.fwd(*pads[:3], ro, rl, *meta)
+    omni_attn_capi.bwd(*pads[:3], ro, pads[3], rl, dq, dk, dv, *meta)
+    o, lse = omni_attention_forward(q, k, v, mask)
+    assert torch.equal(o, ro[:, :, :S]) and torch.equal(lse, rl[:, :, :S])
+    q, k, v = (t.requires_grad_(True) for t in (q, k, v))
+    out = oat.omni_attention(q, k, v, mask)
+    grads = torch.autograd.grad(out, (q, k, v), dout)
+    assert torch.equal(out, ro[:, :, :S])
+    for name, a, b in zip(("dq", "dk", "dv"), grads, (dq, dk, dv)):
+        assert torch.equal(a, b[:, :, :S]), name

@@ -86,6 +86,18 @@ int query_topology(DeviceTopology* out) {
 }  // namespace
 
 namespace {
+// Slabs are dealt to the XCDs round-robin.  Where their number leaves some XCDs with more than 6 % less
+// than others (4 slabs on 8 XCDs: half the device idle), each is dealt in parts of its tiles instead.
+int slab_parts(int n_slabs, int n_xcd) {
+  int parts = 1;
+  while (parts < n_xcd) {
+    const long long n = (long long)n_slabs * parts, most = (n + n_xcd - 1) / n_xcd;
+    if (most * n_xcd * 100 <= n * 106) break;
+    parts *= 2;
+  }
+  return parts;
+}
+
 // [B, H, S, D] contiguous.
 omni_attn_strides contiguous(int H, int S, int D) {
   return {int64_t(H) * S * D, int64_t(S) * D, D};
@@ -155,6 +167,10 @@ int forward(const void* q, const void* k, const void* v, const omni_attn_strides
   p.max_blocks = max_blocks;
   p.seqlen = seqlen_orig < S_pad ? seqlen_orig : S_pad;
   p.H = H;
+  p.QB = QB;
+  p.KB = KB;
+  p.split = fwd_choose_split(D, QB, (long long)B * H * Tq * (QB / 32), Tq * QB);
+  p.tiles = Tq * (QB / fwd_split_rows(p.split, QB));
   p.n_slabs = B * H;
   DeviceTopology topo;
   if (const int e = query_topology(&topo)) {
@@ -173,7 +189,9 @@ int forward(const void* q, const void* k, const void* v, const omni_attn_strides
   // than have their K and V in the XCD's L2 (4 MiB on MI355X) together, when at least two
   // do: a bigger group was 2 % faster still on 4096-token slabs and doubled the L2 misses.
   const int slots_per_xcd = topo.cus_per_xcd * (QB == 128 ? 2 : 4);
-  const int fill = slots_per_xcd / Tq > 1 ? slots_per_xcd / Tq : 1;
+  p.parts = slab_parts(p.n_slabs, X);
+  const int part_tiles = (p.tiles + p.parts - 1) / p.parts;
+  const int fill = slots_per_xcd / part_tiles > 1 ? slots_per_xcd / part_tiles : 1;
   int heads = (H % X == 0) ? H / X : 1;
   const long long slab_kv_bytes = 4LL * S_pad * D;  // K and V, 16-bit
   const long long fit = topo.l2_bytes / slab_kv_bytes;

@@ -63,6 +63,36 @@ struct RowStrides {
   uint32_t row;
 };
 
+// How the walk of a query block is split over waves (FwdShape below says what the numbers are).
+enum class FwdSplit : int {
+  kNone,       // one workgroup per query block
+  kRows32x4,   // 32-row tiles, four groups of one wave
+  kRows64x2,   // 64-row tiles, two groups of two waves
+  kRows64x4,   // 64-row tiles, four groups of two waves (head_dim 128)
+  kRows128x2,  // 128-row tiles, two groups of four waves (head_dim 128)
+};
+constexpr int fwd_split_rows(FwdSplit s, int QB) {
+  return s == FwdSplit::kNone ? QB : (s == FwdSplit::kRows32x4 ? 32 : (s == FwdSplit::kRows128x2 ? 128 : 64));
+}
+
+// Which split?  `rows32`: 32-row tiles of the whole launch, S: rows per slab.  A wave walks a list of up
+// to S / 64 steps of 1.2 us (alone on its SIMD, head_dim 128) to 1.7 us (two per SIMD); the device
+// holds 2048 such waves.  With fewer tiles than that the longest list is the time of the launch, and
+// sharing its steps shortens it; with more, the split costs K/V loads per row (a tile of 32 rows
+// loads four times what one of 128 rows does, against 64 bytes per cycle and compute unit) and the
+// merge, and whole blocks are faster.  The lines lie where the measured times cross (causal and
+// unaligned-span masks, B H = 4 .. 128, S = 256 .. 8192).  Causal, us, whole blocks -> chosen:
+//   D=128  B H=8  S=256 10.0 -> 8.4, S=1024 22.0 -> 13.5, S=2048 38.9 -> 25.6, S=4096 71.8 -> 58.8
+//   D=64   B H=8  S=512 11.7 -> 8.2, S=2048 30.6 -> 17.5, S=4096 56.9 -> 38.0, S=8192 115 -> 99
+inline FwdSplit fwd_choose_split(int D, int QB, long long rows32, int S) {
+  if (rows32 <= (D == 128 ? 256 : 512)) return FwdSplit::kRows32x4;
+  const bool some = (rows32 <= 1024 && S >= 512) || (rows32 <= 2048 && S >= 2048);
+  if (D != 128) return some ? FwdSplit::kRows64x2 : FwdSplit::kNone;
+  if (rows32 <= 768 && S >= 512) return FwdSplit::kRows64x4;
+  if (QB != 128) return some ? FwdSplit::kRows64x2 : FwdSplit::kNone;
+  return (rows32 <= 2048 && S >= 2 * rows32) ? FwdSplit::kRows128x2 : FwdSplit::kNone;
+}
+
 struct FwdParams {
   const uint16_t* q;
   const uint16_t* k;
@@ -84,6 +114,10 @@ struct FwdParams {
   int max_blocks;  // slots per query block
   int seqlen;      // min(seqlen_orig, S): rows/keys at or beyond it are padding
   int H;
+  FwdSplit split;  // how the walks are split over waves
+  int QB, KB;      // block sizes
+  int tiles;       // workgroups per slab (query blocks, or parts of them)
+  int parts;       // parts a slab is dealt to the XCDs in
   int n_slabs;     // B*H
   int n_xcd;       // XCDs (L2 domains) of the device; workgroup ids go round-robin over them
   int slab_group;  // slabs of one XCD that are walked together (>= 1)
@@ -178,19 +212,32 @@ __device__ __forceinline__ float pair_sum(float x) {
   return lo + hi;
 }
 
-template <bool BF16, int D, int QB, int KB>
-struct FwdTraits {
-  static constexpr int kThreads = QB * 2;  // QB/32 waves of 64 lanes
-  // Keys per step.  A 64-row query block has half the waves; at D = 128 its 64-key tiles would
-  // leave LDS room for only two workgroups per CU (one wave per SIMD): it steps by 32 keys, four
-  // workgroups fit and every SIMD has two waves again.  At D <= 64 four workgroups fit with 64-key
-  // tiles, and a step has twice the matrix work per barrier.
-  static constexpr int kStep = (QB == 64 && D == 128) ? 32 : 64;
+// How a workgroup walks: QT query rows of one query block (QT / 32 waves), KG groups of such waves that
+// share the steps of the list (group i takes the steps i, i + KG, ...) and merge their results at the
+// end, STEP keys per step.  QB, KB: the block sizes, 0 where they are not known at compile time.
+template <bool BF16_, int D_, int QB_, int KB_, int QT_, int KG_, int STEP_>
+struct FwdShape {
+  static constexpr bool BF16 = BF16_;
+  static constexpr int D = D_, QB = QB_, KB = KB_, QT = QT_, KG = KG_, kStep = STEP_;
+  static constexpr int kGroupThreads = QT * 2;  // QT/32 waves of 64 lanes
+  static constexpr int kThreads = kGroupThreads * KG;
   static constexpr int kTileElems = kStep * D;
-  // K tiles, V tiles, one mask word per row and 32 keys, one mask byte per row and key in transit
-  static constexpr size_t kLdsBytes = size_t(2) * 2 * kTileElems * sizeof(uint16_t) +
-                                      size_t(QB) * (kStep / 32) * sizeof(uint32_t) + size_t(QB) * kStep;
+  static constexpr bool kLone = QT == 32;  // a group is one wave: its steps need no barriers
+  // per group: K tiles, V tiles, one mask word per row and 32 keys, one mask byte per row and key in
+  // transit
+  static constexpr size_t kTileBytes = size_t(2) * 2 * kTileElems * sizeof(uint16_t);
+  static constexpr size_t kGroupBytes = kTileBytes +
+                                        size_t(QT) * (kStep / 32) * sizeof(uint32_t) + size_t(QT) * kStep;
+  static constexpr size_t kLdsBytes = kGroupBytes * KG;
 };
+
+// One workgroup per query block, all steps in one group.
+// Keys per step.  A 64-row query block has half the waves; at D = 128 its 64-key tiles would
+// leave LDS room for only two workgroups per CU (one wave per SIMD): it steps by 32 keys, four
+// workgroups fit and every SIMD has two waves again.  At D <= 64 four workgroups fit with 64-key
+// tiles, and a step has twice the matrix work per barrier.
+template <bool BF16, int D, int QB, int KB>
+using FwdBlockShape = FwdShape<BF16, D, QB, KB, QB, 1, (QB == 64 && D == 128) ? 32 : 64>;
 
 // One step of the walk: kStep keys starting at row0, with the effective block mode.
 struct StepInfo {
@@ -266,6 +313,12 @@ __device__ __forceinline__ void buffer_to_lds_b32(i32x4_t rsrc, uint32_t lane_of
         "s"(__builtin_amdgcn_readfirstlane(uniform_off))
       : "memory", "m0");
 }
+// Waits until at most N of this wave's vector-memory operations are outstanding (they complete in order).
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  static_assert(N < 64, "six bits");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
 // Block-mask metadata is read-only for the whole launch and every read of it is
 // wave-uniform: reading it through the constant address space makes these scalar loads
 // (SGPR results, no vector-memory latency in the instruction stream).
@@ -299,25 +352,35 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
-template <bool BF16, int D, int QB, int KB>
-__global__ void __launch_bounds__(QB * 2, 2) fwd_kernel(const FwdParams p) {
-  using Traits = FwdTraits<BF16, D, QB, KB>;
-  constexpr int NT = Traits::kThreads;
-  constexpr int STEP = Traits::kStep;
-  constexpr int SPB = KB / STEP;        // steps per KV block
+template <class Shape>
+__device__ __forceinline__ void fwd_walk(const FwdParams& p) {
+  constexpr bool BF16 = Shape::BF16;
+  constexpr int D = Shape::D;
+  constexpr int QT = Shape::QT;
+  constexpr int KG = Shape::KG;
+  constexpr bool LONE = Shape::kLone;
+  constexpr int NT = Shape::kGroupThreads;
+  constexpr int STEP = Shape::kStep;
+  const int QB = Shape::QB != 0 ? Shape::QB : p.QB;
+  const int KB = Shape::KB != 0 ? Shape::KB : p.KB;
+  const int SPB = KB / STEP;            // steps per KV block (a power of two)
   constexpr int NTL = STEP / 32;        // 32-key accumulator tiles of S^T per step
   constexpr int CPR = D / 8;            // 16-byte chunks per row
   constexpr int NCH = STEP * CPR / NT;  // 16-byte chunks per thread per tile
   constexpr int KS = D / 16;            // MFMA k-steps of Q.K
   constexpr int DT = D / 32;            // 32-row tiles of O^T
-  constexpr int TILE = Traits::kTileElems;
+  constexpr int TILE = Shape::kTileElems;
+  constexpr int WQ = QT / 32;           // waves of a group
   static_assert(STEP * CPR % NT == 0, "tile must divide over the workgroup");
 
+  const int w_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kg = KG == 1 ? 0 : w_all / WQ;  // group of the wave (wave-uniform)
+  const int w = KG == 1 ? w_all : w_all % WQ;  // wave of the group
   extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
-  uint16_t* sK = reinterpret_cast<uint16_t*>(lds_raw);           // [2][TILE]
+  uint16_t* sK = reinterpret_cast<uint16_t*>(lds_raw + size_t(kg) * Shape::kGroupBytes);  // [2][TILE]
   uint16_t* sV = sK + 2 * TILE;                                  // [2][TILE]
-  uint32_t* sBits = reinterpret_cast<uint32_t*>(sV + 2 * TILE);  // [QB][NTL]
-  uint8_t* sMaskBytes = reinterpret_cast<uint8_t*>(sBits + QB * NTL);  // [QB][STEP]
+  uint32_t* sBits = reinterpret_cast<uint32_t*>(sV + 2 * TILE);  // [QT][NTL]
+  uint8_t* sMaskBytes = reinterpret_cast<uint8_t*>(sBits + QT * NTL);  // [QT][STEP]
 
   // Workgroup -> (slab, query block).  Consecutive workgroup ids go round-robin over
   // the XCDs.  XCD x takes the slabs bh with bh % n_xcd == x (every batch element's heads
@@ -328,23 +391,30 @@ __global__ void __launch_bounds__(QB * 2, 2) fwd_kernel(const FwdParams p) {
   // each K/V tile is fetched from HBM once and served from the XCD's L2 to the other
   // query blocks.  Inside a group the order is longest-first: query block Tq-1 of each
   // slab of the group, then Tq-2, ...
+  // Where there are too few slabs to go round, a slab is dealt in p.parts parts (part i has the
+  // query tiles i, i + parts, ... from the end): "slab" in the lines below is a part then.
   const int wg = blockIdx.x;
   const int slot = wg / p.n_xcd;
   const int xcd = wg - slot * p.n_xcd;
-  const int slabs_here = (p.n_slabs - xcd + p.n_xcd - 1) / p.n_xcd;
-  if (slot >= slabs_here * p.Tq) return;
-  const int per_group = p.slab_group * p.Tq;
+  const int slabs_here = (p.n_slabs * p.parts - xcd + p.n_xcd - 1) / p.n_xcd;
+  const int part_tiles = (p.tiles + p.parts - 1) / p.parts;
+  if (slot >= slabs_here * part_tiles) return;
+  const int per_group = p.slab_group * part_tiles;
   const int gi = slot / per_group;
   const int in_group = slot - gi * per_group;
   const int g_left = slabs_here - gi * p.slab_group;
   const int g_eff = g_left < p.slab_group ? g_left : p.slab_group;
   const int qrank = in_group / g_eff;
-  const int bh = xcd + p.n_xcd * (gi * p.slab_group + (in_group - qrank * g_eff));
-  const int qb = p.Tq - 1 - qrank;
+  const int dealt = xcd + p.n_xcd * (gi * p.slab_group + (in_group - qrank * g_eff));
+  const int bh = dealt / p.parts;
+  const int qt = p.tiles - 1 - (qrank * p.parts + dealt - bh * p.parts);  // query tile
+  const int q0 = qt * QT;  // first row of this workgroup
+  if (qt < 0 || (KG > 1 && q0 >= p.S)) return;
+  const int qb = KG == 1 ? qt : q0 / QB;
+  const int rb0 = KG == 1 ? 0 : q0 - qb * QB;  // ... inside its query block
 
-  const int tid = threadIdx.x;
+  const int tid = KG == 1 ? threadIdx.x : threadIdx.x - kg * NT;  // thread of the group
   const int lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 5;
   const int c = lane & 31;
 
@@ -356,8 +426,8 @@ __global__ void __launch_bounds__(QB * 2, 2) fwd_kernel(const FwdParams p) {
   const i32x4_t rK = row_resource<D>(p.k, p.k_at, bh, p.H, p.seqlen);
   const i32x4_t rV = row_resource<D>(p.v, p.v_at, bh, p.H, p.seqlen);
 
-  const int q_row = qb * QB + 32 * w + c;  // this lane's query row inside the slab
-  const int q_wave_min = qb * QB + 32 * w;
+  const int q_row = q0 + 32 * w + c;  // this lane's query row inside the slab
+  const int q_wave_min = q0 + 32 * w;
 
   const size_t meta_row = size_t(bh) * p.Tq + qb;
   const size_t meta_off = meta_row * p.max_blocks;
@@ -387,7 +457,40 @@ __global__ void __launch_bounds__(QB * 2, 2) fwd_kernel(const FwdParams p) {
   load_chunk(0);
   int nb = load_uniform(p.kv_num_blocks + meta_row);
   nb = nb < 0 ? 0 : (nb > p.max_blocks ? p.max_blocks : nb);
-  const int nsteps = nb * SPB;
+  int all_steps = nb * SPB;
+  // Groups share the steps of the live slots only (those that allow something), so a list and the same
+  // list with MASKED slots in between give the same result bit for bit.
+  uint64_t rem = 0;  // slots of the chunk in registers that the walk has not passed
+  int block_at = 0, chunk_at = 0;
+  auto live_slots = [&](int chunk) {
+    return __builtin_amdgcn_ballot_w64((chunk * 64 + lane < nb) & (mv_mode != kMasked) & (mv_row0 < p.seqlen));
+  };
+  if constexpr (KG > 1) {
+    if (q0 >= p.seqlen) nb = 0;
+    all_steps = 0;
+    int last_row0 = 0, last_mode = kMasked;
+    for (int chunk = 0; chunk * 64 < nb; ++chunk) {
+      if (chunk > 0) load_chunk(chunk);
+      const uint64_t m = live_slots(chunk);
+      if (chunk == 0) rem = m;
+      if (m != 0) {
+        all_steps += __builtin_popcountll(m) * SPB;
+        const int last = 63 - __builtin_clzll(m);
+        last_row0 = __builtin_amdgcn_readlane(mv_row0, last);
+        last_mode = __builtin_amdgcn_readlane(mv_mode, last);
+      }
+    }
+    if (nb > 64) load_chunk(0);
+    if (all_steps > 0) {
+      // The last block of a list usually holds the diagonal or the end of the sequence: its steps
+      // behind both allow nothing.
+      int last_key = p.seqlen - 1;
+      if (last_mode == kCausal && q0 + QT - 1 < last_key) last_key = q0 + QT - 1;
+      const int useful = last_key < last_row0 ? 0 : (last_key - last_row0) / STEP + 1;
+      all_steps -= SPB - (useful < SPB ? useful : SPB);
+    }
+  }
+  const int nsteps = KG == 1 ? all_steps : (all_steps + KG - 1) / KG;  // iterations of every group
 
   // Q as the B operand of S^T = K.Q^T: lane holds Q[q_row][16s + 8g .. +7].
   u32x4_t qf[KS];
@@ -399,13 +502,31 @@ __global__ void __launch_bounds__(QB * 2, 2) fwd_kernel(const FwdParams p) {
   }
   // Step `it` (clamped to the last step of the walk; steps past the end are only ever
   // used as the address of a tile load whose data nobody reads).
-  auto step_info = [&](int it) {
-    const int itc = it < nsteps ? it : nsteps - 1;
-    const int j = itc / SPB;
-    if (itc == it && itc % SPB == 0 && (j & 63) == 0 && j > 0) load_chunk(j >> 6);
-    const int ln = j & 63;
+  auto step_info = [&](int i) {
+    const int it = KG == 1 ? i : i * KG + kg;
     StepInfo si;
-    si.row0 = __builtin_amdgcn_readlane(mv_row0, ln) + (itc % SPB) * STEP;
+    int ln;
+    if constexpr (KG == 1) {
+      const int itc = it < nsteps ? it : nsteps - 1;
+      const int j = itc / SPB;
+      if (itc == it && itc % SPB == 0 && (j & 63) == 0 && j > 0) load_chunk(j >> 6);
+      ln = j & 63;
+      si.row0 = (itc % SPB) * STEP;
+    } else {
+      if (it >= all_steps) return StepInfo{0, kMasked, -1};  // a step that this group does not have
+      for (const int block = it / SPB;;) {
+        while (rem == 0) {
+          load_chunk(++chunk_at);
+          rem = live_slots(chunk_at);
+        }
+        if (block_at == block) break;
+        rem &= rem - 1;
+        ++block_at;
+      }
+      ln = __builtin_ctzll(rem);
+      si.row0 = (it % SPB) * STEP;
+    }
+    si.row0 += __builtin_amdgcn_readlane(mv_row0, ln);
     si.mode = __builtin_amdgcn_readlane(mv_mode, ln);
     si.pid = __builtin_amdgcn_readlane(mv_pid, ln);
     return si;
@@ -420,9 +541,9 @@ __global__ void __launch_bounds__(QB * 2, 2) fwd_kernel(const FwdParams p) {
   // wave-uniform and goes through the scalar offset of the load.
   constexpr int ROWS_PER_CALL = 64 / CPR;                // rows filled by one wave-wide load
   constexpr int ROW_STRIDE = ROWS_PER_CALL * (NT / 64);  // rows between a thread's loads
-  constexpr int KPER = ROW_STRIDE % 16 == 0 ? 1 : 2;     // distinct K lane offsets
+  constexpr int KPER = ROW_STRIDE % 16 == 0 ? 1 : 16 / ROW_STRIDE;  // distinct K lane offsets
   static_assert((KPER * ROW_STRIDE) % 16 == 0, "K swizzle must repeat over a thread's loads");
-  static_assert(ROW_STRIDE % 8 == 0, "V swizzle must be the same for all loads of a thread");
+  static_assert(ROW_STRIDE % 4 == 0, "V swizzle must be the same for all loads of a thread");
   const int ld_row = tid / CPR;  // row of this thread's first load
   const int ld_pch = tid % CPR;
   auto k_off = [&](int row) { return uint32_t(row) * pitch + uint32_t(ld_pch ^ k_swizzle<D>(row)) * 16u; };
@@ -453,12 +574,12 @@ __global__ void __launch_bounds__(QB * 2, 2) fwd_kernel(const FwdParams p) {
   // so no workgroup barrier is needed.
   constexpr int MCPR = STEP / 16;  // 16-byte chunks per row of mask bytes
   auto prefetch_mask_bytes = [&](int it, const StepInfo& si) {
-    const int half = it % SPB;
-    const i32x4_t rM = make_buffer_resource(p.partial_masks + size_t(si.pid) * (QB * KB), uint32_t(QB * KB));
+    const int half = (KG == 1 ? it : it * KG + kg) % SPB;
+    const i32x4_t rM = make_buffer_resource(p.partial_masks + size_t(si.pid) * size_t(QB * KB), uint32_t(QB * KB));
     const uint32_t dst = lds_offset_of(sMaskBytes) + uint32_t(w) * uint32_t(32 * STEP);
 #pragma unroll
     for (int i = 0; i < MCPR / 2; ++i) {  // 64 / MCPR rows per load
-      const uint32_t row = uint32_t(32 * w + i * (64 / MCPR)) + uint32_t(lane / MCPR);
+      const uint32_t row = uint32_t(rb0 + 32 * w + i * (64 / MCPR)) + uint32_t(lane / MCPR);
       buffer_to_lds_b128(rM, row * uint32_t(KB) + uint32_t(lane % MCPR) * 16u, uint32_t(half * STEP),
                          dst + uint32_t(i) * 1024u);
     }
@@ -467,17 +588,17 @@ __global__ void __launch_bounds__(QB * 2, 2) fwd_kernel(const FwdParams p) {
   // stage: one 4-byte buffer->LDS load per lane puts the step's words of the wave's 32 rows
   // where the byte path parks the words it packs.
   auto prefetch_mask_words = [&](int it, const StepInfo& si) {
-    constexpr uint32_t TILE_WORDS = uint32_t(QB) * (KB / 32);
-    const int half = it % SPB;
+    const uint32_t TILE_WORDS = uint32_t(QB) * uint32_t(KB / 32);
+    const int half = (KG == 1 ? it : it * KG + kg) % SPB;
     const i32x4_t rM = make_buffer_resource(p.partial_bits + size_t(si.pid) * TILE_WORDS, TILE_WORDS * 4u);
     if (lane < 32 * NTL) {
-      const uint32_t row = uint32_t(32 * w + lane / NTL);
+      const uint32_t row = uint32_t(rb0 + 32 * w + lane / NTL);
       buffer_to_lds_b32(rM, (row * uint32_t(KB / 32) + uint32_t(lane % NTL)) * 4u, uint32_t(half * NTL) * 4u,
                         lds_offset_of(sBits) + uint32_t(32 * w * NTL) * 4u);
     }
   };
   auto stage_mask_bits = [&]() {
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the bytes have landed
+    wait_loads<0>();  // the bytes have landed
     // word NTL * row + h of the wave's 32 rows; with one word per row the upper half-wave
     // repeats the lower one
     const int wi = lane % (32 * NTL);
@@ -637,7 +758,9 @@ __global__ void __launch_bounds__(QB * 2, 2) fwd_kernel(const FwdParams p) {
     constexpr int NPV = decltype(first_c)::value != 0 ? 0 : NPV_ALL;
     constexpr int NS = NQK + NPV;  // slots
     constexpr int LSP = (NS / 2) / NL > 0 ? (NS / 2) / NL : 1;  // slots between tile loads
-    static_assert(NL * LSP <= NS, "tile loads must fit in the slots");
+    // ... and no V tile to load: V(0) is on its way already
+    constexpr int L0 = decltype(first_c)::value != 0 ? NCH : 0, NLB = NL - L0;
+    constexpr int LPS = (NLB * LSP + NS - 1) / NS;              // loads per slot that has some
     constexpr int PF = PF_ALL < NS ? PF_ALL : NS;
     constexpr int NMX = 2 * NTL;          // max chunks of 8 scores
     constexpr int NPR = 8 * NTL;          // pairs of exponentials
@@ -718,7 +841,10 @@ __global__ void __launch_bounds__(QB * 2, 2) fwd_kernel(const FwdParams p) {
         st[SET ^ 1][t] = mfma_32x32x16<BF16>(opq[j % PF], qf[s], s == 0 ? zero16 : st[SET ^ 1][t]);
       }
       if constexpr (j + PF < NS) opq[j % PF] = operand(j + PF);
-      if constexpr (j % LSP == 0 && j / LSP < NL) issue_load(j / LSP, SET, k_row0, v_row0);
+      static_for<LPS>([&](auto lc) {
+        constexpr int n = (j / LSP) * LPS + decltype(lc)::value;
+        if constexpr (j % LSP == 0 && n < NLB) issue_load(L0 + n, SET, k_row0, v_row0);
+      });
       constexpr int u_lo = j * NV / NS, u_hi = (j + 1) * NV / NS;
       static_for<u_hi - u_lo>([&](auto dc) { vector_chunk(IntC<u_lo + decltype(dc)::value>{}); });
       __builtin_amdgcn_sched_barrier(0);
@@ -726,39 +852,45 @@ __global__ void __launch_bounds__(QB * 2, 2) fwd_kernel(const FwdParams p) {
     __builtin_amdgcn_s_setprio(0);
   };
 
+  // The tiles (and packed mask words) that were requested an iteration ago have landed, for
+  // every wave that reads them.
+  auto step_barrier = [&]() {
+    wait_loads<0>();
+    if constexpr (!LONE) __syncthreads();
+  };
   // ---- the walk -------------------------------------------------------------------------
   StepInfo cur = {0, kMasked, -1}, nxt = cur, nn = cur;
   if (nsteps > 0) {
     cur = step_info(0);
     nxt = step_info(1);
     nn = step_info(2);
-    // Prologue: K(0) and K(1).
-#pragma unroll
-    for (int i = 0; i < NCH; ++i) {
-      issue_load(NCH + i, 0, cur.row0, 0);
-      issue_load(NCH + i, 1, nxt.row0, 0);
-    }
+    // Prologue: the mask of step 0, K(0), K(1), V(0); the first products wait for K(0) only.
     if (cur.mode == kPartial) {
       if (packed_tiles) {
         prefetch_mask_words(0, cur);
       } else {
         prefetch_mask_bytes(0, cur);
-        stage_mask_bits();
       }
     }
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) issue_load(NCH + i, 0, cur.row0, 0);
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) issue_load(NCH + i, 1, nxt.row0, 0);
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) issue_load(i, 0, 0, cur.row0);
+    wait_loads<2 * NCH>();
+    if constexpr (!LONE) __syncthreads();
 #pragma unroll
     for (int s = 0; s < KS; ++s)
 #pragma unroll
       for (int t = 0; t < NTL; ++t)
         st[0][t] = mfma_32x32x16<BF16>(k_frag(sK, s, t), qf[s], s == 0 ? zero16 : st[0][t]);
+    if (cur.mode == kPartial && !packed_tiles) stage_mask_bits();
   }
 
   auto iteration = [&](auto set_c, auto first_c, int it) {
     constexpr int SET = decltype(set_c)::value;
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this thread's tile loads have landed
-    __syncthreads();
+    step_barrier();
     u32x4_t opq[PF_ALL];
     body_prefetch(IntC<SET>{}, first_c, opq);
     // The common step -- every score allowed, no rescale owed, no PARTIAL tile ahead, no soft cap
@@ -801,8 +933,7 @@ __global__ void __launch_bounds__(QB * 2, 2) fwd_kernel(const FwdParams p) {
 
   // Drain: O^T += V^T . P^T of the last step.
   if (nsteps > 0) {
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
+    step_barrier();
     if (rescale_pending != 0) {
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
@@ -830,7 +961,61 @@ __global__ void __launch_bounds__(QB * 2, 2) fwd_kernel(const FwdParams p) {
   // 32 x D output through LDS -- its own 32 rows of the K buffers, which nobody reads after
   // the barrier of the drain, 16-byte chunks swizzled like a K tile -- and stores whole
   // rows: 64 lanes x 16 bytes = 64 / CPR complete rows per instruction.
-  const float l_tot = pair_sum(l_run);
+  float l_tot = pair_sum(l_run);
+  if constexpr (KG > 1) {
+    // Merge of the groups.  Row maxima and sums go where the mask words and bytes were (a wave
+    // writes and has read its own rows only), the scaled O^T into the tiles once every group is
+    // done with them; then each group adds up and stores its share of the columns.
+    constexpr int UNITS = DT * 4;           // 4-register pieces of a lane's O^T
+    constexpr int MINE = (UNITS + KG - 1) / KG;  // ... that a group stores
+    static_assert(QT * D * 4 <= Shape::kTileBytes && QT * STEP >= QT * 4, "merge layout");
+    auto group_at = [&](int i) { return lds_raw + size_t(i) * Shape::kGroupBytes; };
+    constexpr size_t kStatM = Shape::kTileBytes, kStatL = kStatM + size_t(QT) * NTL * 4;
+    const int row = 32 * w + c;
+    if (g == 0) {
+      reinterpret_cast<float*>(group_at(kg) + kStatM)[row] = m_run;
+      reinterpret_cast<float*>(group_at(kg) + kStatL)[row] = l_tot;
+    }
+    __syncthreads();
+    float m_all = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < KG; ++i) m_all = fmaxf(m_all, reinterpret_cast<const float*>(group_at(i) + kStatM)[row]);
+    const float m_fin = m_all == -INFINITY ? 0.f : m_all;
+    l_tot = 0.f;
+#pragma unroll
+    for (int i = 0; i < KG; ++i)
+      l_tot += reinterpret_cast<const float*>(group_at(i) + kStatL)[row] *
+               __builtin_amdgcn_exp2f(reinterpret_cast<const float*>(group_at(i) + kStatM)[row] - m_fin);
+    const bool live = (q_row < p.seqlen) && (l_tot > 0.f);
+    const float mine = live ? __builtin_amdgcn_exp2f(m_run - m_fin) / l_tot : 0.f;
+    typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+    auto piece_at = [&](int i, int u) {
+      return reinterpret_cast<f32x4_t*>(group_at(i)) + (w * UNITS + u) * 64 + lane;
+    };
+    static_for<UNITS>([&](auto uc) {
+      constexpr int u = decltype(uc)::value, dt = u / 4, r4 = u % 4;
+      f32x4_t x;
+      x[0] = ot[dt][4 * r4 + 0] * mine;
+      x[1] = ot[dt][4 * r4 + 1] * mine;
+      x[2] = ot[dt][4 * r4 + 2] * mine;
+      x[3] = ot[dt][4 * r4 + 3] * mine;
+      *piece_at(kg, u) = x;
+    });
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < MINE; ++n) {
+      const int u = kg * MINE + n;
+      if (UNITS % KG != 0 && u >= UNITS) break;
+      f32x4_t x = *piece_at(0, u);
+#pragma unroll
+      for (int i = 1; i < KG; ++i) x += *piece_at(i, u);
+      const u32x2_t ov = {pack2<BF16>(x[0], x[1]), pack2<BF16>(x[2], x[3])};
+      if (q_row < p.S) *reinterpret_cast<u32x2_t*>(p.o + slab + size_t(q_row) * D + 8 * u + 4 * g) = ov;
+    }
+    if (kg == 0 && g == 0 && q_row < p.S && p.lse != nullptr)
+      p.lse[size_t(bh) * p.S + q_row] = live ? (m_fin + __builtin_amdgcn_logf(l_tot)) * 0.6931471805599453f : -INFINITY;
+    return;
+  }
   const bool live = (q_row < p.seqlen) && (l_tot > 0.f);
   const float inv = live ? 1.f / l_tot : 0.f;
   {
@@ -863,32 +1048,49 @@ __global__ void __launch_bounds__(QB * 2, 2) fwd_kernel(const FwdParams p) {
   }
 }
 
+template <bool BF16, int D, int QB, int KB>
+__global__ void __launch_bounds__(QB * 2, 2) fwd_kernel(const FwdParams p) {
+  fwd_walk<FwdBlockShape<BF16, D, QB, KB>>(p);
+}
+
+// The steps of a list shared by the groups of a workgroup (fwd_choose_split says when).
+template <bool BF16, int D, int QT, int KG, int STEP>
+__global__ void __launch_bounds__(QT * 2 * KG, 2) fwd_ksplit(const FwdParams p) {
+  fwd_walk<FwdShape<BF16, D, 0, 0, QT, KG, STEP>>(p);
+}
+
 // Host-side launch of one instance; returns the hipError_t of the launch itself (the
 // thread's sticky "last error" of earlier, unrelated HIP calls is neither read nor cleared).
 // The dynamic-LDS limit of an instance is raised once per device, not on every launch.
 constexpr int kMaxDevices = 64;
-template <bool BF16, int D, int QB, int KB>
-int launch_fwd(const FwdParams& p, hipStream_t stream) {
-  using Traits = FwdTraits<BF16, D, QB, KB>;
-  auto kern = fwd_kernel<BF16, D, QB, KB>;
+template <class Shape, auto Kernel>
+int launch_fwd_shape(const FwdParams& p, hipStream_t stream) {
   static std::atomic<bool> lds_limit_set[kMaxDevices];
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return int(e);
   const bool cached = dev >= 0 && dev < kMaxDevices;
   if (!cached || !lds_limit_set[dev].load(std::memory_order_acquire)) {
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, int(Traits::kLdsBytes));
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(Kernel),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, int(Shape::kLdsBytes));
     if (e != hipSuccess) return int(e);
     if (cached) lds_limit_set[dev].store(true, std::memory_order_release);
   }
-  const unsigned slabs_per_xcd = unsigned(p.n_slabs + p.n_xcd - 1) / unsigned(p.n_xcd);
-  const dim3 grid(unsigned(p.n_xcd) * slabs_per_xcd * unsigned(p.Tq));
-  const dim3 block(Traits::kThreads);
+  const unsigned slabs_per_xcd = unsigned(p.n_slabs * p.parts + p.n_xcd - 1) / unsigned(p.n_xcd);
+  const dim3 grid(unsigned(p.n_xcd) * slabs_per_xcd * (unsigned(p.tiles + p.parts - 1) / unsigned(p.parts)));
   FwdParams params = p;
   void* args[] = {&params};
-  return int(hipLaunchKernel(reinterpret_cast<const void*>(kern), grid, block, args,
-                             Traits::kLdsBytes, stream));
+  return int(hipLaunchKernel(reinterpret_cast<const void*>(Kernel), grid, dim3(Shape::kThreads), args,
+                             Shape::kLdsBytes, stream));
+}
+
+template <bool BF16, int D, int QB, int KB>
+int launch_fwd(const FwdParams& p, hipStream_t stream) {
+  return launch_fwd_shape<FwdBlockShape<BF16, D, QB, KB>, fwd_kernel<BF16, D, QB, KB>>(p, stream);
+}
+template <bool BF16, int D, int QT, int KG, int STEP>
+int launch_fwd_ksplit(const FwdParams& p, hipStream_t stream) {
+  return launch_fwd_shape<FwdShape<BF16, D, 0, 0, QT, KG, STEP>, fwd_ksplit<BF16, D, QT, KG, STEP>>(p, stream);
 }
 
 }  // namespace omni_attn

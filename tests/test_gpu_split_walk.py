@@ -1,0 +1,46 @@
+"""The forward on problems with few rows, where the steps of a list are shared by groups of waves: one
+case per split, each at sizes where it can go wrong -- lists of more than 64 slots, of fewer steps
+than groups and of none, ragged last blocks, PARTIAL tiles as bytes and as bits, a last block whose
+steps behind the diagonal or the sequence are dropped.  Against the fp32 oracle with its bars (the
+error of a split is that of the operator: rounded weights and results)."""
+import pytest
+import torch
+
+import omni_attn_capi
+from helpers import compare_with_oracle, random_block_metadata
+from oracle.dense_oracle import attention_dense_fp32, dense_mask_from_blocks
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+@pytest.mark.parametrize("D,QB,KB,H,S", [
+    (32, 64, 128, 9, 128), (64, 128, 64, 1, 4480), (128, 128, 128, 3, 384), (128, 64, 64, 5, 192),  # 32 rows, 4 groups
+    (32, 128, 128, 40, 512), (64, 64, 64, 33, 512), (128, 64, 128, 52, 512),                         # 64 rows, 2 groups
+    (128, 128, 64, 20, 512),                                                                         # 64 rows, 4 groups
+    (128, 128, 128, 13, 2048)])                                                                      # 128 rows, 2 groups
+def test_split_walks(dtype, D, QB, KB, H, S, gpu_device):
+    gen = torch.Generator().manual_seed(D + QB + S)
+    q, k, v = (torch.randn(1, H, S, D, generator=gen).to(dtype) for _ in range(3))
+    nb, idx, tys, pidx, pm = random_block_metadata(gen, 1, H, S // QB, S // KB, QB, KB, p_empty=0.15, shuffle=True)
+    # one head causal as a builder lists it, so that the last slot of every list is the diagonal
+    for qb in range(S // QB):
+        n = ((qb + 1) * QB + KB - 1) // KB
+        nb[0, 0, qb] = n
+        idx[0, 0, qb, :n] = torch.arange(n, dtype=torch.int32)
+        tys[0, 0, qb, :n] = 1
+    dev = lambda t: t.to(gpu_device).contiguous()
+    qd, kd, vd, nbd, idxd, tysd, pidxd, pmd = (dev(t) for t in (q, k, v, nb, idx, tys, pidx, pm))
+    for seqlen in (S, S - QB - 13 if S > QB else S - 13):
+        dense = dense_mask_from_blocks(nb, idx, tys, QB, KB, S, S, pidx, pm, seqlen_orig=seqlen)
+        ro, rl = attention_dense_fp32(q, k, v, dense)
+        outs = []
+        for bits in (None, omni_attn_capi.pack_partial_masks(pmd)):
+            o = torch.full_like(qd, float("nan"))
+            lse = torch.full(qd.shape[:3], float("nan"), dtype=torch.float32, device=gpu_device)
+            omni_attn_capi.fwd(qd, kd, vd, o, lse, nbd, idxd, tysd, QB, KB, seqlen, pidxd,
+                               pmd if bits is None else None, partial_bits=bits)
+            torch.cuda.synchronize()
+            compare_with_oracle(o, lse, ro, rl, dtype, f"seqlen {seqlen}, {'bytes' if bits is None else 'bits'}")
+            outs.append((o, lse))
+        assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])

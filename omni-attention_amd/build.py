@@ -51,8 +51,9 @@ RESOURCES_JSON = os.path.join(OBJ, "kernel_resources.json")
 # least this many waves per SIMD (kernels are matched by a substring of their mangled name).
 # The backward kernels and the forward with split lists keep scalar values in spare vector lanes here
 # and there (SGPR spills, no memory behind them): for them only scratch memory and spilled vector registers fail the build.
-MIN_WAVES_PER_SIMD = {"fwd_kernel": 2, "fwd_ksplit": 2, "bwd_dq_kernel": 2, "bwd_dkdv_kernel": 2}
-SGPR_SPILLS_ALLOWED = ("bwd_dq_kernel", "bwd_dkdv_kernel", "fwd_ksplit")
+MIN_WAVES_PER_SIMD = {"fwd_kernel": 2, "fwd_ksplit": 2, "bwd_dq_kernel": 2, "bwd_dq_ksplit": 2,
+                      "bwd_dkdv_kernel": 2, "bwd_dkdv_split": 2}
+SGPR_SPILLS_ALLOWED = ("bwd_dq_", "bwd_dkdv_", "fwd_ksplit")
 NOT_GATED = ("fwd_generic_kernel",)
 
 INSTANCES = [(bf, d) for bf in (0, 1) for d in (32, 64, 128)]

@@ -43,6 +43,40 @@ namespace omni_attn {
 
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
+// How the walk of a KV block is split over waves in the dK/dV kernel.
+enum class DkdvSplit : int {
+  kNone,      // one workgroup per KV block
+  kKeys64x2,  // 64 keys, two groups of waves that share the query steps
+  kKeys32x4,  // 32 keys, four groups (head_dim <= 64)
+};
+
+// Which splits?  The reasons are the forward's (fwd_choose_split): with few rows the longest walk is the
+// time of a launch.  rows32: 32-row tiles of the launch, S: rows per slab.  The lines lie where the
+// measured times cross (causal, unaligned-span and soft-capped, B H = 4 .. 128, S = 256 .. 8192).
+// Both kernels together, causal, us, whole blocks -> chosen (128x128 blocks):
+//   D=128  B H=8  S=512 37.9 -> 29.5, S=1024 59.7 -> 41.0, S=2048 102.9 -> 71.7, S=4096 192.3 -> 154.9
+//   D=64   B H=8  S=512 29.4 -> 20.2, S=1024 46.2 -> 26.5, S=2048  79.7 -> 51.1, S=4096 146.9 -> 103.0
+inline FwdSplit bwd_choose_dq_split(int D, int QB, long long rows32, int S) {
+  if (rows32 <= (D == 128 ? 256 : 512)) return FwdSplit::kRows32x4;
+  bool two;
+  if (D == 128) {
+    two = rows32 <= 640 || (rows32 <= 1024 && S >= (QB == 128 ? 4096 : 1024));
+  } else {
+    two = (rows32 <= 1024 && S >= 512) || (rows32 <= 1536 && S >= 1024) || (rows32 <= 2048 && S >= 4096);
+  }
+  return two ? FwdSplit::kRows64x2 : FwdSplit::kNone;
+}
+inline DkdvSplit bwd_choose_dkdv_split(int D, int KB, bool capped, long long rows32, int S) {
+  if (D != 128 && rows32 <= 256) return DkdvSplit::kKeys32x4;
+  bool two = rows32 <= 512;
+  if (D == 128) {
+    two = two || (rows32 <= 1024 && S >= (KB == 128 ? 4096 : 1024));
+  } else if (!capped) {
+    two = two || (rows32 <= 1536 && S >= 2048) || (rows32 <= 2048 && S >= 4096);
+  }
+  return two ? DkdvSplit::kKeys64x2 : DkdvSplit::kNone;
+}
+
 struct BwdParams {
   const uint16_t* q;
   const uint16_t* k;
@@ -67,6 +101,10 @@ struct BwdParams {
   const uint32_t* partial_bits;
   int num_partial;
   int S, Tq, Tk, max_blocks, seqlen, H, n_slabs;
+  int QB, KB;     // block sizes
+  int parts;      // parts a slab is dealt to the XCDs in
+  FwdSplit dq_split;       // how the walks of the dQ kernel are split over waves
+  DkdvSplit dkdv_split;    // ... and of the dK/dV kernel
   int n_xcd;      // XCDs (L2 domains) of the device; workgroup ids go round-robin over them
   float sl2;      // log2(e) / sqrt(D)
   float scale;    // 1 / sqrt(D)
@@ -162,8 +200,8 @@ __device__ __forceinline__ void bwd_load_tile(i32x4_t rsrc, uint32_t pitch, int 
   if (TOTAL < NT && tid >= TOTAL) return;  // a small tile is loaded by the first waves only
   const int ld_row = tid / CPR, ld_pch = tid % CPR;
   // The swizzle repeats every 16 rows and a thread's loads are ROW_STRIDE rows apart: one or two
-  // per-lane offsets serve all of them, the rest of the address is wave-uniform.
-  constexpr int PER = (NCH == 1 || ROW_STRIDE % 16 == 0) ? 1 : 2;
+  // per-lane offsets (four where a single wave loads) serve all of them, the rest of the address is wave-uniform.
+  constexpr int PER = (NCH == 1 || ROW_STRIDE % 16 == 0) ? 1 : 16 / ROW_STRIDE;
   static_assert(NCH == 1 || (PER * ROW_STRIDE) % 16 == 0, "swizzle must repeat over a thread's loads");
   uint32_t lane_off[PER];
 #pragma unroll
@@ -226,6 +264,42 @@ __device__ __forceinline__ void bwd_store_rows(const f32x16_t (&acc)[D / 32], fl
 }
 
 
+// Sum of the transposed accumulators of KG groups (W waves each, 32 columns = output rows per wave)
+// x factor -> 16-bit rows.  Each group gets a share of the 4-register pieces from the others through LDS,
+// adds up and stores it; `row`: this lane's output row, `stores`: it has one.  LDS: G (G - 1) W
+// (pieces / G) KiB, nobody else may use it any more.
+template <bool BF16, int D, int G, int W>
+__device__ __forceinline__ void bwd_merge_store(const f32x16_t (&acc)[D / 32], float factor, uint8_t* lds, int group,
+                                                int w, int lane, uint16_t* row, bool stores) {
+  constexpr int UNITS = D / 8;                  // 4-register pieces of a lane's accumulators
+  constexpr int SHARE = (UNITS + G - 1) / G;    // ... of a group
+  const int g = lane >> 5;
+  auto piece_at = [&](int to, int from, int n) {
+    const int src = from < to ? from : from - 1;
+    return reinterpret_cast<f32x4_t*>(lds) + (((to * (G - 1) + src) * W + w) * SHARE + n) * 64 + lane;
+  };
+  static_for<UNITS>([&](auto uc) {
+    constexpr int u = decltype(uc)::value, dt = u / 4, r4 = u % 4, to = u / SHARE;
+    if (to != group) {
+      const f32x4_t x = {acc[dt][4 * r4 + 0], acc[dt][4 * r4 + 1], acc[dt][4 * r4 + 2], acc[dt][4 * r4 + 3]};
+      *piece_at(to, group, u % SHARE) = x;
+    }
+  });
+  __syncthreads();
+  static_for<UNITS>([&](auto uc) {
+    constexpr int u = decltype(uc)::value, dt = u / 4, r4 = u % 4, to = u / SHARE;
+    if (to == group) {
+      f32x4_t x = {acc[dt][4 * r4 + 0], acc[dt][4 * r4 + 1], acc[dt][4 * r4 + 2], acc[dt][4 * r4 + 3]};
+      // in the order of the groups, whoever adds: group 0's piece first
+      f32x4_t sum = group == 0 ? x : *piece_at(to, 0, u % SHARE);
+#pragma unroll
+      for (int i = 1; i < G; ++i) sum += i == to ? x : *piece_at(to, i, u % SHARE);
+      const u32x2_t ov = {pack2<BF16>(sum[0] * factor, sum[1] * factor), pack2<BF16>(sum[2] * factor, sum[3] * factor)};
+      if (stores) *reinterpret_cast<u32x2_t*>(row + 8 * u + 4 * g) = ov;
+    }
+  });
+}
+
 // One step of a backward walk.
 struct BwdStepInfo {
   int row0;   // first key row (dQ kernel) / first query row (dK/dV kernel) of the step
@@ -236,41 +310,64 @@ struct BwdStepInfo {
   bool valid;
 };
 
-template <int D, int QB>
-struct BwdDqTraits {
-  static constexpr int kThreads = QB * 2;
-  // keys per step: two 32-key halves whose products and vector work overlap inside a wave
-  static constexpr int kStep = 64;
+// How a workgroup of the dQ kernel walks: QT query rows (QT / 32 waves), KG groups of such waves that
+// share the steps of the list (step n is group n % KG's) and add up at the end, STEP keys per step: 64
+// are two 32-key halves whose products and vector work overlap inside a wave.  QB, KB: the block
+// sizes, 0 where they are not known at compile time.
+template <bool BF16_, bool CAP_, int D_, int QB_, int KB_, int QT_, int KG_, int STEP_>
+struct BwdDqShape {
+  static constexpr bool BF16 = BF16_, CAP = CAP_;
+  static constexpr int D = D_, QB = QB_, KB = KB_, QT = QT_, KG = KG_, kStep = STEP_;
+  static constexpr int kGroupThreads = QT * 2;
+  static constexpr int kThreads = kGroupThreads * KG;
   static constexpr int kTileElems = kStep * D;
   // two sets of two tiles (K, V), or the output staging
-  static constexpr size_t kLdsBytes = (4 * kTileElems > QB * D ? 4 * kTileElems : QB * D) * sizeof(uint16_t);
+  static constexpr size_t kGroupBytes = (4 * kTileElems > QT * D ? 4 * kTileElems : QT * D) * sizeof(uint16_t);
+  static constexpr size_t kMergeBytes = size_t(KG) * (KG - 1) * (QT / 32) * ((D / 8 + KG - 1) / KG) * 1024;
+  static constexpr size_t kLdsBytes = kGroupBytes * KG > kMergeBytes ? kGroupBytes * KG : kMergeBytes;
 };
 
-template <bool BF16, bool CAP, int D, int QB, int KB>
-__global__ void __launch_bounds__(QB * 2, 2) bwd_dq_kernel(const BwdParams p) {
-  using Traits = BwdDqTraits<D, QB>;
-  constexpr int NT = Traits::kThreads;
-  constexpr int STEP = Traits::kStep;
-  constexpr int SPB = KB / STEP;
+template <class Shape>
+__device__ __forceinline__ void bwd_dq_walk(const BwdParams& p) {
+  constexpr bool BF16 = Shape::BF16, CAP = Shape::CAP;
+  constexpr int D = Shape::D;
+  constexpr int QT = Shape::QT;
+  constexpr int KG = Shape::KG;
+  constexpr bool LONE = QT == 32;  // a group is one wave: its steps need no barriers
+  constexpr int NT = Shape::kGroupThreads;
+  constexpr int STEP = Shape::kStep;
+  const int QB = Shape::QB != 0 ? Shape::QB : p.QB;
+  const int KB = Shape::KB != 0 ? Shape::KB : p.KB;
+  const int SPB = KB / STEP;
   constexpr int NTL = STEP / 32;
   constexpr int KS = D / 16;
   constexpr int DT = D / 32;
-  constexpr int TILE = Traits::kTileElems;
+  constexpr int TILE = Shape::kTileElems;
+  constexpr int WQ = QT / 32;
 
+  const int w_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kg = KG == 1 ? 0 : w_all / WQ;     // group of the wave (wave-uniform)
+  const int w = KG == 1 ? w_all : w_all % WQ;  // wave of the group
   extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
-  uint16_t* const lds16 = reinterpret_cast<uint16_t*>(lds_raw);  // [2 sets][K, V][TILE]
+  uint16_t* const lds16 = reinterpret_cast<uint16_t*>(lds_raw + size_t(kg) * Shape::kGroupBytes);  // [2 sets][K, V][TILE]
 
   // Workgroup -> (slab, query block): XCD x takes the slabs bh with bh % n_xcd == x one after
   // the other, longest query block first, so the workgroups that run together on an XCD walk the
   // K/V rows of one or two slabs and share them through that XCD's L2.
+  // (A slab may be dealt in parts, see the forward.)
   const int slot = blockIdx.x / p.n_xcd;
   const int xcd = blockIdx.x - slot * p.n_xcd;
-  if (slot >= ((p.n_slabs - xcd + p.n_xcd - 1) / p.n_xcd) * p.Tq) return;
-  const int bh = xcd + p.n_xcd * (slot / p.Tq);
-  const int qb = p.Tq - 1 - slot % p.Tq;
-  const int tid = threadIdx.x;
+  const int tiles = KG == 1 ? p.Tq : p.Tq * (QB / QT);
+  const int part_tiles = (tiles + p.parts - 1) / p.parts;
+  if (slot >= ((p.n_slabs * p.parts - xcd + p.n_xcd - 1) / p.n_xcd) * part_tiles) return;
+  const int dealt = xcd + p.n_xcd * (slot / part_tiles);
+  const int bh = dealt / p.parts;
+  const int qt = tiles - 1 - ((slot % part_tiles) * p.parts + dealt - bh * p.parts);
+  const int q0 = qt * QT;  // first row of this workgroup
+  if (qt < 0 || (KG > 1 && q0 >= p.S)) return;
+  const int qb = KG == 1 ? qt : q0 / QB;
+  const int tid = KG == 1 ? threadIdx.x : threadIdx.x - kg * NT;  // thread of the group
   const int lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 5, c = lane & 31;
 
   // Rows at or beyond the sequence are never used: the resources of K and V end there (those
@@ -280,8 +377,8 @@ __global__ void __launch_bounds__(QB * 2, 2) bwd_dq_kernel(const BwdParams p) {
   const uint32_t k_pitch = p.k_at.row * 2u, v_pitch = p.v_at.row * 2u;  // bytes from row to row
   const i32x4_t rK = row_resource<D>(p.k, p.k_at, bh, p.H, p.seqlen);
   const i32x4_t rV = row_resource<D>(p.v, p.v_at, bh, p.H, p.seqlen);
-  const int q_row = qb * QB + 32 * w + c;
-  const int q_wave_min = qb * QB + 32 * w;
+  const int q_row = q0 + 32 * w + c;
+  const int q_wave_min = q0 + 32 * w;
   const int qr = q_row < p.S ? q_row : p.S - 1;
   const size_t meta_row = size_t(bh) * p.Tq + qb;
   const size_t meta_off = meta_row * p.max_blocks;
@@ -345,7 +442,7 @@ __global__ void __launch_bounds__(QB * 2, 2) bwd_dq_kernel(const BwdParams p) {
   const bool row_live = q_row < p.seqlen && lse != -INFINITY;
   // exponent offset; +inf for rows without any allowed key so that every weight becomes 0
   const float lse2 = row_live ? lse * 1.4426950408889634f : INFINITY;
-  if (q_row < p.S && g == 0) {
+  if (q_row < p.S && g == 0 && kg == 0) {
     p.ws[size_t(bh) * p.S + q_row] = -delta;
     // The dK/dV kernel starts the accumulator of a row's scores at -LSE * sqrt(D), so that the
     // exponent of a weight is the score times log2(e) / sqrt(D) and nothing else (-inf: every
@@ -368,7 +465,7 @@ __global__ void __launch_bounds__(QB * 2, 2) bwd_dq_kernel(const BwdParams p) {
   // step of a block.
   int gj = 0;  // next slot of the list to look at
   BwdStepInfo g_last = {0, kMasked, -1, 0, 0, false};
-  const int q_last = qb * QB + QB - 1;
+  const int q_last = q0 + QT - 1;
   auto next_step = [&]() {
     if (g_last.valid) {
       const int r = g_last.row0 + STEP, sb = g_last.sub + 1;
@@ -417,6 +514,7 @@ __global__ void __launch_bounds__(QB * 2, 2) bwd_dq_kernel(const BwdParams p) {
   // exp2(score * sl2); that of dP^T starts at -delta.  A soft-capped score is not linear in the
   // product: there S^T starts at zero and offset and mask are applied to the weights.
   constexpr int NSUB = NTL;
+  static_assert(NSUB == 1 || NSUB == 2, "halves of a step");
   constexpr int NTR = 2 * DT;                    // last products of a half
   constexpr int NS = NSUB * (2 * KS + NTR);      // slots of a step
   constexpr int PF = D == 128 ? 2 : 3;           // operand fetch distance in slots (registers are tight at 128)
@@ -499,27 +597,45 @@ __global__ void __launch_bounds__(QB * 2, 2) bwd_dq_kernel(const BwdParams p) {
       if constexpr (n + PF < NS) opq[n % PF] = operand(IntC<n + PF>{});
       // the score gradients of half ch - 1 go beside the products of chain ch: 8 register pairs
       // spread over the chain's slots
-      if constexpr (ch >= 1 && ch <= NSUB) {
+      if constexpr (NSUB == 2 && ch >= 1 && ch <= NSUB) {
         constexpr int lo = sl * 8 / len, hi = (sl + 1) * 8 / len;
         static_for<hi - lo>([&](auto ic) { grads(IntC<ch - 1>{}, IntC<2 * (lo + decltype(ic)::value)>{}); });
       }
       __builtin_amdgcn_sched_barrier(0);
+      if constexpr (NSUB == 1 && n == 2 * KS - 1) {  // a one-half step: nothing to put them under
+        static_for<8>([&](auto ic) { grads(IntC<0>{}, IntC<2 * decltype(ic)::value>{}); });
+        __builtin_amdgcn_sched_barrier(0);
+      }
     });
     __builtin_amdgcn_s_setprio(0);
   };
 
   // Tiles of step i + 1 are loaded while step i is computed: one barrier per step.
-  BwdStepInfo cur = next_step();
+  // A round is KG steps, one of each group (the last round of a walk may have fewer).
+  bool more = false;  // the round that next_round() returned this group's step of has steps
+  auto next_round = [&]() {
+    BwdStepInfo mine = next_step();
+    more = mine.valid;
+    if constexpr (KG > 1) {
+#pragma unroll
+      for (int i = 1; i < KG; ++i) {
+        const BwdStepInfo st = next_step();
+        if (i == kg) mine = st;
+      }
+    }
+    return mine;
+  };
+  BwdStepInfo cur = next_round();
   int set = 0;
   if (cur.valid) issue_loads(cur, 0);
-  while (cur.valid) {
-    const BwdStepInfo nxt = next_step();
+  while (more) {
+    const BwdStepInfo nxt = next_round();
     // mask words of this lane's row: bit j of word t = key row0 + 32 t + j allowed
     uint32_t kw[NTL];
 #pragma unroll
     for (int t = 0; t < NTL; ++t) kw[t] = 0xffffffffu;
     if (cur.mode == kPartial) {
-      const int q_local = q_row - qb * QB;
+      const int q_local = q_row - qb * QB;  // (below QB: the rows of a workgroup are one block's)
 #pragma unroll
       for (int t = 0; t < NTL; ++t) {
         const int kcol = cur.sub * STEP + 32 * t;
@@ -541,14 +657,19 @@ __global__ void __launch_bounds__(QB * 2, 2) bwd_dq_kernel(const BwdParams p) {
       const uint32_t low = n >= 32 ? 0xffffffffu : (n <= 0 ? 0u : ((1u << (n & 31)) - 1u));
       kw[t] &= low;
     });
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this step's tiles (and mask words) have landed
-    __syncthreads();                     // ... for every wave; and the other set is no longer read
+    wait_loads();                  // this step's tiles (and mask words) have landed
+    if constexpr (!LONE) __syncthreads();  // ... for every wave; and the other set is no longer read
     if (nxt.valid) issue_loads(nxt, set ^ 1);
-    compute(set, kw, !(cur.mode == kFull && cur.row0 + STEP <= p.seqlen));
+    if (KG == 1 || cur.valid) compute(set, kw, !(cur.mode == kFull && cur.row0 + STEP <= p.seqlen));
     set ^= 1;
     cur = nxt;
   }
   __syncthreads();  // tiles are dead: the staging area overlaps them
+  if constexpr (KG > 1) {
+    bwd_merge_store<BF16, D, KG, WQ>(dq, p.scale, lds_raw, kg, w, lane,
+                                     p.dq + slab + size_t(q_row < p.S ? q_row : 0) * D, q_row < p.S);
+    return;
+  }
   uint16_t* stage = lds16 + size_t(w) * 32 * D;
   // (the lane number goes through an empty asm: the addresses of the epilogue are then computed
   // here and not kept in registers across the walk, where every register counts)
@@ -557,28 +678,39 @@ __global__ void __launch_bounds__(QB * 2, 2) bwd_dq_kernel(const BwdParams p) {
   bwd_store_rows<BF16, D>(dq, p.scale, stage, p.dq + slab, q_wave_min, p.S, lane_out);
 }
 
-// First step of STEP query rows of query block qb that can contribute to KV block kvb: a CAUSAL
+template <bool BF16, bool CAP, int D, int QB, int KB>
+__global__ void __launch_bounds__(QB * 2, 2) bwd_dq_kernel(const BwdParams p) {
+  bwd_dq_walk<BwdDqShape<BF16, CAP, D, QB, KB, QB, 1, 64>>(p);
+}
+// The steps of a list shared by the groups of a workgroup (fwd_choose_split says when).
+template <bool BF16, bool CAP, int D, int QT, int KG, int STEP>
+__global__ void __launch_bounds__(QT * 2 * KG, 2) bwd_dq_ksplit(const BwdParams p) {
+  bwd_dq_walk<BwdDqShape<BF16, CAP, D, 0, 0, QT, KG, STEP>>(p);
+}
+
+// First step of STEP query rows of a query block that can contribute to the keys from first_key on: a CAUSAL
 // step whose rows all lie above the block's first key contributes nothing (the dK/dV kernel starts
 // a block's walk there, and never stores score gradients for the steps before it).
-template <int QB, int KB, int STEP>
-__device__ __forceinline__ int bwd_first_step(int mode, int kvb, int qb) {
+template <int STEP>
+__device__ __forceinline__ int bwd_first_step(int mode, int first_key, int first_row) {
   if (mode != kCausal) return 0;
-  const int below = kvb * KB - (qb * QB + STEP - 1);  // rows of the block before the first useful step
+  const int below = first_key - (first_row + STEP - 1);  // rows of the block before the first useful step
   return below > 0 ? (below + STEP - 1) / STEP : 0;
 }
 
-template <int D, int KB>
-struct BwdDkdvTraits {
-  static constexpr int kKeyGroups = KB / 32;       // 32 keys per wave
-  static constexpr int kRoleThreads = KB * 2;      // one wave per key group in each of the two roles
-  static constexpr int kThreads = KB * 4;
-  // Query rows per step.  At head_dim 128 with 128-key blocks: 64, worked as two 32-row halves
-  // whose products and vector work overlap inside a wave (one workgroup of eight waves per
-  // compute unit, two waves per SIMD).  Elsewhere 32, so that two workgroups share a compute
-  // unit: a 64-key workgroup has four waves, and at head_dim <= 64 the products of a step are so
-  // short that four waves per SIMD hide more than longer steps gain (measured at head_dim 64:
-  // 64-row steps at two waves per SIMD take 1.3 x the time of 32-row steps at four).
-  static constexpr int kStep = (KB == 128 && D == 128) ? 64 : 32;
+// How a workgroup of the dK/dV kernel works: NKG key groups of 32 keys (of one KV block) with two waves
+// each, G groups of such waves that share the steps (step n is group n % G's) and add up at the end, STEP
+// query rows per step.  QB, KB: the block sizes, 0 where they are not known at compile time.
+template <bool BF16_, bool CAP_, int D_, int QB_, int KB_, int NKG_, int G_, int STEP_>
+struct BwdDkdvShape {
+  static constexpr bool BF16 = BF16_, CAP = CAP_;
+  static constexpr int D = D_, QB = QB_, KB = KB_, G = G_;
+  static constexpr int kKeyGroups = NKG_;          // 32 keys per wave
+  static constexpr int kKeys = NKG_ * 32;          // keys of the workgroup
+  static constexpr int kRoleThreads = kKeys * 2;   // one wave per key group in each of the two roles
+  static constexpr int kGroupThreads = kKeys * 4;
+  static constexpr int kThreads = kGroupThreads * G;
+  static constexpr int kStep = STEP_;
   static constexpr int kSub = kStep / 32;
   static constexpr int kTileElems = kStep * D;
   // three sets of two tiles (Q, dO) -- the output staging overlaps them
@@ -588,17 +720,37 @@ struct BwdDkdvTraits {
   static constexpr size_t kHandBytes = size_t(2) * kKeyGroups * kSub * 2 * 64 * 16;
   // -delta and the exponent offsets of the rows of three steps
   static constexpr size_t kRowBytes = size_t(6) * kStep * sizeof(float);
-  static constexpr size_t kFixedBytes = kTileBytes + kHandBytes + kRowBytes;
+  static constexpr size_t kGroupBytes = kTileBytes + kHandBytes + kRowBytes;
+  static constexpr size_t kFixedBytes = kGroupBytes * G;
+  static_assert(size_t(G) * (G - 1) * 2 * kKeyGroups * ((D / 8 + G - 1) / G) * 1024 <= kFixedBytes, "merge in LDS");
   // per 64-slot word of a slab's metadata: the bitmap of the slots that list this KV block (8
-  // bytes) and mode / tile index of the first (4 bytes).  The launch asks for the words its
-  // metadata needs, so small problems fit two workgroups per compute unit; metadata with more
-  // words than fit is worked through in windows of kMaxBitmapWords.
+  // bytes) and mode / tile index of the first (4 bytes); behind them the table of steps (8 bytes each),
+  // room for one match per word and for one word full of matches.  The launch asks for the words
+  // its metadata needs, so small problems fit two workgroups per compute unit; metadata with more
+  // words (or matches) than fit is worked through in windows.
   static constexpr size_t kLdsLimit = size_t(160) * 1024;
-  static constexpr int kMaxBitmapWords =
-      (kLdsLimit - kFixedBytes) / 12 < 4096 ? int((kLdsLimit - kFixedBytes) / 12) : 4096;
-  static constexpr size_t lds_bytes(size_t bitmap_words) { return kFixedBytes + bitmap_words * 12; }
-  static constexpr size_t kLdsBytes = lds_bytes(kMaxBitmapWords);
+  static constexpr int table_steps(int words, int steps_per_block) { return (words + 64) * steps_per_block; }
+  static constexpr size_t lds_bytes(int words, int steps_per_block) {
+    return kFixedBytes + size_t((words + 1) / 2) * 24 + size_t(table_steps(words, steps_per_block)) * 8 + 8;
+  }
+  static constexpr int kMaxStepsPerBlock = 128 / kStep;
+  static constexpr int fitting_words() {
+    int n = 4096;
+    while (lds_bytes(n, kMaxStepsPerBlock) > kLdsLimit) --n;
+    return n;
+  }
+  static constexpr int kMaxBitmapWords = fitting_words();
+  static constexpr size_t kLdsBytes = lds_bytes(kMaxBitmapWords, kMaxStepsPerBlock);
 };
+// One workgroup per KV block, all steps in one group.  Query rows per step: at head_dim 128 with
+// 128-key blocks 64, worked as two 32-row halves
+// whose products and vector work overlap inside a wave (one workgroup of eight waves per
+// compute unit, two waves per SIMD).  Elsewhere 32, so that two workgroups share a compute
+// unit: a 64-key workgroup has four waves, and at head_dim <= 64 the products of a step are so
+// short that four waves per SIMD hide more than longer steps gain (measured at head_dim 64:
+// 64-row steps at two waves per SIMD take 1.3 x the time of 32-row steps at four).
+template <bool BF16, bool CAP, int D, int QB, int KB>
+using BwdDkdvBlockShape = BwdDkdvShape<BF16, CAP, D, QB, KB, KB / 32, 1, (KB == 128 && D == 128) ? 64 : 32>;
 
 // Two 16-bit values of a word -> fp32 (exact).
 template <bool BF16>
@@ -629,15 +781,20 @@ __device__ __forceinline__ void unpack2(uint32_t w, float& lo, float& hi) {
 // the operand three slots ahead and a share of the vector work of the half whose first
 // product has just finished, with a scheduling fence after each slot: the weights of half u are
 // computed under the products of half u + 1 (or under the second products of half 0).
-template <bool BF16, bool CAP, int D, int QB, int KB>
-__global__ void __launch_bounds__(KB * 4, D == 128 ? 2 : 4) bwd_dkdv_kernel(const BwdParams p) {
-  using Traits = BwdDkdvTraits<D, KB>;
+template <class Traits>
+__device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
+  constexpr bool BF16 = Traits::BF16, CAP = Traits::CAP;
+  constexpr int D = Traits::D;
+  constexpr int G = Traits::G;
+  constexpr int KT = Traits::kKeys;
+  const int QB = Traits::QB != 0 ? Traits::QB : p.QB;
+  const int KB = Traits::KB != 0 ? Traits::KB : p.KB;
   constexpr int NKG = Traits::kKeyGroups;
   constexpr int RT = Traits::kRoleThreads;
-  constexpr int NW = Traits::kThreads / 64;
+  constexpr int NW = Traits::kThreads / 64;  // waves of the workgroup
   constexpr int STEP = Traits::kStep;
   constexpr int NSUB = Traits::kSub;
-  constexpr int NSTEPS = QB / STEP;  // steps per query block
+  const int NSTEPS = QB / STEP;      // steps per query block
   constexpr int KS = D / 16;         // products of a 32-row half: KS for S (or dP) ...
   constexpr int DT = D / 32;
   constexpr int NTR = 2 * DT;        // ... and as many for dV^T (or dK^T)
@@ -645,28 +802,37 @@ __global__ void __launch_bounds__(KB * 4, D == 128 ? 2 : 4) bwd_dkdv_kernel(cons
   constexpr int SPC = 16 / KS;       // scores of a half whose vector work goes beside one product
   constexpr int TILE = Traits::kTileElems;
   constexpr int PF = 3 < NS ? 3 : NS;  // operand fetch distance in slots
-  constexpr bool PRIO = KB == 64;      // raise the wave priority around the products (it pays
+  constexpr bool PRIO = KT == 64 || G > 1;  // raise the wave priority around the products (it pays
                                        // with two workgroups per compute unit)
-  static_assert(NTR == KS && QB % STEP == 0 && 16 % KS == 0, "slot layout");
+  static_assert(NTR == KS && 16 % KS == 0, "slot layout");
 
   extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
-  uint16_t* const lds16 = reinterpret_cast<uint16_t*>(lds_raw);  // [3 sets][Q, dO][TILE]
-  uint32_t* const sHand = reinterpret_cast<uint32_t*>(lds_raw + Traits::kTileBytes);
-  float* const sNd = reinterpret_cast<float*>(lds_raw + Traits::kTileBytes + Traits::kHandBytes);  // [3 sets][STEP] -delta
+  const int w_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int group = G == 1 ? 0 : w_all / (2 * NKG);     // group of the wave (wave-uniform)
+  const int w = G == 1 ? w_all : w_all % (2 * NKG);     // wave of the group
+  uint8_t* const lds_group = lds_raw + size_t(group) * Traits::kGroupBytes;
+  uint16_t* const lds16 = reinterpret_cast<uint16_t*>(lds_group);  // [3 sets][Q, dO][TILE]
+  uint32_t* const sHand = reinterpret_cast<uint32_t*>(lds_group + Traits::kTileBytes);
+  float* const sNd = reinterpret_cast<float*>(lds_group + Traits::kTileBytes + Traits::kHandBytes);  // [3 sets][STEP] -delta
   float* const sL2 = sNd + 3 * STEP;                                         // [3 sets][STEP] exponent offsets
-  uint64_t* const sMatch = reinterpret_cast<uint64_t*>(sL2 + 3 * STEP);
+  uint64_t* const sMatch = reinterpret_cast<uint64_t*>(lds_raw + Traits::kFixedBytes);
 
   // Workgroup -> (slab, KV block): XCD x takes the slabs bh with bh % n_xcd == x one after the
   // other, so the workgroups that run together on an XCD read the Q and dO rows of one slab and
   // share them through that XCD's L2.
   const int slot = blockIdx.x / p.n_xcd;
   const int xcd = blockIdx.x - slot * p.n_xcd;
-  if (slot >= ((p.n_slabs - xcd + p.n_xcd - 1) / p.n_xcd) * p.Tk) return;
-  const int bh = xcd + p.n_xcd * (slot / p.Tk);
-  const int kvb = slot % p.Tk;
-  const int tid = threadIdx.x;
+  const int tiles = G == 1 ? p.Tk : p.Tk * (KB / KT);
+  const int part_tiles = (tiles + p.parts - 1) / p.parts;
+  if (slot >= ((p.n_slabs * p.parts - xcd + p.n_xcd - 1) / p.n_xcd) * part_tiles) return;
+  const int dealt = xcd + p.n_xcd * (slot / part_tiles);
+  const int bh = dealt / p.parts;
+  const int kt = (slot % part_tiles) * p.parts + dealt - bh * p.parts;
+  const int key0 = kt * KT;  // first key of this workgroup
+  if (kt >= tiles || (G > 1 && key0 >= p.S)) return;
+  const int kvb = G == 1 ? kt : key0 / KB;
+  const int tid = G == 1 ? threadIdx.x : threadIdx.x - group * Traits::kGroupThreads;  // thread of the group
   const int lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool grad_role = w >= NKG;        // wave-uniform
   const int kg = grad_role ? w - NKG : w;  // key group of the wave
   const int rtid = tid - (grad_role ? RT : 0);
@@ -680,7 +846,8 @@ __global__ void __launch_bounds__(KB * 4, D == 128 ? 2 : 4) bwd_dkdv_kernel(cons
   const i32x4_t rD = row_resource<D>(p.dout, p.dout_at, bh, p.H, p.seqlen);
   const i32x4_t rNd = make_buffer_resource(p.ws + size_t(bh) * p.S, uint32_t(p.S) * 4u);
   const i32x4_t rL2 = make_buffer_resource(p.ws + size_t(p.n_slabs) * p.S + size_t(bh) * p.S, uint32_t(p.S) * 4u);
-  const int key_wave_min = kvb * KB + 32 * kg;
+  const int key_wave_min = key0 + 32 * kg;
+  const int kcol = key_wave_min - kvb * KB;  // ... inside its block
   const int key = key_wave_min + c;  // this lane's key row inside the slab
   const bool key_live = key < p.seqlen;
   const bool has_partial = p.partial_idx != nullptr && (p.partial_masks != nullptr || p.partial_bits != nullptr);
@@ -690,6 +857,10 @@ __global__ void __launch_bounds__(KB * 4, D == 128 ? 2 : 4) bwd_dkdv_kernel(cons
   // words of the bitmap held in LDS at a time (what the launch sized the allocation for)
   const int win_words = n_words < Traits::kMaxBitmapWords ? n_words : Traits::kMaxBitmapWords;
   int32_t* const sFirst = reinterpret_cast<int32_t*>(sMatch + win_words);
+  typedef __attribute__((ext_vector_type(2))) int32_t i32x2_t;
+  // one entry per step: first query row; mode in the low two bits, tile index above
+  i32x2_t* const sSteps = reinterpret_cast<i32x2_t*>(sFirst + ((win_words + 1) & ~1));
+  const int table_steps = Traits::table_steps(win_words, NSTEPS);
 
   // This lane's key as B operand: K for a weight wave, V for a gradient wave (zeros for a key
   // beyond the sequence).
@@ -715,7 +886,7 @@ __global__ void __launch_bounds__(KB * 4, D == 128 ? 2 : 4) bwd_dkdv_kernel(cons
     // together (every slot inside the list's width is loaded; kv_num_blocks cuts afterwards).
     // The first window, scanned while few registers are live, takes four; later ones one.
     constexpr int SCAN = decltype(scan_c)::value;
-    for (int word0 = base + w * SCAN; word0 < end; word0 += NW * SCAN) {
+    for (int word0 = base + w_all * SCAN; word0 < end; word0 += NW * SCAN) {
       int32_t raw[SCAN], ty[SCAN], pid[SCAN], nbv[SCAN];
 #pragma unroll
       for (int u = 0; u < SCAN; ++u) {
@@ -751,69 +922,74 @@ __global__ void __launch_bounds__(KB * 4, D == 128 ? 2 : 4) bwd_dkdv_kernel(cons
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) acc[dt] = zero16;
 
-  // The walk: the matches in ascending (query block, slot) order, each as NSTEPS steps of STEP
-  // query rows, skipping steps beyond the sequence and CAUSAL steps entirely above the diagonal.
-  // Inside a match the next step is the previous one moved on by STEP query rows (a CAUSAL step
-  // that is valid stays valid further down; only the end of the sequence can end a match early):
-  // that path is a handful of scalar instructions; the bitmap is only read at the first step of a
-  // match.  The generator ends at the end of the window LDS holds and goes on from there once the
-  // next window has been scanned.
-  int gw = -1, g_qb = 0, g_ch = -1;  // word gw = (g_qb, g_ch)
+  // The walk: the matches in ascending (query block, slot) order, each as NSTEPS steps of STEP query
+  // rows, skipping steps beyond the sequence and CAUSAL steps entirely above the diagonal (both cut a
+  // match's steps from one end).  The first wave turns the window's bitmap into a table of steps, a
+  // lane per word, so that the loop gets a step with one LDS read, requested an iteration ahead
+  // (a generator that found the next step from the bitmap cost every wave 500 - 700 cycles per
+  // step).  Returns the number of steps; `end` moves to the first word that is not in the table.
+  int32_t* const s_table = reinterpret_cast<int32_t*>(sSteps + table_steps);  // steps, end
+  auto steps_of = [&](int32_t info, int first_row, int& sub0) {
+    sub0 = bwd_first_step<STEP>(info & 3, key0, first_row);
+    const int rows = p.seqlen - first_row;
+    const int subs = rows <= 0 ? 0 : (rows + STEP - 1) / STEP;
+    const int n = (subs < NSTEPS ? subs : NSTEPS) - sub0;
+    return n > 0 ? n : 0;
+  };
+  auto build_table = [&](int base, int& end) {
+    if (w_all == 0) {
+      int n = 0;
+      for (int w0 = base; w0 < end; w0 += 64) {
+        const int word = w0 + lane;
+        uint64_t bits = word < end ? sMatch[word - base] : 0;
+        const int qb = word / chunks, ch = word - qb * chunks;
+        const int first_row = qb * QB;
+        // information of the match that is the lowest bit of `left`
+        auto info_of = [&](uint64_t left) {
+          if (left == bits) return sFirst[word - base];
+          const size_t o = (meta_slab + qb) * p.max_blocks + ch * 64 + __builtin_ctzll(left);
+          const int32_t pid = has_partial ? p.partial_idx[o] : -1;
+          const int32_t mode = bwd_slot_mode(p.types[o], pid, has_partial, p.num_partial);
+          return (mode == kPartial ? pid << 2 : 0) | mode;
+        };
+        int count = 0, sub0;
+        for (uint64_t left = bits; left != 0; left &= left - 1) count += steps_of(info_of(left), first_row, sub0);
+        int upto = count;  // inclusive sum over the lanes
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+          const int other = __shfl_up(upto, d, 64);
+          upto += lane >= d ? other : 0;
+        }
+        const bool fits = n + upto <= table_steps;
+        if (fits) {
+          int at = n + upto - count;
+          for (uint64_t left = bits; left != 0; left &= left - 1) {
+            const int32_t info = info_of(left);
+            const int k = steps_of(info, first_row, sub0);
+            for (int i = 0; i < k; ++i) sSteps[at++] = i32x2_t{first_row + (sub0 + i) * STEP, info};
+          }
+        }
+        const uint64_t all_fit = __builtin_amdgcn_ballot_w64(fits);
+        if (~all_fit != 0) {  // (only lists that name a block many times get here)
+          const int m = __builtin_ctzll(~all_fit);
+          if (m > 0) n += __shfl(upto, m - 1, 64);
+          end = w0 + m < end ? w0 + m : end;
+          break;
+        }
+        n += __shfl(upto, 63, 64);
+      }
+      if (lane == 0) {
+        s_table[0] = n;
+        s_table[1] = end;
+      }
+    }
+    __syncthreads();
+    end = __builtin_amdgcn_readfirstlane(s_table[1]);
+    return __builtin_amdgcn_readfirstlane(s_table[0]);
+  };
   int win_base = 0, win_end = win_words;  // the words of the slab the window holds
   scan_window(IntC<4>{}, 0, win_end);
-  uint64_t gbits = 0;
-  bool g_first = true;
-  BwdStepInfo g_last = {0, kMasked, -1, 0, 0, false};
-  auto next_step = [&]() {
-    if (g_last.valid) {
-      const int r = g_last.row0 + STEP, sb = g_last.sub + 1;
-      if (bool(int(sb < NSTEPS) & int(r < p.seqlen))) {
-        g_last.row0 = r;
-        g_last.sub = sb;
-        return g_last;
-      }
-    }
-    g_last.valid = false;
-    for (;;) {
-      while (gbits == 0) {
-        if (++gw >= win_end) return g_last;
-        if (++g_ch == chunks) {
-          g_ch = 0;
-          ++g_qb;
-        }
-        const uint64_t m = sMatch[gw - win_base];
-        // (readfirstlane returns a signed int: go through uint32_t so that bit 31 does not sign-extend)
-        gbits = (uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(m >> 32))))) << 32) |
-                uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(m)))));
-        g_first = true;
-      }
-      int mode, pid;
-      if (g_first) {
-        const int32_t info = __builtin_amdgcn_readfirstlane(sFirst[gw - win_base]);
-        mode = info & 3;
-        pid = mode == kPartial ? info >> 2 : -1;
-      } else {  // a further match in the same 64 slots
-        const size_t o = (meta_slab + g_qb) * p.max_blocks + g_ch * 64 + __builtin_ctzll(gbits);
-        const int32_t ty = load_uniform(p.types + o);
-        pid = has_partial ? load_uniform(p.partial_idx + o) : -1;
-        mode = bwd_slot_mode(ty, pid, has_partial, p.num_partial);
-      }
-      gbits &= gbits - 1;
-      g_first = false;
-      // first step of the match that contributes: CAUSAL steps entirely above the diagonal and
-      // steps beyond the sequence do not
-      const int sub = bwd_first_step<QB, KB, STEP>(mode, kvb, g_qb);
-      const int q0 = g_qb * QB + sub * STEP;
-      if (sub >= NSTEPS || q0 >= p.seqlen) continue;
-      g_last.row0 = q0;
-      g_last.mode = mode;
-      g_last.pid = pid;
-      g_last.blk = g_qb;
-      g_last.sub = sub;
-      g_last.valid = true;
-      return g_last;
-    }
-  };
+  int n_steps = build_table(0, win_end);
   const uint32_t lds_tiles = lds_offset_of(lds16);
   const uint32_t hand_lane = lds_offset_of(sHand) + uint32_t(kg) * (NSUB * 2048u) + uint32_t(lane) * 16u;
   const uint32_t lds_nd = lds_offset_of(sNd), lds_l2 = lds_offset_of(sL2);
@@ -822,14 +998,18 @@ __global__ void __launch_bounds__(KB * 4, D == 128 ? 2 : 4) bwd_dkdv_kernel(cons
   auto hand_at = [&](int par, int u, int half) {
     return hand_lane + uint32_t(par) * (NKG * NSUB * 2048u) + uint32_t(u) * 2048u + uint32_t(half) * 1024u;
   };
+  struct Step {
+    int row0, info;
+    bool valid;
+  };
   // The rows of step j + 1 are loaded during iteration j: Q and the exponent offsets by the
   // weight waves, dO and -delta by the gradient waves.
-  auto load_q = [&](const BwdStepInfo& st, int set) {
+  auto load_q = [&](const Step& st, int set) {
     bwd_load_tile<D, RT, STEP>(rQ, q_pitch, st.row0, tile_at(set, 0), rtid, kg);
     if (rtid < STEP)
       buffer_to_lds_b32(rL2, uint32_t(rtid) * 4u, uint32_t(st.row0) * 4u, lds_l2 + uint32_t(set * STEP) * 4u);
   };
-  auto load_do = [&](const BwdStepInfo& st, int set) {
+  auto load_do = [&](const Step& st, int set) {
     bwd_load_tile<D, RT, STEP>(rD, do_pitch, st.row0, tile_at(set, 1), rtid, kg);
     if (rtid < STEP)
       buffer_to_lds_b32(rNd, uint32_t(rtid) * 4u, uint32_t(st.row0) * 4u, lds_nd + uint32_t(set * STEP) * 4u);
@@ -1011,9 +1191,9 @@ __global__ void __launch_bounds__(KB * 4, D == 128 ? 2 : 4) bwd_dkdv_kernel(cons
     const int rl = lane & 31;
     uint32_t roww;
     if (p.partial_bits != nullptr) {
-      roww = p.partial_bits[(size_t(pid) * QB + q_local0 + rl) * (KB / 32) + kg];
+      roww = p.partial_bits[(size_t(pid) * QB + q_local0 + rl) * (KB / 32) + kcol / 32];
     } else {
-      const uint8_t* mp = p.partial_masks + (size_t(pid) * QB + q_local0 + rl) * KB + 32 * kg;
+      const uint8_t* mp = p.partial_masks + (size_t(pid) * QB + q_local0 + rl) * KB + kcol;
       roww = bwd_pack32(*reinterpret_cast<const u32x4_t*>(mp), *reinterpret_cast<const u32x4_t*>(mp + 16));
     }
     uint32_t col = 0;
@@ -1031,42 +1211,58 @@ __global__ void __launch_bounds__(KB * 4, D == 128 ? 2 : 4) bwd_dkdv_kernel(cons
   // windows: the steps of a window are worked off completely before the next one is scanned.
   auto run = [&](auto role_c) {
     constexpr bool GRAD = decltype(role_c)::value;
-    const BwdStepInfo none = {0, kMasked, -1, 0, 0, false};
+    // A round is G steps, one of each group.  A window's last round may have fewer: the next
+    // window's first one goes on with the group whose turn it is.
+    int turn = 0;
     for (;;) {
-      BwdStepInfo prev = none, cur = next_step();
+      const int rounds = (n_steps + turn + G - 1) / G;
+      auto index_of = [&](int j) { return j * G + group - turn; };  // of this group's step of round j
+      auto request = [&](int j) {
+        const int t = index_of(j);
+        return sSteps[t < 0 || t >= n_steps ? 0 : t];
+      };
+      auto receive = [&](i32x2_t e, int j) {
+        const int t = index_of(j);
+        const int e0 = e[0], e1 = e[1];
+        return Step{__builtin_amdgcn_readfirstlane(e0), __builtin_amdgcn_readfirstlane(e1), t >= 0 && t < n_steps};
+      };
+      Step prev = {0, kMasked, false}, cur = receive(request(0), 0);
+      i32x2_t coming = request(1);
       int s_prev = 2, s_cur = 0, s_nxt = 1;  // tile sets of steps j - 1, j, j + 1
       if (cur.valid) {
         if constexpr (!GRAD) load_q(cur, 0); else load_do(cur, 0);
       }
-      for (int j = 0; cur.valid || prev.valid; ++j) {
-        const BwdStepInfo nxt = cur.valid ? next_step() : none;
+      const int iterations = rounds > 0 ? rounds + 1 : 0;
+      for (int j = 0; j < iterations; ++j) {
+        const Step nxt = receive(coming, j + 1);
+        coming = request(j + 2);
         // mask words of this lane's key: bit i of word u = query row row0 + 32 u + i attends it
         uint32_t kw[NSUB];
-  #pragma unroll
+#pragma unroll
         for (int u = 0; u < NSUB; ++u) kw[u] = 0;
+        const int mode = cur.info & 3;
+        // (wave-uniform) a FULL step whose keys are all inside the sequence needs no mask
+        const bool masked = CAP || !(mode == kFull && key_wave_min + 32 <= p.seqlen);
         if constexpr (!GRAD) {
-          if (cur.valid) {
-  #pragma unroll
+          if (cur.valid && masked) {
+#pragma unroll
             for (int u = 0; u < NSUB; ++u) {
               uint32_t m = key_live ? 0xffffffffu : 0u;
-              if (cur.mode == kCausal) {  // rows at or after the key
+              if (mode == kCausal) {  // rows at or after the key
                 const int n = key - (cur.row0 + 32 * u);
                 m &= n <= 0 ? 0xffffffffu : (n >= 32 ? 0u : (0xffffffffu << (n & 31)));
               }
-              if (cur.mode == kPartial) m &= partial_column(cur.pid, cur.row0 + 32 * u - cur.blk * QB);
+              if (mode == kPartial) m &= partial_column(cur.info >> 2, (cur.row0 & (QB - 1)) + 32 * u);
               kw[u] = m >> (4 * g);
             }
           }
         }
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the tile this wave loaded has landed
+        wait_loads();  // the tile this wave loaded has landed
         __syncthreads();  // ... everybody's have; the hand-over of step j - 1 is written; the set
                           // about to be overwritten (step j - 2) is no longer read
         if constexpr (!GRAD) {
           if (nxt.valid) load_q(nxt, s_nxt);
-          if (cur.valid) {
-            // (wave-uniform) a FULL step whose keys are all inside the sequence needs no mask
-            weight_step(s_cur, j & 1, kw, !(cur.mode == kFull && key_wave_min + 32 <= p.seqlen));
-          }
+          if (cur.valid) weight_step(s_cur, j & 1, kw, masked);
         } else {
           if (nxt.valid) load_do(nxt, s_nxt);
           if (prev.valid) grad_step(s_prev, (j + 1) & 1);
@@ -1079,13 +1275,20 @@ __global__ void __launch_bounds__(KB * 4, D == 128 ? 2 : 4) bwd_dkdv_kernel(cons
         s_nxt = t3;
       }
       if (__builtin_expect(win_end >= n_words, 1)) break;
-      // (rare) more words of metadata than the bitmap holds: the next window
+      // (rare) more words of metadata, or matches, than LDS holds: the next window
+      turn = (turn + n_steps) % G;
       win_base = win_end;
       win_end = win_base + win_words < n_words ? win_base + win_words : n_words;
       scan_window(IntC<1>{}, win_base, win_end);
-      gw = win_base - 1;
+      n_steps = build_table(win_base, win_end);
     }
     __syncthreads();
+    if constexpr (G > 1) {
+      const size_t row = slab + size_t(key < p.S ? key : 0) * D;
+      bwd_merge_store<BF16, D, G, 2 * NKG>(acc, GRAD ? p.scale : 1.f, lds_raw, group, w, lane,
+                                           (GRAD ? p.dk : p.dv) + row, key < p.S);
+      return;
+    }
     uint16_t* stage = lds16 + size_t(w) * 32 * D;
     if constexpr (!GRAD) {
       bwd_store_rows<BF16, D>(acc, 1.f, stage, p.dv + slab, key_wave_min, p.S, lane);
@@ -1100,39 +1303,82 @@ __global__ void __launch_bounds__(KB * 4, D == 128 ? 2 : 4) bwd_dkdv_kernel(cons
   }
 }
 
-constexpr int kBwdMaxDevices = 64;
-
 template <bool BF16, bool CAP, int D, int QB, int KB>
-int launch_bwd_cap(const BwdParams& p, hipStream_t stream) {
-  using TQ = BwdDqTraits<D, QB>;
-  using TK = BwdDkdvTraits<D, KB>;
-  auto kq = bwd_dq_kernel<BF16, CAP, D, QB, KB>;
-  auto kk = bwd_dkdv_kernel<BF16, CAP, D, QB, KB>;
-  static std::atomic<bool> lds_limit_set[kBwdMaxDevices];
+__global__ void __launch_bounds__(KB * 4, D == 128 ? 2 : 4) bwd_dkdv_kernel(const BwdParams p) {
+  bwd_dkdv_walk<BwdDkdvBlockShape<BF16, CAP, D, QB, KB>>(p);
+}
+// The query rows of a KV block shared by the groups of a workgroup.
+template <bool BF16, bool CAP, int D, int NKG, int G>
+__global__ void __launch_bounds__(NKG * 128 * G, D == 128 ? 2 : 4) bwd_dkdv_split(const BwdParams p) {
+  bwd_dkdv_walk<BwdDkdvShape<BF16, CAP, D, 0, 0, NKG, G, 32>>(p);
+}
+
+// Launch of one backward kernel; its dynamic-LDS limit is raised once per device.
+template <auto Kernel>
+int launch_bwd_kernel(const BwdParams& p, int tiles, int threads, size_t lds, size_t max_lds, hipStream_t stream) {
+  static std::atomic<bool> lds_limit_set[kMaxDevices];
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return int(e);
-  const bool cached = dev >= 0 && dev < kBwdMaxDevices;
+  const bool cached = dev >= 0 && dev < kMaxDevices;
   if (!cached || !lds_limit_set[dev].load(std::memory_order_acquire)) {
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(kq), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            int(TQ::kLdsBytes));
-    if (e != hipSuccess) return int(e);
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(kk), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            int(TK::kLdsBytes));
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(Kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            int(max_lds));
     if (e != hipSuccess) return int(e);
     if (cached) lds_limit_set[dev].store(true, std::memory_order_release);
   }
-  const unsigned slabs_per_xcd = unsigned(p.n_slabs + p.n_xcd - 1) / unsigned(p.n_xcd);
+  const unsigned slabs_per_xcd = unsigned(p.n_slabs * p.parts + p.n_xcd - 1) / unsigned(p.n_xcd);
+  const dim3 grid(unsigned(p.n_xcd) * slabs_per_xcd * (unsigned(tiles + p.parts - 1) / unsigned(p.parts)));
   BwdParams params = p;
   void* args[] = {&params};
+  return int(hipLaunchKernel(reinterpret_cast<const void*>(Kernel), grid, dim3(threads), args, lds, stream));
+}
+
+template <bool BF16, bool CAP, int D, int QB, int KB>
+int launch_dq(const BwdParams& p, hipStream_t stream) {
+  using Shape = BwdDqShape<BF16, CAP, D, QB, KB, QB, 1, 64>;
+  return launch_bwd_kernel<bwd_dq_kernel<BF16, CAP, D, QB, KB>>(p, p.Tq, Shape::kThreads, Shape::kLdsBytes,
+                                                                Shape::kLdsBytes, stream);
+}
+template <bool BF16, bool CAP, int D, int QT, int KG, int STEP>
+int launch_dq_ksplit(const BwdParams& p, hipStream_t stream) {
+  using Shape = BwdDqShape<BF16, CAP, D, 0, 0, QT, KG, STEP>;
+  return launch_bwd_kernel<bwd_dq_ksplit<BF16, CAP, D, QT, KG, STEP>>(p, p.Tq * (p.QB / QT), Shape::kThreads,
+                                                                      Shape::kLdsBytes, Shape::kLdsBytes, stream);
+}
+
+template <class Shape, auto Kernel>
+int launch_dkdv_shape(const BwdParams& p, int tiles, hipStream_t stream) {
   const size_t n_words = size_t(p.Tq) * size_t((p.max_blocks + 63) / 64);
-  const size_t dkdv_lds = TK::lds_bytes(n_words < size_t(TK::kMaxBitmapWords) ? n_words : size_t(TK::kMaxBitmapWords));
-  const dim3 dkdv_grid(unsigned(p.n_xcd) * slabs_per_xcd * unsigned(p.Tk));
-  const dim3 dq_grid(unsigned(p.n_xcd) * slabs_per_xcd * unsigned(p.Tq));
-  e = hipLaunchKernel(reinterpret_cast<const void*>(kq), dq_grid, dim3(TQ::kThreads), args, TQ::kLdsBytes, stream);
-  if (e != hipSuccess) return int(e);
-  e = hipLaunchKernel(reinterpret_cast<const void*>(kk), dkdv_grid, dim3(TK::kThreads), args, dkdv_lds, stream);
-  return int(e);
+  const size_t lds = Shape::lds_bytes(n_words < size_t(Shape::kMaxBitmapWords) ? int(n_words) : Shape::kMaxBitmapWords,
+                                      p.QB / Shape::kStep);
+  return launch_bwd_kernel<Kernel>(p, tiles, Shape::kThreads, lds, Shape::kLdsBytes, stream);
+}
+template <bool BF16, bool CAP, int D, int QB, int KB>
+int launch_dkdv(const BwdParams& p, hipStream_t stream) {
+  return launch_dkdv_shape<BwdDkdvBlockShape<BF16, CAP, D, QB, KB>, bwd_dkdv_kernel<BF16, CAP, D, QB, KB>>(p, p.Tk,
+                                                                                                          stream);
+}
+template <bool BF16, bool CAP, int D, int NKG, int G>
+int launch_dkdv_split(const BwdParams& p, hipStream_t stream) {
+  return launch_dkdv_shape<BwdDkdvShape<BF16, CAP, D, 0, 0, NKG, G, 32>, bwd_dkdv_split<BF16, CAP, D, NKG, G>>(
+      p, p.Tk * (p.KB / (32 * NKG)), stream);
+}
+
+template <bool BF16, bool CAP, int D, int QB, int KB>
+int launch_bwd_cap(const BwdParams& p, hipStream_t stream) {
+  int e;
+  switch (p.dq_split) {
+    case FwdSplit::kRows32x4: e = launch_dq_ksplit<BF16, CAP, D, 32, 4, 32>(p, stream); break;
+    case FwdSplit::kRows64x2: e = launch_dq_ksplit<BF16, CAP, D, 64, 2, 64>(p, stream); break;
+    default: e = launch_dq<BF16, CAP, D, QB, KB>(p, stream); break;
+  }
+  if (e != 0) return e;
+  if constexpr (D != 128) {
+    if (p.dkdv_split == DkdvSplit::kKeys32x4) return launch_dkdv_split<BF16, CAP, D, 1, 4>(p, stream);
+  }
+  if (p.dkdv_split == DkdvSplit::kKeys64x2) return launch_dkdv_split<BF16, CAP, D, 2, 2>(p, stream);
+  return launch_dkdv<BF16, CAP, D, QB, KB>(p, stream);
 }
 
 // The soft-capped instances are separate kernels: the extra arithmetic per score would

@@ -346,12 +346,18 @@ int backward(const void* q, const void* k, const void* v, const void* o, const v
   p.seqlen = seqlen_orig < S_pad ? seqlen_orig : S_pad;
   p.H = H;
   p.n_slabs = B * H;
+  p.QB = QB;
+  p.KB = KB;
+  const long long rows32 = (long long)B * H * Tq * (QB / 32);
+  p.dq_split = bwd_choose_dq_split(D, QB, rows32, Tq * QB);
+  p.dkdv_split = bwd_choose_dkdv_split(D, KB, softcap > 0.f, rows32, Tq * QB);
   DeviceTopology topo;
   if (const int e = query_topology(&topo)) {
     g_last_hip_error = e;
     return OMNI_ATTN_ERR_LAUNCH;
   }
   p.n_xcd = topo.n_xcd;
+  p.parts = slab_parts(p.n_slabs, p.n_xcd);
   p.scale = float(1.0 / std::sqrt(double(D)));
   p.sl2 = float(1.4426950408889634 / std::sqrt(double(D)));
   p.softcap = softcap;

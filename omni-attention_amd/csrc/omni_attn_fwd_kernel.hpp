@@ -313,11 +313,12 @@ __device__ __forceinline__ void buffer_to_lds_b32(i32x4_t rsrc, uint32_t lane_of
         "s"(__builtin_amdgcn_readfirstlane(uniform_off))
       : "memory", "m0");
 }
-// Waits until at most N of this wave's vector-memory operations are outstanding (they complete in order).
-template <int N>
+// Waits until this wave's vector-memory operations are complete.  (The builtin, not inline asm: the
+// compiler then knows that its own loads have landed too, and does not wait for them again behind
+// tile loads that have been issued since.)
 __device__ __forceinline__ void wait_loads() {
-  static_assert(N < 64, "six bits");
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  asm volatile("" ::: "memory");
 }
 // Block-mask metadata is read-only for the whole launch and every read of it is
 // wave-uniform: reading it through the constant address space makes these scalar loads
@@ -598,7 +599,7 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
     }
   };
   auto stage_mask_bits = [&]() {
-    wait_loads<0>();  // the bytes have landed
+    wait_loads();  // the bytes have landed
     // word NTL * row + h of the wave's 32 rows; with one word per row the upper half-wave
     // repeats the lower one
     const int wi = lane % (32 * NTL);
@@ -758,9 +759,7 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
     constexpr int NPV = decltype(first_c)::value != 0 ? 0 : NPV_ALL;
     constexpr int NS = NQK + NPV;  // slots
     constexpr int LSP = (NS / 2) / NL > 0 ? (NS / 2) / NL : 1;  // slots between tile loads
-    // ... and no V tile to load: V(0) is on its way already
-    constexpr int L0 = decltype(first_c)::value != 0 ? NCH : 0, NLB = NL - L0;
-    constexpr int LPS = (NLB * LSP + NS - 1) / NS;              // loads per slot that has some
+    constexpr int LPS = (NL * LSP + NS - 1) / NS;               // loads per slot that has some
     constexpr int PF = PF_ALL < NS ? PF_ALL : NS;
     constexpr int NMX = 2 * NTL;          // max chunks of 8 scores
     constexpr int NPR = 8 * NTL;          // pairs of exponentials
@@ -843,7 +842,7 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
       if constexpr (j + PF < NS) opq[j % PF] = operand(j + PF);
       static_for<LPS>([&](auto lc) {
         constexpr int n = (j / LSP) * LPS + decltype(lc)::value;
-        if constexpr (j % LSP == 0 && n < NLB) issue_load(L0 + n, SET, k_row0, v_row0);
+        if constexpr (j % LSP == 0 && n < NL) issue_load(n, SET, k_row0, v_row0);
       });
       constexpr int u_lo = j * NV / NS, u_hi = (j + 1) * NV / NS;
       static_for<u_hi - u_lo>([&](auto dc) { vector_chunk(IntC<u_lo + decltype(dc)::value>{}); });
@@ -855,7 +854,7 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   // The tiles (and packed mask words) that were requested an iteration ago have landed, for
   // every wave that reads them.
   auto step_barrier = [&]() {
-    wait_loads<0>();
+    wait_loads();
     if constexpr (!LONE) __syncthreads();
   };
   // ---- the walk -------------------------------------------------------------------------
@@ -864,28 +863,26 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
     cur = step_info(0);
     nxt = step_info(1);
     nn = step_info(2);
-    // Prologue: the mask of step 0, K(0), K(1), V(0); the first products wait for K(0) only.
+    // Prologue: K(0) and K(1).
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      issue_load(NCH + i, 0, cur.row0, 0);
+      issue_load(NCH + i, 1, nxt.row0, 0);
+    }
     if (cur.mode == kPartial) {
       if (packed_tiles) {
         prefetch_mask_words(0, cur);
       } else {
         prefetch_mask_bytes(0, cur);
+        stage_mask_bits();
       }
     }
-#pragma unroll
-    for (int i = 0; i < NCH; ++i) issue_load(NCH + i, 0, cur.row0, 0);
-#pragma unroll
-    for (int i = 0; i < NCH; ++i) issue_load(NCH + i, 1, nxt.row0, 0);
-#pragma unroll
-    for (int i = 0; i < NCH; ++i) issue_load(i, 0, 0, cur.row0);
-    wait_loads<2 * NCH>();
-    if constexpr (!LONE) __syncthreads();
+    step_barrier();
 #pragma unroll
     for (int s = 0; s < KS; ++s)
 #pragma unroll
       for (int t = 0; t < NTL; ++t)
         st[0][t] = mfma_32x32x16<BF16>(k_frag(sK, s, t), qf[s], s == 0 ? zero16 : st[0][t]);
-    if (cur.mode == kPartial && !packed_tiles) stage_mask_bits();
   }
 
   auto iteration = [&](auto set_c, auto first_c, int it) {

@@ -44,3 +44,23 @@ def test_split_walks(dtype, D, QB, KB, H, S, gpu_device):
             compare_with_oracle(o, lse, ro, rl, dtype, f"seqlen {seqlen}, {'bytes' if bits is None else 'bits'}")
             outs.append((o, lse))
         assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
+@pytest.mark.parametrize("softcap", [0.0, 5.0])
+@pytest.mark.parametrize("D,QB,KB,H,S", [
+    (32, 64, 128, 9, 128), (64, 128, 64, 1, 4480), (128, 128, 128, 3, 384), (64, 64, 64, 5, 192),  # 32 rows / keys, 4 groups
+    (32, 128, 128, 40, 512), (64, 64, 128, 36, 512), (128, 64, 64, 20, 512), (128, 128, 64, 20, 512),  # 64 rows / keys, 2
+    (64, 128, 128, 18, 2048)])
+def test_split_walks_backward(softcap, D, QB, KB, H, S, gpu_device):
+    """The backward of such problems: gradients against autograd through the dense oracle, at the bars of
+    the other backward tests; rows and keys behind the sequence get zeros."""
+    from oracle.dense_oracle import attention_dense_grads
+    from test_gpu_backward import check_grads, run_fwd_bwd
+    dtype = torch.bfloat16 if D == 128 else torch.float16
+    gen = torch.Generator().manual_seed(D + QB + S + 1)
+    q, k, v, dout = (torch.randn(1, H, S, D, generator=gen).to(dtype) for _ in range(4))
+    nb, idx, tys, pidx, pm = random_block_metadata(gen, 1, H, S // QB, S // KB, QB, KB, p_empty=0.15, shuffle=True)
+    for seqlen in (S, S - QB - 13 if S > QB else S - 13):
+        got = run_fwd_bwd(q, k, v, dout, nb, idx, tys, QB, KB, seqlen, pidx, pm, device=gpu_device, softcap=softcap)
+        dense = dense_mask_from_blocks(nb, idx, tys, QB, KB, S, S, pidx, pm, seqlen_orig=seqlen)
+        check_grads(got[:3], attention_dense_grads(q, k, v, dense, dout, softcap=softcap), dtype, f"seqlen {seqlen}")

@@ -7,21 +7,23 @@
 // cores, at the precision of a scalar kernel: products of 16-bit operands summed in fp32, and
 // weights that enter the second product with (at least) 22 significant bits.
 //
-// One workgroup owns up to 32 query rows of one query block; its four waves share the keys of the
+// One workgroup owns up to 32 query rows of one query block; its waves share the keys of the
 // block's list: the listed keys are one sequence of positions, slot * KB + offset; step n is the
 // positions 32 n .. 32 n + 31 (of one block or of several, for any KB) and wave w takes the steps
-// w, w + 4, ...  A wave has its own running maximum, sum and O^T accumulators; they are merged
+// w, w + waves, ...  A wave has its own running maximum, sum and O^T accumulators; they are merged
 // through LDS at the end.  No workgroup barrier until then.
 //
 // S^T = K.Q^T and O^T = V^T.P^T with v_mfma_f32_32x32x16 as in the tuned forward: a lane owns a query
-// row.  K fragments come straight from global memory into registers (a step's rows are used by one
-// wave only, so LDS would share nothing), V goes through a wave-private LDS tile for its transposed
-// read.  A weight is a sum of 16-bit parts with one product each: two for fp16 (scaled by 2^14
+// row; the K and V rows of a step go to tiles of the wave in LDS, straight from global memory where rows
+// lie on 16-byte boundaries (the rows of the next step are requested as soon as the products have read
+// a tile).  A weight is a sum of 16-bit parts with one product each: two for fp16 (scaled by 2^8
 // first, so that small weights stay out of the subnormals), three for bf16.
 //
-// Bound by the latency of a step (loads, two matrix chains, the softmax and the split of the weights
-// on the vector pipe) times a quarter of the steps of the longest list.  B=1 H=8 S=2048 D=96 fp16,
-// causal in 32x32 blocks: 33 us; one wave per row with vector arithmetic and two passes took 1938 us.
+// Bound by the latency of a step (two matrix chains, the softmax and the split of the weights on the
+// vector pipe) times the steps of the longest list over the waves; from 192 columns on by LDS (a step
+// of 32 rows reads each K and V byte once for 32 query rows).  B=1 H=8 S=2048 D=96 fp16, causal in 32x32
+// blocks: 24 us; with K fragments loaded straight into registers (32 rows x 32 bytes per load) and
+// masks evaluated on every step 34 us; one wave per row with vector arithmetic 1938 us.
 #include "../../include/omni_attn_gfx950.h"
 
 #include <hip/hip_runtime.h>
@@ -52,7 +54,6 @@ typedef __attribute__((ext_vector_type(2))) uint32_t u32x2_t;
 
 enum : int { kMasked = 0, kCausal = 1, kFull = 2, kPartial = 3 };
 constexpr int kMaxD = 256;
-constexpr int kWaves = 4;
 
 struct GenericParams {
   const uint16_t* q;
@@ -69,10 +70,11 @@ struct GenericParams {
   int num_partial;
   int S, D, H, Tq, Tk, max_blocks, QB, KB, seqlen;
   int kb_eff;         // keys of a block that can be inside the sequence: min(KB, S)
-  int adv_slot, adv_off;  // 32 kWaves positions = adv_slot blocks of kb_eff keys + adv_off keys
+  int adv_slot, adv_off;  // 32 positions per wave = adv_slot blocks of kb_eff keys + adv_off keys
   int q_tiles;        // 32-row tiles per query block
   int o_vec;          // rows of o start on 8-byte boundaries and D is a multiple of 8
   int mask_words;     // four keys of a tile row may be read as one 32-bit word
+  int whole;          // a step never crosses a block (blocks of 32 n keys, mask_words)
   unsigned n_slabs;   // B * H
   float scale, sl2, softcap;
 };
@@ -83,11 +85,15 @@ struct GenericParams {
 // the repeated columns of the result are not stored.
 __device__ __forceinline__ int chunk_start(int d0, int D) { return d0 + 8 <= D ? d0 : D - 8; }
 
-// The chunk of `row` at column d0.  SMALL: head dimensions below 8, zeros behind the row.
-template <bool SMALL>
+// How rows are read: straight to LDS (rows of k and v on 16-byte boundaries, D a multiple of 8), by
+// 16-byte loads at any alignment, or element by element (head dimensions below 8).
+enum class Rows : int { kDirect, kWide, kSmall };
+
+// The chunk of `row` at column d0 (kSmall: zeros behind the row).
+template <Rows R>
 __device__ __forceinline__ u32x4_t load8(const uint16_t* row, int d0, int D) {
   u32x4_t r;
-  if constexpr (SMALL) {
+  if constexpr (R == Rows::kSmall) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int d = d0 + 2 * i;
@@ -98,6 +104,33 @@ __device__ __forceinline__ u32x4_t load8(const uint16_t* row, int d0, int D) {
     __builtin_memcpy(&r, row + chunk_start(d0, D), 16);
   }
   return r;
+}
+
+// 16 bytes per lane from a buffer straight into LDS, at lds_base + 16 * lane; a lane whose offset lies
+// beyond the buffer writes zeros.  (Inline asm, so that reads of other tiles are not ordered behind it;
+// completion is waited for explicitly.)
+__device__ __forceinline__ void buffer_to_lds(i32x4_t rsrc, uint32_t lane_off, uint32_t uniform_off,
+                                              uint32_t lds_base) {
+  i32x4_t r;
+  r[0] = __builtin_amdgcn_readfirstlane(rsrc[0]);
+  r[1] = __builtin_amdgcn_readfirstlane(rsrc[1]);
+  r[2] = __builtin_amdgcn_readfirstlane(rsrc[2]);
+  r[3] = __builtin_amdgcn_readfirstlane(rsrc[3]);
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "buffer_load_dwordx4 %1, %2, %3 offen lds"
+      :
+      : "s"(__builtin_amdgcn_readfirstlane(lds_base)), "v"(lane_off), "s"(r),
+        "s"(__builtin_amdgcn_readfirstlane(uniform_off))
+      : "memory", "m0");
+}
+// At most N vector-memory operations of this wave are outstanding.
+template <int N>
+__device__ __forceinline__ void wait_but() {
+  static_assert(N < 64, "six bits");
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+  asm volatile("" ::: "memory");
 }
 
 template <bool BF16>
@@ -111,20 +144,20 @@ __device__ __forceinline__ f32x16_t mfma(u32x4_t a, u32x4_t b, f32x16_t c) {
   }
 }
 
-// One 16-bit part of a pair of values; the values become what is left of them (exact).
+// One 16-bit part of a pair of non-negative values, cut off towards zero; the values become what is left
+// of them (exact: after three bf16 parts nothing is left).
 template <bool BF16>
 __device__ __forceinline__ uint32_t split_part(float& lo, float& hi) {
   if constexpr (BF16) {
-    const __bf16 a = (__bf16)lo, b = (__bf16)hi;
-    lo -= float(a);
-    hi -= float(b);
-    const bf16x2_t v = {a, b};
-    return __builtin_bit_cast(uint32_t, v);
+    const uint32_t a = __builtin_bit_cast(uint32_t, lo), b = __builtin_bit_cast(uint32_t, hi);
+    lo -= __builtin_bit_cast(float, a & 0xffff0000u);
+    hi -= __builtin_bit_cast(float, b & 0xffff0000u);
+    return __builtin_amdgcn_perm(b, a, 0x07060302u);  // upper halves of both
   } else {
-    const _Float16 a = (_Float16)lo, b = (_Float16)hi;
-    lo -= float(a);
-    hi -= float(b);
-    const f16x2_t v = {a, b};
+    const auto v = __builtin_amdgcn_cvt_pkrtz(lo, hi);
+    const f16x2_t h = __builtin_bit_cast(f16x2_t, v);
+    lo = __builtin_fmaf(float(h[0]), -1.f, lo);
+    hi = __builtin_fmaf(float(h[1]), -1.f, hi);
     return __builtin_bit_cast(uint32_t, v);
   }
 }
@@ -142,31 +175,34 @@ __device__ __forceinline__ uint16_t from_float(float x) {
 // The other half-wave's value (lane ^ 32).
 __device__ __forceinline__ float other_half(float x) { return __shfl_xor(x, 32, 64); }
 
-// DT: 32-column tiles of the head dimension.
-template <int DT>
+// DT: 32-column tiles of the head dimension; NW: waves.
+template <int DT, int NW>
 struct GenericTraits {
-  static constexpr int kRowBytes = 64 * (DT | 1);  // an odd multiple of 64: four consecutive rows
-                                                   // of a transposed read lie on different banks
-  static constexpr int kVBytes = 32 * kRowBytes;
-  static constexpr int kGroup = DT < kWaves ? DT : kWaves;  // output tiles merged per pass
-  static constexpr size_t kMergeBytes = size_t(kWaves) * kGroup * 4096;
-  static constexpr size_t kTiles = size_t(kWaves) * kVBytes > kMergeBytes ? size_t(kWaves) * kVBytes : kMergeBytes;
-  // From 128 columns on Q lives in LDS (shared by the waves) instead of in registers, of which the
-  // rows of the next step and the accumulators leave too few.
-  static constexpr bool kQInLds = DT >= 4;
-  static constexpr size_t kQBytes = kQInLds ? size_t(kVBytes) : 0;
+  static constexpr int kRowBytes = 64 * DT;
+  static constexpr int kTileBytes = 32 * kRowBytes;
+  static constexpr int kGroup = DT < NW ? DT : NW;  // output tiles merged per pass
+  static constexpr size_t kMergeBytes = size_t(NW) * kGroup * 4096;
+  // K and V of every wave; the merge overlaps them
+  static constexpr size_t kTiles = size_t(NW) * 2 * kTileBytes > kMergeBytes ? size_t(NW) * 2 * kTileBytes : kMergeBytes;
+  // With 97 - 128 columns (eight waves, 256 registers each) and from 193 on Q lives in LDS, shared by the waves.
+  static constexpr bool kQInLds = DT == 4 || DT >= 7;
+  static constexpr size_t kQBytes = kQInLds ? size_t(kTileBytes) : 0;
   // behind the tiles: Q; per wave, compare key, offset inside the block and tile of 32 keys; and
   // the maximum and sum of 32 rows
-  static constexpr size_t kLdsBytes = kTiles + kQBytes + kWaves * (32 * 12 + 32 * 8);
+  static constexpr size_t kLdsBytes = kTiles + kQBytes + NW * (32 * 12 + 32 * 8);
 };
 
-template <bool BF16, int DT, bool SMALL>
-__global__ void __launch_bounds__(64 * kWaves, DT <= 4 ? 2 : 1) fwd_generic_kernel(const GenericParams p) {
-  using Traits = GenericTraits<DT>;
+template <bool BF16, int DT, int NW, Rows R>
+__global__ void __launch_bounds__(64 * NW, (DT <= 4 || NW == 8) ? 2 : 1) fwd_generic_kernel(const GenericParams p) {
+  using Traits = GenericTraits<DT, NW>;
   constexpr int KS = 2 * DT;
-  constexpr int RS = Traits::kRowBytes;
+  constexpr int C = 4 * DT;     // 16-byte chunks of a tile row
+  constexpr int NLD = 2 * DT;   // chunks of a tile per lane
   constexpr int PARTS = BF16 ? 3 : 2;
-  constexpr float kShift = BF16 ? 0.f : 14.f;  // log2 of the factor on the weights
+  constexpr float kShift = BF16 ? 0.f : 8.f;  // log2 of the factor on the weights
+  // The reference point of the exponentials follows the running maximum when that is more than this
+  // ahead (log2): weights stay below 2^(kSlack + kShift), and the sums are rarely rescaled.
+  constexpr float kSlack = 6.f;
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
 
   const unsigned wg = blockIdx.x;
@@ -183,12 +219,13 @@ __global__ void __launch_bounds__(64 * kWaves, DT <= 4 ? 2 : 1) fwd_generic_kern
   const bool q_here = q_local < p.QB && q_idx < p.S;  // a row of this tile
   const bool q_live = q_here && q_idx < p.seqlen;
 
-  uint8_t* const sV = lds + size_t(w) * Traits::kVBytes;
+  uint8_t* const sK = lds + size_t(w) * 2 * Traits::kTileBytes;
+  uint8_t* const sV = sK + Traits::kTileBytes;
   uint8_t* const sQ = lds + Traits::kTiles;
   int32_t* const sKey = reinterpret_cast<int32_t*>(lds + Traits::kTiles + Traits::kQBytes) + w * 96;
   int32_t* const sOff = sKey + 32;
   int32_t* const sPid = sKey + 64;
-  float* const sStat = reinterpret_cast<float*>(lds + Traits::kTiles + Traits::kQBytes + kWaves * 384);  // [2][kWaves][32]
+  float* const sStat = reinterpret_cast<float*>(lds + Traits::kTiles + Traits::kQBytes + NW * 384);  // [2][NW][32]
 
   const int64_t b = int64_t(bh) / p.H, h = int64_t(bh) - b * p.H;
   const uint16_t* const q_slab = p.q + b * p.q_at.batch + h * p.q_at.head;
@@ -196,24 +233,46 @@ __global__ void __launch_bounds__(64 * kWaves, DT <= 4 ? 2 : 1) fwd_generic_kern
   const uint16_t* const v_slab = p.v + b * p.v_at.batch + h * p.v_at.head;
   const size_t mrow = bh * p.Tq + qb;
   const size_t moff = mrow * p.max_blocks;
+  const bool has_partial = p.partial_idx != nullptr && p.partial_masks != nullptr;
+
+  // Block metadata in registers: lane i holds slot 64 chunk + i of the list (block index, and mode in
+  // the low two bits with the tile index above).
+  int32_t mv_idx = 0, mv_info = kMasked, chunk_at = 0;
+  auto info_of = [&](int type, int pid) {
+    int mode = (type == kCausal || type == kFull || type == kPartial) ? type : int(kMasked);
+    if (mode == kPartial && (pid < 0 || pid >= p.num_partial)) mode = kMasked;  // attn_naive.cu:119-131
+    return (mode == kPartial ? pid << 2 : 0) | mode;
+  };
+  auto load_chunk = [&](int chunk) {
+    const int j = chunk * 64 + lane;
+    const size_t o = moff + size_t(j < p.max_blocks ? j : 0);
+    mv_idx = p.kv_indices[o];
+    mv_info = info_of(p.types[o], has_partial ? p.partial_idx[o] : -1);
+    chunk_at = chunk;
+  };
+  load_chunk(0);
   int nb = p.kv_num_blocks[mrow];
   nb = nb < 0 ? 0 : (nb > p.max_blocks ? p.max_blocks : nb);
   if (qb * p.QB + row0 >= p.seqlen) nb = 0;  // only padding rows: zeros (attn_naive.cu:64-72)
-  const bool has_partial = p.partial_idx != nullptr && p.partial_masks != nullptr;
 
-  // chunk (16 bytes) `ch` of row r of a tile: XORed with bits 2 and 3 of the row
-  auto tile_at = [](int r, int ch) { return r * RS + ((ch ^ ((r >> 2) & 3)) * 16); };
+  // Chunk (16 bytes) `ch` of row r of a tile.  The XOR keeps 16 consecutive rows of one chunk (K, Q) and
+  // four consecutive chunks of four consecutive rows (transposed reads of V) on different banks.
+  auto swizzle = [](int r) {
+    const int low = (r >> 2) & 3;
+    return DT % 2 == 1 ? low : (DT % 4 == 2 ? (low | ((r >> 1) & 1) << 2) : (low | (r & 3) << 2));
+  };
+  auto tile_at = [&](int r, int ch) { return r * Traits::kRowBytes + (ch ^ swizzle(r)) * 16; };
   // Q as B operand: lane holds Q[row][16 s + 8 g .. +7]
   u32x4_t qf[Traits::kQInLds ? 1 : KS];
   {
     const uint16_t* qrow = q_slab + int64_t(q_live ? q_idx : 0) * p.q_at.row;
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
-      if (Traits::kQInLds && s % kWaves != w) continue;
+      if (Traits::kQInLds && s % NW != w) continue;
       const int d0 = 16 * s + 8 * g;
-      u32x4_t x = load8<SMALL>(qrow, d0, p.D);
+      u32x4_t x = load8<R == Rows::kDirect ? Rows::kWide : R>(qrow, d0, p.D);
       if (!q_live || d0 >= p.D) x = u32x4_t{0u, 0u, 0u, 0u};
-      if (!SMALL && d0 < p.D) {
+      if (R != Rows::kSmall && d0 < p.D) {
         const int repeats = d0 - chunk_start(d0, p.D);  // leading columns that the chunk before has
 #pragma unroll
         for (int i = 0; i < 4; ++i)
@@ -235,57 +294,118 @@ __global__ void __launch_bounds__(64 * kWaves, DT <= 4 ? 2 : 1) fwd_generic_kern
     }
   };
 
-  // Position of this lane's key (lanes c and c + 32 follow the same key) in the current step, and
-  // the block metadata of the step that is loaded next.
+  // Position of this lane's key (lanes c and c + 32 follow the same key) in the wave's next step.
   int slot, off;
   {
     const int pos = 32 * w + c;
     slot = pos / p.kb_eff;
     off = pos - slot * p.kb_eff;
   }
-  int32_t m_idx = 0, m_type = kMasked, m_pid = -1;
-  auto load_meta = [&]() {
-    const bool in = slot < nb;
-    const size_t o = moff + size_t(in ? slot : 0);
-    m_idx = p.kv_indices[o];
-    m_type = in ? p.types[o] : int32_t(kMasked);
-    m_pid = has_partial ? p.partial_idx[o] : -1;
-  };
-  // The key of this lane in the step whose metadata has just been loaded.  `cmp`: the key is
-  // allowed for the query rows >= cmp (all of them for FULL and PARTIAL, none for a key that does
-  // not exist, lies beyond the sequence or belongs to a skipped slot).
+  // The key of this lane.  `cmp`: the key is allowed for the query rows >= cmp (all of them for FULL and
+  // PARTIAL, none for a key that does not exist, lies beyond the sequence or belongs to a skipped slot).
   struct Key {
     int row, cmp, off, pid;
-    bool live;
   };
-  auto resolve = [&]() {
-    Key k;
-    const int kvb = m_idx < 0 ? 0 : (m_idx >= p.Tk ? p.Tk - 1 : m_idx);
-    int mode = m_type;
-    if (mode == kPartial && (m_pid < 0 || m_pid >= p.num_partial)) mode = kMasked;  // :119-131
+  auto next_key = [&]() {
+    const int first = __builtin_amdgcn_readfirstlane(slot), last = __builtin_amdgcn_readlane(slot, 31);
+    if ((first >> 6) != chunk_at) load_chunk(first >> 6);
+    int idx = __shfl(mv_idx, slot & 63, 64), info = __shfl(mv_info, slot & 63, 64);
+    if ((last >> 6) != (first >> 6) && (slot >> 6) != (first >> 6)) {  // the step runs into the next chunk
+      const size_t o = moff + size_t(slot < p.max_blocks ? slot : 0);
+      idx = p.kv_indices[o];
+      info = info_of(p.types[o], has_partial ? p.partial_idx[o] : -1);
+    }
+    const int mode = slot < nb ? info & 3 : int(kMasked);
+    const int kvb = idx < 0 ? 0 : (idx >= p.Tk ? p.Tk - 1 : idx);
     const long long row = (long long)kvb * p.KB + off;
-    k.live = (mode == kCausal || mode == kFull || mode == kPartial) && row < p.seqlen;
-    k.row = k.live ? int(row) : 0;
-    k.cmp = !k.live ? 0x7fffffff : (mode == kCausal ? int(row) : -1);
-    k.pid = (k.live && mode == kPartial) ? m_pid : -1;
+    const bool live = mode != kMasked && row < p.seqlen;
+    Key k;
+    k.row = live ? int(row) : -1;
+    k.cmp = !live ? 0x7fffffff : (mode == kCausal ? int(row) : -1);
+    k.pid = (live && mode == kPartial) ? info >> 2 : -1;
     k.off = off;
-    return k;
-  };
-  auto advance = [&]() {
     slot += p.adv_slot;
     off += p.adv_off;
     if (off >= p.kb_eff) {
       off -= p.kb_eff;
       ++slot;
     }
+    return k;
   };
 
-  constexpr bool kPrefetchV = DT < 8;  // (at 256 columns the registers do not hold a step's V rows as well)
-  u32x4_t kf[KS], vf[KS];
-  auto load_rows = [&](const uint16_t* base, int64_t pitch, const Key& k, u32x4_t (&dst)[KS]) {
-    const uint16_t* row = base + int64_t(k.row) * pitch;
+  // A step of one block (p.whole) is uniform over the wave: its first key, mode, tile and offset.
+  struct Block {
+    int row0, mode, pid, off;
+  };
+  auto next_block = [&]() {
+    const int first = __builtin_amdgcn_readfirstlane(slot), at = __builtin_amdgcn_readfirstlane(off);
+    if ((first >> 6) != chunk_at) load_chunk(first >> 6);
+    const int idx = __builtin_amdgcn_readlane(mv_idx, first & 63), info = __builtin_amdgcn_readlane(mv_info, first & 63);
+    const int kvb = idx < 0 ? 0 : (idx >= p.Tk ? p.Tk - 1 : idx);
+    const long long row0 = (long long)kvb * p.KB + at;  // (beyond the sequence: nothing is allowed)
+    Block k;
+    k.mode = row0 < p.seqlen ? info & 3 : int(kMasked);
+    k.row0 = k.mode != kMasked ? int(row0) : 0;
+    k.pid = info >> 2;
+    k.off = at;
+    slot += p.adv_slot;
+    off += p.adv_off;
+    if (off >= p.kb_eff) {
+      off -= p.kb_eff;
+      ++slot;
+    }
+    return k;
+  };
+
+  // Rows of a step into a tile: lane l takes the chunks l, l + 64, ... of the tile, in the order they
+  // lie in LDS.  from[i]: row of the operand that chunk i of this lane comes from, -1 for zeros; of a
+  // whole step only the first row matters (base) and from[i] counts from there.
+  int from[NLD], base = 0;
+  auto take_rows = [&](const Key& k) {
 #pragma unroll
-    for (int s = 0; s < KS; ++s) dst[s] = load8<SMALL>(row, 16 * s + 8 * g, p.D);
+    for (int i = 0; i < NLD; ++i) from[i] = __shfl(k.row, (i * 64 + lane) / C, 64);
+  };
+#pragma unroll
+  for (int i = 0; i < NLD; ++i) from[i] = (i * 64 + lane) / C;
+  auto resource = [&](const uint16_t* slab, int64_t pitch) {
+    const uint64_t a = reinterpret_cast<uint64_t>(slab);
+    i32x4_t r;
+    r[0] = __builtin_amdgcn_readfirstlane(int32_t(uint32_t(a)));
+    r[1] = __builtin_amdgcn_readfirstlane(int32_t(uint32_t(a >> 32) & 0xffffu));
+    r[2] = __builtin_amdgcn_readfirstlane(int32_t(uint32_t((int64_t(p.seqlen) - 1) * pitch + p.D) * 2u));
+    r[3] = 0x00020000;
+    return r;
+  };
+  const i32x4_t rK = resource(k_slab, p.k_at.row), rV = resource(v_slab, p.v_at.row);
+  // byte offsets of this lane's chunks inside the rows, and of its rows in a whole step
+  uint32_t cols[NLD];
+#pragma unroll
+  for (int i = 0; i < NLD; ++i) {
+    const int id = i * 64 + lane;
+    cols[i] = uint32_t(chunk_start(((id % C) ^ swizzle(id / C)) * 8, p.D)) * 2u;
+  }
+  auto load_tile = [&](const uint16_t* slab, const i32x4_t& rsrc, int64_t pitch, uint8_t* dst) {
+    if constexpr (R == Rows::kDirect) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the tile has been read
+      const uint32_t to = uint32_t(size_t((__attribute__((address_space(3))) void*)dst));
+      const uint32_t pitch2 = uint32_t(pitch * 2);
+#pragma unroll
+      for (int i = 0; i < NLD; ++i) {
+        uint32_t at = uint32_t(from[i]) * pitch2 + cols[i];
+        if (!p.whole) at = from[i] < 0 ? 0xffffffffu : at;
+        buffer_to_lds(rsrc, at, uint32_t(base) * pitch2, to + uint32_t(i) * 1024u);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < NLD; ++i) {
+        const int id = i * 64 + lane;
+        const int row = from[i] + base;  // (base is 0 unless the step is whole)
+        const bool none = from[i] < 0 || row >= p.seqlen;
+        u32x4_t x = load8<R>(slab + int64_t(none ? 0 : row) * pitch, ((id % C) ^ swizzle(id / C)) * 8, p.D);
+        if (none) x = u32x4_t{0u, 0u, 0u, 0u};
+        *reinterpret_cast<u32x4_t*>(dst + size_t(id) * 16) = x;
+      }
+    }
   };
 
   const f32x16_t zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -297,79 +417,125 @@ __global__ void __launch_bounds__(64 * kWaves, DT <= 4 ? 2 : 1) fwd_generic_kern
   // A wave is done when the first position of its step is beyond the list.
   auto more = [&]() { return __builtin_amdgcn_readfirstlane(slot) < nb; };
   bool go = more() && p.seqlen > 0;
-  Key cur = {0, 0x7fffffff, 0, -1, false};
+  Key cur = {-1, 0x7fffffff, 0, -1};
+  Block blk = {0, kMasked, 0, 0};
+  auto advance = [&]() {
+    if (p.whole) {
+      blk = next_block();
+      base = blk.row0;
+    } else {
+      cur = next_key();
+      take_rows(cur);
+    }
+  };
   if (go) {
-    load_meta();
-    cur = resolve();
-    load_rows(k_slab, p.k_at.row, cur, kf);
-    if (kPrefetchV) load_rows(v_slab, p.v_at.row, cur, vf);
     advance();
-    load_meta();
+    load_tile(k_slab, rK, p.k_at.row, sK);
+    load_tile(v_slab, rV, p.v_at.row, sV);
   }
+  const int q_first = qb * p.QB + row0;  // first row of the workgroup
   while (go) {
-    if (!kPrefetchV) load_rows(v_slab, p.v_at.row, cur, vf);
-    // what the softmax needs to know about the 32 keys, by key
-    if (g == 0) {
-      sKey[c] = cur.cmp;
-      sOff[c] = cur.off;
-      sPid[c] = cur.pid;
-    }
-    const bool any_partial = __builtin_amdgcn_ballot_w64(cur.pid >= 0) != 0;
-    f32x16_t st = zero16;
+    // Allowed keys of this step as bits: register r (key 8 (r / 4) + 4 g + r % 4) is bit r.
+    uint32_t keep = 0xffffu;
+    bool masked;  // (uniform) some of them are not allowed
+    if (p.whole) {
+      masked = !(blk.row0 + 32 <= p.seqlen && (blk.mode == kFull || (blk.mode == kCausal && blk.row0 + 31 <= q_first)));
+      if (masked) {
+        if (blk.mode == kPartial) {  // attn_naive.cu:143-154: any non-zero byte of the tile = attend
+          const uint8_t* t = p.partial_masks + (size_t(blk.pid) * p.QB + (q_here ? q_local : 0)) * p.KB + blk.off + 4 * g;
+          uint32_t word[4];
 #pragma unroll
-    for (int s = 0; s < KS; ++s) st = mfma<BF16>(kf[s], q_frag(s), st);
-    // V rows into the wave's tile
+          for (int r4 = 0; r4 < 4; ++r4) word[r4] = *reinterpret_cast<const uint32_t*>(t + 8 * r4);
+          keep = 0;
 #pragma unroll
-    for (int s = 0; s < KS; ++s)
-      *reinterpret_cast<u32x4_t*>(sV + tile_at(c, 2 * s + g)) = cur.live ? vf[s] : u32x4_t{0u, 0u, 0u, 0u};
-    // registers are free: the rows of the wave's next step, and the metadata of the one after it
-    go = more();
-    Key nxt = cur;
-    if (go) {
-      nxt = resolve();
-      load_rows(k_slab, p.k_at.row, nxt, kf);
-      if (kPrefetchV) load_rows(v_slab, p.v_at.row, nxt, vf);
-      advance();
-      load_meta();
-    }
-    // scores: register r is key 8 (r / 4) + 4 g + r % 4 of the step
-    float mx = -INFINITY;
+          for (int r4 = 0; r4 < 4; ++r4) {
+            uint32_t x = word[r4];
+            x |= x >> 4;
+            x |= x >> 2;
+            x |= x >> 1;
+            keep |= (((x & 0x01010101u) * 0x01020408u) >> 24) << (4 * r4);
+          }
+        }
+        int limit = p.seqlen - 1;
+        if (blk.mode == kCausal) limit = limit < q_idx ? limit : q_idx;
+        if (blk.mode == kMasked) limit = -1;
+        const int n = limit - blk.row0 - 4 * g + 1;  // leading keys of this half-wave's pattern that are allowed
 #pragma unroll
-    for (int r4 = 0; r4 < 4; ++r4) {
-      const i32x4_t cmp = *reinterpret_cast<const i32x4_t*>(sKey + 8 * r4 + 4 * g);
-      uint32_t bits = 0x01010101u;
-      if (any_partial) {  // :143-154: any non-zero byte of the tile = attend
-        const i32x4_t pid = *reinterpret_cast<const i32x4_t*>(sPid + 8 * r4 + 4 * g);
-        const i32x4_t po = *reinterpret_cast<const i32x4_t*>(sOff + 8 * r4 + 4 * g);
-        const int ql = q_here ? q_local : 0;
-        if (p.mask_words) {  // the four keys are neighbours in one block
-          const int p0 = pid[0], o0 = po[0];
-          if (p0 >= 0) bits = *reinterpret_cast<const uint32_t*>(p.partial_masks + (size_t(p0) * p.QB + ql) * p.KB + o0);
-        } else {
-          bits = 0;
+        for (int r4 = 0; r4 < 4; ++r4) {
+          const int m = n - 8 * r4;
+          const uint32_t four = m >= 4 ? 15u : (m <= 0 ? 0u : (1u << m) - 1u);
+          keep &= ~((15u & ~four) << (4 * r4));
+        }
+      }
+    } else {
+      // what is known about the 32 keys, by key
+      if (g == 0) {
+        sKey[c] = cur.cmp;
+        sOff[c] = cur.off;
+        sPid[c] = cur.pid;
+      }
+      const bool any_partial = __builtin_amdgcn_ballot_w64(cur.pid >= 0) != 0;
+      masked = any_partial || __builtin_amdgcn_ballot_w64(cur.cmp > q_first) != 0;
+      if (masked) {
+        keep = 0;
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+          const i32x4_t cmp = *reinterpret_cast<const i32x4_t*>(sKey + 8 * r4 + 4 * g);
+          uint32_t bytes = 0x01010101u;
+          if (any_partial) {
+            const i32x4_t pid = *reinterpret_cast<const i32x4_t*>(sPid + 8 * r4 + 4 * g);
+            const i32x4_t po = *reinterpret_cast<const i32x4_t*>(sOff + 8 * r4 + 4 * g);
+            const int ql = q_here ? q_local : 0;
+            if (p.mask_words) {  // the four keys are neighbours in one block
+              const int p0 = pid[0], o0 = po[0];
+              if (p0 >= 0)
+                bytes = *reinterpret_cast<const uint32_t*>(p.partial_masks + (size_t(p0) * p.QB + ql) * p.KB + o0);
+            } else {
+              bytes = 0;
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                const int pi = pid[i], oi = po[i];
+                const uint32_t byte = pi >= 0 ? p.partial_masks[(size_t(pi) * p.QB + ql) * p.KB + oi] : 1u;
+                bytes |= byte << (8 * i);
+              }
+            }
+          }
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const int pi = pid[i], oi = po[i];
-            const uint32_t byte = pi >= 0 ? p.partial_masks[(size_t(pi) * p.QB + ql) * p.KB + oi] : 1u;
-            bits |= byte << (8 * i);
+            const int ci = cmp[i];
+            keep |= uint32_t(ci <= q_idx && ((bytes >> (8 * i)) & 0xffu) != 0) << (4 * r4 + i);
           }
         }
       }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float s = st[4 * r4 + i];
-        if (p.softcap > 0.f) s = tanhf(s * p.scale / p.softcap) * p.softcap;
-        s *= p.sl2;
-        const int ci = cmp[i];
-        s = (ci <= q_idx && ((bits >> (8 * i)) & 0xffu) != 0) ? s : -INFINITY;
-        st[4 * r4 + i] = s;
-        mx = fmaxf(mx, s);
-      }
     }
+    if constexpr (R == Rows::kDirect) wait_but<NLD>();  // K is there (V was requested after it)
+    f32x16_t st = zero16;
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+      st = mfma<BF16>(*reinterpret_cast<const u32x4_t*>(sK + tile_at(c, 2 * s + g)), q_frag(s), st);
+    asm volatile("" : "+v"(keep));  // (the mask's own loads are waited for here, not behind the next request)
+    // K has been read: the rows of the wave's next step
+    go = more();
+    if (go) {
+      advance();
+      load_tile(k_slab, rK, p.k_at.row, sK);
+    }
+    if (p.softcap > 0.f) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) st[r] = tanhf(st[r] * p.scale / p.softcap) * p.softcap;
+    }
+    if (masked) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) st[r] = (keep >> r) & 1u ? st[r] : -INFINITY;
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) mx = fmaxf(mx, st[r]);
+    mx *= p.sl2;
     mx = fmaxf(mx, other_half(mx));
-    const float m_new = fmaxf(m_run, mx);
-    const float m_ref = m_new == -INFINITY ? 0.f : m_new;
-    if (__builtin_amdgcn_ballot_w64(m_new > m_run) != 0) {
+    if (__builtin_amdgcn_ballot_w64(mx > m_run + kSlack) != 0) {
+      const float m_new = fmaxf(m_run, mx);
+      const float m_ref = m_new == -INFINITY ? 0.f : m_new;
       const float alpha = __builtin_amdgcn_exp2f(m_run - m_ref);
       l_run *= alpha;
 #pragma unroll
@@ -378,18 +544,26 @@ __global__ void __launch_bounds__(64 * kWaves, DT <= 4 ? 2 : 1) fwd_generic_kern
         for (int r = 0; r < 16; ++r) ot[dt][r] *= alpha;
       m_run = m_new;
     }
+    const float m_ref = m_run == -INFINITY ? 0.f : m_run;
     u32x4_t pb[PARTS][2];
     float sum = 0.f;
 #pragma unroll
     for (int r = 0; r < 16; r += 2) {
-      float p0 = __builtin_amdgcn_exp2f(st[r] - (m_ref - kShift));
-      float p1 = __builtin_amdgcn_exp2f(st[r + 1] - (m_ref - kShift));
+      float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[r], p.sl2, kShift - m_ref));
+      float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[r + 1], p.sl2, kShift - m_ref));
       sum += p0;
       sum += p1;
 #pragma unroll
       for (int n = 0; n < PARTS; ++n) pb[n][r >> 3][(r & 7) >> 1] = split_part<BF16>(p0, p1);
     }
     l_run += sum;
+    if constexpr (R == Rows::kDirect) {  // V is there (the next K was requested after it)
+      if (go) {
+        wait_but<NLD>();
+      } else {
+        wait_but<0>();
+      }
+    }
     // O^T += V^T.P^T: k-slot e of lane group g in 16-key half ts is key 16 ts + 8 (e / 4) + 4 g + e % 4
     const int i16 = c & 15, j16 = c >> 4;
 #pragma unroll
@@ -409,7 +583,7 @@ __global__ void __launch_bounds__(64 * kWaves, DT <= 4 ? 2 : 1) fwd_generic_kern
         for (int n = 0; n < PARTS; ++n) ot[dt] = mfma<BF16>(a, pb[n][ts], ot[dt]);
       }
     }
-    cur = nxt;
+    if (go) load_tile(v_slab, rV, p.v_at.row, sV);
   }
 
   // Merge: row maxima and sums of the waves, then the O^T tiles, kGroup at a time: every wave
@@ -417,17 +591,17 @@ __global__ void __launch_bounds__(64 * kWaves, DT <= 4 ? 2 : 1) fwd_generic_kern
   l_run += other_half(l_run);
   if (g == 0) {
     sStat[w * 32 + c] = m_run;
-    sStat[(kWaves + w) * 32 + c] = l_run;
+    sStat[(NW + w) * 32 + c] = l_run;
   }
   __syncthreads();
   float m_all = -INFINITY;
 #pragma unroll
-  for (int i = 0; i < kWaves; ++i) m_all = fmaxf(m_all, sStat[i * 32 + c]);
+  for (int i = 0; i < NW; ++i) m_all = fmaxf(m_all, sStat[i * 32 + c]);
   const float m_fin = m_all == -INFINITY ? 0.f : m_all;
   float l_all = 0.f;
 #pragma unroll
-  for (int i = 0; i < kWaves; ++i)
-    l_all += sStat[(kWaves + i) * 32 + c] * __builtin_amdgcn_exp2f(sStat[i * 32 + c] - m_fin);
+  for (int i = 0; i < NW; ++i)
+    l_all += sStat[(NW + i) * 32 + c] * __builtin_amdgcn_exp2f(sStat[i * 32 + c] - m_fin);
   const bool some = q_live && l_all > 0.f;
   const float inv = some ? 1.f / l_all : 0.f;  // :283-288; rows without a key: zeros (:177-183)
   const float mine = __builtin_amdgcn_exp2f(m_run - m_fin) * inv;
@@ -450,32 +624,32 @@ __global__ void __launch_bounds__(64 * kWaves, DT <= 4 ? 2 : 1) fwd_generic_kern
       }
     }
     __syncthreads();
-    if (w < G && d0 + w < DT) {
+    // pieces (tile, four registers) of the group, dealt to the waves
+    for (int u = w; u < 4 * G; u += NW) {
+      const int i = u >> 2, r4 = u & 3;
+      if (d0 + i >= DT) break;
+      f32x4_t x = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < NW; ++j)
+        x += *reinterpret_cast<const f32x4_t*>(stage + ((size_t(j) * G + i) * 4 + r4) * 256 + lane * 4);
+      if (!q_live) x = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      const int d = 32 * (d0 + i) + 8 * r4 + 4 * g;
       uint16_t* orow = p.o + (bh * p.S + q_idx) * p.D;
+      uint16_t hv[4];
 #pragma unroll
-      for (int r4 = 0; r4 < 4; ++r4) {
-        f32x4_t x = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int i = 0; i < kWaves; ++i)
-          x += *reinterpret_cast<const f32x4_t*>(stage + ((size_t(i) * G + w) * 4 + r4) * 256 + lane * 4);
-        if (!q_live) x = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        const int d = 32 * (d0 + w) + 8 * r4 + 4 * g;
-        uint16_t h[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) h[j] = from_float<BF16>(x[j]);
-        if (q_here) {
-          if (p.o_vec) {  // D is a multiple of 8: four columns are inside together
-            if (d < p.D) {
-              const u32x2_t two = {uint32_t(h[0]) | uint32_t(h[1]) << 16, uint32_t(h[2]) | uint32_t(h[3]) << 16};
-              *reinterpret_cast<u32x2_t*>(orow + d) = two;
-            }
-          } else {
-            const int chunk = d & ~7;
-            const int col = SMALL ? d : chunk_start(chunk, p.D) + (d & 7);
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-              if (chunk < p.D && col + j < p.D && col + j >= chunk) orow[col + j] = h[j];
+      for (int j = 0; j < 4; ++j) hv[j] = from_float<BF16>(x[j]);
+      if (q_here) {
+        if (p.o_vec) {  // D is a multiple of 8: four columns are inside together
+          if (d < p.D) {
+            const u32x2_t two = {uint32_t(hv[0]) | uint32_t(hv[1]) << 16, uint32_t(hv[2]) | uint32_t(hv[3]) << 16};
+            *reinterpret_cast<u32x2_t*>(orow + d) = two;
           }
+        } else {
+          const int chunk = d & ~7;
+          const int col = R == Rows::kSmall ? d : chunk_start(chunk, p.D) + (d & 7);
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (chunk < p.D && col + j < p.D && col + j >= chunk) orow[col + j] = hv[j];
         }
       }
     }
@@ -484,11 +658,12 @@ __global__ void __launch_bounds__(64 * kWaves, DT <= 4 ? 2 : 1) fwd_generic_kern
 
 constexpr int kMaxDevices = 64;
 
-template <bool BF16, int DT, bool SMALL>
+template <bool BF16, int DT, int NW, Rows R>
 int launch(const GenericParams& p, unsigned grid, hipStream_t stream) {
-  auto kern = fwd_generic_kernel<BF16, DT, SMALL>;
+  auto kern = fwd_generic_kernel<BF16, DT, NW, R>;
   const void* fn = reinterpret_cast<const void*>(kern);
-  constexpr int lds = int(GenericTraits<DT>::kLdsBytes);
+  constexpr int lds = int(GenericTraits<DT, NW>::kLdsBytes);
+  static_assert(lds <= 160 * 1024, "LDS of a compute unit");
   if (lds > 48 * 1024) {  // the dynamic-LDS limit of an instance is raised once per device
     static std::atomic<bool> raised[kMaxDevices];
     int dev = 0;
@@ -502,15 +677,24 @@ int launch(const GenericParams& p, unsigned grid, hipStream_t stream) {
     }
   }
   GenericParams params = p;
+  params.adv_slot = 32 * NW / p.kb_eff;
+  params.adv_off = 32 * NW % p.kb_eff;
   void* args[] = {&params};
-  return int(hipLaunchKernel(fn, dim3(grid), dim3(64 * kWaves), args, lds, stream));
+  return int(hipLaunchKernel(fn, dim3(grid), dim3(64 * NW), args, lds, stream));
+}
+
+template <bool BF16, int DT>
+int launch_rows(const GenericParams& p, Rows rows, unsigned grid, hipStream_t s) {
+  constexpr int NW = DT <= 4 ? 8 : 4;  // what the tiles leave room for in LDS
+  return rows == Rows::kDirect ? launch<BF16, DT, NW, Rows::kDirect>(p, grid, s)
+                               : launch<BF16, DT, NW, Rows::kWide>(p, grid, s);
 }
 
 template <bool BF16, int... I>
-int launch_tiles(const GenericParams& p, unsigned grid, hipStream_t s, std::integer_sequence<int, I...>) {
-  if (p.D < 8) return launch<BF16, 1, true>(p, grid, s);
+int launch_tiles(const GenericParams& p, Rows rows, unsigned grid, hipStream_t s, std::integer_sequence<int, I...>) {
+  if (rows == Rows::kSmall) return launch<BF16, 1, 4, Rows::kSmall>(p, grid, s);
   int rc = int(hipErrorInvalidValue);
-  ((((p.D + 31) / 32 == I + 1) ? (void)(rc = launch<BF16, I + 1, false>(p, grid, s)) : (void)0), ...);
+  ((((p.D + 31) / 32 == I + 1) ? (void)(rc = launch_rows<BF16, I + 1>(p, rows, grid, s)) : (void)0), ...);
   return rc;
 }
 
@@ -566,10 +750,10 @@ int forward_generic(const void* q, const void* k, const void* v, const omni_attn
   p.KB = KB;
   p.seqlen = seqlen_orig < S_pad ? seqlen_orig : S_pad;
   p.kb_eff = KB < S_pad ? KB : S_pad;
-  p.adv_slot = 32 * kWaves / p.kb_eff;
-  p.adv_off = 32 * kWaves % p.kb_eff;
   p.q_tiles = ((QB < S_pad ? QB : S_pad) + 31) / 32;
   p.mask_words = KB % 4 == 0 && p.kb_eff % 4 == 0 && !misaligned(partial_masks_or_null, 4);
+  p.whole = KB % 32 == 0 && !misaligned(partial_masks_or_null, 4);
+  if (p.whole) p.kb_eff = KB;  // (the keys of a block behind the sequence are masked like any others)
   p.n_slabs = unsigned(B) * unsigned(H);
   p.scale = float(1.0 / std::sqrt(double(D)));
   p.softcap = softcap;
@@ -578,10 +762,16 @@ int forward_generic(const void* q, const void* k, const void* v, const omni_attn
   p.o_vec = D % 8 == 0 && !misaligned(o, 8);
   const long long grid = (long long)B * H * Tq * p.q_tiles;
   if (grid > 0x7fffffffLL) return OMNI_ATTN_ERR_TOO_LARGE;
+  const auto direct = [&](const void* ptr, const omni_attn_strides& at) {  // 32-bit offsets inside a slab
+    return !misaligned(ptr, 16) && at.batch % 8 == 0 && at.head % 8 == 0 && at.row % 8 == 0 && at.row >= D &&
+           (long long)p.seqlen * at.row * 2 < 0xffffff00LL;
+  };
+  const Rows reads = D < 8 ? Rows::kSmall
+                           : (D % 8 == 0 && direct(k, k_at) && direct(v, v_at) ? Rows::kDirect : Rows::kWide);
   const auto tiles = std::make_integer_sequence<int, kMaxD / 32>{};
   const int e = dtype == OMNI_ATTN_DTYPE_BF16
-                    ? launch_tiles<true>(p, unsigned(grid), static_cast<hipStream_t>(stream), tiles)
-                    : launch_tiles<false>(p, unsigned(grid), static_cast<hipStream_t>(stream), tiles);
+                    ? launch_tiles<true>(p, reads, unsigned(grid), static_cast<hipStream_t>(stream), tiles)
+                    : launch_tiles<false>(p, reads, unsigned(grid), static_cast<hipStream_t>(stream), tiles);
   if (e != 0) {
     omni_attn::record_hip_error(e);
     return OMNI_ATTN_ERR_LAUNCH;

@@ -19,6 +19,9 @@
 // a tile).  A weight is a sum of 16-bit parts with one product each: two for fp16 (scaled by 2^8
 // first, so that small weights stay out of the subnormals), three for bf16.
 //
+// A key that a row may not attend to never reaches it, whatever its V row holds (0 * infinity would):
+// a wave whose sums end up infinite or NaN walks its list once more and leaves out the zero weights.
+//
 // Bound by the latency of a step (two matrix chains, the softmax and the split of the weights on the
 // vector pipe) times the steps of the longest list over the waves; from 192 columns on by LDS (a step
 // of 32 rows reads each K and V byte once for 32 query rows).  B=1 H=8 S=2048 D=96 fp16, causal in 32x32
@@ -31,6 +34,7 @@
 
 #include <atomic>
 #include <cmath>
+#include <type_traits>
 #include <utility>
 
 namespace omni_attn {
@@ -172,6 +176,16 @@ __device__ __forceinline__ uint16_t from_float(float x) {
   }
 }
 
+// One 16-bit value as a float (the inverse of a part of split_part).
+template <bool BF16>
+__device__ __forceinline__ float to_float(uint32_t bits) {
+  if constexpr (BF16) {
+    return __builtin_bit_cast(float, bits << 16);
+  } else {
+    return float(__builtin_bit_cast(_Float16, uint16_t(bits)));
+  }
+}
+
 // The other half-wave's value (lane ^ 32).
 __device__ __forceinline__ float other_half(float x) { return __shfl_xor(x, 32, 64); }
 
@@ -193,7 +207,7 @@ struct GenericTraits {
 };
 
 template <bool BF16, int DT, int NW, Rows R>
-__global__ void __launch_bounds__(64 * NW, (DT <= 4 || NW == 8) ? 2 : 1) fwd_generic_kernel(const GenericParams p) {
+__global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2 : 1)) fwd_generic_kernel(const GenericParams p) {
   using Traits = GenericTraits<DT, NW>;
   constexpr int KS = 2 * DT;
   constexpr int C = 4 * DT;     // 16-byte chunks of a tile row
@@ -384,7 +398,7 @@ __global__ void __launch_bounds__(64 * NW, (DT <= 4 || NW == 8) ? 2 : 1) fwd_gen
     const int id = i * 64 + lane;
     cols[i] = uint32_t(chunk_start(((id % C) ^ swizzle(id / C)) * 8, p.D)) * 2u;
   }
-  auto load_tile = [&](const uint16_t* slab, const i32x4_t& rsrc, int64_t pitch, uint8_t* dst) {
+  auto load_tile = [&](auto again, const uint16_t* slab, const i32x4_t& rsrc, int64_t pitch, uint8_t* dst) {
     if constexpr (R == Rows::kDirect) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the tile has been read
       const uint32_t to = uint32_t(size_t((__attribute__((address_space(3))) void*)dst));
@@ -396,9 +410,12 @@ __global__ void __launch_bounds__(64 * NW, (DT <= 4 || NW == 8) ? 2 : 1) fwd_gen
         buffer_to_lds(rsrc, at, uint32_t(base) * pitch2, to + uint32_t(i) * 1024u);
       }
     } else {
+      int l = lane;
+      if constexpr (decltype(again)::value) asm volatile("" : "+v"(l));  // (addresses worked out anew)
 #pragma unroll
       for (int i = 0; i < NLD; ++i) {
-        const int id = i * 64 + lane;
+        if constexpr (decltype(again)::value) __builtin_amdgcn_sched_barrier(0);
+        const int id = i * 64 + l;
         const int row = from[i] + base;  // (base is 0 unless the step is whole)
         const bool none = from[i] < 0 || row >= p.seqlen;
         u32x4_t x = load8<R>(slab + int64_t(none ? 0 : row) * pitch, ((id % C) ^ swizzle(id / C)) * 8, p.D);
@@ -428,162 +445,220 @@ __global__ void __launch_bounds__(64 * NW, (DT <= 4 || NW == 8) ? 2 : 1) fwd_gen
       take_rows(cur);
     }
   };
-  if (go) {
+  auto first_rows = [&](auto again) {
     advance();
-    load_tile(k_slab, rK, p.k_at.row, sK);
-    load_tile(v_slab, rV, p.v_at.row, sV);
-  }
+    load_tile(again, k_slab, rK, p.k_at.row, sK);
+    load_tile(again, v_slab, rV, p.v_at.row, sV);
+  };
   const int q_first = qb * p.QB + row0;  // first row of the workgroup
-  while (go) {
-    // Allowed keys of this step as bits: register r (key 8 (r / 4) + 4 g + r % 4) is bit r.
-    uint32_t keep = 0xffffu;
-    bool masked;  // (uniform) some of them are not allowed
-    if (p.whole) {
-      masked = !(blk.row0 + 32 <= p.seqlen && (blk.mode == kFull || (blk.mode == kCausal && blk.row0 + 31 <= q_first)));
-      if (masked) {
-        if (blk.mode == kPartial) {  // attn_naive.cu:143-154: any non-zero byte of the tile = attend
-          const uint8_t* t = p.partial_masks + (size_t(blk.pid) * p.QB + (q_here ? q_local : 0)) * p.KB + blk.off + 4 * g;
-          uint32_t word[4];
+  // `again`: the second walk of a wave whose first met an infinity or a NaN in V (or overflowed); rare, so
+  // that it may be slow.  (Code of its own: a branch in one loop doubles the registers of the sums.)
+  auto walk = [&](auto again) {
+    while (go) {
+      // Allowed keys of this step as bits: register r (key 8 (r / 4) + 4 g + r % 4) is bit r.
+      uint32_t keep = 0xffffu;
+      bool masked;  // (uniform) some of them are not allowed
+      if (p.whole) {
+        masked = !(blk.row0 + 32 <= p.seqlen && (blk.mode == kFull || (blk.mode == kCausal && blk.row0 + 31 <= q_first)));
+        if (masked) {
+          if (blk.mode == kPartial) {  // attn_naive.cu:143-154: any non-zero byte of the tile = attend
+            const uint8_t* t = p.partial_masks + (size_t(blk.pid) * p.QB + (q_here ? q_local : 0)) * p.KB + blk.off + 4 * g;
+            uint32_t word[4];
 #pragma unroll
-          for (int r4 = 0; r4 < 4; ++r4) word[r4] = *reinterpret_cast<const uint32_t*>(t + 8 * r4);
+            for (int r4 = 0; r4 < 4; ++r4) word[r4] = *reinterpret_cast<const uint32_t*>(t + 8 * r4);
+            keep = 0;
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4) {
+              uint32_t x = word[r4];
+              x |= x >> 4;
+              x |= x >> 2;
+              x |= x >> 1;
+              keep |= (((x & 0x01010101u) * 0x01020408u) >> 24) << (4 * r4);
+            }
+          }
+          int limit = p.seqlen - 1;
+          if (blk.mode == kCausal) limit = limit < q_idx ? limit : q_idx;
+          if (blk.mode == kMasked) limit = -1;
+          const int n = limit - blk.row0 - 4 * g + 1;  // leading keys of this half-wave's pattern that are allowed
+#pragma unroll
+          for (int r4 = 0; r4 < 4; ++r4) {
+            const int m = n - 8 * r4;
+            const uint32_t four = m >= 4 ? 15u : (m <= 0 ? 0u : (1u << m) - 1u);
+            keep &= ~((15u & ~four) << (4 * r4));
+          }
+        }
+      } else {
+        // what is known about the 32 keys, by key
+        if (g == 0) {
+          sKey[c] = cur.cmp;
+          sOff[c] = cur.off;
+          sPid[c] = cur.pid;
+        }
+        const bool any_partial = __builtin_amdgcn_ballot_w64(cur.pid >= 0) != 0;
+        masked = any_partial || __builtin_amdgcn_ballot_w64(cur.cmp > q_first) != 0;
+        if (masked) {
           keep = 0;
 #pragma unroll
           for (int r4 = 0; r4 < 4; ++r4) {
-            uint32_t x = word[r4];
-            x |= x >> 4;
-            x |= x >> 2;
-            x |= x >> 1;
-            keep |= (((x & 0x01010101u) * 0x01020408u) >> 24) << (4 * r4);
+            const i32x4_t cmp = *reinterpret_cast<const i32x4_t*>(sKey + 8 * r4 + 4 * g);
+            uint32_t bytes = 0x01010101u;
+            if (any_partial) {
+              const i32x4_t pid = *reinterpret_cast<const i32x4_t*>(sPid + 8 * r4 + 4 * g);
+              const i32x4_t po = *reinterpret_cast<const i32x4_t*>(sOff + 8 * r4 + 4 * g);
+              const int ql = q_here ? q_local : 0;
+              if (p.mask_words) {  // the four keys are neighbours in one block
+                const int p0 = pid[0], o0 = po[0];
+                if (p0 >= 0)
+                  bytes = *reinterpret_cast<const uint32_t*>(p.partial_masks + (size_t(p0) * p.QB + ql) * p.KB + o0);
+              } else {
+                bytes = 0;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                  const int pi = pid[i], oi = po[i];
+                  const uint32_t byte = pi >= 0 ? p.partial_masks[(size_t(pi) * p.QB + ql) * p.KB + oi] : 1u;
+                  bytes |= byte << (8 * i);
+                }
+              }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const int ci = cmp[i];
+              keep |= uint32_t(ci <= q_idx && ((bytes >> (8 * i)) & 0xffu) != 0) << (4 * r4 + i);
+            }
           }
         }
-        int limit = p.seqlen - 1;
-        if (blk.mode == kCausal) limit = limit < q_idx ? limit : q_idx;
-        if (blk.mode == kMasked) limit = -1;
-        const int n = limit - blk.row0 - 4 * g + 1;  // leading keys of this half-wave's pattern that are allowed
+      }
+      if constexpr (R == Rows::kDirect) wait_but<NLD>();  // K is there (V was requested after it)
+      f32x16_t st = zero16;
 #pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4) {
-          const int m = n - 8 * r4;
-          const uint32_t four = m >= 4 ? 15u : (m <= 0 ? 0u : (1u << m) - 1u);
-          keep &= ~((15u & ~four) << (4 * r4));
+      for (int s = 0; s < KS; ++s)
+        st = mfma<BF16>(*reinterpret_cast<const u32x4_t*>(sK + tile_at(c, 2 * s + g)), q_frag(s), st);
+      asm volatile("" : "+v"(keep));  // (the mask's own loads are waited for here, not behind the next request)
+      // K has been read: the rows of the wave's next step
+      go = more();
+      if (go) {
+        advance();
+        load_tile(again, k_slab, rK, p.k_at.row, sK);
+      }
+      if (p.softcap > 0.f) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) st[r] = tanhf(st[r] * p.scale / p.softcap) * p.softcap;
+      }
+      if (masked) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) st[r] = (keep >> r) & 1u ? st[r] : -INFINITY;
+      }
+      float mx = -INFINITY;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, st[r]);
+      mx *= p.sl2;
+      mx = fmaxf(mx, other_half(mx));
+      if (__builtin_amdgcn_ballot_w64(mx > m_run + kSlack) != 0) {
+        const float m_new = fmaxf(m_run, mx);
+        const float m_ref = m_new == -INFINITY ? 0.f : m_new;
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_ref);
+        l_run *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) ot[dt][r] *= alpha;
+        m_run = m_new;
+      }
+      const float m_ref = m_run == -INFINITY ? 0.f : m_run;
+      u32x4_t pb[PARTS][2];
+      float sum = 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; r += 2) {
+        float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[r], p.sl2, kShift - m_ref));
+        float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[r + 1], p.sl2, kShift - m_ref));
+        sum += p0;
+        sum += p1;
+#pragma unroll
+        for (int n = 0; n < PARTS; ++n) pb[n][r >> 3][(r & 7) >> 1] = split_part<BF16>(p0, p1);
+      }
+      l_run += sum;
+      if constexpr (R == Rows::kDirect) {  // V is there (the next K was requested after it)
+        if (go) {
+          wait_but<NLD>();
+        } else {
+          wait_but<0>();
         }
       }
-    } else {
-      // what is known about the 32 keys, by key
-      if (g == 0) {
-        sKey[c] = cur.cmp;
-        sOff[c] = cur.off;
-        sPid[c] = cur.pid;
-      }
-      const bool any_partial = __builtin_amdgcn_ballot_w64(cur.pid >= 0) != 0;
-      masked = any_partial || __builtin_amdgcn_ballot_w64(cur.cmp > q_first) != 0;
-      if (masked) {
-        keep = 0;
+      // O^T += V^T.P^T: k-slot e of lane group g in 16-key half ts is key 16 ts + 8 (e / 4) + 4 g + e % 4
+      const int i16 = c & 15, j16 = c >> 4;
+      if constexpr (decltype(again)::value) {
+        // one key after the other, without those of weight zero (from the parts: as exact as the products)
+#pragma unroll 1
+        for (int key = 0; key < 32; ++key) {
+          const int r = (key >> 3) * 4 + (key & 3);  // its register in half-wave (key / 4) % 2
+          float weight = 0.f;
 #pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4) {
-          const i32x4_t cmp = *reinterpret_cast<const i32x4_t*>(sKey + 8 * r4 + 4 * g);
-          uint32_t bytes = 0x01010101u;
-          if (any_partial) {
-            const i32x4_t pid = *reinterpret_cast<const i32x4_t*>(sPid + 8 * r4 + 4 * g);
-            const i32x4_t po = *reinterpret_cast<const i32x4_t*>(sOff + 8 * r4 + 4 * g);
-            const int ql = q_here ? q_local : 0;
-            if (p.mask_words) {  // the four keys are neighbours in one block
-              const int p0 = pid[0], o0 = po[0];
-              if (p0 >= 0)
-                bytes = *reinterpret_cast<const uint32_t*>(p.partial_masks + (size_t(p0) * p.QB + ql) * p.KB + o0);
-            } else {
-              bytes = 0;
+          for (int n = 0; n < PARTS; ++n) {
+            uint32_t pair = 0;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) pair = i == (r >> 1) ? pb[n][i >> 2][i & 3] : pair;
+            weight += to_float<BF16>((r & 1 ? pair >> 16 : pair) & 0xffffu);
+          }
+          weight = __shfl(weight, c + 32 * ((key >> 2) & 1), 64);
+          // (the fences keep this path from costing the first walk registers)
+          int turn = swizzle(key) * 16;
+          const uint8_t* row = sV + key * Traits::kRowBytes;
+          asm volatile("" : "+v"(turn));
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt) {
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4) {
+              __builtin_amdgcn_sched_barrier(0);
+              const u32x2_t four = *reinterpret_cast<const u32x2_t*>(row + ((4 * dt + r4) * 16 ^ turn) + 8 * g);
 #pragma unroll
               for (int i = 0; i < 4; ++i) {
-                const int pi = pid[i], oi = po[i];
-                const uint32_t byte = pi >= 0 ? p.partial_masks[(size_t(pi) * p.QB + ql) * p.KB + oi] : 1u;
-                bytes |= byte << (8 * i);
+                const uint32_t pair = four[i >> 1];
+                const float x = to_float<BF16>((i & 1 ? pair >> 16 : pair) & 0xffffu), y = ot[dt][4 * r4 + i];
+                ot[dt][4 * r4 + i] = weight != 0.f ? __builtin_fmaf(weight, x, y) : y;
               }
             }
           }
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int ci = cmp[i];
-            keep |= uint32_t(ci <= q_idx && ((bytes >> (8 * i)) & 0xffu) != 0) << (4 * r4 + i);
-          }
         }
       }
-    }
-    if constexpr (R == Rows::kDirect) wait_but<NLD>();  // K is there (V was requested after it)
-    f32x16_t st = zero16;
 #pragma unroll
-    for (int s = 0; s < KS; ++s)
-      st = mfma<BF16>(*reinterpret_cast<const u32x4_t*>(sK + tile_at(c, 2 * s + g)), q_frag(s), st);
-    asm volatile("" : "+v"(keep));  // (the mask's own loads are waited for here, not behind the next request)
-    // K has been read: the rows of the wave's next step
-    go = more();
-    if (go) {
-      advance();
-      load_tile(k_slab, rK, p.k_at.row, sK);
-    }
-    if (p.softcap > 0.f) {
+      for (int ts = 0; ts < (decltype(again)::value ? 0 : 2); ++ts) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) st[r] = tanhf(st[r] * p.scale / p.softcap) * p.softcap;
-    }
-    if (masked) {
+        for (int dt = 0; dt < DT; ++dt) {
+          const int chunk = 2 * (2 * dt + j16) + ((i16 & 3) >> 1);
+          const int r0 = 16 * ts + 4 * g + (i16 >> 2), r1 = r0 + 8;
+          const uint8_t* a0 = sV + tile_at(r0, chunk) + (i16 & 1) * 8;
+          const uint8_t* a1 = sV + tile_at(r1, chunk) + (i16 & 1) * 8;
+          const u32x2_t lo = __builtin_bit_cast(
+              u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(a0)));
+          const u32x2_t hi = __builtin_bit_cast(
+              u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(a1)));
+          const u32x4_t a = {lo[0], lo[1], hi[0], hi[1]};
 #pragma unroll
-      for (int r = 0; r < 16; ++r) st[r] = (keep >> r) & 1u ? st[r] : -INFINITY;
-    }
-    float mx = -INFINITY;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) mx = fmaxf(mx, st[r]);
-    mx *= p.sl2;
-    mx = fmaxf(mx, other_half(mx));
-    if (__builtin_amdgcn_ballot_w64(mx > m_run + kSlack) != 0) {
-      const float m_new = fmaxf(m_run, mx);
-      const float m_ref = m_new == -INFINITY ? 0.f : m_new;
-      const float alpha = __builtin_amdgcn_exp2f(m_run - m_ref);
-      l_run *= alpha;
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) ot[dt][r] *= alpha;
-      m_run = m_new;
-    }
-    const float m_ref = m_run == -INFINITY ? 0.f : m_run;
-    u32x4_t pb[PARTS][2];
-    float sum = 0.f;
-#pragma unroll
-    for (int r = 0; r < 16; r += 2) {
-      float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[r], p.sl2, kShift - m_ref));
-      float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[r + 1], p.sl2, kShift - m_ref));
-      sum += p0;
-      sum += p1;
-#pragma unroll
-      for (int n = 0; n < PARTS; ++n) pb[n][r >> 3][(r & 7) >> 1] = split_part<BF16>(p0, p1);
-    }
-    l_run += sum;
-    if constexpr (R == Rows::kDirect) {  // V is there (the next K was requested after it)
-      if (go) {
-        wait_but<NLD>();
-      } else {
-        wait_but<0>();
+          for (int n = 0; n < PARTS; ++n) ot[dt] = mfma<BF16>(a, pb[n][ts], ot[dt]);
+        }
       }
+      if (go) load_tile(again, v_slab, rV, p.v_at.row, sV);
     }
-    // O^T += V^T.P^T: k-slot e of lane group g in 16-key half ts is key 16 ts + 8 (e / 4) + 4 g + e % 4
-    const int i16 = c & 15, j16 = c >> 4;
+  };
+  if (go) {
+    first_rows(std::false_type{});
+    walk(std::false_type{});
+    float probe = 0.f;  // becomes NaN with any sum that is not finite
 #pragma unroll
-    for (int ts = 0; ts < 2; ++ts) {
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        const int chunk = 2 * (2 * dt + j16) + ((i16 & 3) >> 1);
-        const int r0 = 16 * ts + 4 * g + (i16 >> 2), r1 = r0 + 8;
-        const uint8_t* a0 = sV + tile_at(r0, chunk) + (i16 & 1) * 8;
-        const uint8_t* a1 = sV + tile_at(r1, chunk) + (i16 & 1) * 8;
-        const u32x2_t lo = __builtin_bit_cast(
-            u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(a0)));
-        const u32x2_t hi = __builtin_bit_cast(
-            u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(a1)));
-        const u32x4_t a = {lo[0], lo[1], hi[0], hi[1]};
+      for (int r = 0; r < 16; ++r) probe = __builtin_fmaf(ot[dt][r], 0.f, probe);
+    if (__builtin_amdgcn_ballot_w64(probe != probe) != 0) {
 #pragma unroll
-        for (int n = 0; n < PARTS; ++n) ot[dt] = mfma<BF16>(a, pb[n][ts], ot[dt]);
-      }
+      for (int dt = 0; dt < DT; ++dt) ot[dt] = zero16;
+      l_run = 0.f;
+      m_run += kSlack;  // no score is beyond this: weights stay below 2^kShift, nothing is rescaled
+      slot = (32 * w + c) / p.kb_eff;
+      off = 32 * w + c - slot * p.kb_eff;
+      go = true;
+      first_rows(std::true_type{});
+      walk(std::true_type{});
     }
-    if (go) load_tile(v_slab, rV, p.v_at.row, sV);
   }
 
   // Merge: row maxima and sums of the waves, then the O^T tiles, kGroup at a time: every wave
@@ -603,6 +678,7 @@ __global__ void __launch_bounds__(64 * NW, (DT <= 4 || NW == 8) ? 2 : 1) fwd_gen
   for (int i = 0; i < NW; ++i)
     l_all += sStat[(NW + i) * 32 + c] * __builtin_amdgcn_exp2f(sStat[i * 32 + c] - m_fin);
   const bool some = q_live && l_all > 0.f;
+  const bool empty = !q_live || m_all == -INFINITY;  // no score above minus infinity (:177-183)
   const float inv = some ? 1.f / l_all : 0.f;  // :283-288; rows without a key: zeros (:177-183)
   const float mine = __builtin_amdgcn_exp2f(m_run - m_fin) * inv;
   if (w == 0 && g == 0 && q_here && p.lse)
@@ -632,7 +708,7 @@ __global__ void __launch_bounds__(64 * NW, (DT <= 4 || NW == 8) ? 2 : 1) fwd_gen
 #pragma unroll
       for (int j = 0; j < NW; ++j)
         x += *reinterpret_cast<const f32x4_t*>(stage + ((size_t(j) * G + i) * 4 + r4) * 256 + lane * 4);
-      if (!q_live) x = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      if (empty) x = f32x4_t{0.f, 0.f, 0.f, 0.f};
       const int d = 32 * (d0 + i) + 8 * r4 + 4 * g;
       uint16_t* orow = p.o + (bh * p.S + q_idx) * p.D;
       uint16_t hv[4];
@@ -764,7 +840,7 @@ int forward_generic(const void* q, const void* k, const void* v, const omni_attn
   if (grid > 0x7fffffffLL) return OMNI_ATTN_ERR_TOO_LARGE;
   const auto direct = [&](const void* ptr, const omni_attn_strides& at) {  // 32-bit offsets inside a slab
     return !misaligned(ptr, 16) && at.batch % 8 == 0 && at.head % 8 == 0 && at.row % 8 == 0 && at.row >= D &&
-           (long long)p.seqlen * at.row * 2 < 0xffffff00LL;
+           ((long long)p.seqlen + 31) * at.row * 2 < 0xffffff00LL;  // (a step may run 31 rows past the sequence)
   };
   const Rows reads = D < 8 ? Rows::kSmall
                            : (D % 8 == 0 && direct(k, k_at) && direct(v, v_at) ? Rows::kDirect : Rows::kWide);

@@ -93,3 +93,42 @@ def test_generic_kernel_edges_of_tiles_and_chunks(QB, KB, D, gpu_device):
         assert (o.float().cpu() - wo).abs().max().item() <= 2.0 ** -10, (QB, KB, D, seqlen)
         live = ~torch.isinf(wl)
         assert (lse.cpu()[live] - wl[live]).abs().max().item() <= 2e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+@pytest.mark.parametrize("QB,KB,D,S", [(16, 16, 5, 80), (32, 32, 64, 160), (48, 48, 96, 144), (128, 128, 161, 256),
+                                       (64, 32, 256, 192), (32, 32, 250, 96)])
+def test_values_of_keys_that_are_not_allowed_never_reach_a_row(dtype, QB, KB, D, S, gpu_device):
+    """Infinities, NaNs and large values in V: rows that may not attend to those keys get what
+    they get without them, rows that may get the infinity, the NaN or the (finite) average.  A query row
+    of NaNs has no score: zeros, and no logsumexp."""
+    from omni_attn_torch import create_causal_omni_block_mask
+    gen = torch.Generator().manual_seed(D)
+    q, k, v = (torch.randn(1, 1, S, D, generator=gen).to(dtype) for _ in range(3))
+    m = create_causal_omni_block_mask(1, 1, S, S, QB, KB, device="cpu")
+    args = (m.kv_num_blocks, m.kv_indices, m.block_mask_types, QB, KB, S, None, None, gpu_device)
+    clean, lse0 = run_generic(q, k, v, *args)
+    bad = v.clone()
+    at_inf, at_nan = S // 2 + 3, S - 6
+    bad[..., at_inf, 0] = float("inf")
+    bad[..., at_nan, 2] = float("nan")
+    o, lse = run_generic(q, k, bad, *args)
+    assert (lse - lse0).abs().max().item() <= 2e-5
+    # (the second walk sums in another order: an ulp of |o| < 4 apart at the most, and half of one is usual)
+    ulp = 2.0 ** -9 if dtype == torch.float16 else 2.0 ** -6
+    assert (o - clean).float()[..., :at_inf, :].abs().max().item() <= ulp
+    assert bool((o[..., at_inf:, 0] == float("inf")).all()) and bool(o[..., at_nan:, 2].isnan().all())
+    rest = (o - clean).float()[..., at_inf:, :]
+    rest[..., 0] = 0
+    rest[..., at_nan - at_inf:, 2] = 0
+    assert rest.abs().max().item() <= ulp
+    # a large value as every V is its own average (1e-2: rounding of the result and sums in fp32)
+    large = 60000.0 if dtype == torch.float16 else 2.0 ** 116
+    o, _ = run_generic(q, k, torch.full_like(v, large), *args)
+    assert bool(((o.float() / large - 1).abs() <= 1e-2).all())
+    nan_row = q.clone()
+    nan_row[..., 7, :] = float("nan")
+    o, lse = run_generic(nan_row, k, v, *args)
+    assert bool((o[..., 7, :] == 0).all()) and bool(torch.isneginf(lse[..., 7]).all())
+    keep = torch.arange(S) != 7
+    assert (o - clean).float()[..., keep, :].abs().max().item() <= ulp

@@ -463,9 +463,9 @@ torch::Tensor launch_forward(torch::Tensor& q, torch::Tensor& k, torch::Tensor& 
   q = in_rows(q, m.q_len + m.KB, generic);
   k = in_rows(k, m.q_len + m.KB, generic);
   v = in_rows(v, m.q_len + m.KB, generic);
-  if (!generic && k.stride(2) != v.stride(2)) {  // one row stride for both
-    k = k.contiguous();
-    v = v.contiguous();
+  if (!generic && k.stride(2) != v.stride(2)) {  // one row stride for both (clones: of one row any stride is contiguous)
+    k = k.clone(at::MemoryFormat::Contiguous);
+    v = v.clone(at::MemoryFormat::Contiguous);
   }
   torch::Tensor out = torch::empty({B, H, S, D}, q.options());
   if (lse) *lse = torch::empty({B, H, S}, q.options().dtype(torch::kFloat32));

@@ -168,3 +168,16 @@ def test_operands_are_read_where_they_lie(S, QB, KB, D, layout, gpu_device):
     assert torch.equal(out, ro[:, :, :S])
     for name, a, b in zip(("dq", "dk", "dv"), grads, (dq, dk, dv)):
         assert torch.equal(a, b[:, :, :S]), name
+
+
+@pytest.mark.parametrize("S", [1, 5])
+def test_keys_and_values_with_different_row_strides(S, gpu_device):
+    """K as a model's projection leaves it, V contiguous: also for a single row, whose stride says nothing."""
+    B, H, D = 2, 3, 64
+    gen = torch.Generator().manual_seed(S)
+    q, v = (torch.randn(B, H, S, D, generator=gen).half().to(gpu_device) for _ in range(2))
+    k = torch.randn(B, S, H, D, generator=gen).half().to(gpu_device).transpose(1, 2)
+    m = oat.create_causal_omni_block_mask(B, H, S, S, 128, 128, device=gpu_device)
+    out = oat.omni_attention_shared_kv_swizzle(q, k, v, m)
+    ref, _ = attention_dense_fp32(q.cpu(), k.cpu(), v.cpu(), torch.tril(torch.ones(S, S, dtype=torch.bool)))
+    assert (out.float().cpu() - ref).abs().max().item() <= 2e-3

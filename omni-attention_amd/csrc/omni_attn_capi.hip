@@ -200,6 +200,19 @@ int forward(const void* q, const void* k, const void* v, const omni_attn_strides
     while ((H / X) % heads != 0) --heads;  // whole batch elements per group sequence
   }
   p.slab_group = heads * ((fill + heads - 1) / heads);
+  // With fewer than four groups' worth of workgroups, the last group's longest lists, which start when
+  // the group before runs out, are a large part of the launch: all slabs are walked together then,
+  // unless they make two groups that fill the slots alike (there the masks of a group count for more).
+  // D=64 causal, us, in groups -> together: B H=40 S=2048 (groups of 4 and 1) 42.2 -> 34.7, B H=64 S=1536
+  // (6 and 2) 41.2 -> 31.2, B H=48 S=3000 (2, 2 and 2) 85.4 -> 77.6, B H=96 S=2048 (4, 4 and 4) 80.0 ->
+  // 71.9; two even groups, B H=128 S=1024, 31.1 -> 31.7 (unaligned spans 36.5 -> 39.3).
+  const long long slabs = ((long long)p.n_slabs * p.parts + X - 1) / X;  // (or parts) of one XCD
+  const bool even_pair = slabs == 2LL * p.slab_group && 10LL * p.slab_group * part_tiles >= 9LL * slots_per_xcd;
+  p.flat_first = 0;
+  if (p.slab_group < slabs && slabs <= 64 && slabs * part_tiles < 4LL * slots_per_xcd && !even_pair) {
+    p.slab_group = int(slabs);
+    p.flat_first = p.n_slabs > H;  // batch elements may have masks of their own
+  }
   p.softcap = softcap;
   p.cap_c2 = softcap > 0.f ? float(2.0 * 1.4426950408889634 / (std::sqrt(double(D)) * double(softcap))) : 0.f;
   p.sl2 = softcap > 0.f ? float(1.4426950408889634) : float(1.4426950408889634 / std::sqrt(double(D)));

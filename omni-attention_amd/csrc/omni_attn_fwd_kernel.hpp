@@ -80,17 +80,32 @@ constexpr int fwd_split_rows(FwdSplit s, int QB) {
 // holds 2048 such waves.  With fewer tiles than that the longest list is the time of the launch, and
 // sharing its steps shortens it; with more, the split costs K/V loads per row (a tile of 32 rows
 // loads four times what one of 128 rows does, against 64 bytes per cycle and compute unit) and the
-// merge, and whole blocks are faster.  The lines lie where the measured times cross (causal and
-// unaligned-span masks, B H = 4 .. 128, S = 256 .. 8192).  Causal, us, whole blocks -> chosen:
-//   D=128  B H=8  S=256 10.0 -> 8.4, S=1024 22.0 -> 13.5, S=2048 38.9 -> 25.6, S=4096 71.8 -> 58.8
-//   D=64   B H=8  S=512 11.7 -> 8.2, S=2048 30.6 -> 17.5, S=4096 56.9 -> 38.0, S=8192 115 -> 99
+// merge, and whole blocks are faster.  A workgroup of eight waves (kRows64x4, kRows128x2) has a compute
+// unit to itself: beyond 256 of them only what starts last and is short may be left over, so those
+// need lists long against the start and end of a workgroup.  The lines lie where the measured times
+// cross (causal and unaligned-span masks, B H = 4 .. 128, S = 256 .. 8192).  Causal, us, whole blocks ->
+// chosen:
+//   D=128  B H=8   S=256 10.0 -> 8.4, S=1024 22.0 -> 13.5, S=2048 38.9 -> 25.6, S=4096 71.8 -> 58.8
+//          B H=24  S=1024 22.5 -> 21.1, S=1536 32.3 -> 29.3;  B H=32 S=1237 28.5 -> 25.2
+//          B H=20 S=2048 41.7 (kRows64x2 36.8; unaligned spans 42.9, 46.2)
+//          B H=40  S=512 14.2 (kRows64x4 18.4), S=1024 25.0 (kRows64x2 24.1; unaligned spans 24.9, 27.3)
+//   D=64   B H=8   S=512 11.7 -> 8.2, S=2048 30.6 -> 17.5, S=4096 56.9 -> 38.0, S=8192 115 -> 99
+//          B H=24  S=1536 24.8 -> 18.6;  B H=32 S=1237 21.5 -> 17.3;  B H=48 S=1024 18.5 (kRows64x2 19.3)
 inline FwdSplit fwd_choose_split(int D, int QB, long long rows32, int S) {
   if (rows32 <= (D == 128 ? 256 : 512)) return FwdSplit::kRows32x4;
   const bool some = (rows32 <= 1024 && S >= 512) || (rows32 <= 2048 && S >= 2048);
-  if (D != 128) return some ? FwdSplit::kRows64x2 : FwdSplit::kNone;
-  if (rows32 <= 768 && S >= 512) return FwdSplit::kRows64x4;
-  if (QB != 128) return some ? FwdSplit::kRows64x2 : FwdSplit::kNone;
-  return (rows32 <= 2048 && S >= 2 * rows32) ? FwdSplit::kRows128x2 : FwdSplit::kNone;
+  if (QB != 128) {
+    if (D == 128 && rows32 <= 768 && S >= 512) return FwdSplit::kRows64x4;
+    return some ? FwdSplit::kRows64x2 : FwdSplit::kNone;
+  }
+  if (D != 128) {
+    const bool more = (rows32 <= 1280 && S >= 1024) || (rows32 <= 1536 && S >= 1536);
+    return some || more ? FwdSplit::kRows64x2 : FwdSplit::kNone;
+  }
+  if ((rows32 <= 512 && S >= 512) || (rows32 <= 768 && S >= 1152)) return FwdSplit::kRows64x4;
+  if (rows32 <= 768 && S >= 1024) return FwdSplit::kRows64x2;
+  if ((rows32 <= 1152 && S >= 1152) || (rows32 <= 2048 && S >= 2 * rows32)) return FwdSplit::kRows128x2;
+  return (rows32 <= 1280 && S >= 1152 && S < 1536) ? FwdSplit::kRows64x2 : FwdSplit::kNone;
 }
 
 struct FwdParams {
@@ -121,6 +136,7 @@ struct FwdParams {
   int n_slabs;     // B*H
   int n_xcd;       // XCDs (L2 domains) of the device; workgroup ids go round-robin over them
   int slab_group;  // slabs of one XCD that are walked together (>= 1)
+  int flat_first;  // (at most 64 slabs per XCD) slabs without short lists go first
   float sl2;       // log2(e) / sqrt(D); log2(e) when scores are soft-capped (they are scaled there)
   float softcap;   // > 0: scores s / sqrt(D) are replaced by softcap * tanh(s / sqrt(D) / softcap)
   float cap_c2;    // 2 * log2(e) / (sqrt(D) * softcap)
@@ -400,13 +416,40 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   const int slabs_here = (p.n_slabs * p.parts - xcd + p.n_xcd - 1) / p.n_xcd;
   const int part_tiles = (p.tiles + p.parts - 1) / p.parts;
   if (slot >= slabs_here * part_tiles) return;
+  // Batch elements may have different masks.  Slabs whose first query block lists more than half of the
+  // KV blocks (nothing is masked, say: all their lists are long) go first, so that the launch ends with
+  // short lists: a load at the start of a workgroup, and a sequence of groups for either kind.  Where all
+  // slabs are one group: a third of the batch unmasked, D=128 B H=64 S=1536, 67.1 us in groups, 75.6 as one,
+  // 63.2 as one with this.  With many groups the load costs 1-2 % and the end of the launch is small.
+  uint64_t kind = 0;  // bit i: slab i of this XCD is of the kind that is dealt here (0: all are)
+  int at = slot, slabs_kind = slabs_here;
+  if (p.flat_first) {
+    const int i = threadIdx.x & 63;
+    bool flat = false;
+    if (i < slabs_here)
+      flat = 2 * p.kv_num_blocks[size_t((xcd + p.n_xcd * i) / p.parts) * size_t(p.Tq)] > p.Tk;
+    const uint64_t flats = __builtin_amdgcn_ballot_w64(flat);
+    const int n = __builtin_popcountll(flats);
+    if (n != 0 && n != slabs_here) {
+      const bool early = slot < n * part_tiles;
+      kind = __builtin_amdgcn_ballot_w64(i < slabs_here && flat == early);
+      at = early ? slot : slot - n * part_tiles;
+      slabs_kind = early ? n : slabs_here - n;
+    }
+  }
   const int per_group = p.slab_group * part_tiles;
-  const int gi = slot / per_group;
-  const int in_group = slot - gi * per_group;
-  const int g_left = slabs_here - gi * p.slab_group;
+  const int gi = at / per_group;
+  const int in_group = at - gi * per_group;
+  const int g_left = slabs_kind - gi * p.slab_group;
   const int g_eff = g_left < p.slab_group ? g_left : p.slab_group;
   const int qrank = in_group / g_eff;
-  const int dealt = xcd + p.n_xcd * (gi * p.slab_group + (in_group - qrank * g_eff));
+  int pick = gi * p.slab_group + (in_group - qrank * g_eff);  // which slab of its kind
+  if (kind != 0) {
+    const int i = threadIdx.x & 63;
+    const int rank = __builtin_amdgcn_mbcnt_hi(uint32_t(kind >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(kind), 0u));
+    pick = __builtin_ctzll(__builtin_amdgcn_ballot_w64(((kind >> i) & 1) != 0 && rank == pick));
+  }
+  const int dealt = xcd + p.n_xcd * pick;
   const int bh = dealt / p.parts;
   const int qt = p.tiles - 1 - (qrank * p.parts + dealt - bh * p.parts);  // query tile
   const int q0 = qt * QT;  // first row of this workgroup

@@ -64,3 +64,21 @@ def test_split_walks_backward(softcap, D, QB, KB, H, S, gpu_device):
         got = run_fwd_bwd(q, k, v, dout, nb, idx, tys, QB, KB, seqlen, pidx, pm, device=gpu_device, softcap=softcap)
         dense = dense_mask_from_blocks(nb, idx, tys, QB, KB, S, S, pidx, pm, seqlen_orig=seqlen)
         check_grads(got[:3], attention_dense_grads(q, k, v, dense, dout, softcap=softcap), dtype, f"seqlen {seqlen}")
+
+
+@pytest.mark.parametrize("H,S", [(10, 2048), (12, 1500)])
+def test_slabs_walked_together_with_different_masks(H, S, gpu_device):
+    """A batch of which one element attends everything, in a launch whose slabs form one group: every query
+    block is computed exactly once, whichever order the lists' lengths give."""
+    from omni_attn_torch import create_omni_block_mask_from_prefix_lengths, omni_attention_forward
+    gen = torch.Generator().manual_seed(H)
+    B, D = 4, 32
+    q, k, v = (torch.randn(B, H, S, D, generator=gen).half() for _ in range(3))
+    prefix = torch.arange(1, S + 1).repeat(B, 1)
+    prefix[1] = S
+    prefix[2, :300] = 300
+    m = create_omni_block_mask_from_prefix_lengths(prefix.to(gpu_device), H, S, S, 128, 128)
+    o, lse = omni_attention_forward(q.to(gpu_device), k.to(gpu_device), v.to(gpu_device), m)
+    allow = torch.arange(S).view(1, 1, S) < prefix.unsqueeze(-1)
+    ro, rl = attention_dense_fp32(q, k, v, allow.unsqueeze(1))
+    compare_with_oracle(o, lse, ro, rl, torch.float16, f"H={H} S={S}")

@@ -105,6 +105,8 @@ struct BwdParams {
   int parts;      // parts a slab is dealt to the XCDs in
   FwdSplit dq_split;       // how the walks of the dQ kernel are split over waves
   DkdvSplit dkdv_split;    // ... and of the dK/dV kernel
+  int slab_group;  // slabs of one XCD that are walked together (>= 1)
+  int flat_first;  // (at most 64 slabs per XCD) slabs without short lists go first
   int n_xcd;      // XCDs (L2 domains) of the device; workgroup ids go round-robin over them
   float sl2;      // log2(e) / sqrt(D)
   float scale;    // 1 / sqrt(D)
@@ -351,18 +353,15 @@ __device__ __forceinline__ void bwd_dq_walk(const BwdParams& p) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
   uint16_t* const lds16 = reinterpret_cast<uint16_t*>(lds_raw + size_t(kg) * Shape::kGroupBytes);  // [2 sets][K, V][TILE]
 
-  // Workgroup -> (slab, query block): XCD x takes the slabs bh with bh % n_xcd == x one after
-  // the other, longest query block first, so the workgroups that run together on an XCD walk the
-  // K/V rows of one or two slabs and share them through that XCD's L2.
+  // Workgroup -> (slab, query block): XCD x takes the slabs bh with bh % n_xcd == x in groups,
+  // longest query blocks of a group first, so the workgroups that run together on an XCD walk the
+  // K/V rows of a few slabs and share them through that XCD's L2.
   // (A slab may be dealt in parts, see the forward.)
-  const int slot = blockIdx.x / p.n_xcd;
-  const int xcd = blockIdx.x - slot * p.n_xcd;
   const int tiles = KG == 1 ? p.Tq : p.Tq * (QB / QT);
-  const int part_tiles = (tiles + p.parts - 1) / p.parts;
-  if (slot >= ((p.n_slabs * p.parts - xcd + p.n_xcd - 1) / p.n_xcd) * part_tiles) return;
-  const int dealt = xcd + p.n_xcd * (slot / part_tiles);
-  const int bh = dealt / p.parts;
-  const int qt = tiles - 1 - ((slot % part_tiles) * p.parts + dealt - bh * p.parts);
+  const Dealt deal = deal_slab(p, tiles, p.slab_group, p.flat_first != 0);
+  if (deal.slab < 0) return;
+  const int bh = deal.slab / p.parts;
+  const int qt = tiles - 1 - (deal.rank * p.parts + deal.slab - bh * p.parts);
   const int q0 = qt * QT;  // first row of this workgroup
   if (qt < 0 || (KG > 1 && q0 >= p.S)) return;
   const int qb = KG == 1 ? qt : q0 / QB;
@@ -817,17 +816,14 @@ __device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
   float* const sL2 = sNd + 3 * STEP;                                         // [3 sets][STEP] exponent offsets
   uint64_t* const sMatch = reinterpret_cast<uint64_t*>(lds_raw + Traits::kFixedBytes);
 
-  // Workgroup -> (slab, KV block): XCD x takes the slabs bh with bh % n_xcd == x one after the
-  // other, so the workgroups that run together on an XCD read the Q and dO rows of one slab and
-  // share them through that XCD's L2.
-  const int slot = blockIdx.x / p.n_xcd;
-  const int xcd = blockIdx.x - slot * p.n_xcd;
+  // Workgroup -> (slab, KV block): XCD x takes the slabs bh with bh % n_xcd == x in groups, first KV
+  // blocks (the longest walks of a causal mask) first, so the workgroups that run together on an XCD
+  // read the Q and dO rows of a few slabs and share them through that XCD's L2.
   const int tiles = G == 1 ? p.Tk : p.Tk * (KB / KT);
-  const int part_tiles = (tiles + p.parts - 1) / p.parts;
-  if (slot >= ((p.n_slabs * p.parts - xcd + p.n_xcd - 1) / p.n_xcd) * part_tiles) return;
-  const int dealt = xcd + p.n_xcd * (slot / part_tiles);
-  const int bh = dealt / p.parts;
-  const int kt = (slot % part_tiles) * p.parts + dealt - bh * p.parts;
+  const Dealt deal = deal_slab(p, tiles, p.slab_group, p.flat_first != 0);
+  if (deal.slab < 0) return;
+  const int bh = deal.slab / p.parts;
+  const int kt = deal.rank * p.parts + deal.slab - bh * p.parts;
   const int key0 = kt * KT;  // first key of this workgroup
   if (kt >= tiles || (G > 1 && key0 >= p.S)) return;
   const int kvb = G == 1 ? kt : key0 / KB;

@@ -371,6 +371,15 @@ int backward(const void* q, const void* k, const void* v, const void* o, const v
   }
   p.n_xcd = topo.n_xcd;
   p.parts = slab_parts(p.n_slabs, p.n_xcd);
+  // Slabs of one XCD that are walked together, longest tiles first: about eight.  One after the other,
+  // the longest lists of the last slab began when the device ran empty; with all of 16 or more together
+  // their rows leave the L2.  Both kernels, us, one / 4 / 8 / all at a time: causal D=64 B H=64 S=2048
+  // 203 / 160 / 153 / 155, B H=256 650 / 608 / 596 / 615; images D=128 B H=128 S=2500 914 / 886 / 885 /
+  // 917; unaligned spans D=128 B H=256 S=2048 1276 / 1223 / 1246 / 1334.
+  const long long slabs = ((long long)p.n_slabs * p.parts + p.n_xcd - 1) / p.n_xcd;  // (or parts)
+  const long long groups = (slabs + 3) / 8 > 1 ? (slabs + 3) / 8 : 1;
+  p.slab_group = int((slabs + groups - 1) / groups);
+  p.flat_first = slabs > 1 && slabs <= 64 && p.n_slabs > H;  // batch elements may have masks of their own
   p.scale = float(1.0 / std::sqrt(double(D)));
   p.sl2 = float(1.4426950408889634 / std::sqrt(double(D)));
   p.softcap = softcap;

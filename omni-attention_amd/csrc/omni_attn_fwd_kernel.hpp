@@ -369,6 +369,56 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
+// Which slab (or part of one) a workgroup has, and which of its tiles, longest first; slab -1: none.
+// `tiles` per slab, `group` slabs are walked together (the kernels say why); Params: of the forward or the
+// backward.
+struct Dealt {
+  int slab, rank;
+};
+template <class Params>
+__device__ __forceinline__ Dealt deal_slab(const Params& p, int tiles, int group, bool flat_first) {
+  const int wg = blockIdx.x;
+  const int slot = wg / p.n_xcd;
+  const int xcd = wg - slot * p.n_xcd;
+  const int slabs_here = (p.n_slabs * p.parts - xcd + p.n_xcd - 1) / p.n_xcd;
+  const int part_tiles = (tiles + p.parts - 1) / p.parts;
+  if (slot >= slabs_here * part_tiles) return {-1, 0};
+  // Batch elements may have different masks.  Slabs whose first query block lists more than half of the
+  // KV blocks (nothing is masked, say: all their lists are long) go first, so that the launch ends with
+  // short lists: a load at the start of a workgroup, and a sequence of groups for either kind.  Where all
+  // slabs are one group: a third of the batch unmasked, D=128 B H=64 S=1536, 67.1 us in groups, 75.6 as one,
+  // 63.2 as one with this.  With many groups the load costs 1-2 % and the end of the launch is small.
+  uint64_t kind = 0;  // bit i: slab i of this XCD is of the kind that is dealt here (0: all are)
+  int at = slot, slabs_kind = slabs_here;
+  if (flat_first) {
+    const int i = threadIdx.x & 63;
+    bool flat = false;
+    if (i < slabs_here)
+      flat = 2 * p.kv_num_blocks[size_t((xcd + p.n_xcd * i) / p.parts) * size_t(p.Tq)] > p.Tk;
+    const uint64_t flats = __builtin_amdgcn_ballot_w64(flat);
+    const int n = __builtin_popcountll(flats);
+    if (n != 0 && n != slabs_here) {
+      const bool early = slot < n * part_tiles;
+      kind = __builtin_amdgcn_ballot_w64(i < slabs_here && flat == early);
+      at = early ? slot : slot - n * part_tiles;
+      slabs_kind = early ? n : slabs_here - n;
+    }
+  }
+  const int per_group = group * part_tiles;
+  const int gi = at / per_group;
+  const int in_group = at - gi * per_group;
+  const int g_left = slabs_kind - gi * group;
+  const int g_eff = g_left < group ? g_left : group;
+  const int qrank = in_group / g_eff;
+  int pick = gi * group + (in_group - qrank * g_eff);  // which slab of its kind
+  if (kind != 0) {
+    const int i = threadIdx.x & 63;
+    const int rank = __builtin_amdgcn_mbcnt_hi(uint32_t(kind >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(kind), 0u));
+    pick = __builtin_ctzll(__builtin_amdgcn_ballot_w64(((kind >> i) & 1) != 0 && rank == pick));
+  }
+  return {xcd + p.n_xcd * pick, qrank};
+}
+
 template <class Shape>
 __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   constexpr bool BF16 = Shape::BF16;
@@ -410,48 +460,10 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   // slab of the group, then Tq-2, ...
   // Where there are too few slabs to go round, a slab is dealt in p.parts parts (part i has the
   // query tiles i, i + parts, ... from the end): "slab" in the lines below is a part then.
-  const int wg = blockIdx.x;
-  const int slot = wg / p.n_xcd;
-  const int xcd = wg - slot * p.n_xcd;
-  const int slabs_here = (p.n_slabs * p.parts - xcd + p.n_xcd - 1) / p.n_xcd;
-  const int part_tiles = (p.tiles + p.parts - 1) / p.parts;
-  if (slot >= slabs_here * part_tiles) return;
-  // Batch elements may have different masks.  Slabs whose first query block lists more than half of the
-  // KV blocks (nothing is masked, say: all their lists are long) go first, so that the launch ends with
-  // short lists: a load at the start of a workgroup, and a sequence of groups for either kind.  Where all
-  // slabs are one group: a third of the batch unmasked, D=128 B H=64 S=1536, 67.1 us in groups, 75.6 as one,
-  // 63.2 as one with this.  With many groups the load costs 1-2 % and the end of the launch is small.
-  uint64_t kind = 0;  // bit i: slab i of this XCD is of the kind that is dealt here (0: all are)
-  int at = slot, slabs_kind = slabs_here;
-  if (p.flat_first) {
-    const int i = threadIdx.x & 63;
-    bool flat = false;
-    if (i < slabs_here)
-      flat = 2 * p.kv_num_blocks[size_t((xcd + p.n_xcd * i) / p.parts) * size_t(p.Tq)] > p.Tk;
-    const uint64_t flats = __builtin_amdgcn_ballot_w64(flat);
-    const int n = __builtin_popcountll(flats);
-    if (n != 0 && n != slabs_here) {
-      const bool early = slot < n * part_tiles;
-      kind = __builtin_amdgcn_ballot_w64(i < slabs_here && flat == early);
-      at = early ? slot : slot - n * part_tiles;
-      slabs_kind = early ? n : slabs_here - n;
-    }
-  }
-  const int per_group = p.slab_group * part_tiles;
-  const int gi = at / per_group;
-  const int in_group = at - gi * per_group;
-  const int g_left = slabs_kind - gi * p.slab_group;
-  const int g_eff = g_left < p.slab_group ? g_left : p.slab_group;
-  const int qrank = in_group / g_eff;
-  int pick = gi * p.slab_group + (in_group - qrank * g_eff);  // which slab of its kind
-  if (kind != 0) {
-    const int i = threadIdx.x & 63;
-    const int rank = __builtin_amdgcn_mbcnt_hi(uint32_t(kind >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(kind), 0u));
-    pick = __builtin_ctzll(__builtin_amdgcn_ballot_w64(((kind >> i) & 1) != 0 && rank == pick));
-  }
-  const int dealt = xcd + p.n_xcd * pick;
-  const int bh = dealt / p.parts;
-  const int qt = p.tiles - 1 - (qrank * p.parts + dealt - bh * p.parts);  // query tile
+  const Dealt deal = deal_slab(p, p.tiles, p.slab_group, p.flat_first != 0);
+  if (deal.slab < 0) return;
+  const int bh = deal.slab / p.parts;
+  const int qt = p.tiles - 1 - (deal.rank * p.parts + deal.slab - bh * p.parts);  // query tile
   const int q0 = qt * QT;  // first row of this workgroup
   if (qt < 0 || (KG > 1 && q0 >= p.S)) return;
   const int qb = KG == 1 ? qt : q0 / QB;

@@ -82,3 +82,22 @@ def test_slabs_walked_together_with_different_masks(H, S, gpu_device):
     allow = torch.arange(S).view(1, 1, S) < prefix.unsqueeze(-1)
     ro, rl = attention_dense_fp32(q, k, v, allow.unsqueeze(1))
     compare_with_oracle(o, lse, ro, rl, torch.float16, f"H={H} S={S}")
+
+
+@pytest.mark.parametrize("H,S", [(10, 600), (16, 300)])
+def test_backward_of_slabs_walked_together_with_different_masks(H, S, gpu_device):
+    """As above for the backward: 5 slabs per XCD in one group, and 14 in two."""
+    from omni_attn_torch import create_omni_block_mask_from_prefix_lengths, omni_attention
+    from oracle.dense_oracle import attention_dense_grads
+    from test_gpu_backward import check_grads
+    gen = torch.Generator().manual_seed(H + 1)
+    B, D = (4, 32) if H == 10 else (7, 32)
+    q, k, v, dout = (torch.randn(B, H, S, D, generator=gen).half() for _ in range(4))
+    prefix = torch.arange(1, S + 1).repeat(B, 1)
+    prefix[1] = S
+    prefix[2, :150] = 150
+    m = create_omni_block_mask_from_prefix_lengths(prefix.to(gpu_device), H, S, S, 64, 64)
+    leaves = [t.to(gpu_device).requires_grad_(True) for t in (q, k, v)]
+    got = torch.autograd.grad(omni_attention(*leaves, m), leaves, dout.to(gpu_device))
+    allow = (torch.arange(S).view(1, 1, S) < prefix.unsqueeze(-1)).unsqueeze(1).expand(B, H, S, S)
+    check_grads(got, attention_dense_grads(q, k, v, allow, dout), torch.float16, f"H={H} S={S}")

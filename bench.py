@@ -334,7 +334,13 @@ def operator_overhead(name, seed, dev, calls=200):
             capi()
         torch.cuda.synchronize()
     op_ms, capi_ms = wall(op), wall(capi)
+    # a short kernel ends before the host has issued the next: 1 GiB fills (at least 0.13 ms each) hold
+    # the stream back until its queue is full (an issue takes up to 12 us), so that the events
+    # bracket launches back to back
+    ballast = torch.empty(1 << 28, dtype=torch.int32, device=dev)
     a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    for _ in range(2 + int(calls * 0.012 / 0.13)):
+        ballast.fill_(0)
     a.record(stream)
     for _ in range(calls):
         capi()

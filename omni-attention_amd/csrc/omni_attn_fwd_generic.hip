@@ -25,7 +25,7 @@
 // Bound by the latency of a step (two matrix chains, the softmax and the split of the weights on the
 // vector pipe) times the steps of the longest list over the waves; from 192 columns on by LDS (a step
 // of 32 rows reads each K and V byte once for 32 query rows).  B=1 H=8 S=2048 D=96 fp16, causal in 32x32
-// blocks: 24 us; with K fragments loaded straight into registers (32 rows x 32 bytes per load) and
+// blocks: 25 us; with K fragments loaded straight into registers (32 rows x 32 bytes per load) and
 // masks evaluated on every step 34 us; one wave per row with vector arithmetic 1938 us.
 #include "../../include/omni_attn_gfx950.h"
 

@@ -458,6 +458,7 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   // each K/V tile is fetched from HBM once and served from the XCD's L2 to the other
   // query blocks.  Inside a group the order is longest-first: query block Tq-1 of each
   // slab of the group, then Tq-2, ...
+  // (Launches of few rounds walk all slabs of an XCD as one group.)
   // Where there are too few slabs to go round, a slab is dealt in p.parts parts (part i has the
   // query tiles i, i + parts, ... from the end): "slab" in the lines below is a part then.
   const Dealt deal = deal_slab(p, p.tiles, p.slab_group, p.flat_first != 0);

@@ -56,6 +56,8 @@ enum class DkdvSplit : int {
 // Both kernels together, causal, us, whole blocks -> chosen (128x128 blocks):
 //   D=128  B H=8  S=512 37.9 -> 29.5, S=1024 59.7 -> 41.0, S=2048 102.9 -> 71.7, S=4096 192.3 -> 154.9
 //   D=64   B H=8  S=512 29.4 -> 20.2, S=1024 46.2 -> 26.5, S=2048  79.7 -> 51.1, S=4096 146.9 -> 103.0
+//   dK/dV split, B H=16: D=64 S=1157 45.8 -> 39.0 (soft-capped spans 64.9 -> 58.9), S=1536 56.2 -> 47.3;
+//   D=128 S=1157 57.8 -> 50.9; not at B H=24 S=1024 D=64 (41.9, 37.3; spans 42.1, 43.5; soft-capped 56.5, 62.9)
 inline FwdSplit bwd_choose_dq_split(int D, int QB, long long rows32, int S) {
   if (rows32 <= (D == 128 ? 256 : 512)) return FwdSplit::kRows32x4;
   bool two;
@@ -68,11 +70,11 @@ inline FwdSplit bwd_choose_dq_split(int D, int QB, long long rows32, int S) {
 }
 inline DkdvSplit bwd_choose_dkdv_split(int D, int KB, bool capped, long long rows32, int S) {
   if (D != 128 && rows32 <= 256) return DkdvSplit::kKeys32x4;
-  bool two = rows32 <= 512;
+  bool two = rows32 <= 512 || (rows32 <= 640 && S >= 1152);
   if (D == 128) {
     two = two || (rows32 <= 1024 && S >= (KB == 128 ? 4096 : 1024));
   } else if (!capped) {
-    two = two || (rows32 <= 1536 && S >= 2048) || (rows32 <= 2048 && S >= 4096);
+    two = two || (rows32 <= 768 && S >= 1152) || (rows32 <= 1536 && S >= 2048) || (rows32 <= 2048 && S >= 4096);
   }
   return two ? DkdvSplit::kKeys64x2 : DkdvSplit::kNone;
 }

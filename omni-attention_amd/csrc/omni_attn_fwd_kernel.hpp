@@ -570,7 +570,7 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
       ln = j & 63;
       si.row0 = (itc % SPB) * STEP;
     } else {
-      if (it >= all_steps) return StepInfo{0, kMasked, -1};  // a step that this group does not have
+      if (it >= all_steps) return StepInfo{0, kMasked, -1};  // a step that this group does not have (see the drain)
       for (const int block = it / SPB;;) {
         while (rem == 0) {
           load_chunk(++chunk_at);
@@ -1001,10 +1001,14 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
         ot[dt] = mfma_32x32x16<BF16>(v_frag(sV + SET * TILE, j), pb[SET][ts >> 1][ts & 1], ot[dt]);
       }
     };
-    if ((nsteps - 1) & 1) {
-      drain(IntC<1>{});
-    } else {
-      drain(IntC<0>{});
+    // (A group without a step in the last round has weights of zero and whatever tile its loads were
+    // pointed at: rows that the list may not hold, and zero times an infinity would reach the result.)
+    if (KG == 1 || (nsteps - 1) * KG + kg < all_steps) {
+      if ((nsteps - 1) & 1) {
+        drain(IntC<1>{});
+      } else {
+        drain(IntC<0>{});
+      }
     }
   }
 

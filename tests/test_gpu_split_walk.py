@@ -46,6 +46,42 @@ def test_split_walks(dtype, D, QB, KB, H, S, gpu_device):
         assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
 
 
+@pytest.mark.parametrize("D,QB,KB,H,S", [
+    (32, 128, 64, 2, 1024), (64, 64, 64, 1, 4480), (128, 128, 128, 1, 1152),   # 32 rows, 4 groups
+    (32, 128, 64, 40, 512), (64, 64, 64, 33, 512), (128, 64, 128, 52, 512),    # 64 rows, 2 groups
+    (128, 128, 64, 20, 512),                                                   # 64 rows, 4 groups
+    (128, 128, 64, 13, 2048)])                                                 # 128 rows, 2 groups
+def test_rows_outside_the_list_never_reach_the_output(D, QB, KB, H, S, gpu_device):
+    """Windows that leave out the first keys, with lists of every length modulo the groups: what the keys and
+    values of blocks that are not listed hold (infinities, NaNs) changes no bit of the result."""
+    gen = torch.Generator().manual_seed(D + QB + S)
+    q, k, v = (torch.randn(1, H, S, D, generator=gen).half().to(gpu_device) for _ in range(3))
+    Tq, Tk = S // QB, S // KB
+    nb = torch.zeros(1, H, Tq, dtype=torch.int32)
+    idx, tys = (torch.zeros(1, H, Tq, Tk, dtype=torch.int32) for _ in range(2))
+    for qb in range(Tq):
+        last = min(((qb + 1) * QB - 1) // KB, Tk - 1)
+        n = max(0, min(last, 1 + qb % 9))  # of the blocks 1 .. last; CAUSAL cuts the last one
+        nb[:, :, qb] = n
+        idx[:, :, qb, :n] = torch.arange(last - n + 1, last + 1, dtype=torch.int32)
+        tys[:, :, qb, :n] = 1
+    seqlen = S - 13
+    args = (nb.to(gpu_device), idx.to(gpu_device), tys.to(gpu_device), QB, KB, seqlen)
+    results = []
+    for bad in (None, float("inf"), float("nan")):
+        if bad is not None:
+            k[:, :, :KB] = bad
+            v[:, :, :KB] = bad
+        o = torch.full_like(q, float("nan"))
+        lse = torch.full(q.shape[:3], float("nan"), dtype=torch.float32, device=gpu_device)
+        omni_attn_capi.fwd(q, k, v, o, lse, *args)
+        torch.cuda.synchronize()
+        results.append((o, lse))
+    assert torch.isfinite(results[0][0]).all()
+    for o, lse in results[1:]:
+        assert torch.equal(o, results[0][0]) and torch.equal(lse, results[0][1])
+
+
 @pytest.mark.parametrize("softcap", [0.0, 5.0])
 @pytest.mark.parametrize("D,QB,KB,H,S", [
     (32, 64, 128, 9, 128), (64, 128, 64, 1, 4480), (128, 128, 128, 3, 384), (64, 64, 64, 5, 192),  # 32 rows / keys, 4 groups

@@ -4,8 +4,8 @@
 // (omni-attn-mma/mma/attn_naive.cu:21-302, launcher :305-408) takes any Q_BLOCK / KV_BLOCK and
 // any head_dim up to 256 (`float out[256]`, :189-190); its MMA kernels take only
 // {64, 128}^2 x {32, 64, 128}.  This kernel keeps that generality and the slot rules, on the matrix
-// cores, at the precision of a scalar kernel: products of 16-bit operands summed in fp32, and
-// weights that enter the second product with (at least) 22 significant bits.
+// cores, at the precision of a scalar kernel: products of 16-bit operands summed in fp32, and fp32
+// weights that enter the second product with all their bits.
 //
 // One workgroup owns up to 32 query rows of one query block; its waves share the keys of the
 // block's list: the listed keys are one sequence of positions, slot * KB + offset; step n is the
@@ -16,8 +16,9 @@
 // S^T = K.Q^T and O^T = V^T.P^T with v_mfma_f32_32x32x16 as in the tuned forward: a lane owns a query
 // row; the K and V rows of a step go to tiles of the wave in LDS, straight from global memory where rows
 // lie on 16-byte boundaries (the rows of the next step are requested as soon as the products have read
-// a tile).  A weight is a sum of 16-bit parts with one product each: two for fp16 (scaled by 2^8
-// first, so that small weights stay out of the subnormals), three for bf16.
+// a tile).  A weight is a sum of three 16-bit parts with one product each.  fp16 has few exponents: weights
+// are scaled by 2^11 first, and those below 2^-12 of the reference (scores of a peaked row) leave a rest
+// that goes through two more products of the steps that have any.
 //
 // A key that a row may not attend to never reaches it, whatever its V row holds (0 * infinity would):
 // a wave whose sums end up infinite or NaN walks its list once more and leaves out the zero weights.
@@ -25,8 +26,10 @@
 // Bound by the latency of a step (two matrix chains, the softmax and the split of the weights on the
 // vector pipe) times the steps of the longest list over the waves; from 192 columns on by LDS (a step
 // of 32 rows reads each K and V byte once for 32 query rows).  B=1 H=8 S=2048 D=96 fp16, causal in 32x32
-// blocks: 25 us; with K fragments loaded straight into registers (32 rows x 32 bytes per load) and
-// masks evaluated on every step 34 us; one wave per row with vector arithmetic 1938 us.
+// blocks, launches back to back: 30 us (bf16 29), 38 where queries are four times as large (every row
+// peaked, a rest in most steps); D=95, rows at any alignment, 43.  Two parts per weight, cut off after 22 bits
+// and at 2^-32 of the reference: 28 us, but not the scalar kernel's sum.  One wave per row with vector
+// arithmetic: 1934 us.
 #include "../../include/omni_attn_gfx950.h"
 
 #include <hip/hip_runtime.h>
@@ -212,11 +215,11 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
   constexpr int KS = 2 * DT;
   constexpr int C = 4 * DT;     // 16-byte chunks of a tile row
   constexpr int NLD = 2 * DT;   // chunks of a tile per lane
-  constexpr int PARTS = BF16 ? 3 : 2;
-  constexpr float kShift = BF16 ? 0.f : 8.f;  // log2 of the factor on the weights
-  // The reference point of the exponentials follows the running maximum when that is more than this
-  // ahead (log2): weights stay below 2^(kSlack + kShift), and the sums are rarely rescaled.
-  constexpr float kSlack = 6.f;
+  constexpr int PARTS = 3;
+  // The reference point of the exponentials follows the running maximum when that is more than kSlack
+  // ahead (log2), so that the sums are rarely rescaled; kShift: log2 of the factor on the weights, which stay
+  // below 2^(kSlack + kShift), inside fp16's range.
+  constexpr float kSlack = BF16 ? 6.f : 4.f, kShift = BF16 ? 0.f : 11.f;
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
 
   const unsigned wg = blockIdx.x;
@@ -411,7 +414,8 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
       }
     } else {
       int l = lane;
-      if constexpr (decltype(again)::value) asm volatile("" : "+v"(l));  // (addresses worked out anew)
+      // (addresses worked out anew: kept over the walk they cost it registers, which the fp16 form has none left of)
+      if constexpr (decltype(again)::value || (DT == 8 && !BF16)) asm volatile("" : "+v"(l));
 #pragma unroll
       for (int i = 0; i < NLD; ++i) {
         if constexpr (decltype(again)::value) __builtin_amdgcn_sched_barrier(0);
@@ -544,9 +548,17 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
 #pragma unroll
         for (int r = 0; r < 16; ++r) st[r] = tanhf(st[r] * p.scale / p.softcap) * p.softcap;
       }
+      float mn = INFINITY;  // the lowest allowed score of this lane (fp16, for the rests of the weights)
       if (masked) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) st[r] = (keep >> r) & 1u ? st[r] : -INFINITY;
+        for (int r = 0; r < 16; ++r) {
+          const bool kept = (keep >> r) & 1u;
+          if constexpr (!BF16) mn = fminf(mn, kept ? st[r] : INFINITY);
+          st[r] = kept ? st[r] : -INFINITY;
+        }
+      } else if constexpr (!BF16) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mn = fminf(mn, st[r]);
       }
       float mx = -INFINITY;
 #pragma unroll
@@ -565,16 +577,20 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
         m_run = m_new;
       }
       const float m_ref = m_run == -INFINITY ? 0.f : m_run;
+      // The weights, in place of the scores, and their parts.
       u32x4_t pb[PARTS][2];
-      float sum = 0.f;
-#pragma unroll
-      for (int r = 0; r < 16; r += 2) {
-        float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[r], p.sl2, kShift - m_ref));
-        float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[r + 1], p.sl2, kShift - m_ref));
-        sum += p0;
-        sum += p1;
+      auto split = [&](int r) {
+        float p0 = st[r], p1 = st[r + 1];
 #pragma unroll
         for (int n = 0; n < PARTS; ++n) pb[n][r >> 3][(r & 7) >> 1] = split_part<BF16>(p0, p1);
+      };
+      float sum = 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float x = __builtin_amdgcn_exp2f(__builtin_fmaf(st[r], p.sl2, kShift - m_ref));
+        sum += x;
+        st[r] = x;
+        if (!decltype(again)::value && (r & 1)) split(r - 1);
       }
       l_run += sum;
       if constexpr (R == Rows::kDirect) {  // V is there (the next K was requested after it)
@@ -587,18 +603,13 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
       // O^T += V^T.P^T: k-slot e of lane group g in 16-key half ts is key 16 ts + 8 (e / 4) + 4 g + e % 4
       const int i16 = c & 15, j16 = c >> 4;
       if constexpr (decltype(again)::value) {
-        // one key after the other, without those of weight zero (from the parts: as exact as the products)
+        // one key after the other, without those of weight zero
 #pragma unroll 1
         for (int key = 0; key < 32; ++key) {
           const int r = (key >> 3) * 4 + (key & 3);  // its register in half-wave (key / 4) % 2
           float weight = 0.f;
 #pragma unroll
-          for (int n = 0; n < PARTS; ++n) {
-            uint32_t pair = 0;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) pair = i == (r >> 1) ? pb[n][i >> 2][i & 3] : pair;
-            weight += to_float<BF16>((r & 1 ? pair >> 16 : pair) & 0xffffu);
-          }
+          for (int i = 0; i < 16; ++i) weight = i == r ? st[i] : weight;
           weight = __shfl(weight, c + 32 * ((key >> 2) & 1), 64);
           // (the fences keep this path from costing the first walk registers)
           int turn = swizzle(key) * 16;
@@ -620,21 +631,62 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
           }
         }
       }
-#pragma unroll
-      for (int ts = 0; ts < (decltype(again)::value ? 0 : 2); ++ts) {
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
+      if constexpr (!decltype(again)::value) {
+        auto v_frag = [&](const uint8_t* tile, int ts, int dt) {
           const int chunk = 2 * (2 * dt + j16) + ((i16 & 3) >> 1);
           const int r0 = 16 * ts + 4 * g + (i16 >> 2), r1 = r0 + 8;
-          const uint8_t* a0 = sV + tile_at(r0, chunk) + (i16 & 1) * 8;
-          const uint8_t* a1 = sV + tile_at(r1, chunk) + (i16 & 1) * 8;
+          const uint8_t* a0 = tile + tile_at(r0, chunk) + (i16 & 1) * 8;
+          const uint8_t* a1 = tile + tile_at(r1, chunk) + (i16 & 1) * 8;
           const u32x2_t lo = __builtin_bit_cast(
               u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(a0)));
           const u32x2_t hi = __builtin_bit_cast(
               u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(a1)));
-          const u32x4_t a = {lo[0], lo[1], hi[0], hi[1]};
+          return u32x4_t{lo[0], lo[1], hi[0], hi[1]};
+        };
 #pragma unroll
-          for (int n = 0; n < PARTS; ++n) ot[dt] = mfma<BF16>(a, pb[n][ts], ot[dt]);
+        for (int ts = 0; ts < 2; ++ts) {
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt) {
+            const u32x4_t a = v_frag(sV, ts, dt);
+#pragma unroll
+            for (int n = 0; n < PARTS; ++n) ot[dt] = mfma<BF16>(a, pb[n][ts], ot[dt]);
+          }
+        }
+        // Weights below 1/2 (2^-(1 + kShift) of the reference) may have bits below 2^-24, where fp16 ends: that rest,
+        // times 2^39, in two rounded parts.  (Nothing above 2^-74 of the reference is dropped; beside a maximum that
+        // a V row of zeros belongs to, small weights are the result.)
+        if (!BF16 && __builtin_amdgcn_ballot_w64(__builtin_fmaf(mn, p.sl2, kShift - m_ref) < -1.f) != 0) {
+          u32x4_t part[2][2];
+#pragma unroll
+          for (int r = 0; r < 16; r += 2) {
+            float p0 = st[r], p1 = st[r + 1];
+            asm volatile("" : "+v"(p0), "+v"(p1));  // (nothing of this path is worked out before it)
+            p0 = __builtin_amdgcn_fractf(p0 * 0x1p24f) * 0x1p15f;
+            p1 = __builtin_amdgcn_fractf(p1 * 0x1p24f) * 0x1p15f;
+#pragma unroll
+            for (int n = 0; n < 2; ++n) {
+              const f16x2_t h = {(_Float16)p0, (_Float16)p1};
+              part[n][r >> 3][(r & 7) >> 1] = __builtin_bit_cast(uint32_t, h);
+              p0 -= float(h[0]);
+              p1 -= float(h[1]);
+            }
+          }
+          int fresh = 0;  // (an offset that the compiler knows nothing about: it would otherwise keep the
+          asm volatile("" : "+v"(fresh));  // fragments of this path in registers for the products below)
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt) {
+            __builtin_amdgcn_sched_barrier(0);
+            f32x16_t add = zero16;
+#pragma unroll
+            for (int ts = 0; ts < 2; ++ts) {
+              const u32x4_t a = v_frag(sV + fresh, ts, dt);
+#pragma unroll
+              for (int n = 0; n < 2; ++n) add = mfma<BF16>(a, part[n][ts], add);
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) ot[dt][r] = __builtin_fmaf(add[r], 0x1p-39f, ot[dt][r]);
+          }
+          __builtin_amdgcn_sched_barrier(0);
         }
       }
       if (go) load_tile(again, v_slab, rV, p.v_at.row, sV);

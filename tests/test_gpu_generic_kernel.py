@@ -132,3 +132,33 @@ def test_values_of_keys_that_are_not_allowed_never_reach_a_row(dtype, QB, KB, D,
     assert bool((o[..., 7, :] == 0).all()) and bool(torch.isneginf(lse[..., 7]).all())
     keep = torch.arange(S) != 7
     assert (o - clean).float()[..., keep, :].abs().max().item() <= ulp
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+@pytest.mark.parametrize("D", [5, 96, 250, 256])
+def test_small_weights_reach_the_result(dtype, D, gpu_device):
+    """A row whose largest weight meets a V row of zeros: the result is the sum of weights of 2^-8 down to
+    2^-44 of it times large values.  Weights are fp32 numbers and none is dropped, so the error is the
+    rounding of the result (half an ulp: 2^-11 or 2^-8 of it, 2^-25 where it is an fp16 subnormal) and that of
+    exponents below 64 in fp32 (64 * 2^-23 * ln 2 = 2^-17.5, of the score and of its maximum)."""
+    exps = torch.tensor([8.0, 15, 20, 26, 31, 36, 40, 44])  # of key block i, which query block i sees; its first key: 0
+    n, blk = exps.numel(), 32
+    S = n * blk
+    want = -exps.repeat_interleave(blk)
+    want[::blk] = 0
+    want *= D ** 0.5 / 1.4426950408889634
+    q, k, v = torch.zeros(1, 1, S, D), torch.zeros(1, 1, S, D), torch.full((1, 1, S, D), 60000.0)
+    v[:, :, ::blk] = 0
+    q[..., 0] = 1.0
+    q[..., 1] = 2.0 ** -8  # (a score is the sum of two rounded parts)
+    k[0, 0, :, 0] = want.to(dtype).float()
+    k[0, 0, :, 1] = (want - k[0, 0, :, 0]) * 2.0 ** 8
+    q, k, v = (t.to(dtype) for t in (q, k, v))
+    nb = torch.ones(1, 1, n, dtype=torch.int32)
+    idx = torch.arange(n, dtype=torch.int32).view(1, 1, n, 1)
+    o, _ = run_generic(q, k, v, nb, idx, torch.full_like(idx, 2), blk, blk, S, None, None, gpu_device)
+    block = torch.arange(S) // blk
+    scores = q.double() @ k.double().transpose(2, 3).contiguous() / D ** 0.5
+    ref = torch.softmax(scores.masked_fill(block != block.unsqueeze(1), float("-inf")), -1) @ v.double()
+    ulp, least = (2.0 ** -11, 2.0 ** -25) if dtype == torch.float16 else (2.0 ** -8, 0.0)
+    assert bool(((o.double().cpu() - ref).abs() <= ref * (ulp + 2.0 ** -16) + least).all())

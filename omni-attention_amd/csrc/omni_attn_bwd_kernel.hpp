@@ -37,6 +37,7 @@
 // their operands through its L2.
 #pragma once
 
+#include "omni_attn_bwd_plan.hpp"
 #include "omni_attn_fwd_kernel.hpp"
 
 namespace omni_attn {
@@ -107,6 +108,7 @@ struct BwdParams {
   int parts;      // parts a slab is dealt to the XCDs in
   FwdSplit dq_split;       // how the walks of the dQ kernel are split over waves
   DkdvSplit dkdv_split;    // ... and of the dK/dV kernel
+  int win_words, table_steps;  // metadata words and steps that the dK/dV kernel holds in LDS (dkdv_plan)
   int slab_group;  // slabs of one XCD that are walked together (>= 1)
   int flat_first;  // (at most 64 slabs per XCD) slabs without short lists go first
   int n_xcd;      // XCDs (L2 domains) of the device; workgroup ids go round-robin over them
@@ -724,24 +726,10 @@ struct BwdDkdvShape {
   static constexpr size_t kGroupBytes = kTileBytes + kHandBytes + kRowBytes;
   static constexpr size_t kFixedBytes = kGroupBytes * G;
   static_assert(size_t(G) * (G - 1) * 2 * kKeyGroups * ((D / 8 + G - 1) / G) * 1024 <= kFixedBytes, "merge in LDS");
-  // per 64-slot word of a slab's metadata: the bitmap of the slots that list this KV block (8
-  // bytes) and mode / tile index of the first (4 bytes); behind them the table of steps (8 bytes each),
-  // room for one match per word and for one word full of matches.  The launch asks for the words
-  // its metadata needs, so small problems fit two workgroups per compute unit; metadata with more
-  // words (or matches) than fit is worked through in windows.
-  static constexpr size_t kLdsLimit = size_t(160) * 1024;
-  static constexpr int table_steps(int words, int steps_per_block) { return (words + 64) * steps_per_block; }
-  static constexpr size_t lds_bytes(int words, int steps_per_block) {
-    return kFixedBytes + size_t((words + 1) / 2) * 24 + size_t(table_steps(words, steps_per_block)) * 8 + 8;
-  }
-  static constexpr int kMaxStepsPerBlock = 128 / kStep;
-  static constexpr int fitting_words() {
-    int n = 4096;
-    while (lds_bytes(n, kMaxStepsPerBlock) > kLdsLimit) --n;
-    return n;
-  }
-  static constexpr int kMaxBitmapWords = fitting_words();
-  static constexpr size_t kLdsBytes = lds_bytes(kMaxBitmapWords, kMaxStepsPerBlock);
+  // workgroups that a compute unit's registers hold (waves per SIMD: 2 at head_dim 128, 4 at 64, 5 at 32)
+  static constexpr int kWavesFit = (D == 128 ? 2 : (D == 64 ? 4 : 5)) * 256 / kThreads;
+  static_assert(kWavesFit >= 1 && kFixedBytes + dkdv_word_bytes(64) + kDkdvTail + kDkdvMinTable * 8 <= kLdsOfComputeUnit,
+                "a workgroup fits a compute unit");
 };
 // One workgroup per KV block, all steps in one group.  Query rows per step: at head_dim 128 with
 // 128-key blocks 64, worked as two 32-row halves
@@ -852,13 +840,12 @@ __device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
   const size_t meta_slab = size_t(bh) * p.Tq;
   const int chunks = (p.max_blocks + 63) / 64;  // 64-slot words per query block
   const int n_words = p.Tq * chunks;
-  // words of the bitmap held in LDS at a time (what the launch sized the allocation for)
-  const int win_words = n_words < Traits::kMaxBitmapWords ? n_words : Traits::kMaxBitmapWords;
+  const int win_words = p.win_words;  // words of the bitmap held in LDS at a time
   int32_t* const sFirst = reinterpret_cast<int32_t*>(sMatch + win_words);
   typedef __attribute__((ext_vector_type(2))) int32_t i32x2_t;
   // one entry per step: first query row; mode in the low two bits, tile index above
   i32x2_t* const sSteps = reinterpret_cast<i32x2_t*>(sFirst + ((win_words + 1) & ~1));
-  const int table_steps = Traits::table_steps(win_words, NSTEPS);
+  const int table_steps = p.table_steps;
 
   // This lane's key as B operand: K for a weight wave, V for a gradient wave (zeros for a key
   // beyond the sequence).
@@ -925,8 +912,10 @@ __device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
   // match's steps from one end).  The first wave turns the window's bitmap into a table of steps, a
   // lane per word, so that the loop gets a step with one LDS read, requested an iteration ahead
   // (a generator that found the next step from the bitmap cost every wave 500 - 700 cycles per
-  // step).  Returns the number of steps; `end` moves to the first word that is not in the table.
-  int32_t* const s_table = reinterpret_cast<int32_t*>(sSteps + table_steps);  // steps, end
+  // step).  A table holds table_steps of them, a piece of the window's walk.  Returns their number;
+  // behind the table stay the word that the next piece begins with (or `end`), the number of the window's
+  // steps before that word, and that of the next piece's first step.
+  int32_t* const s_table = reinterpret_cast<int32_t*>(sSteps + table_steps);  // steps, word, before, next
   auto steps_of = [&](int32_t info, int first_row, int& sub0) {
     sub0 = bwd_first_step<STEP>(info & 3, key0, first_row);
     const int rows = p.seqlen - first_row;
@@ -934,10 +923,15 @@ __device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
     const int n = (subs < NSTEPS ? subs : NSTEPS) - sub0;
     return n > 0 ? n : 0;
   };
-  auto build_table = [&](int base, int& end) {
+  auto build_table = [&](int base, int end, bool first_piece) {
     if (w_all == 0) {
-      int n = 0;
-      for (int w0 = base; w0 < end; w0 += 64) {
+      int w0 = base, n = 0, first = 0;
+      if (!first_piece) {
+        w0 = s_table[1];
+        n = s_table[2];
+        first = s_table[3];
+      }
+      for (; w0 < end; w0 += 64) {
         const int word = w0 + lane;
         uint64_t bits = word < end ? sMatch[word - base] : 0;
         const int qb = word / chunks, ch = word - qb * chunks;
@@ -958,36 +952,30 @@ __device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
           const int other = __shfl_up(upto, d, 64);
           upto += lane >= d ? other : 0;
         }
-        const bool fits = n + upto <= table_steps;
-        if (fits) {
-          int at = n + upto - count;
-          for (uint64_t left = bits; left != 0; left &= left - 1) {
-            const int32_t info = info_of(left);
-            const int k = steps_of(info, first_row, sub0);
-            for (int i = 0; i < k; ++i) sSteps[at++] = i32x2_t{first_row + (sub0 + i) * STEP, info};
-          }
+        int at = n + upto - count - first;  // entry of this lane's first step
+        for (uint64_t left = bits; left != 0 && at < table_steps; left &= left - 1) {
+          const int32_t info = info_of(left);
+          const int k = steps_of(info, first_row, sub0);
+          for (int i = 0; i < k; ++i, ++at)
+            if (at >= 0 && at < table_steps) sSteps[at] = i32x2_t{first_row + (sub0 + i) * STEP, info};
         }
-        const uint64_t all_fit = __builtin_amdgcn_ballot_w64(fits);
-        if (~all_fit != 0) {  // (only lists that name a block many times get here)
-          const int m = __builtin_ctzll(~all_fit);
-          if (m > 0) n += __shfl(upto, m - 1, 64);
-          end = w0 + m < end ? w0 + m : end;
-          break;
-        }
-        n += __shfl(upto, 63, 64);
+        const int all = __builtin_amdgcn_readfirstlane(__shfl(upto, 63, 64));
+        if (n + all - first > table_steps) break;  // (these words have steps of the next piece)
+        n += all;
       }
       if (lane == 0) {
-        s_table[0] = n;
-        s_table[1] = end;
+        s_table[0] = w0 < end ? table_steps : n - first;
+        s_table[1] = w0 < end ? w0 : end;
+        s_table[2] = n;
+        s_table[3] = first + table_steps;
       }
     }
     __syncthreads();
-    end = __builtin_amdgcn_readfirstlane(s_table[1]);
     return __builtin_amdgcn_readfirstlane(s_table[0]);
   };
-  int win_base = 0, win_end = win_words;  // the words of the slab the window holds
+  int win_base = 0, win_end = win_words < n_words ? win_words : n_words;  // the words of the slab the window holds
   scan_window(IntC<4>{}, 0, win_end);
-  int n_steps = build_table(0, win_end);
+  int n_steps = build_table(0, win_end, true);
   const uint32_t lds_tiles = lds_offset_of(lds16);
   const uint32_t hand_lane = lds_offset_of(sHand) + uint32_t(kg) * (NSUB * 2048u) + uint32_t(lane) * 16u;
   const uint32_t lds_nd = lds_offset_of(sNd), lds_l2 = lds_offset_of(sL2);
@@ -1272,13 +1260,18 @@ __device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
         s_cur = s_nxt;
         s_nxt = t3;
       }
-      if (__builtin_expect(win_end >= n_words, 1)) break;
-      // (rare) more words of metadata, or matches, than LDS holds: the next window
+      const bool window_done = __builtin_amdgcn_readfirstlane(s_table[1]) >= win_end;
+      if (__builtin_expect(window_done && win_end >= n_words, 1)) break;
+      // more steps, or more words of metadata, than LDS holds: the next piece of the window, or the next window
       turn = (turn + n_steps) % G;
-      win_base = win_end;
-      win_end = win_base + win_words < n_words ? win_base + win_words : n_words;
-      scan_window(IntC<1>{}, win_base, win_end);
-      n_steps = build_table(win_base, win_end);
+      if (window_done) {
+        win_base = win_end;
+        win_end = win_base + win_words < n_words ? win_base + win_words : n_words;
+        scan_window(IntC<1>{}, win_base, win_end);
+      } else {
+        __syncthreads();  // nobody reads the table any more
+      }
+      n_steps = build_table(win_base, win_end, window_done);
     }
     __syncthreads();
     if constexpr (G > 1) {
@@ -1347,10 +1340,12 @@ int launch_dq_ksplit(const BwdParams& p, hipStream_t stream) {
 
 template <class Shape, auto Kernel>
 int launch_dkdv_shape(const BwdParams& p, int tiles, hipStream_t stream) {
-  const size_t n_words = size_t(p.Tq) * size_t((p.max_blocks + 63) / 64);
-  const size_t lds = Shape::lds_bytes(n_words < size_t(Shape::kMaxBitmapWords) ? int(n_words) : Shape::kMaxBitmapWords,
-                                      p.QB / Shape::kStep);
-  return launch_bwd_kernel<Kernel>(p, tiles, Shape::kThreads, lds, Shape::kLdsBytes, stream);
+  const long long n_words = (long long)p.Tq * ((p.max_blocks + 63) / 64);
+  const DkdvPlan plan = dkdv_plan(Shape::kFixedBytes, Shape::kWavesFit, n_words, p.QB / Shape::kStep);
+  BwdParams with = p;
+  with.win_words = plan.words;
+  with.table_steps = plan.steps;
+  return launch_bwd_kernel<Kernel>(with, tiles, Shape::kThreads, plan.bytes, kLdsOfComputeUnit, stream);
 }
 template <bool BF16, bool CAP, int D, int QB, int KB>
 int launch_dkdv(const BwdParams& p, hipStream_t stream) {

@@ -203,19 +203,18 @@ def test_wide_block_lists_backward(gpu_device):
     assert (got[3].float().cpu() - fwd_ref).abs().max().item() <= 2e-3
 
 
-@pytest.mark.parametrize("dtype,D,QB,KB,S,W,windows", [
-    (torch.bfloat16, 128, 128, 128, 2048, 64 * 400, 3),   # 16 x 400 = 6400 words, 2602 held at a time
-    (torch.float16, 64, 64, 64, 1024, 64 * 300, 2),       # 16 x 300 = 4800 words, 4096 at a time
-    (torch.float16, 128, 64, 64, 1024, 64 * 300, 2),
+@pytest.mark.parametrize("dtype,D,QB,KB,H,S,W,held,windows", [
+    (torch.bfloat16, 128, 128, 128, 11, 2048, 64 * 400, 2516, 3),   # whole blocks; 16 x 400 = 6400 words
+    (torch.float16, 64, 64, 64, 2, 1024, 64 * 300, 3752, 2),        # four groups; 16 x 300 = 4800 words
+    (torch.float16, 128, 64, 64, 2, 1024, 64 * 300, 3880, 2),       # two groups
 ])
-def test_metadata_beyond_one_bitmap_window(dtype, D, QB, KB, S, W, windows, gpu_device):
+def test_metadata_beyond_one_bitmap_window(dtype, D, QB, KB, H, S, W, held, windows, gpu_device):
     """More 64-slot words of metadata per slab than the dK/dV kernel's match bitmap holds in LDS:
     the kernel scans and walks them window by window (the boundaries fall inside a query block's
     list), and the gradients are those of the same blocks in a narrow list."""
     gen = torch.Generator().manual_seed(115)
-    H = 2
     words = (S // QB) * (W // 64)
-    assert windows == -(-words // (2602 if (D, KB) == (128, 128) else 4096))
+    assert windows == -(-words // held)  # (words held at a time at most)
     q, k, v, dout = (torch.randn(1, H, S, D, generator=gen).to(dtype) for _ in range(4))
     nb, idx, tys, pidx, pm = scattered_lists(gen, H, S, QB, KB, W)
     got = run_fwd_bwd(q, k, v, dout, nb, idx, tys, QB, KB, S - 5, pidx, pm, device=gpu_device, softcap=0.0)
@@ -230,6 +229,40 @@ def test_metadata_beyond_one_bitmap_window(dtype, D, QB, KB, S, W, windows, gpu_
     got2 = run_fwd_bwd(q, k, v, dout, nb2, narrow[0], narrow[1], QB, KB, S - 5, narrow[2], pm, device=gpu_device)
     for name, a, b in zip(("dQ", "dK", "dV"), got[:3], got2[:3]):
         assert torch.equal(a, b), f"{name} differs between the wide and the narrow list"
+
+
+@pytest.mark.parametrize("dtype,D,QB,KB,H,copies,W", [
+    (torch.float16, 64, 64, 64, 64, 8, 64 * 32),       # whole blocks: 256 steps per KV block, about 160 in the table
+    (torch.bfloat16, 128, 64, 64, 2, 64, 64 * 400),    # two groups: two windows of 1024 steps, 1150 and less in the table
+    (torch.float16, 32, 64, 64, 2, 16, 64 * 56),       # four groups: 512 steps, about 320 in the table
+])
+def test_walks_of_more_steps_than_the_table_holds(dtype, D, QB, KB, H, copies, W, gpu_device):
+    """Lists that name every block several times, in as many words of metadata as leave the dK/dV kernel's table
+    of steps little room: the walk goes piece by piece.  Equal multiplicity changes no weight, so the gradients
+    are those of the dense attention; the same list without its MASKED slots gives the same bits."""
+    gen = torch.Generator().manual_seed(D + copies)
+    S = 1024
+    Tq, Tk = S // QB, S // KB
+    q, k, v, dout = (torch.randn(1, H, S, D, generator=gen).to(dtype) for _ in range(4))
+    real = Tk * copies
+    blocks = torch.stack([torch.randperm(real, generator=gen) % Tk for _ in range(Tq)]).to(torch.int32)
+    at = torch.stack([torch.randperm(W, generator=gen)[:real].sort().values for _ in range(Tq)])
+    idx = torch.zeros(Tq, W, dtype=torch.int32).scatter_(1, at, blocks)
+    tys = torch.zeros(Tq, W, dtype=torch.int32).scatter_(1, at, torch.ones_like(blocks))  # CAUSAL
+    per_head = lambda t: t.expand(1, H, *t.shape).contiguous()
+    seqlen = S - 5
+    grads = []
+    for i, t in ((idx, tys), (blocks, torch.ones_like(blocks))):
+        nb = torch.full((1, H, Tq), i.shape[1], dtype=torch.int32)
+        grads.append(run_fwd_bwd(q, k, v, dout, nb, per_head(i), per_head(t), QB, KB, seqlen, device=gpu_device)[:3])
+    rows = torch.arange(S)
+    allow = (rows <= rows.unsqueeze(1)) & (rows < seqlen) & (rows < seqlen).unsqueeze(1)
+    heads = range(min(H, 2))
+    for h in heads:
+        ref = attention_dense_grads(*(t[:, h:h + 1] for t in (q, k, v)), allow.expand(1, 1, S, S), dout[:, h:h + 1])
+        check_grads([t[:, h:h + 1] for t in grads[0]], ref, dtype, f"head {h}")
+    for name, a, b in zip(("dQ", "dK", "dV"), *grads):
+        assert torch.equal(a, b), f"{name} differs without the MASKED slots"
 
 
 def test_c2_full_size_backward_on_sampled_slabs(gpu_device):

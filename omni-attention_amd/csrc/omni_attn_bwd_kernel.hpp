@@ -44,42 +44,6 @@ namespace omni_attn {
 
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
-// How the walk of a KV block is split over waves in the dK/dV kernel.
-enum class DkdvSplit : int {
-  kNone,      // one workgroup per KV block
-  kKeys64x2,  // 64 keys, two groups of waves that share the query steps
-  kKeys32x4,  // 32 keys, four groups (head_dim <= 64)
-};
-
-// Which splits?  The reasons are the forward's (fwd_choose_split): with few rows the longest walk is the
-// time of a launch.  rows32: 32-row tiles of the launch, S: rows per slab.  The lines lie where the
-// measured times cross (causal, unaligned-span and soft-capped, B H = 4 .. 128, S = 256 .. 8192).
-// Both kernels together, causal, us, whole blocks -> chosen (128x128 blocks):
-//   D=128  B H=8  S=512 37.9 -> 29.5, S=1024 59.7 -> 41.0, S=2048 102.9 -> 71.7, S=4096 192.3 -> 154.9
-//   D=64   B H=8  S=512 29.4 -> 20.2, S=1024 46.2 -> 26.5, S=2048  79.7 -> 51.1, S=4096 146.9 -> 103.0
-//   dK/dV split, B H=16: D=64 S=1157 45.8 -> 39.0 (soft-capped spans 64.9 -> 58.9), S=1536 56.2 -> 47.3;
-//   D=128 S=1157 57.8 -> 50.9; not at B H=24 S=1024 D=64 (41.9, 37.3; spans 42.1, 43.5; soft-capped 56.5, 62.9)
-inline FwdSplit bwd_choose_dq_split(int D, int QB, long long rows32, int S) {
-  if (rows32 <= (D == 128 ? 256 : 512)) return FwdSplit::kRows32x4;
-  bool two;
-  if (D == 128) {
-    two = rows32 <= 640 || (rows32 <= 1024 && S >= (QB == 128 ? 4096 : 1024));
-  } else {
-    two = (rows32 <= 1024 && S >= 512) || (rows32 <= 1536 && S >= 1024) || (rows32 <= 2048 && S >= 4096);
-  }
-  return two ? FwdSplit::kRows64x2 : FwdSplit::kNone;
-}
-inline DkdvSplit bwd_choose_dkdv_split(int D, int KB, bool capped, long long rows32, int S) {
-  if (D != 128 && rows32 <= 256) return DkdvSplit::kKeys32x4;
-  bool two = rows32 <= 512 || (rows32 <= 640 && S >= 1152);
-  if (D == 128) {
-    two = two || (rows32 <= 1024 && S >= (KB == 128 ? 4096 : 1024));
-  } else if (!capped) {
-    two = two || (rows32 <= 768 && S >= 1152) || (rows32 <= 1536 && S >= 2048) || (rows32 <= 2048 && S >= 4096);
-  }
-  return two ? DkdvSplit::kKeys64x2 : DkdvSplit::kNone;
-}
-
 struct BwdParams {
   const uint16_t* q;
   const uint16_t* k;

@@ -169,8 +169,6 @@ int forward(const void* q, const void* k, const void* v, const omni_attn_strides
   p.H = H;
   p.QB = QB;
   p.KB = KB;
-  p.split = fwd_choose_split(D, QB, (long long)B * H * Tq * (QB / 32), Tq * QB);
-  p.tiles = Tq * (QB / fwd_split_rows(p.split, QB));
   p.n_slabs = B * H;
   DeviceTopology topo;
   if (const int e = query_topology(&topo)) {
@@ -190,6 +188,9 @@ int forward(const void* q, const void* k, const void* v, const omni_attn_strides
   // do: a bigger group was 2 % faster still on 4096-token slabs and doubled the L2 misses.
   const int slots_per_xcd = topo.cus_per_xcd * (QB == 128 ? 2 : 4);
   p.parts = slab_parts(p.n_slabs, X);
+  const long long busiest = ((long long)p.n_slabs * p.parts + X - 1) / X * ((Tq * QB / 128 + p.parts - 1) / p.parts);
+  p.split = fwd_choose_split(D, QB, (long long)B * H * Tq * (QB / 32), Tq * QB, busiest, topo.cus_per_xcd);
+  p.tiles = Tq * (QB / fwd_split_rows(p.split, QB));
   const int part_tiles = (p.tiles + p.parts - 1) / p.parts;
   const int fill = slots_per_xcd / part_tiles > 1 ? slots_per_xcd / part_tiles : 1;
   int heads = (H % X == 0) ? H / X : 1;
@@ -363,7 +364,7 @@ int backward(const void* q, const void* k, const void* v, const void* o, const v
   p.KB = KB;
   const long long rows32 = (long long)B * H * Tq * (QB / 32);
   p.dq_split = bwd_choose_dq_split(D, QB, rows32, Tq * QB);
-  p.dkdv_split = bwd_choose_dkdv_split(D, KB, softcap > 0.f, rows32, Tq * QB);
+  p.dkdv_split = bwd_choose_dkdv_split(D, softcap > 0.f, rows32, Tq * QB);
   DeviceTopology topo;
   if (const int e = query_topology(&topo)) {
     g_last_hip_error = e;

@@ -39,6 +39,8 @@
 #include <atomic>
 #include <utility>
 
+#include "omni_attn_split_rules.hpp"
+
 namespace omni_attn {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
@@ -62,51 +64,6 @@ struct RowStrides {
   int64_t b, h;
   uint32_t row;
 };
-
-// How the walk of a query block is split over waves (FwdShape below says what the numbers are).
-enum class FwdSplit : int {
-  kNone,       // one workgroup per query block
-  kRows32x4,   // 32-row tiles, four groups of one wave
-  kRows64x2,   // 64-row tiles, two groups of two waves
-  kRows64x4,   // 64-row tiles, four groups of two waves (head_dim 128)
-  kRows128x2,  // 128-row tiles, two groups of four waves (head_dim 128)
-};
-constexpr int fwd_split_rows(FwdSplit s, int QB) {
-  return s == FwdSplit::kNone ? QB : (s == FwdSplit::kRows32x4 ? 32 : (s == FwdSplit::kRows128x2 ? 128 : 64));
-}
-
-// Which split?  `rows32`: 32-row tiles of the whole launch, S: rows per slab.  A wave walks a list of up
-// to S / 64 steps of 1.2 us (alone on its SIMD, head_dim 128) to 1.7 us (two per SIMD); the device
-// holds 2048 such waves.  With fewer tiles than that the longest list is the time of the launch, and
-// sharing its steps shortens it; with more, the split costs K/V loads per row (a tile of 32 rows
-// loads four times what one of 128 rows does, against 64 bytes per cycle and compute unit) and the
-// merge, and whole blocks are faster.  A workgroup of eight waves (kRows64x4, kRows128x2) has a compute
-// unit to itself: beyond 256 of them only what starts last and is short may be left over, so those
-// need lists long against the start and end of a workgroup.  The lines lie where the measured times
-// cross (causal and unaligned-span masks, B H = 4 .. 128, S = 256 .. 8192).  Causal, us, whole blocks ->
-// chosen:
-//   D=128  B H=8   S=256 10.0 -> 8.4, S=1024 22.0 -> 13.5, S=2048 38.9 -> 25.6, S=4096 71.8 -> 58.8
-//          B H=24  S=1024 22.5 -> 21.1, S=1536 32.3 -> 29.3;  B H=32 S=1237 28.5 -> 25.2
-//          B H=20 S=2048 41.7 (kRows64x2 36.8; unaligned spans 42.9, 46.2)
-//          B H=40  S=512 14.2 (kRows64x4 18.4), S=1024 25.0 (kRows64x2 24.1; unaligned spans 24.9, 27.3)
-//   D=64   B H=8   S=512 11.7 -> 8.2, S=2048 30.6 -> 17.5, S=4096 56.9 -> 38.0, S=8192 115 -> 99
-//          B H=24  S=1536 24.8 -> 18.6;  B H=32 S=1237 21.5 -> 17.3;  B H=48 S=1024 18.5 (kRows64x2 19.3)
-inline FwdSplit fwd_choose_split(int D, int QB, long long rows32, int S) {
-  if (rows32 <= (D == 128 ? 256 : 512)) return FwdSplit::kRows32x4;
-  const bool some = (rows32 <= 1024 && S >= 512) || (rows32 <= 2048 && S >= 2048);
-  if (QB != 128) {
-    if (D == 128 && rows32 <= 768 && S >= 512) return FwdSplit::kRows64x4;
-    return some ? FwdSplit::kRows64x2 : FwdSplit::kNone;
-  }
-  if (D != 128) {
-    const bool more = (rows32 <= 1280 && S >= 1024) || (rows32 <= 1536 && S >= 1536);
-    return some || more ? FwdSplit::kRows64x2 : FwdSplit::kNone;
-  }
-  if ((rows32 <= 512 && S >= 512) || (rows32 <= 768 && S >= 1152)) return FwdSplit::kRows64x4;
-  if (rows32 <= 768 && S >= 1024) return FwdSplit::kRows64x2;
-  if ((rows32 <= 1152 && S >= 1152) || (rows32 <= 2048 && S >= 2 * rows32)) return FwdSplit::kRows128x2;
-  return (rows32 <= 1280 && S >= 1152 && S < 1536) ? FwdSplit::kRows64x2 : FwdSplit::kNone;
-}
 
 struct FwdParams {
   const uint16_t* q;

@@ -1,0 +1,107 @@
+// Where the walks of a launch with few rows are split over more waves.  (Host arithmetic, no device code.)
+#pragma once
+
+namespace omni_attn {
+
+// How the walk of a query block is split over waves (FwdShape says what the numbers are).
+enum class FwdSplit : int {
+  kNone,       // one workgroup per query block
+  kRows32x4,   // 32-row tiles, four groups of one wave
+  kRows64x2,   // 64-row tiles, two groups of two waves
+  kRows64x4,   // 64-row tiles, four groups of two waves (head_dim 128)
+  kRows128x2,  // 128-row tiles, two groups of four waves (head_dim 128)
+};
+constexpr int fwd_split_rows(FwdSplit s, int QB) {
+  return s == FwdSplit::kNone ? QB : (s == FwdSplit::kRows32x4 ? 32 : (s == FwdSplit::kRows128x2 ? 128 : 64));
+}
+
+// Which split?  `rows32`: 32-row tiles of the whole launch, S: rows per slab; `busiest`: 128-row tiles dealt
+// to the XCD that has most, `cus`: compute units of an XCD.  A wave walks a list of up
+// to S / 64 steps of 1.2 us (alone on its SIMD, head_dim 128) to 1.7 us (two per SIMD); the device
+// holds 2048 such waves.  With fewer tiles than that the longest list is the time of the launch, and
+// sharing its steps shortens it; with more, the split costs K/V loads per row (a tile of 32 rows
+// loads four times what one of 128 rows does, against 64 bytes per cycle and compute unit) and the
+// merge, and whole blocks are faster.  A workgroup of eight waves (kRows64x4, kRows128x2) has a compute
+// unit to itself: what does not start in the first round starts late, so those need one round, or
+// lists long against the start and end of a workgroup.  The lines lie where the split gains on some masks
+// and costs none of them more than runs differ by, as a rule (causal, two layouts of unaligned spans, and
+// images of 1024 tokens; B H = 4 .. 64, S = 512 .. 8192).  Whole blocks, us, and the split against them:
+//   D=128  kRows64x4   B H=16 S=1024 22-24 (-20 .. -23 %), S=1152 24 (-21, one layout +5); B H=12 S=2048 38-41
+//                      (-23 .. +3), B H=8 S=3072 54-58 (-21 .. -36); beyond: B H=20 S=1152 24 (-3 .. +24)
+//          kRows64x2   B H=20 S=1152 24 (0 .. -7), B H=24 S=1024 22-24 (-4 .. -10); beyond: B H=32 S=1237 30-35
+//                      (-6 .. -12), but S=1280 30 (-11 .. +11) and S=1408 32 (-6 .. +25)
+//          kRows128x2  B H=20 S=1300 28-34 (-7 .. -17), B H=16 S=2048 38-42 (-8 .. -11), B H=14 S=2500 48-61 (-15
+//                      .. -23), B H=12 S=4096 79-85 (-18 .. 0), B H=8 S=8192 169-175 (-2 .. -14); beyond: B H=26
+//                      S=1152 26 (+10 .. +26; 39 workgroups for 32 compute units), B H=16 S=4096 89-96 (-9 .. +14)
+//   64-row blocks: kRows64x4  B H=16 S=1237 31-40 (-34 .. -40), B H=12 S=2048 48 (-20 .. -38); kRows64x2  B H=40
+//                      S=512 16 (-12), B H=24 S=1024 27 (-23), B H=20 S=2048 50-56 (-18 .. -26)
+//   D=64   kRows64x2   B H=64 S=512 11-13 (-11 .. +3), B H=32 S=1024 18-20 (-4 .. -21), S=1237 21-28 (-14 .. -27),
+//                      B H=20 S=2048 31-34 (-6 .. -24), B H=16 S=3072 45-49 (-8 .. -23), S=4096 60-65 (-8 .. +3);
+//                      beyond: B H=40 S=1024 18-20 (0 .. +19), B H=24 S=2048 32-34 (-10 .. +16)
+//   D=32   kRows64x2   B H=40 S=1024 16-18 (-3 .. -16), B H=32 S=1536 21-24 (-10 .. -21), S=2048 28-33 (-14 .. +1)
+inline FwdSplit fwd_choose_split(int D, int QB, long long rows32, int S, long long busiest, int cus) {
+  if (rows32 <= (D == 128 ? 256 : 512)) return FwdSplit::kRows32x4;
+  const bool some = (rows32 <= 1024 && S >= 512) || (rows32 <= 1280 && S >= 2048) || (rows32 <= 2048 && S >= 2 * rows32);
+  const bool lone = (rows32 <= 512 && S >= 512) || (rows32 <= 640 && S >= 1152) || (rows32 <= 768 && S >= 1536);
+  if (QB != 128) {
+    if (D == 128 && (lone || (rows32 <= 768 && S >= 1152))) return FwdSplit::kRows64x4;
+    return some ? FwdSplit::kRows64x2 : FwdSplit::kNone;
+  }
+  if (D != 128) {
+    const bool more = D == 64 ? rows32 <= 1280 && S >= 1152
+                              : (rows32 <= 1280 && S >= 1024) || (rows32 <= 1536 && S >= 1536) || (rows32 <= 2048 && S >= 2048);
+    return some || more ? FwdSplit::kRows64x2 : FwdSplit::kNone;
+  }
+  if (lone) return FwdSplit::kRows64x4;
+  if (rows32 <= 768 && S >= 1024) return FwdSplit::kRows64x2;
+  const bool one_round = busiest <= cus || (S >= 1280 && 8 * busiest <= 9LL * cus);
+  const bool long_lists = S >= 2048 && (rows32 <= 1152 || (rows32 <= 1280 && S >= 2 * rows32) ||
+                                        (rows32 <= 2048 && 5LL * S >= 13 * rows32));
+  return (rows32 <= 1152 && S >= 1152 && one_round) || long_lists ? FwdSplit::kRows128x2 : FwdSplit::kNone;
+}
+
+// How the walk of a KV block is split over waves in the dK/dV kernel.
+enum class DkdvSplit : int {
+  kNone,      // one workgroup per KV block
+  kKeys64x2,  // 64 keys, two groups of waves that share the query steps
+  kKeys32x4,  // 32 keys, four groups (head_dim <= 64)
+};
+
+// Which splits?  The reasons are the forward's (fwd_choose_split): with few rows the longest walk is the
+// time of a launch.  rows32: 32-row tiles of the launch, S: rows per slab.  The lines lie where a split gains
+// on some masks and costs none more than runs differ by, as a rule (causal, unaligned spans, images of 1024
+// tokens; B H = 4 .. 64, S = 512 .. 4096).  Both kernels together, causal, us, whole blocks -> chosen:
+//   D=128  B H=8  S=512 37.9 -> 29.5, S=1024 59.7 -> 41.0, S=2048 102.9 -> 71.7, S=4096 192.3 -> 154.9
+//   D=64   B H=8  S=512 29.4 -> 20.2, S=1024 46.2 -> 26.5, S=2048  79.7 -> 51.1, S=4096 146.9 -> 103.0
+// The operator's backward at the lines (causal, spans, images), whole blocks, us, and the split of that kernel:
+//   dQ     D=128  B H=20 S=1024 62 (-2 .. -10 %), B H=8 S=4096 177-217 (-12 .. +3); 64-row blocks: B H=16 S=2048
+//                 107-140 (-7 .. +1), S=1024 beyond: B H=32 68-85 (+1 .. +5)
+//          D=64   B H=40 S=1024 52-59 (-3 .. +1), B H=32 S=1237 58-72 (-6 .. -12), B H=24 S=2048 87-106 (-7 .. +3), B H=16
+//                 S=4096 167-211 (-3 .. +2); 64-row blocks B H=32 S=1237 57-69 (-7 .. -13), B H=16 S=4096 172-225 (-8 .. 0)
+//   dK/dV  D=128  B H=16 S=1237 62-73 (-1 .. -13), B H=8 S=4096 176-216 (-10 .. +2); 64-key blocks B H=12 S=1237 62-71
+//                 (-8 .. -12), B H=8 S=4096 184-226 (-10 .. +1); beyond: B H=20 S=1237 69-86 (+1 .. +9)
+//          D=64   B H=16 S=1237 51-60 (-4 .. -15), soft-capped 68-77 (-10), B H=12 S=2048 71-81 (-4 .. -17), B H=20 S=2048
+//                 75-95 (0 .. -13); 64-key blocks 73-90 (-3 .. +9); beyond: B H=24 S=2048 78-106 (-2 .. +9), B H=12
+//                 S=4096 136-170 (-7 .. +6)
+inline FwdSplit bwd_choose_dq_split(int D, int QB, long long rows32, int S) {
+  if (rows32 <= (D == 128 ? 256 : 512)) return FwdSplit::kRows32x4;
+  bool two;
+  if (D == 128) {
+    two = rows32 <= 640 || (rows32 <= 1024 && S >= (QB == 128 ? 4096 : 2048));
+  } else {
+    two = (rows32 <= 1024 && S >= 512) || (rows32 <= 1536 && S >= 1024) || (rows32 <= 2048 && S >= 4096);
+  }
+  return two ? FwdSplit::kRows64x2 : FwdSplit::kNone;
+}
+inline DkdvSplit bwd_choose_dkdv_split(int D, bool capped, long long rows32, int S) {
+  if (D != 128 && rows32 <= 256) return DkdvSplit::kKeys32x4;
+  bool two = rows32 <= 512 || (rows32 <= 640 && S >= 1152);
+  if (D == 128) {
+    two = two || (rows32 <= 1024 && S >= 4096);
+  } else if (!capped) {
+    two = two || (rows32 <= 768 && S >= 1152) || (rows32 <= 1280 && S >= 2048);
+  }
+  return two ? DkdvSplit::kKeys64x2 : DkdvSplit::kNone;
+}
+
+}  // namespace omni_attn

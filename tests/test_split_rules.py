@@ -1,0 +1,61 @@
+"""The rules that split the walks of launches with few rows (csrc/omni_attn_split_rules.hpp, compiled alone).  The
+reason for a split is few rows and long lists: a launch with fewer rows of the same length, or with longer
+lists of as many rows, is split too wherever this one is.  No line is drawn around a size."""
+import os
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "omni-attention_amd", "csrc")
+
+PROGRAM = r"""
+#include "omni_attn_split_rules.hpp"
+#include <cstdio>
+using namespace omni_attn;
+int main() {
+  for (int kind = 0; kind < 6; ++kind)    // forward: busiest XCD of 20, 34 and 60 tiles; dQ; dK/dV, soft-capped
+    for (int D = 32; D <= 128; D *= 2)
+      for (int block = 64; block <= 128; block += 64)
+        for (int S = 64; S <= 16384; S += 64) {
+          printf("%d %d %d %d ", kind, D, block, S);
+          for (long long rows = 16; rows <= 4096; rows += 16) {
+            bool split;
+            if (kind < 3)
+              split = fwd_choose_split(D, block, rows, S, kind == 0 ? 20 : (kind == 1 ? 34 : 60), 32) != FwdSplit::kNone;
+            else if (kind == 3)
+              split = bwd_choose_dq_split(D, block, rows, S) != FwdSplit::kNone;
+            else
+              split = bwd_choose_dkdv_split(D, kind == 5, rows, S) != DkdvSplit::kNone;
+            putchar(split ? '1' : '0');
+          }
+          putchar('\n');
+        }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    d = tmp_path_factory.mktemp("rules")
+    (d / "rules.cpp").write_text(PROGRAM)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I", CSRC, "-o", str(d / "rules"), str(d / "rules.cpp")], check=True)
+    out = subprocess.run([str(d / "rules")], check=True, capture_output=True, text=True).stdout
+    table = {}
+    for line in out.splitlines():
+        kind, D, block, S, bits = line.split()
+        table.setdefault((int(kind), int(D), int(block)), []).append((int(S), bits))
+    return table
+
+
+@pytest.mark.parametrize("kind", range(6), ids=["fwd-one-round", "fwd-a-little-more", "fwd-more", "dq", "dkdv", "dkdv-capped"])
+def test_fewer_rows_and_longer_lists_stay_split(rules, kind):
+    for (k, D, block), by_length in rules.items():
+        if k != kind:
+            continue
+        shortest = None  # rows (in steps of 16) up to which the shorter lists are split
+        for S, bits in sorted(by_length):
+            upto = bits.find("0") if "0" in bits else len(bits)
+            assert "1" not in bits[upto:], (D, block, S, "rows")
+            assert shortest is None or upto >= shortest, (D, block, S, "length")
+            shortest = upto
+        assert 0 < upto < len(bits)  # (with the longest lists: some, and not all)

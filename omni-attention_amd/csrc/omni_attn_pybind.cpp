@@ -310,7 +310,8 @@ class HostNumber {
       return;
     }
     void* mem = nullptr;
-    const hipError_t e = hipHostMalloc(&mem, 64, hipHostMallocDefault);
+    // (portable: a word taken under one device is handed to calls on any)
+    const hipError_t e = hipHostMalloc(&mem, 64, hipHostMallocPortable | hipHostMallocMapped);
     if (e != hipSuccess) throw std::runtime_error(std::string("omni_attn: hipHostMalloc: ") + hipGetErrorString(e));
     slot_ = static_cast<int32_t*>(mem);
     slot_[0] = slot_[1] = slot_[2] = 0;

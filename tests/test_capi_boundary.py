@@ -134,3 +134,11 @@ def test_kernel_resources_of_the_built_library():
                "a.hpp:1:1: remark:     ScratchSize [bytes/lane]: 8 [-Rpass-analysis=kernel-resource-usage]\n"
                "a.hpp:1:1: remark:     Occupancy [waves/SIMD]: 5 [-Rpass-analysis=kernel-resource-usage]\n")
     assert build.parse_resource_remarks(remarks) == {"kern_a": {"vgprs": 77, "scratch_bytes": 8, "waves_per_simd": 5}}
+
+
+def test_host_memory_of_the_module_is_usable_from_every_device():
+    """Words that a kernel reports a number through are kept between calls in one list, whatever device the
+    call is on: the memory has to be taken as portable (one device cannot show the difference)."""
+    text = open(os.path.join(PKG, "csrc", "omni_attn_pybind.cpp")).read()
+    calls = re.findall(r"hipHostMalloc\(([^;]*)\);", text)
+    assert calls and all("hipHostMallocPortable" in c for c in calls)

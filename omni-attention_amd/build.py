@@ -52,9 +52,17 @@ RESOURCES_JSON = os.path.join(OBJ, "kernel_resources.json")
 # The backward kernels and the forward with split lists keep scalar values in spare vector lanes here
 # and there (SGPR spills, no memory behind them): for them only scratch memory and spilled vector registers fail the build.
 MIN_WAVES_PER_SIMD = {"fwd_kernel": 2, "fwd_ksplit": 2, "bwd_dq_kernel": 2, "bwd_dq_ksplit": 2,
-                      "bwd_dkdv_kernel": 2, "bwd_dkdv_split": 2}
-SGPR_SPILLS_ALLOWED = ("bwd_dq_", "bwd_dkdv_", "fwd_ksplit")
-NOT_GATED = ("fwd_generic_kernel",)
+                      "bwd_dkdv_kernel": 2, "bwd_dkdv_split": 2, "fwd_generic_kernel": 1,
+                      "ELi8ELNS_4Rows": 2}  # (its forms of eight waves)
+SGPR_SPILLS_ALLOWED = ("bwd_dq_", "bwd_dkdv_", "fwd_ksplit", "fwd_generic_kernel")
+# The generic kernel beyond 128 columns has one wave per SIMD and keeps some values in accumulation registers
+# (counted as spilled vector registers, no memory behind them): scratch memory is what counts.  Three forms
+# that read rows at any alignment have some: up to 32 columns and 97 - 128 in fp16 (two registers' worth; at B=1 H=8
+# S=2048 D=125 48.5 us, 52.9 without, where the addresses of the loads are worked out anew in every step) and 225 -
+# 256 in bf16 (B=1 H=4 S=1500 D=250 90.5, 103.5 us without).
+VGPR_SPILLS_ALLOWED = ("fwd_generic_kernel",)
+SCRATCH_ALLOWED = {"fwd_generic_kernelILb0ELi1ELi8ELNS_4RowsE1E": 8, "fwd_generic_kernelILb0ELi4ELi8ELNS_4RowsE1E": 8,
+                   "fwd_generic_kernelILb1ELi8ELi4ELNS_4RowsE1E": 88}
 
 INSTANCES = [(bf, d) for bf in (0, 1) for d in (32, 64, 128)]
 LIB_NAME = "libomni_attn_gfx950.so"
@@ -86,10 +94,10 @@ def check_resources(kernels):
     """Raise if a kernel uses scratch memory, spills, or falls below its waves per SIMD."""
     problems = []
     for name, r in sorted(kernels.items()):
-        if any(tag in name for tag in NOT_GATED):
-            continue
         sgpr_spills = 0 if any(tag in name for tag in SGPR_SPILLS_ALLOWED) else r.get("sgpr_spills", 0)
-        if r.get("scratch_bytes", 0) or r.get("vgpr_spills", 0) or sgpr_spills:
+        vgpr_spills = 0 if any(tag in name for tag in VGPR_SPILLS_ALLOWED) else r.get("vgpr_spills", 0)
+        scratch = max([n for tag, n in SCRATCH_ALLOWED.items() if tag in name] + [0])
+        if r.get("scratch_bytes", 0) > scratch or vgpr_spills or sgpr_spills:
             problems.append("%s: scratch %d B/lane, %d VGPR / %d SGPR spills" % (
                 name, r.get("scratch_bytes", 0), r.get("vgpr_spills", 0), r.get("sgpr_spills", 0)))
         for pattern, waves in MIN_WAVES_PER_SIMD.items():

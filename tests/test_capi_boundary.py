@@ -129,6 +129,15 @@ def test_kernel_resources_of_the_built_library():
     low = {"k_fwd_kernel_x": {"scratch_bytes": 0, "vgpr_spills": 0, "sgpr_spills": 0, "waves_per_simd": 1}}
     with pytest.raises(RuntimeError, match="waves per SIMD"):
         build.check_resources(low)
+    # the generic kernel too: scratch memory beyond the forms that are known to have some, or a lost wave of eight
+    generic = {k: dict(v) for k, v in kernels.items() if "fwd_generic_kernel" in k}
+    assert len(generic) == 34
+    for name, r in generic.items():
+        with pytest.raises(RuntimeError, match="scratch"):
+            build.check_resources({name: dict(r, scratch_bytes=r["scratch_bytes"] + 96)})
+        if "ELi8ELNS_4Rows" in name:  # eight waves
+            with pytest.raises(RuntimeError, match="waves per SIMD"):
+                build.check_resources({name: dict(r, waves_per_simd=1)})
     remarks = ("a.hpp:1:1: remark: Function Name: kern_a [-Rpass-analysis=kernel-resource-usage]\n"
                "a.hpp:1:1: remark:     VGPRs: 77 [-Rpass-analysis=kernel-resource-usage]\n"
                "a.hpp:1:1: remark:     ScratchSize [bytes/lane]: 8 [-Rpass-analysis=kernel-resource-usage]\n"

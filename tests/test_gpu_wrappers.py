@@ -181,3 +181,23 @@ def test_keys_and_values_with_different_row_strides(S, gpu_device):
     out = oat.omni_attention_shared_kv_swizzle(q, k, v, m)
     ref, _ = attention_dense_fp32(q.cpu(), k.cpu(), v.cpu(), torch.tril(torch.ones(S, S, dtype=torch.bool)))
     assert (out.float().cpu() - ref).abs().max().item() <= 2e-3
+
+
+@pytest.mark.parametrize("S", [256, 200])
+@pytest.mark.parametrize("rows", ["bhsd", "bshd"])
+def test_operands_changed_before_the_backward_are_noticed(S, rows, gpu_device):
+    """The backward reads q, k and v where they lie, whatever their length and strides: changing one in place
+    after the forward is an error and no wrong gradient."""
+    gen = torch.Generator().manual_seed(S)
+    B, H, D = 1, 2, 64
+    shape = (B, S, H, D) if rows == "bshd" else (B, H, S, D)
+    place = lambda t: t.transpose(1, 2) if rows == "bshd" else t
+    leaves = [torch.randn(*shape, generator=gen).half().to(gpu_device).requires_grad_(True) for _ in range(3)]
+    mask = create_causal_omni_block_mask(B, H, S, S, 128, 128, device=gpu_device)
+    for changed in range(3):
+        operands = [t * 1 for t in leaves]  # (leaves that need gradients may not be changed in place)
+        out = oat.omni_attention(*(place(t) for t in operands), mask)
+        with torch.no_grad():
+            operands[changed].add_(1)
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            out.sum().backward()

@@ -82,8 +82,9 @@ def test_c3_partial_shrunk_backward(packed, gpu_device):
 @pytest.mark.parametrize("D", [32, 64, 128])
 @pytest.mark.parametrize("QB,KB", [(128, 128), (128, 64), (64, 128), (64, 64)])
 def test_random_metadata_backward(dtype, D, QB, KB, softcap, gpu_device):
-    """Every instance of both backward kernels, plain and soft-capped (byte tiles, every slot kind,
-    a sequence that ends inside a block)."""
+    """Every block shape, head_dim and type, plain and soft-capped (byte tiles, every slot kind,
+    a sequence that ends inside a block).  Four slabs: the walks are split over waves; the whole-block
+    instances of both kernels are tests/test_gpu_whole_blocks.py."""
     gen = torch.Generator().manual_seed(7000 + 10 * D + QB + KB // 64)
     B, H, S = 2, 2, 512
     q, k, v, dout = (torch.randn(B, H, S, D, generator=gen).to(dtype) for _ in range(4))

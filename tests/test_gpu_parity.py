@@ -129,7 +129,8 @@ def test_config_full_size(name, gpu_device):
 def test_random_metadata_all_slot_kinds(dtype, D, QB, KB, gpu_device):
     """FULL / CAUSAL (on and off the diagonal) / PARTIAL with bits / PARTIAL without bits /
     MASKED slots, unordered kv_indices, empty query blocks, fully masked rows inside
-    listed blocks, for every (Q_BLOCK, KV_BLOCK, head_dim, dtype) instance."""
+    listed blocks, for every (Q_BLOCK, KV_BLOCK, head_dim, dtype).  (Four slabs: the walks are split over
+    waves; whole blocks are tests/test_gpu_whole_blocks.py.)"""
     gen = torch.Generator().manual_seed(1000 * D + 10 * QB + KB)
     B, H, S = 2, 2, 512
     q, k, v = (torch.randn(B, H, S, D, generator=gen).to(dtype) for _ in range(3))

@@ -63,6 +63,39 @@ def test_whole_block_walks(dtype, D, QB, KB, gpu_device):
                 assert (t[:, :, seqlen:] == 0).all(), what
 
 
+@pytest.mark.parametrize("D", [128, 64])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+@pytest.mark.parametrize("gain", [4.0, 12.0])
+def test_reference_points_that_move_often(dtype, gain, D, gpu_device):
+    """Scores whose running maximum keeps jumping by far more than the slack of the reference point: the rescale
+    of O in whole-block walks.  Bars as in test_gpu_parity's test of such scores, whose three slabs are split: rows return
+    single V entries, so an ulp of the value more than usual, and the logsumexp relative to its size."""
+    from helpers import TOL_O
+    gen = torch.Generator().manual_seed(int(gain) * 7 + D)
+    H, S, QB, KB, copies = 3, 1536, 128, 128, 15
+    assert H * copies * S // 32 > 2048
+    q = (torch.randn(1, H, S, D, generator=gen) * gain).to(dtype)
+    k, v = (torch.randn(1, H, S, D, generator=gen).to(dtype) for _ in range(2))
+    k[:, 1] -= 0.5 * q[:, 1].float().mean(1, keepdim=True).to(dtype)  # head 1: mostly negative scores
+    nb, idx, tys, pidx, pm = random_block_metadata(gen, 1, H, S // QB, S // KB, QB, KB, p_empty=0.2, shuffle=True)
+    many = lambda t: t.to(gpu_device).repeat(1, copies, *[1] * (t.dim() - 2)).contiguous()
+    qd = many(q)
+    o = torch.full_like(qd, float("nan"))
+    lse = torch.full(qd.shape[:3], float("nan"), dtype=torch.float32, device=gpu_device)
+    omni_attn_capi.fwd(qd, many(k), many(v), o, lse, many(nb), many(idx), many(tys), QB, KB, S, many(pidx),
+                       pm.to(gpu_device))
+    torch.cuda.synchronize()
+    for t in (o, lse):
+        assert torch.equal(t, t[:, :H].repeat(1, copies, *[1] * (t.dim() - 2)))
+    wo, wl = attention_dense_fp32(q, k, v, dense_mask_from_blocks(nb, idx, tys, QB, KB, S, S, pidx, pm))
+    o32, l32 = o[:, :H].float().cpu(), lse[:, :H].cpu()
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    assert ((o32 - wo).abs() - ulp * wo.abs()).max().item() <= TOL_O[dtype]
+    empty = torch.isinf(wl)
+    assert torch.equal(torch.isinf(l32), empty) and (o32[empty] == 0).all()
+    assert ((l32 - wl)[~empty].abs() / wl[~empty].abs().clamp(min=1.0)).max().item() <= TOL_LSE
+
+
 @pytest.mark.parametrize("S,QB,KB,D", [(500, 128, 128, 128), (450, 128, 64, 64), (500, 64, 128, 32), (390, 64, 64, 128)])
 def test_operands_are_read_where_they_lie(S, QB, KB, D, gpu_device):
     """A projection's [B, S, H, D] result against contiguous operands padded by hand: the same bits.  Rows behind

@@ -43,7 +43,7 @@ MFMA_PEAK_TFLOPS = 2500.0  # MI355X dense bf16 / fp16 MFMA
 # sources the run was made with; a figure whose hash is not the hash of the sources in this tree
 # describes another kernel and is not reported.
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "fwd_kernel_hbm_traffic.md")
-KERNEL_SOURCES = ("omni_attn_fwd_kernel.hpp", "omni_attn_fwd_inst.hip", "omni_attn_capi.hip")
+KERNEL_SOURCES = ("omni_attn_fwd_kernel.hpp", "omni_attn_split_rules.hpp", "omni_attn_fwd_inst.hip", "omni_attn_capi.hip")
 
 
 def kernel_source_hash() -> str:

@@ -376,7 +376,8 @@ int backward(const void* q, const void* k, const void* v, const void* o, const v
   // the longest lists of the last slab began when the device ran empty; with all of 16 or more together
   // their rows leave the L2.  Both kernels, us, one / 4 / 8 / all at a time: causal D=64 B H=64 S=2048
   // 203 / 160 / 153 / 155, B H=256 650 / 608 / 596 / 615; images D=128 B H=128 S=2500 914 / 886 / 885 /
-  // 917; unaligned spans D=128 B H=256 S=2048 1276 / 1223 / 1246 / 1334.
+  // 917; unaligned spans D=128 B H=256 S=2048 1276 / 1223 / 1246 / 1334.  Read from HBM, causal B H=256 S=2048,
+  // both kernels, MiB, one / 8 / all 32: D=64 585 / 780 / 2421, D=128 1169 / 1849 / 5034.
   const long long slabs = ((long long)p.n_slabs * p.parts + p.n_xcd - 1) / p.n_xcd;  // (or parts)
   const long long groups = (slabs + 3) / 8 > 1 ? (slabs + 3) / 8 : 1;
   p.slab_group = int((slabs + groups - 1) / groups);

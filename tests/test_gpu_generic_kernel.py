@@ -156,9 +156,11 @@ def test_small_weights_reach_the_result(dtype, D, gpu_device):
     q, k, v = (t.to(dtype) for t in (q, k, v))
     nb = torch.ones(1, 1, n, dtype=torch.int32)
     idx = torch.arange(n, dtype=torch.int32).view(1, 1, n, 1)
-    o, _ = run_generic(q, k, v, nb, idx, torch.full_like(idx, 2), blk, blk, S, None, None, gpu_device)
-    block = torch.arange(S) // blk
+    at = torch.arange(S)
+    block = at // blk
     scores = q.double() @ k.double().transpose(2, 3).contiguous() / D ** 0.5
-    ref = torch.softmax(scores.masked_fill(block != block.unsqueeze(1), float("-inf")), -1) @ v.double()
     ulp, least = (2.0 ** -11, 2.0 ** -25) if dtype == torch.float16 else (2.0 ** -8, 0.0)
-    assert bool(((o.double().cpu() - ref).abs() <= ref * (ulp + 2.0 ** -16) + least).all())
+    for kind, allow in ((2, block == block.unsqueeze(1)), (1, (block == block.unsqueeze(1)) & (at <= at.unsqueeze(1)))):
+        o, _ = run_generic(q, k, v, nb, idx, torch.full_like(idx, kind), blk, blk, S, None, None, gpu_device)
+        ref = torch.softmax(scores.masked_fill(~allow, float("-inf")), -1) @ v.double()
+        assert bool(((o.double().cpu() - ref).abs() <= ref * (ulp + 2.0 ** -16) + least).all()), kind

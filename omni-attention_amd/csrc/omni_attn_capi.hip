@@ -157,7 +157,7 @@ int forward(const void* q, const void* k, const void* v, const omni_attn_strides
   if ((long long)num_partial * QB * KB > 0x7fffffffLL * 64) return OMNI_ATTN_ERR_TOO_LARGE;
   const bool has_partial = partial_idx_or_null != nullptr && num_partial > 0 &&
                            (partial_masks_or_null != nullptr || partial_bits_or_null != nullptr);
-  p.partial_idx = has_partial ? partial_idx_or_null : nullptr;
+  p.partial_idx = has_partial ? partial_idx_or_null : block_mask_types;  // (read, and not looked at, without tiles)
   p.partial_masks = has_partial ? partial_masks_or_null : nullptr;
   p.partial_bits = has_partial ? partial_bits_or_null : nullptr;
   p.num_partial = has_partial ? num_partial : 0;

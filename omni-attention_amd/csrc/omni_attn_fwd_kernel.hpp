@@ -75,7 +75,7 @@ struct FwdParams {
   const int32_t* kv_num_blocks;  // [B,H,Tq]
   const int32_t* kv_indices;     // [B,H,Tq,max_blocks]
   const int32_t* types;          // [B,H,Tq,max_blocks]
-  const int32_t* partial_idx;    // [B,H,Tq,max_blocks] or null
+  const int32_t* partial_idx;    // [B,H,Tq,max_blocks] (any such array where num_partial is 0)
   const uint8_t* partial_masks;  // [P,QB,KB] bytes or null
   const uint32_t* partial_bits;  // [P,QB,KB/32] words (bit j of word c = key 32c + j) or null;
                                  // at most one of partial_masks / partial_bits is set
@@ -453,14 +453,13 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   // blocks).  The loads of a chunk do not depend on the block count, so the first chunk,
   // the count and Q are all in flight together at the start of the kernel.
   const bool packed_tiles = p.partial_bits != nullptr;
-  const bool has_partial = p.partial_idx != nullptr && (p.partial_masks != nullptr || packed_tiles);
   int32_t mv_row0 = 0, mv_mode = kMasked, mv_pid = -1;
   auto load_chunk = [&](int chunk) {
     const int j = chunk * 64 + lane;
     const size_t o = meta_off + size_t(j < p.max_blocks ? j : 0);
     const int32_t kvb_raw = p.kv_indices[o];
     const int32_t ty = p.types[o];
-    const int32_t pid = has_partial ? p.partial_idx[o] : -1;
+    const int32_t pid = p.partial_idx[o];
     const int32_t kvb = kvb_raw < 0 ? 0 : (kvb_raw >= p.Tk ? p.Tk - 1 : kvb_raw);
     int32_t mode = (ty == kCausal || ty == kFull || ty == kPartial) ? ty : int32_t(kMasked);
     if (ty == kPartial && (pid < 0 || pid >= p.num_partial)) mode = kMasked;
@@ -522,10 +521,10 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
     int ln;
     if constexpr (KG == 1) {
       const int itc = it < nsteps ? it : nsteps - 1;
-      const int j = itc / SPB;
-      if (itc == it && itc % SPB == 0 && (j & 63) == 0 && j > 0) load_chunk(j >> 6);
+      const int j = unsigned(itc) / unsigned(SPB), sub = unsigned(itc) % unsigned(SPB);
+      if (itc == it && sub == 0 && (j & 63) == 0 && j > 0) load_chunk(j >> 6);
       ln = j & 63;
-      si.row0 = (itc % SPB) * STEP;
+      si.row0 = sub * STEP;
     } else {
       if (it >= all_steps) return StepInfo{0, kMasked, -1};  // a step that this group does not have (see the drain)
       for (const int block = it / SPB;;) {
@@ -679,12 +678,17 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
 #pragma unroll
       for (int s2 = 0; s2 < 2; ++s2) pb[a][t][s2] = u32x4_t{0u, 0u, 0u, 0u};
     }
-  float m_run = -INFINITY;  // reference point of the exponentials, log2 domain (score * sl2)
+  // reference point of the exponentials, log2 domain (score * sl2); -inf: the row has seen no key so far
+  float m_run = q_row < p.seqlen ? -INFINITY : 0.f;  // (a row of zeros beyond the sequence needs none)
+  float m_ref = 0.f;        // what exponents are taken against: m_run, or 0 where that is -inf
   float l_run = 0.f;        // this lane's share of the running row sum
   // When the reference point moves, the rescale of O waits until the top of the next
   // iteration: the PV product that is in flight still belongs to the old reference.
   float alpha_pending = 1.f;
-  uint64_t rescale_pending = 0;  // wave-uniform: lanes whose row outgrew the reference
+  // What is owed before the next step (wave-uniform): that rescale; a look at the row maxima, because
+  // some row has no reference yet or has outgrown the one it has.
+  constexpr uint32_t kOwesRescale = 1, kOwesLook = 2;
+  uint32_t owed = kOwesLook;
 
   // ---- one iteration of the pipeline ----------------------------------------------------
   // SET = it % 2.  Reads K(it+1) from sK[SET^1] into st[SET^1], V(it-1) from sV[SET^1] with
@@ -694,7 +698,16 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   constexpr int NPV_ALL = (STEP / 16) * DT; // MFMAs of O^T
   constexpr int NL = 2 * NCH;     // tile loads per thread
   constexpr int PF_ALL = 3;       // operand fetch distance in slots
-  constexpr float kSlack = 6.f;
+  // The reference point of a row's exponentials only has to stay near the running maximum -- the
+  // result is the same sum with a different common factor -- so the slots do not look at the maximum
+  // at all: a step takes the reference as it is, and its row sums (a lane's 32 weights) tell whether a
+  // row has outgrown it.  Beyond kGrown the maxima are looked at before the next step, and the reference of
+  // rows that are more than 2^kSlack ahead moves; beyond kRedo the step itself is done again from its
+  // scores, which are still in registers (16-bit weights end at 65504; sums and O^T are far from fp32's end).
+  // Looked at in every step, on the vector pipe, the maxima cost 27 of a step's 157 vector
+  // instructions: B=2 H=32 S=4096 D=128 interleaved 316 -> 301 us, B=4 H=16 S=2048 D=64 causal 54.6 -> 51.2,
+  // B=2 H=16 S=8192 D=32 interleaved 259 -> 233.
+  constexpr float kSlack = 6.f, kGrown = 0x1p10f, kRedo = 0x1p13f;
 
   // Mask of a step whose 32x64 tile is not entirely allowed, applied to S^T before the
   // iteration that does its softmax: disallowed scores become -inf.  Register r of tile t
@@ -748,6 +761,63 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
     });
   };
 
+  // Row maximum of a step's scores, in the log2 domain (the row lives in lanes c and c + 32).
+  auto step_max = [&](auto set_c) {
+    constexpr int SET = decltype(set_c)::value;
+    float a = vmax(st[SET][0][0], st[SET][0][1]), b = vmax(st[SET][0][2], st[SET][0][3]);
+    static_for<8 * NTL - 2>([&](auto ic) {
+      constexpr int e = 2 * decltype(ic)::value + 4;
+      float& m = e & 2 ? b : a;
+      m = vmax3(m, st[SET][e / 16][e % 16], st[SET][e / 16][e % 16 + 1]);
+    });
+    return pair_max(vmax(a, b)) * p.sl2;
+  };
+  // Pair i of a step's weights, packed for the second product and added to the sums.
+  auto weights = [&](auto set_c, auto ic, float& s0, float& s1) {
+    constexpr int SET = decltype(set_c)::value, i = decltype(ic)::value;
+    constexpr int t = i / 8, r = 2 * (i % 8);
+    const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[SET][t][r], p.sl2, -m_ref));
+    const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[SET][t][r + 1], p.sl2, -m_ref));
+    if constexpr (i == 0) {
+      s0 = p0;
+      s1 = p1;
+    } else {
+      s0 += p0;
+      s1 += p1;
+    }
+    uint32_t packed = pack2<BF16>(p0, p1);
+    pin(packed);
+    pb[SET][t][r >> 3][(r & 7) >> 1] = packed;
+    pin(s0, s1);
+  };
+  // The reference becomes m_new (at least the old one); returns the factor for what was summed against
+  // the old one (exactly 0 for a row that has not seen a key yet: its sums are still 0).
+  auto set_reference = [&](float m_new) {
+    m_ref = m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = __builtin_amdgcn_exp2f(m_run - m_ref);
+    l_run *= alpha;
+    m_run = m_new;
+    return alpha;
+  };
+  auto look_again = [&]() { return __builtin_amdgcn_ballot_w64(m_run == -INFINITY) != 0 ? kOwesLook : 0u; };
+  auto look = [&](auto set_c) {
+    const float m_cand = step_max(set_c);
+    owed = 0;
+    if (__builtin_amdgcn_ballot_w64(m_cand > m_run + kSlack) != 0) {
+      alpha_pending = set_reference(vmax(m_run, m_cand));
+      owed = kOwesRescale;
+    }
+    owed |= look_again();
+  };
+  auto redo = [&](auto set_c, float& sum) {
+    const float alpha = set_reference(vmax(m_run, step_max(set_c)));
+    alpha_pending = owed & kOwesRescale ? alpha_pending * alpha : alpha;
+    float s0, s1;
+    static_for<8 * NTL>([&](auto ic) { weights(set_c, ic, s0, s1); });
+    sum = s0 + s1;
+    owed = kOwesRescale | look_again();
+  };
+
   // The first operands of an iteration are fetched right after the barrier, ahead of everything
   // else that happens between two bodies: their LDS latency runs under that bookkeeping.
   auto body_prefetch = [&](auto set_c, auto first_c, u32x4_t* opq) {
@@ -774,70 +844,12 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
     constexpr int LSP = (NS / 2) / NL > 0 ? (NS / 2) / NL : 1;  // slots between tile loads
     constexpr int LPS = (NL * LSP + NS - 1) / NS;               // loads per slot that has some
     constexpr int PF = PF_ALL < NS ? PF_ALL : NS;
-    constexpr int NMX = 2 * NTL;          // max chunks of 8 scores
     constexpr int NPR = 8 * NTL;          // pairs of exponentials
-    constexpr int NV = NMX + 1 + NPR;     // vector chunks: max, reference, exponentials
     const uint16_t* tK = sK + (SET ^ 1) * TILE;
     const uint16_t* tV = sV + (SET ^ 1) * TILE;
     auto operand = [&](int n) { return n < NPV ? v_frag(tV, n) : k_frag(tK, (n - NPV) / NTL, (n - NPV) % NTL); };
 
-    float mxa, mxb, m_ref = 0.f, rs0, rs1;
-    auto vector_chunk = [&](auto uc) {
-      constexpr int u = decltype(uc)::value;
-      if constexpr (u < 0) {
-      } else if constexpr (u < NMX) {
-        static_for<4>([&](auto ec) {
-          constexpr int e = 8 * u + 2 * decltype(ec)::value;
-          if constexpr (u == 0 && e == 0) {
-            mxa = vmax(st[SET][0][0], st[SET][0][1]);
-          } else if constexpr (u == 1 && e == 8) {
-            mxb = vmax(st[SET][0][8], st[SET][0][9]);
-          } else if constexpr ((u & 1) != 0) {
-            mxb = vmax3(mxb, st[SET][e / 16][e % 16], st[SET][e / 16][e % 16 + 1]);
-          } else {
-            mxa = vmax3(mxa, st[SET][e / 16][e % 16], st[SET][e / 16][e % 16 + 1]);
-          }
-        });
-      } else if constexpr (u == NMX) {
-        // The reference point m_run of the exponentials only has to stay within 2^kSlack of
-        // the true running max (P then stays below 2^kSlack, exact in fp32 and well inside
-        // the 16-bit types' range), so it is moved -- and O, l rescaled -- only when some
-        // row of the wave outgrows it by more than that.  The decision is wave-uniform; the
-        // result is the same sum with a different common factor.  (Written without
-        // branches: an unmoved reference gives a factor of exactly 1, or of 0 for a row that
-        // has not seen a key yet and whose sums are still 0.)
-        const float mx = pair_max(vmax(mxa, mxb));  // the row lives in lanes c and c+32
-        const float m_cand = mx * p.sl2;
-        const uint64_t movers = __builtin_amdgcn_ballot_w64(m_cand > m_run + kSlack);
-        const bool move = movers != 0;
-        const float m_new = move ? vmax(m_run, m_cand) : m_run;
-        m_ref = m_new == -INFINITY ? 0.f : m_new;
-        const float alpha = __builtin_amdgcn_exp2f(m_run - m_ref);
-        l_run *= alpha;
-        m_run = m_new;
-        alpha_pending = move ? alpha : alpha_pending;
-        rescale_pending |= movers;
-        pin(l_run, alpha_pending);
-      } else {
-        constexpr int i = u - NMX - 1;
-        constexpr int t = i / 8, r = 2 * (i % 8);
-        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[SET][t][r], p.sl2, -m_ref));
-        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[SET][t][r + 1], p.sl2, -m_ref));
-        if constexpr (i == 0) {
-          rs0 = p0;
-          rs1 = p1;
-        } else {
-          rs0 += p0;
-          rs1 += p1;
-        }
-        uint32_t packed = pack2<BF16>(p0, p1);
-        pin(packed);
-        pb[SET][t][r >> 3][(r & 7) >> 1] = packed;
-        pin(rs0, rs1);
-        if constexpr (i == NPR - 1) l_run += rs0 + rs1;
-      }
-    };
-
+    float rs0, rs1;
     // The slots run at a raised wave priority and everything between two bodies (barrier, rescale,
     // mask, metadata of the next steps) at the default one: the other wave of the SIMD, from the
     // other workgroup of the compute unit, is then not held up by this wave's bookkeeping while
@@ -857,11 +869,12 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
         constexpr int n = (j / LSP) * LPS + decltype(lc)::value;
         if constexpr (j % LSP == 0 && n < NL) issue_load(n, SET, k_row0, v_row0);
       });
-      constexpr int u_lo = j * NV / NS, u_hi = (j + 1) * NV / NS;
-      static_for<u_hi - u_lo>([&](auto dc) { vector_chunk(IntC<u_lo + decltype(dc)::value>{}); });
+      constexpr int i_lo = j * NPR / NS, i_hi = (j + 1) * NPR / NS;
+      static_for<i_hi - i_lo>([&](auto dc) { weights(set_c, IntC<i_lo + decltype(dc)::value>{}, rs0, rs1); });
       __builtin_amdgcn_sched_barrier(0);
     });
     __builtin_amdgcn_s_setprio(0);
+    return rs0 + rs1;
   };
 
   // The tiles (and packed mask words) that were requested an iteration ago have landed, for
@@ -906,17 +919,18 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
     // The common step -- every score allowed, no rescale owed, no PARTIAL tile ahead, no soft cap
     // -- goes from the barrier into the slots over one scalar condition and one branch.
     const bool next_partial = it + 1 < nsteps && nxt.mode == kPartial;
-    const bool plain = (rescale_pending == 0) & !(p.softcap > 0.f) & unmasked(cur) & !next_partial;
+    const bool plain = (owed == 0) & !(p.softcap > 0.f) & unmasked(cur) & !next_partial;
     if (!plain) {
-      if (rescale_pending != 0) {
+      if (owed & kOwesRescale) {
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
           for (int r = 0; r < 16; ++r) ot[dt][r] *= alpha_pending;
-        rescale_pending = 0;
+        owed &= ~kOwesRescale;
       }
       if (p.softcap > 0.f) apply_softcap(IntC<SET>{});
       if (!unmasked(cur)) apply_mask(IntC<SET>{}, cur);
+      if (owed & kOwesLook) look(set_c);
       if (next_partial) {
         if (packed_tiles) {
           prefetch_mask_words(it + 1, nxt);
@@ -925,7 +939,12 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
         }
       }
     }
-    body(IntC<SET>{}, first_c, nn.row0, cur.row0, opq);
+    float sum = body(set_c, first_c, nn.row0, cur.row0, opq);
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(sum <= kGrown)) != 0, 0)) {
+      owed |= kOwesLook;
+      if (__builtin_amdgcn_ballot_w64(!(sum <= kRedo)) != 0) redo(set_c, sum);
+    }
+    l_run += sum;
     if (next_partial && !packed_tiles) stage_mask_bits();
     const StepInfo n3 = step_info(it + 3);
     cur = nxt;
@@ -944,7 +963,7 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   // Drain: O^T += V^T . P^T of the last step.
   if (nsteps > 0) {
     step_barrier();
-    if (rescale_pending != 0) {
+    if (owed & kOwesRescale) {
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll

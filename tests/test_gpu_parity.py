@@ -311,6 +311,44 @@ def test_wide_score_range_moves_the_reference_often(dtype, gain, D, gpu_device):
     assert rel_l <= TOL_LSE, f"gain {gain}: LSE relative error {rel_l:.3e}"
 
 
+@pytest.mark.parametrize("D,QB,KB,H,S", [(32, 128, 128, 2, 1024), (64, 64, 128, 40, 512), (64, 128, 128, 70, 1024),
+                                         (128, 128, 128, 3, 1024), (128, 64, 64, 40, 1024), (128, 128, 64, 68, 1024)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+def test_scores_that_outgrow_the_reference(dtype, D, QB, KB, H, S, gpu_device):
+    """Scores that change by 2^3 .. 2^60 from step to step, up and down: steps that only make the next one look at its
+    maxima, and steps that are done again (weights past the 16-bit types).  Odd heads start with
+    blocks that half the rows may not see, before keys with scores near 2^-200."""
+    gen = torch.Generator().manual_seed(D + QB + S)
+    q = 1.0 + 0.05 * torch.randn(1, H, S, D, generator=gen)
+    k = 0.2 * torch.randn(1, H, S, D, generator=gen)
+    v = torch.randn(1, H, S, D, generator=gen)
+    jumps = torch.tensor([3.0, 7.0, 9.0, 11.0, 12.5, 14.0, 20.0, 60.0, -5.0, -30.0])
+    level = jumps[torch.randint(len(jumps), (H, S // 32), generator=gen)].cumsum(1).clamp(-200.0, 300.0)
+    level[1::2] -= 250.0  # (log2 of the weights, one level per 32 keys)
+    k += (level.repeat_interleave(32, 1) / (1.4427 * D ** 0.5)).view(1, H, S, 1)
+    q, k, v = q.to(dtype), k.to(dtype), v.to(dtype)
+    Tq, Tk = S // QB, S // KB
+    nb = torch.full((1, H, Tq), Tk, dtype=torch.int32)
+    idx = torch.arange(Tk, dtype=torch.int32).expand(1, H, Tq, Tk).contiguous()
+    tys = torch.full((1, H, Tq, Tk), 2, dtype=torch.int32)
+    pidx = torch.full((1, H, Tq, Tk), -1, dtype=torch.int32)
+    tys[:, 1::2, :, :2], pidx[:, 1::2, :, :2] = 3, 0
+    tile = torch.zeros(1, QB, KB, dtype=torch.bool)
+    tile[:, ::2] = True
+    args = (nb, idx, tys, QB, KB, S - 13, pidx, tile)
+    o, lse = run_kernel(q, k, v, *args, device=gpu_device)
+    dense = dense_mask_from_blocks(nb, idx, tys, QB, KB, S, S, pidx, tile, seqlen_orig=S - 13)
+    ro, rl = attention_dense_fp32(q, k, v, dense)
+    # (rows are single V entries here: one ulp of the result beside the bar, as above)
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    o32, l32 = o.float().cpu(), lse.cpu()
+    assert torch.isfinite(o32).all()
+    assert ((o32 - ro).abs() - ulp * ro.abs()).max().item() <= TOL_O[dtype]
+    live = ~torch.isinf(rl)
+    assert torch.equal(~torch.isinf(l32), live)
+    assert ((l32 - rl)[live].abs() / rl[live].abs().clamp(min=1.0)).max().item() <= TOL_LSE
+
+
 def sparse_rows_bf16_case():
     """B=2 H=9 S=1152 D=128 128/128 bf16, standard-normal operands, 80 % of the blocks left out
     and shuffled lists: many rows attend one, two or a handful of keys, so outputs are single V

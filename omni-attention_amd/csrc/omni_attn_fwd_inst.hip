@@ -21,7 +21,7 @@ int launch_fwd_blocks<OMNI_INST_BF16 != 0, OMNI_INST_D>(const FwdParams& p, int 
   constexpr bool BF = OMNI_INST_BF16 != 0;
   constexpr int D = OMNI_INST_D;
   switch (p.split) {
-    case FwdSplit::kRows32x4: return launch_fwd_ksplit<BF, D, 32, 4, 32>(p, stream);
+    case FwdSplit::kRows32x4: return launch_fwd_ksplit<BF, D, 32, 4, D == 128 ? 32 : 64>(p, stream);
     case FwdSplit::kRows64x2: return launch_fwd_ksplit<BF, D, 64, 2, D == 128 ? 32 : 64>(p, stream);
 #if OMNI_INST_D == 128
     case FwdSplit::kRows64x4: return launch_fwd_ksplit<BF, D, 64, 4, 32>(p, stream);

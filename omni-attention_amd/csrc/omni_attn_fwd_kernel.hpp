@@ -196,13 +196,22 @@ struct FwdShape {
   static constexpr int kThreads = kGroupThreads * KG;
   static constexpr int kTileElems = kStep * D;
   static constexpr bool kLone = QT == 32;  // a group is one wave: its steps need no barriers
+  static constexpr int kSets = kLone ? 1 : 2;  // tiles of K, and of V
   // per group: K tiles, V tiles, one mask word per row and 32 keys, one mask byte per row and key in
   // transit
-  static constexpr size_t kTileBytes = size_t(2) * 2 * kTileElems * sizeof(uint16_t);
+  static constexpr size_t kTileBytes = size_t(kSets) * 2 * kTileElems * sizeof(uint16_t);
   static constexpr size_t kGroupBytes = kTileBytes +
                                         size_t(QT) * (kStep / 32) * sizeof(uint32_t) + size_t(QT) * kStep;
   static constexpr size_t kLdsBytes = kGroupBytes * KG;
 };
+
+// A lone wave is bound by its own instructions (about one in five cycles) and by what a step costs beside
+// its slots, so its steps are long: 64 keys at head_dim <= 64.  What leaves LDS room for that (and for two
+// workgroups per compute unit) is one tile of K and one of V: a step fetches all its operands first, and
+// the loads of the next tiles go out once they are in registers.  Two tiles each, steps of 32 keys, one
+// tile load per instruction group, us -> now: B H=8 D=64 S=512 7.3 -> 6.6, S=2048 16.0 -> 13.5, B H=4 S=4096 26.4 -> 21.5;
+// D=32 B H=8 S=2048 13.4 -> 9.7; D=128 (32 keys) B H=4 S=2048 18.6 -> 16.2.  Eight groups of 32 rows: 6.6 -> 8.1
+// at S=512, 8.5 -> 9.0 at S=1024 (the merge, and a workgroup of eight waves).
 
 // One workgroup per query block, all steps in one group.
 // Keys per step.  A 64-row query block has half the waves; at D = 128 its 64-key tiles would
@@ -268,6 +277,30 @@ __device__ __forceinline__ void buffer_to_lds_b128(i32x4_t rsrc, uint32_t lane_o
         "s"(__builtin_amdgcn_readfirstlane(uniform_off))
       : "memory", "m0");
 }
+// Four such loads, 1 KiB of LDS apart.
+__device__ __forceinline__ void buffer_to_lds_4xb128(i32x4_t rsrc, const uint32_t (&lane_off)[4],
+                                                     const uint32_t (&uniform_off)[4], uint32_t lds_base) {
+  i32x4_t r;
+  r[0] = __builtin_amdgcn_readfirstlane(rsrc[0]);
+  r[1] = __builtin_amdgcn_readfirstlane(rsrc[1]);
+  r[2] = __builtin_amdgcn_readfirstlane(rsrc[2]);
+  r[3] = __builtin_amdgcn_readfirstlane(rsrc[3]);
+  // (the instruction offset counts for both addresses)
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "buffer_load_dwordx4 %1, %5, %6 offen lds\n\t"
+      "buffer_load_dwordx4 %2, %5, %7 offen offset:1024 lds\n\t"
+      "buffer_load_dwordx4 %3, %5, %8 offen offset:2048 lds\n\t"
+      "buffer_load_dwordx4 %4, %5, %9 offen offset:3072 lds"
+      :
+      : "s"(__builtin_amdgcn_readfirstlane(lds_base)), "v"(lane_off[0]), "v"(lane_off[1]), "v"(lane_off[2]),
+        "v"(lane_off[3]), "s"(r), "s"(__builtin_amdgcn_readfirstlane(uniform_off[0])),
+        "s"(__builtin_amdgcn_readfirstlane(uniform_off[1] - 1024u)),
+        "s"(__builtin_amdgcn_readfirstlane(uniform_off[2] - 2048u)),
+        "s"(__builtin_amdgcn_readfirstlane(uniform_off[3] - 3072u))
+      : "memory", "m0");
+}
 // 4 bytes per lane: the dword of lane l lands at lds_base + 4 * l (lanes switched off by the
 // execution mask neither load nor store).
 __device__ __forceinline__ void buffer_to_lds_b32(i32x4_t rsrc, uint32_t lane_off,
@@ -291,6 +324,13 @@ __device__ __forceinline__ void buffer_to_lds_b32(i32x4_t rsrc, uint32_t lane_of
 // tile loads that have been issued since.)
 __device__ __forceinline__ void wait_loads() {
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  asm volatile("" ::: "memory");
+}
+// ... all but the N that were issued last.
+template <int N>
+__device__ __forceinline__ void wait_loads_but() {
+  static_assert(N < 64, "six bits");
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
   asm volatile("" ::: "memory");
 }
 // Block-mask metadata is read-only for the whole launch and every read of it is
@@ -401,9 +441,10 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   const int kg = KG == 1 ? 0 : w_all / WQ;  // group of the wave (wave-uniform)
   const int w = KG == 1 ? w_all : w_all % WQ;  // wave of the group
   extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
-  uint16_t* sK = reinterpret_cast<uint16_t*>(lds_raw + size_t(kg) * Shape::kGroupBytes);  // [2][TILE]
-  uint16_t* sV = sK + 2 * TILE;                                  // [2][TILE]
-  uint32_t* sBits = reinterpret_cast<uint32_t*>(sV + 2 * TILE);  // [QT][NTL]
+  constexpr int SETS = Shape::kSets;
+  uint16_t* sK = reinterpret_cast<uint16_t*>(lds_raw + size_t(kg) * Shape::kGroupBytes);  // [SETS][TILE]
+  uint16_t* sV = sK + SETS * TILE;                                  // [SETS][TILE]
+  uint32_t* sBits = reinterpret_cast<uint32_t*>(sV + SETS * TILE);  // [QT][NTL]
   uint8_t* sMaskBytes = reinterpret_cast<uint8_t*>(sBits + QT * NTL);  // [QT][STEP]
 
   // Workgroup -> (slab, query block).  Consecutive workgroup ids go round-robin over
@@ -472,29 +513,39 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   nb = nb < 0 ? 0 : (nb > p.max_blocks ? p.max_blocks : nb);
   int all_steps = nb * SPB;
   // Groups share the steps of the live slots only (those that allow something), so a list and the same
-  // list with MASKED slots in between give the same result bit for bit.
-  uint64_t rem = 0;  // slots of the chunk in registers that the walk has not passed
-  int block_at = 0, chunk_at = 0;
-  auto live_slots = [&](int chunk) {
-    return __builtin_amdgcn_ballot_w64((chunk * 64 + lane < nb) & (mv_mode != kMasked) & (mv_row0 < p.seqlen));
+  // list with MASKED slots in between give the same result bit for bit: the live slots of a chunk are
+  // moved to the lanes 0, 1, ...
+  const int sub_bits = KG == 1 ? 0 : 31 - __builtin_clz(SPB);
+  int chunk_at = 0, live_before = 0, live_here = 0;  // chunk in registers; live slots before it and of it
+  auto take_live = [&](int chunk) {
+    const bool live = (chunk * 64 + lane < nb) & (mv_mode != kMasked) & (mv_row0 < p.seqlen);
+    const uint64_t m = __builtin_amdgcn_ballot_w64(live);
+    const int rank = __builtin_amdgcn_mbcnt_hi(uint32_t(m >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(m), 0u));
+    const int rest = __builtin_popcountll(m) + lane - rank;  // (slots that are not live go behind)
+    const int to = (live ? rank : rest) * 4;
+    mv_row0 = __builtin_amdgcn_ds_permute(to, mv_row0);
+    mv_mode = __builtin_amdgcn_ds_permute(to, mv_mode);
+    mv_pid = __builtin_amdgcn_ds_permute(to, mv_pid);
+    live_here = __builtin_popcountll(m);
   };
   if constexpr (KG > 1) {
     if (q0 >= p.seqlen) nb = 0;
-    all_steps = 0;
-    int last_row0 = 0, last_mode = kMasked;
+    int live = 0, last_row0 = 0, last_mode = kMasked;
     for (int chunk = 0; chunk * 64 < nb; ++chunk) {
       if (chunk > 0) load_chunk(chunk);
-      const uint64_t m = live_slots(chunk);
-      if (chunk == 0) rem = m;
-      if (m != 0) {
-        all_steps += __builtin_popcountll(m) * SPB;
-        const int last = 63 - __builtin_clzll(m);
-        last_row0 = __builtin_amdgcn_readlane(mv_row0, last);
-        last_mode = __builtin_amdgcn_readlane(mv_mode, last);
+      take_live(chunk);
+      if (live_here != 0) {
+        live += live_here;
+        last_row0 = __builtin_amdgcn_readlane(mv_row0, live_here - 1);
+        last_mode = __builtin_amdgcn_readlane(mv_mode, live_here - 1);
       }
     }
-    if (nb > 64) load_chunk(0);
-    if (all_steps > 0) {
+    if (nb > 64) {
+      load_chunk(0);
+      take_live(0);
+    }
+    all_steps = live << sub_bits;
+    if (live > 0) {
       // The last block of a list usually holds the diagonal or the end of the sequence: its steps
       // behind both allow nothing.
       int last_key = p.seqlen - 1;
@@ -527,17 +578,14 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
       si.row0 = sub * STEP;
     } else {
       if (it >= all_steps) return StepInfo{0, kMasked, -1};  // a step that this group does not have (see the drain)
-      for (const int block = it / SPB;;) {
-        while (rem == 0) {
-          load_chunk(++chunk_at);
-          rem = live_slots(chunk_at);
-        }
-        if (block_at == block) break;
-        rem &= rem - 1;
-        ++block_at;
+      const int block = it >> sub_bits;
+      while (block >= live_before + live_here) {
+        live_before += live_here;
+        load_chunk(++chunk_at);
+        take_live(chunk_at);
       }
-      ln = __builtin_ctzll(rem);
-      si.row0 = (it % SPB) * STEP;
+      ln = block - live_before;
+      si.row0 = (it & (SPB - 1)) * STEP;
     }
     si.row0 += __builtin_amdgcn_readlane(mv_row0, ln);
     si.mode = __builtin_amdgcn_readlane(mv_mode, ln);
@@ -578,6 +626,17 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
     const uint32_t row = uint32_t(is_v ? v_row0 : k_row0) + uint32_t(i * ROW_STRIDE);
     buffer_to_lds_b128(is_v ? rV : rK, is_v ? voff : koff[i % KPER], row * pitch, dst);
   };
+  // Four of a lone wave's loads (rows ROW_STRIDE apart, which are 1 KiB of its tile).
+  auto issue_four = [&](bool is_v, int part, int row0, uint32_t lds_tile) {
+    uint32_t lane_off[4], uniform_off[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      lane_off[i] = is_v ? voff : koff[i % KPER];
+      uniform_off[i] = uint32_t(row0 + (4 * part + i) * ROW_STRIDE) * pitch;
+    }
+    buffer_to_lds_4xb128(is_v ? rV : rK, lane_off, uniform_off, lds_tile + uint32_t(part) * 4096u);
+  };
+  static_assert(!LONE || (NCH % 4 == 0 && 4 % KPER == 0), "loads of a lone wave come in fours");
 
   // PARTIAL blocks, in two stages so that no load latency is exposed.  One iteration ahead
   // each wave fetches the STEP mask bytes of its 32 rows for that step straight into LDS
@@ -587,7 +646,7 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   // so no workgroup barrier is needed.
   constexpr int MCPR = STEP / 16;  // 16-byte chunks per row of mask bytes
   auto prefetch_mask_bytes = [&](int it, const StepInfo& si) {
-    const int half = (KG == 1 ? it : it * KG + kg) % SPB;
+    const int half = (KG == 1 ? it : it * KG + kg) & (SPB - 1);
     const i32x4_t rM = make_buffer_resource(p.partial_masks + size_t(si.pid) * size_t(QB * KB), uint32_t(QB * KB));
     const uint32_t dst = lds_offset_of(sMaskBytes) + uint32_t(w) * uint32_t(32 * STEP);
 #pragma unroll
@@ -602,7 +661,7 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   // where the byte path parks the words it packs.
   auto prefetch_mask_words = [&](int it, const StepInfo& si) {
     const uint32_t TILE_WORDS = uint32_t(QB) * uint32_t(KB / 32);
-    const int half = (KG == 1 ? it : it * KG + kg) % SPB;
+    const int half = (KG == 1 ? it : it * KG + kg) & (SPB - 1);
     const i32x4_t rM = make_buffer_resource(p.partial_bits + size_t(si.pid) * TILE_WORDS, TILE_WORDS * 4u);
     if (lane < 32 * NTL) {
       const uint32_t row = uint32_t(rb0 + 32 * w + lane / NTL);
@@ -610,8 +669,7 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
                         lds_offset_of(sBits) + uint32_t(32 * w * NTL) * 4u);
     }
   };
-  auto stage_mask_bits = [&]() {
-    wait_loads();  // the bytes have landed
+  auto stage_mask_bits = [&]() {  // (the bytes have landed)
     // word NTL * row + h of the wave's 32 rows; with one word per row the upper half-wave
     // repeats the lower one
     const int wi = lane % (32 * NTL);
@@ -697,7 +755,7 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   constexpr int NQK = NTL * KS;            // MFMAs of S^T
   constexpr int NPV_ALL = (STEP / 16) * DT; // MFMAs of O^T
   constexpr int NL = 2 * NCH;     // tile loads per thread
-  constexpr int PF_ALL = 3;       // operand fetch distance in slots
+  constexpr int PF_ALL = LONE ? NQK + NPV_ALL : 3;  // operand fetch distance in slots
   // The reference point of a row's exponentials only has to stay near the running maximum -- the
   // result is the same sum with a different common factor -- so the slots do not look at the maximum
   // at all: a step takes the reference as it is, and its row sums (a lane's 32 weights) tell whether a
@@ -818,6 +876,9 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
     owed = kOwesRescale | look_again();
   };
 
+  // The operands that were requested from a lone wave's tiles are in registers: the tiles may be overwritten.
+  auto tile_read = [&]() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
+
   // The first operands of an iteration are fetched right after the barrier, ahead of everything
   // else that happens between two bodies: their LDS latency runs under that bookkeeping.
   auto body_prefetch = [&](auto set_c, auto first_c, u32x4_t* opq) {
@@ -825,8 +886,8 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
     constexpr int NPV = decltype(first_c)::value != 0 ? 0 : NPV_ALL;
     constexpr int NS = NQK + NPV;
     constexpr int PF = PF_ALL < NS ? PF_ALL : NS;
-    const uint16_t* tK = sK + (SET ^ 1) * TILE;
-    const uint16_t* tV = sV + (SET ^ 1) * TILE;
+    const uint16_t* tK = LONE ? (NPV == 0 ? sV : sK) : sK + (SET ^ 1) * TILE;  // (K(1) of a lone wave waits in V's tile)
+    const uint16_t* tV = LONE ? sV : sV + (SET ^ 1) * TILE;
     static_for<PF>([&](auto nc) {
       constexpr int n = decltype(nc)::value;
       if constexpr (n < NPV) {
@@ -867,8 +928,19 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
       if constexpr (j + PF < NS) opq[j % PF] = operand(j + PF);
       static_for<LPS>([&](auto lc) {
         constexpr int n = (j / LSP) * LPS + decltype(lc)::value;
-        if constexpr (j % LSP == 0 && n < NL) issue_load(n, SET, k_row0, v_row0);
+        if constexpr (!LONE && j % LSP == 0 && n < NL) issue_load(n, SET, k_row0, v_row0);
       });
+      if constexpr (LONE) {  // K(it + 2) and V(it), once the operands have left the tiles
+        constexpr int J0 = NS / 4, FOURS = NL / 4, PER = (FOURS + NS - J0 - 1) / (NS - J0);
+        if constexpr (j == J0) tile_read();
+        static_for<PER>([&](auto lc) {
+          constexpr int n = (j - J0) * PER + decltype(lc)::value;
+          if constexpr (n >= 0 && n < FOURS) {
+            constexpr bool is_v = n < FOURS / 2;
+            issue_four(is_v, n % (FOURS / 2), is_v ? v_row0 : k_row0, is_v ? lds_v0 : lds_k0);
+          }
+        });
+      }
       constexpr int i_lo = j * NPR / NS, i_hi = (j + 1) * NPR / NS;
       static_for<i_hi - i_lo>([&](auto dc) { weights(set_c, IntC<i_lo + decltype(dc)::value>{}, rs0, rs1); });
       __builtin_amdgcn_sched_barrier(0);
@@ -890,16 +962,24 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
     nxt = step_info(1);
     nn = step_info(2);
     // Prologue: K(0) and K(1).
+    if constexpr (LONE) {
 #pragma unroll
-    for (int i = 0; i < NCH; ++i) {
-      issue_load(NCH + i, 0, cur.row0, 0);
-      issue_load(NCH + i, 1, nxt.row0, 0);
+      for (int i = 0; i < NCH / 4; ++i) issue_four(false, i, cur.row0, lds_k0);
+#pragma unroll
+      for (int i = 0; i < NCH / 4; ++i) issue_four(false, i, nxt.row0, lds_v0);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NCH; ++i) {
+        issue_load(NCH + i, 0, cur.row0, 0);
+        issue_load(NCH + i, 1, nxt.row0, 0);
+      }
     }
     if (cur.mode == kPartial) {
       if (packed_tiles) {
         prefetch_mask_words(0, cur);
       } else {
         prefetch_mask_bytes(0, cur);
+        wait_loads();
         stage_mask_bits();
       }
     }
@@ -945,7 +1025,10 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
       if (__builtin_amdgcn_ballot_w64(!(sum <= kRedo)) != 0) redo(set_c, sum);
     }
     l_run += sum;
-    if (next_partial && !packed_tiles) stage_mask_bits();
+    if (next_partial && !packed_tiles) {
+      wait_loads_but<LONE ? NL : 0>();  // (a lone wave has requested its tiles behind the bytes)
+      stage_mask_bits();
+    }
     const StepInfo n3 = step_info(it + 3);
     cur = nxt;
     nxt = nn;
@@ -974,7 +1057,7 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
 #pragma unroll
       for (int j = 0; j < NPV_ALL; ++j) {
         const int ts = j / DT, dt = j % DT;
-        ot[dt] = mfma_32x32x16<BF16>(v_frag(sV + SET * TILE, j), pb[SET][ts >> 1][ts & 1], ot[dt]);
+        ot[dt] = mfma_32x32x16<BF16>(v_frag(LONE ? sV : sV + SET * TILE, j), pb[SET][ts >> 1][ts & 1], ot[dt]);
       }
     };
     // (A group without a step in the last round has weights of zero and whatever tile its loads were

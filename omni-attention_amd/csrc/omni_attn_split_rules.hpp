@@ -6,7 +6,7 @@ namespace omni_attn {
 // How the walk of a query block is split over waves (FwdShape says what the numbers are).
 enum class FwdSplit : int {
   kNone,       // one workgroup per query block
-  kRows32x4,   // 32-row tiles, four groups of one wave
+  kRows32x4,   // 32-row tiles, four groups of one wave (steps without barriers)
   kRows64x2,   // 64-row tiles, two groups of two waves
   kRows64x4,   // 64-row tiles, four groups of two waves (head_dim 128)
   kRows128x2,  // 128-row tiles, two groups of four waves (head_dim 128)
@@ -26,7 +26,9 @@ constexpr int fwd_split_rows(FwdSplit s, int QB) {
 // lists long against the start and end of a workgroup.  The lines lie where the split gains on some masks
 // and costs none of them more than runs differ by, as a rule (causal, two layouts of unaligned spans, and
 // images of 1024 tokens; B H = 4 .. 64, S = 512 .. 8192).  Whole blocks, us, and the split against them:
-//   D=128  kRows64x4   B H=16 S=1024 22-24 (-20 .. -23 %), S=1152 24 (-21, one layout +5); B H=12 S=2048 38-41
+//   D=128  kRows32x4   against kRows64x4: B H=8 S=1536 19-20 (-9 .. -17 %), B H=12 S=1024 15-16 (-12 .. -18), B H=5
+//                      S=3000 30-43 (-3 .. -7), B H=2 S=8192 66-71 (-3 .. -5); beyond: B H=8 S=2048 23-24 (-3 .. +12)
+//          kRows64x4   B H=16 S=1024 22-24 (-20 .. -23 %), S=1152 24 (-21, one layout +5); B H=12 S=2048 38-41
 //                      (-23 .. +3), B H=8 S=3072 54-58 (-21 .. -36); beyond: B H=20 S=1152 24 (-3 .. +24)
 //          kRows64x2   B H=20 S=1152 24 (0 .. -7), B H=24 S=1024 22-24 (-4 .. -10); beyond: B H=32 S=1237 30-35
 //                      (-6 .. -12), but S=1280 30 (-11 .. +11) and S=1408 32 (-6 .. +25)
@@ -35,12 +37,17 @@ constexpr int fwd_split_rows(FwdSplit s, int QB) {
 //                      S=1152 26 (+10 .. +26; 39 workgroups for 32 compute units), B H=16 S=4096 89-96 (-9 .. +14)
 //   64-row blocks: kRows64x4  B H=16 S=1237 31-40 (-34 .. -40), B H=12 S=2048 48 (-20 .. -38); kRows64x2  B H=40
 //                      S=512 16 (-12), B H=24 S=1024 27 (-23), B H=20 S=2048 50-56 (-18 .. -26)
-//   D=64   kRows64x2   B H=64 S=512 11-13 (-11 .. +3), B H=32 S=1024 18-20 (-4 .. -21), S=1237 21-28 (-14 .. -27),
+//   D=64   kRows32x4   against kRows64x2: B H=16 S=1024 11 (-10), B H=8 S=2048 17 (-22), B H=4 S=4096 29 (-25);
+//                      beyond: B H=20 S=1024 12 (+31)
+//          kRows64x2   B H=64 S=512 11-13 (-11 .. +3), B H=32 S=1024 18-20 (-4 .. -21), S=1237 21-28 (-14 .. -27),
 //                      B H=20 S=2048 31-34 (-6 .. -24), B H=16 S=3072 45-49 (-8 .. -23), S=4096 60-65 (-8 .. +3);
 //                      beyond: B H=40 S=1024 18-20 (0 .. +19), B H=24 S=2048 32-34 (-10 .. +16)
-//   D=32   kRows64x2   B H=40 S=1024 16-18 (-3 .. -16), B H=32 S=1536 21-24 (-10 .. -21), S=2048 28-33 (-14 .. +1)
+//   D=32   kRows32x4   against kRows64x2: B H=16 S=1237 11-16 (-17 .. -29), B H=6 S=4096 25-27 (-17 .. -26); beyond: B H=8
+//                      S=4096 25-27 (-3 .. +7)
+//          kRows64x2   B H=40 S=1024 16-18 (-3 .. -16), B H=32 S=1536 21-24 (-10 .. -21), S=2048 28-33 (-14 .. +1)
 inline FwdSplit fwd_choose_split(int D, int QB, long long rows32, int S, long long busiest, int cus) {
-  if (rows32 <= (D == 128 ? 256 : 512)) return FwdSplit::kRows32x4;
+  const int one_round_32 = D == 128 ? 384 : (D == 64 ? 512 : 768);
+  if (rows32 <= one_round_32 || (D == 128 && rows32 <= 512 && S >= 2560)) return FwdSplit::kRows32x4;
   const bool some = (rows32 <= 1024 && S >= 512) || (rows32 <= 1280 && S >= 2048) || (rows32 <= 2048 && S >= 2 * rows32);
   const bool lone = (rows32 <= 512 && S >= 512) || (rows32 <= 640 && S >= 1152) || (rows32 <= 768 && S >= 1536);
   if (QB != 128) {

@@ -46,6 +46,13 @@ def test_split_walks(dtype, D, QB, KB, H, S, gpu_device):
         assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
 
 
+@pytest.mark.parametrize("D,QB,KB,H,S", [(32, 64, 64, 5, 4480), (128, 64, 64, 1, 8384), (64, 64, 128, 3, 448)])
+def test_lone_waves(D, QB, KB, H, S, gpu_device):
+    """Lists of up to 131 slots for waves that walk alone (live slots of several chunks moved together), and
+    lists of fewer steps than groups."""
+    test_split_walks(torch.float16, D, QB, KB, H, S - S % KB, gpu_device)
+
+
 @pytest.mark.parametrize("D,QB,KB,H,S", [
     (32, 128, 64, 2, 1024), (64, 64, 64, 1, 4480), (128, 128, 128, 1, 1152),   # 32 rows, 4 groups
     (32, 128, 64, 40, 512), (64, 64, 64, 33, 512), (128, 64, 128, 52, 512),    # 64 rows, 2 groups

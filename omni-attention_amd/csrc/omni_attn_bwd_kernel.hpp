@@ -33,6 +33,11 @@
 // exponentials of one half run under the products of the other inside one wave.  Offsets
 // (-LSE sqrt(D), -delta) and masks (-inf) go into the accumulators the products start from, so a
 // weight is one multiplication and one exp2 and an unmasked step carries no mask instruction.
+// Masks of PARTIAL steps come with the step's tiles, straight into LDS, and a step whose tile leaves nothing out
+// for the rows inside the sequence runs as an unmasked one: where the length is no multiple of the block, every block of
+// the last list is PARTIAL.  (Requested by the step that uses them, a memory latency each, and always applied:
+// forward and backward, us, before -> now, B=1 H=8 S=3000 D=128 images 230 -> 196, B=4 H=8 S=1157 D=64 85 -> 72,
+// soft-capped 95 -> 86, of which 4 from two vector instructions less per capped weight and masks only where needed.)
 // Workgroups are dealt to the XCDs by slab, so the workgroups that run together on an XCD share
 // their operands through its L2.
 #pragma once
@@ -58,12 +63,12 @@ struct BwdParams {
   // workspace [2][B,H,S], written by the dQ kernel and read by the dK/dV kernel: plane 0 is
   // -delta = -rowsum(dO . O); plane 1 the offset of the row's scores, -LSE * sqrt(D), -inf for a
   // row without any allowed key or beyond the sequence (every weight of such a row becomes 0) --
-  // or, in the soft-capped instances, the exponent offset LSE * log2(e), +inf for such a row
+  // or, in the soft-capped instances, the exponent offset (cap - LSE) * log2(e), -inf for such a row
   float* ws;
   const int32_t* kv_num_blocks;
   const int32_t* kv_indices;
   const int32_t* types;
-  const int32_t* partial_idx;
+  const int32_t* partial_idx;  // null where no tiles are stored
   const uint8_t* partial_masks;
   const uint32_t* partial_bits;
   int num_partial;
@@ -80,6 +85,7 @@ struct BwdParams {
   float scale;    // 1 / sqrt(D)
   float softcap;  // > 0: the forward replaced x = s / sqrt(D) by softcap * tanh(x / softcap)
   float cap_c2;   // 2 * log2(e) / (sqrt(D) * softcap)
+  float cap_l2;   // softcap * log2(e)
 };
 
 // sqrt(D) for the head dimensions of the instances.
@@ -88,20 +94,25 @@ struct SqrtOf {
   static constexpr float value = D == 128 ? 11.313708498984761f : (D == 64 ? 8.f : 5.656854249492381f);
 };
 
-// Weight and score-gradient factor of one score.  Plain: p = exp2(s * sl2 - lse2), factor 1.
-// Soft-capped: t = tanh(s / sqrt(D) / cap), p = exp2(cap * t * log2 e - lse2), factor 1 - t^2
-// (the derivative of cap * tanh(x / cap) with respect to x).
-template <bool CAP>
-__device__ __forceinline__ void bwd_weight(float s, float lse2, const BwdParams& p, float& w, float& dfac) {
-  if constexpr (CAP) {
-    const float ex = __builtin_amdgcn_exp2f(s * p.cap_c2);
-    const float t = __builtin_fmaf(__builtin_amdgcn_rcpf(ex + 1.f), -2.f, 1.f);
-    w = __builtin_amdgcn_exp2f(__builtin_fmaf(t, p.softcap * 1.4426950408889634f, -lse2));
-    dfac = __builtin_fmaf(-t, t, 1.f);
-  } else {
-    w = __builtin_amdgcn_exp2f(__builtin_fmaf(s, p.sl2, -lse2));
-    dfac = 1.f;
-  }
+// The kernel's arguments, read again where they are used: what only a rare path needs is not kept in scalar
+// registers over the walk (there are none left: they would be spilled to vector lanes and read back in every step).
+__device__ __forceinline__ const __attribute__((address_space(4))) BwdParams& params_again() {
+  auto* at = (const __attribute__((address_space(4))) BwdParams*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(at));
+  return *at;
+}
+
+// Soft-capped scores: with r = 1 / (exp(2 s / sqrt(D) / cap) + 1) the capped score is cap (1 - 2 r), its
+// derivative 4 r (1 - r).  A weight is exp2(off - 2 cap log2(e) r), off = cap log2(e) - lse log2(e).
+__device__ __forceinline__ float capped_r(float s, const BwdParams& p) {
+  return __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(s * p.cap_c2) + 1.f);
+}
+// Pair of 16-bit values of registers r, r + 1, zero where the mask word (shifted by 4 g) forbids them.
+template <int R>
+__device__ __forceinline__ uint32_t keep_pair(uint32_t pair, uint32_t kw) {
+  constexpr int bit = 8 * (R >> 2) + (R & 3);
+  const uint32_t lo = uint32_t(__builtin_amdgcn_sbfe(int(kw), bit, 1)), hi = uint32_t(__builtin_amdgcn_sbfe(int(kw), bit + 1, 1));
+  return pair & ((lo & 0xffffu) | (hi & 0xffff0000u));
 }
 
 // LDS reads at a byte address.  A fragment's address is (tile + lane part) ^ (k-step bits) + a
@@ -109,6 +120,9 @@ __device__ __forceinline__ void bwd_weight(float s, float lse2, const BwdParams&
 // repeat every 16 rows, so rows and tiles are immediate offsets and a fragment costs one XOR.
 __device__ __forceinline__ u32x4_t lds_b128_at(uint32_t addr) {
   return *(const __attribute__((address_space(3))) u32x4_t*)(addr);
+}
+__device__ __forceinline__ uint32_t lds_u32_at(uint32_t addr) {
+  return *(const __attribute__((address_space(3))) uint32_t*)(addr);
 }
 __device__ __forceinline__ f32x4_t lds_f32x4_at(uint32_t addr) {
   return *(const __attribute__((address_space(3))) f32x4_t*)(addr);
@@ -183,20 +197,6 @@ __device__ __forceinline__ void bwd_load_tile(i32x4_t rsrc, uint32_t pitch, int 
   for (int i = 0; i < NCH; ++i)
     buffer_to_lds_b128(rsrc, lane_off[i % PER], uint32_t(row0 + i * ROW_STRIDE) * pitch,
                        lds_tile + uint32_t(w) * 1024u + uint32_t(i) * (NT * 16u));
-}
-
-// 32 mask bytes -> 32 bits (any non-zero byte = 1), byte i -> bit i.
-__device__ __forceinline__ uint32_t bwd_pack32(const u32x4_t m0, const u32x4_t m1) {
-  uint32_t word = 0;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    uint32_t bytes = i < 4 ? m0[i] : m1[i - 4];
-    bytes |= bytes >> 4;
-    bytes |= bytes >> 2;
-    bytes |= bytes >> 1;
-    word |= (((bytes & 0x01010101u) * 0x01020408u) >> 24) << (4 * i);
-  }
-  return word;
 }
 
 // Effective mode of a slot, as the forward decides it.
@@ -291,8 +291,9 @@ struct BwdDqShape {
   static constexpr int kGroupThreads = QT * 2;
   static constexpr int kThreads = kGroupThreads * KG;
   static constexpr int kTileElems = kStep * D;
-  // two sets of two tiles (K, V), or the output staging
-  static constexpr size_t kGroupBytes = (4 * kTileElems > QT * D ? 4 * kTileElems : QT * D) * sizeof(uint16_t);
+  // two sets of two tiles (K, V), or the output staging; then one byte per row and key of a PARTIAL step
+  static constexpr size_t kTileBytes = (4 * kTileElems > QT * D ? 4 * kTileElems : QT * D) * sizeof(uint16_t);
+  static constexpr size_t kGroupBytes = kTileBytes + size_t(QT) * kStep;
   static constexpr size_t kMergeBytes = size_t(KG) * (KG - 1) * (QT / 32) * ((D / 8 + KG - 1) / KG) * 1024;
   static constexpr size_t kLdsBytes = kGroupBytes * KG > kMergeBytes ? kGroupBytes * KG : kMergeBytes;
 };
@@ -349,7 +350,7 @@ __device__ __forceinline__ void bwd_dq_walk(const BwdParams& p) {
   const int qr = q_row < p.S ? q_row : p.S - 1;
   const size_t meta_row = size_t(bh) * p.Tq + qb;
   const size_t meta_off = meta_row * p.max_blocks;
-  const bool has_partial = p.partial_idx != nullptr && (p.partial_masks != nullptr || p.partial_bits != nullptr);
+  const bool has_partial = p.partial_idx != nullptr;
 
   // Block metadata in registers, as in the forward: lane i holds block 64 * chunk + i of the list.
   int32_t mv_kvb = 0, mv_info = kMasked;  // info: effective mode in the low two bits, tile index above
@@ -407,16 +408,14 @@ __device__ __forceinline__ void bwd_dq_walk(const BwdParams& p) {
   const float delta = pair_sum(dsum);  // the row lives in lanes c and c + 32
   const float lse = p.lse[size_t(bh) * p.S + qr];
   const bool row_live = q_row < p.seqlen && lse != -INFINITY;
-  // exponent offset; +inf for rows without any allowed key so that every weight becomes 0
-  const float lse2 = row_live ? lse * 1.4426950408889634f : INFINITY;
+  // What a row's exponents start from; -inf for rows without any allowed key so that every weight becomes 0.
+  // The dK/dV kernel, too, starts the accumulator of a row's scores at -LSE * sqrt(D), so that the
+  // exponent of a weight is the score times log2(e) / sqrt(D) and nothing else.  A soft-capped score is not
+  // linear in the product: there it is the offset of the exponent itself.
+  const float row_start = !row_live ? -INFINITY : (CAP ? __builtin_fmaf(lse, -1.4426950408889634f, p.cap_l2) : -lse * SqrtOf<D>::value);
   if (q_row < p.S && g == 0 && kg == 0) {
     p.ws[size_t(bh) * p.S + q_row] = -delta;
-    // The dK/dV kernel starts the accumulator of a row's scores at -LSE * sqrt(D), so that the
-    // exponent of a weight is the score times log2(e) / sqrt(D) and nothing else (-inf: every
-    // weight of the row is 0).  A soft-capped score is not linear in the product: there the
-    // plane holds the offset itself.
-    p.ws[size_t(p.n_slabs) * p.S + size_t(bh) * p.S + q_row] =
-        CAP ? lse2 : (row_live ? -lse * SqrtOf<D>::value : -INFINITY);
+    p.ws[size_t(p.n_slabs) * p.S + size_t(bh) * p.S + q_row] = row_start;
   }
 
   const f32x16_t zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -462,7 +461,7 @@ __device__ __forceinline__ void bwd_dq_walk(const BwdParams& p) {
     }
     return g_last;
   };
-  const uint32_t lds_tiles = lds_offset_of(lds16);
+  const uint32_t lds_tiles = lds_offset_of(lds_raw) + uint32_t(kg) * uint32_t(Shape::kGroupBytes);
   auto issue_loads = [&](const BwdStepInfo& st, int set) {
     const uint32_t base = lds_tiles + uint32_t(set) * (2u * TILE * 2u);
     bwd_load_tile<D, NT, STEP>(rK, k_pitch, st.row0, base, tid, w);
@@ -479,13 +478,14 @@ __device__ __forceinline__ void bwd_dq_walk(const BwdParams& p) {
   // last products of half 0).  The accumulator of S^T starts at the row's offset -LSE * sqrt(D) --
   // at -inf where the step's mask forbids the pair (`masked`, wave-uniform) -- so that a weight is
   // exp2(score * sl2); that of dP^T starts at -delta.  A soft-capped score is not linear in the
-  // product: there S^T starts at zero and offset and mask are applied to the weights.
+  // product: there S^T starts at zero, the offset goes into the exponents and the mask onto dS.
   constexpr int NSUB = NTL;
   static_assert(NSUB == 1 || NSUB == 2, "halves of a step");
   constexpr int NTR = 2 * DT;                    // last products of a half
   constexpr int NS = NSUB * (2 * KS + NTR);      // slots of a step
   constexpr int PF = D == 128 ? 2 : 3;           // operand fetch distance in slots (registers are tight at 128)
-  const float row_off = CAP ? lse2 : (row_live ? -lse * SqrtOf<D>::value : -INFINITY);
+  // (capped: the derivative's factor 4 comes with the exponent)
+  const float row_off = CAP ? row_start + 2.f : row_start;
   const float neg_delta = -delta;
   auto compute = [&](int set, const uint32_t (&kw)[NTL], bool masked) {
     const uint32_t base = lds_tiles + uint32_t(set) * (2u * TILE * 2u);
@@ -510,14 +510,11 @@ __device__ __forceinline__ void bwd_dq_walk(const BwdParams& p) {
     // the score gradients of registers r, r + 1 of half u
     auto grads = [&](auto uc, auto rc) {
       constexpr int u = decltype(uc)::value, r = decltype(rc)::value;
-      float w0, w1, f0 = 1.f, f1 = 1.f;
+      float w0, w1;
       if constexpr (CAP) {
-        bwd_weight<true>(st[u][r], row_off, p, w0, f0);
-        bwd_weight<true>(st[u][r + 1], row_off, p, w1, f1);
-        const uint32_t b0 = __builtin_bit_cast(uint32_t, w0) & keep_bits(uc, rc);
-        const uint32_t b1 = __builtin_bit_cast(uint32_t, w1) & keep_bits(uc, IntC<r + 1>{});
-        w0 = __builtin_bit_cast(float, b0) * f0;
-        w1 = __builtin_bit_cast(float, b1) * f1;
+        const float r0 = capped_r(st[u][r], p), r1 = capped_r(st[u][r + 1], p);
+        w0 = __builtin_amdgcn_exp2f(__builtin_fmaf(r0, -2.f * p.cap_l2, row_off)) * __builtin_fmaf(-r0, r0, r0);
+        w1 = __builtin_amdgcn_exp2f(__builtin_fmaf(r1, -2.f * p.cap_l2, row_off)) * __builtin_fmaf(-r1, r1, r1);
       } else {
         w0 = __builtin_amdgcn_exp2f(st[u][r] * p.sl2);
         w1 = __builtin_amdgcn_exp2f(st[u][r + 1] * p.sl2);
@@ -559,6 +556,14 @@ __device__ __forceinline__ void bwd_dq_walk(const BwdParams& p) {
         }
       } else {
         constexpr int u = ch - NSUB, ts = sl / DT, dt = sl % DT;
+        if constexpr (CAP && sl == 0) {
+          if (masked)
+            static_for<8>([&](auto ic) {
+              constexpr int i = decltype(ic)::value;
+              const uint32_t pair = dsb[u][i >> 2][i & 3];
+              dsb[u][i >> 2][i & 3] = keep_pair<2 * i>(pair, kw[u]);
+            });
+        }
         dq[dt] = mfma_32x32x16<BF16>(opq[n % PF], dsb[u][ts], dq[dt]);
       }
       if constexpr (n + PF < NS) opq[n % PF] = operand(IntC<n + PF>{});
@@ -592,42 +597,90 @@ __device__ __forceinline__ void bwd_dq_walk(const BwdParams& p) {
     }
     return mine;
   };
+  // PARTIAL steps: the mask bytes of the wave's 32 rows, or the packed words, are requested with the tiles,
+  // straight into LDS; a lane packs the 32 bytes of its row and of key half g and gets the other half's word
+  // from the lane that has it.  (Writer and reader are the same wave.)
+  const uint32_t lds_mask = lds_tiles + uint32_t(Shape::kTileBytes) + uint32_t(w) * (32u * STEP);
+  const int row_in_block = q0 + 32 * w - qb * QB;  // first row of the wave in its query block
+  auto request_mask = [&](const BwdStepInfo& st) {
+    const auto& pp = params_again();
+    int l = lane;  // (addresses are worked out here, not kept in registers over the walk)
+    asm volatile("" : "+v"(l));
+    if (pp.partial_bits != nullptr) {
+      const uint32_t words = uint32_t(QB) * uint32_t(KB / 32);
+      const i32x4_t rM = make_buffer_resource(pp.partial_bits + size_t(st.pid) * words, words * 4u);
+      if (l < 32 * NTL)
+        buffer_to_lds_b32(rM, (uint32_t(row_in_block + l % 32) * uint32_t(KB / 32) + uint32_t(l / 32)) * 4u,
+                          uint32_t(st.sub * NTL) * 4u, lds_mask);
+    } else {
+      constexpr int MCPR = STEP / 16;  // 16-byte chunks per row
+      const i32x4_t rM = make_buffer_resource(pp.partial_masks + size_t(st.pid) * size_t(QB * KB), uint32_t(QB * KB));
+#pragma unroll
+      for (int i = 0; i < MCPR / 2; ++i)
+        buffer_to_lds_b128(rM, uint32_t(row_in_block + i * (64 / MCPR) + l / MCPR) * uint32_t(KB) + uint32_t(l % MCPR) * 16u,
+                           uint32_t(st.sub * STEP), lds_mask + uint32_t(i) * 1024u);
+    }
+  };
+  auto take_mask = [&](uint32_t (&kw)[NTL]) {
+    const auto& pp = params_again();
+    int l = lane;
+    asm volatile("" : "+v"(l));
+    uint32_t mine;  // word g (of two; the only one otherwise) of row c
+    if (pp.partial_bits != nullptr) {
+      mine = lds_u32_at(lds_mask + 4u * uint32_t(NTL == 2 ? l : l % 32));
+    } else {
+      const uint32_t at = lds_mask + uint32_t((l % 32) * STEP + (NTL == 2 ? (l & 32) : 0));
+      mine = pack_mask_bytes(lds_b128_at(at), lds_b128_at(at + 16u));
+    }
+    if constexpr (NTL == 2) {
+      float w0, w1;
+      pair_split(__builtin_bit_cast(float, mine), w0, w1);
+      kw[0] = __builtin_bit_cast(uint32_t, w0);
+      kw[1] = __builtin_bit_cast(uint32_t, w1);
+    } else {
+      kw[0] = mine;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (read before the next request overwrites it)
+  };
   BwdStepInfo cur = next_round();
   int set = 0;
-  if (cur.valid) issue_loads(cur, 0);
+  if (cur.valid) {
+    issue_loads(cur, 0);
+    if (cur.mode == kPartial) request_mask(cur);
+  }
   while (more) {
     const BwdStepInfo nxt = next_round();
-    // mask words of this lane's row: bit j of word t = key row0 + 32 t + j allowed
+    wait_loads();  // the tiles (and mask) that this wave loaded have landed
+    // Mask words of this lane's row: bit j of word t = key row0 + 32 t + j allowed.  `masked`: something is left
+    // out for the rows of this wave (that a length which is no multiple of the block makes every block of the last
+    // list PARTIAL, because of the rows beyond it, costs a look at the words).
     uint32_t kw[NTL];
+    bool masked = false;
+    if (__builtin_expect(!(cur.mode == kFull && cur.row0 + STEP <= p.seqlen), 0)) {
+      if (cur.mode == kPartial) {
+        take_mask(kw);
+      } else {
 #pragma unroll
-    for (int t = 0; t < NTL; ++t) kw[t] = 0xffffffffu;
-    if (cur.mode == kPartial) {
-      const int q_local = q_row - qb * QB;  // (below QB: the rows of a workgroup are one block's)
-#pragma unroll
-      for (int t = 0; t < NTL; ++t) {
-        const int kcol = cur.sub * STEP + 32 * t;
-        if (p.partial_bits != nullptr) {
-          kw[t] = p.partial_bits[(size_t(cur.pid) * QB + q_local) * (KB / 32) + kcol / 32];
-        } else {
-          const uint8_t* mp = p.partial_masks + (size_t(cur.pid) * QB + q_local) * KB + kcol;
-          kw[t] = bwd_pack32(*reinterpret_cast<const u32x4_t*>(mp), *reinterpret_cast<const u32x4_t*>(mp + 16));
-        }
+        for (int t = 0; t < NTL; ++t) kw[t] = 0xffffffffu;
       }
+      int limit = p.seqlen - 1;
+      if (cur.mode == kCausal) limit = limit < q_row ? limit : q_row;
+      uint32_t all = 0xffffffffu;
+      static_for<NTL>([&](auto tc) {
+        constexpr int t = decltype(tc)::value;
+        const int n = limit - cur.row0 - 32 * t + 1;
+        kw[t] &= n >= 32 ? 0xffffffffu : (n <= 0 ? 0u : ((1u << (n & 31)) - 1u));
+        all &= kw[t];
+        kw[t] >>= 4 * g;
+      });
+      masked = __builtin_amdgcn_ballot_w64(all != 0xffffffffu && q_row < p.seqlen) != 0;
     }
-    int limit = p.seqlen - 1;
-    if (cur.mode == kCausal) limit = limit < q_row ? limit : q_row;
-    const int lim_l = limit - cur.row0 - 4 * g;
-    static_for<NTL>([&](auto tc) {
-      constexpr int t = decltype(tc)::value;
-      kw[t] >>= 4 * g;
-      const int n = lim_l - 32 * t + 1;
-      const uint32_t low = n >= 32 ? 0xffffffffu : (n <= 0 ? 0u : ((1u << (n & 31)) - 1u));
-      kw[t] &= low;
-    });
-    wait_loads();                  // this step's tiles (and mask words) have landed
     if constexpr (!LONE) __syncthreads();  // ... for every wave; and the other set is no longer read
-    if (nxt.valid) issue_loads(nxt, set ^ 1);
-    if (KG == 1 || cur.valid) compute(set, kw, !(cur.mode == kFull && cur.row0 + STEP <= p.seqlen));
+    if (nxt.valid) {
+      issue_loads(nxt, set ^ 1);
+      if (__builtin_expect(nxt.mode == kPartial, 0)) request_mask(nxt);
+    }
+    if (KG == 1 || cur.valid) compute(set, kw, masked);
     set ^= 1;
     cur = nxt;
   }
@@ -687,7 +740,9 @@ struct BwdDkdvShape {
   static constexpr size_t kHandBytes = size_t(2) * kKeyGroups * kSub * 2 * 64 * 16;
   // -delta and the exponent offsets of the rows of three steps
   static constexpr size_t kRowBytes = size_t(6) * kStep * sizeof(float);
-  static constexpr size_t kGroupBytes = kTileBytes + kHandBytes + kRowBytes;
+  // one mask byte per row and key of a PARTIAL step
+  static constexpr size_t kMaskBytes = size_t(kStep) * kKeys;
+  static constexpr size_t kGroupBytes = kTileBytes + kHandBytes + kRowBytes + kMaskBytes;
   static constexpr size_t kFixedBytes = kGroupBytes * G;
   static_assert(size_t(G) * (G - 1) * 2 * kKeyGroups * ((D / 8 + G - 1) / G) * 1024 <= kFixedBytes, "merge in LDS");
   // workgroups that a compute unit's registers hold (waves per SIMD: 2 at head_dim 128, 4 at 64, 5 at 32)
@@ -765,9 +820,12 @@ __device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
   const int w = G == 1 ? w_all : w_all % (2 * NKG);     // wave of the group
   uint8_t* const lds_group = lds_raw + size_t(group) * Traits::kGroupBytes;
   uint16_t* const lds16 = reinterpret_cast<uint16_t*>(lds_group);  // [3 sets][Q, dO][TILE]
-  uint32_t* const sHand = reinterpret_cast<uint32_t*>(lds_group + Traits::kTileBytes);
-  float* const sNd = reinterpret_cast<float*>(lds_group + Traits::kTileBytes + Traits::kHandBytes);  // [3 sets][STEP] -delta
-  float* const sL2 = sNd + 3 * STEP;                                         // [3 sets][STEP] exponent offsets
+  // (byte addresses in LDS are integers: a pointer that goes through the generic address space is checked for null)
+  const uint32_t lds_tiles = lds_offset_of(lds_raw) + uint32_t(group) * uint32_t(Traits::kGroupBytes);
+  const uint32_t lds_hand = lds_tiles + uint32_t(Traits::kTileBytes);
+  const uint32_t lds_nd = lds_hand + uint32_t(Traits::kHandBytes);  // [3 sets][STEP] -delta
+  const uint32_t lds_l2 = lds_nd + 3u * STEP * 4u;                  // [3 sets][STEP] exponent offsets
+  const uint32_t lds_masks = lds_nd + uint32_t(Traits::kRowBytes);  // [key groups][STEP][32]
   uint64_t* const sMatch = reinterpret_cast<uint64_t*>(lds_raw + Traits::kFixedBytes);
 
   // Workgroup -> (slab, KV block): XCD x takes the slabs bh with bh % n_xcd == x in groups, first KV
@@ -800,7 +858,6 @@ __device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
   const int kcol = key_wave_min - kvb * KB;  // ... inside its block
   const int key = key_wave_min + c;  // this lane's key row inside the slab
   const bool key_live = key < p.seqlen;
-  const bool has_partial = p.partial_idx != nullptr && (p.partial_masks != nullptr || p.partial_bits != nullptr);
   const size_t meta_slab = size_t(bh) * p.Tq;
   const int chunks = (p.max_blocks + 63) / 64;  // 64-slot words per query block
   const int n_words = p.Tq * chunks;
@@ -829,8 +886,9 @@ __device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
   // kept beside it (a list names a block once, except for duplicates and clamped indices).  The
   // words [base, end) of the slab go to entries 0 .. end - base of the window; every wave of the
   // workgroup calls this at the same point (the barriers are the workgroup's).
-  auto scan_window = [&](auto scan_c, int base, int end) {
+  auto scan_window = [&](auto scan_c, const auto& pp, int base, int end) {
     __syncthreads();  // nobody reads the previous window any more
+    const bool has_partial = pp.partial_idx != nullptr;
     // A wave takes SCAN consecutive words per pass and has the loads of all of them in flight
     // together (every slot inside the list's width is loaded; kv_num_blocks cuts afterwards).
     // The first window, scanned while few registers are live, takes four; later ones one.
@@ -842,20 +900,20 @@ __device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
         const int word = word0 + u < end ? word0 + u : end - 1;  // (a repeat of the last word: ignored below)
         const int qb = word / chunks, ch = word - qb * chunks;
         const int slot = ch * 64 + lane;
-        const size_t o = (meta_slab + qb) * p.max_blocks + (slot < p.max_blocks ? slot : p.max_blocks - 1);
-        raw[u] = p.kv_indices[o];
-        ty[u] = p.types[o];
-        pid[u] = has_partial ? p.partial_idx[o] : -1;
-        nbv[u] = p.kv_num_blocks[meta_slab + qb];
+        const size_t o = (meta_slab + qb) * pp.max_blocks + (slot < pp.max_blocks ? slot : pp.max_blocks - 1);
+        raw[u] = pp.kv_indices[o];
+        ty[u] = pp.types[o];
+        pid[u] = has_partial ? pp.partial_idx[o] : -1;
+        nbv[u] = pp.kv_num_blocks[meta_slab + qb];
       }
 #pragma unroll
       for (int u = 0; u < SCAN; ++u) {
         const int word = word0 + u;
         if (word >= end) break;
         const int ch = word % chunks;
-        const int nb = nbv[u] < 0 ? 0 : (nbv[u] > p.max_blocks ? p.max_blocks : nbv[u]);
-        const int32_t idx = raw[u] < 0 ? 0 : (raw[u] >= p.Tk ? p.Tk - 1 : raw[u]);
-        const int32_t mode = bwd_slot_mode(ty[u], pid[u], has_partial, p.num_partial);
+        const int nb = nbv[u] < 0 ? 0 : (nbv[u] > pp.max_blocks ? pp.max_blocks : nbv[u]);
+        const int32_t idx = raw[u] < 0 ? 0 : (raw[u] >= pp.Tk ? pp.Tk - 1 : raw[u]);
+        const int32_t mode = bwd_slot_mode(ty[u], pid[u], has_partial, pp.num_partial);
         const bool hit = ch * 64 + lane < nb && idx == kvb && mode != kMasked;
         const int32_t info = (mode == kPartial ? pid[u] << 2 : 0) | mode;
         const uint64_t bits = __builtin_amdgcn_ballot_w64(hit);
@@ -887,8 +945,9 @@ __device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
     const int n = (subs < NSTEPS ? subs : NSTEPS) - sub0;
     return n > 0 ? n : 0;
   };
-  auto build_table = [&](int base, int end, bool first_piece) {
+  auto build_table = [&](const auto& pp, int base, int end, bool first_piece) {
     if (w_all == 0) {
+      const bool has_partial = pp.partial_idx != nullptr;
       int w0 = base, n = 0, first = 0;
       if (!first_piece) {
         w0 = s_table[1];
@@ -903,9 +962,9 @@ __device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
         // information of the match that is the lowest bit of `left`
         auto info_of = [&](uint64_t left) {
           if (left == bits) return sFirst[word - base];
-          const size_t o = (meta_slab + qb) * p.max_blocks + ch * 64 + __builtin_ctzll(left);
-          const int32_t pid = has_partial ? p.partial_idx[o] : -1;
-          const int32_t mode = bwd_slot_mode(p.types[o], pid, has_partial, p.num_partial);
+          const size_t o = (meta_slab + qb) * pp.max_blocks + ch * 64 + __builtin_ctzll(left);
+          const int32_t pid = has_partial ? pp.partial_idx[o] : -1;
+          const int32_t mode = bwd_slot_mode(pp.types[o], pid, has_partial, pp.num_partial);
           return (mode == kPartial ? pid << 2 : 0) | mode;
         };
         int count = 0, sub0;
@@ -938,11 +997,9 @@ __device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
     return __builtin_amdgcn_readfirstlane(s_table[0]);
   };
   int win_base = 0, win_end = win_words < n_words ? win_words : n_words;  // the words of the slab the window holds
-  scan_window(IntC<4>{}, 0, win_end);
-  int n_steps = build_table(0, win_end, true);
-  const uint32_t lds_tiles = lds_offset_of(lds16);
-  const uint32_t hand_lane = lds_offset_of(sHand) + uint32_t(kg) * (NSUB * 2048u) + uint32_t(lane) * 16u;
-  const uint32_t lds_nd = lds_offset_of(sNd), lds_l2 = lds_offset_of(sL2);
+  scan_window(IntC<4>{}, p, 0, win_end);
+  int n_steps = build_table(p, 0, win_end, true);
+  const uint32_t hand_lane = lds_hand + uint32_t(kg) * (NSUB * 2048u) + uint32_t(lane) * 16u;
   auto tile_at = [&](int set, int which) { return lds_tiles + uint32_t(set * 2 + which) * (TILE * 2u); };
   // the four words of half `half` of 32-row half u of the step with parity par
   auto hand_at = [&](int par, int u, int half) {
@@ -1011,15 +1068,11 @@ __device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
         constexpr int r = SPC * i + 2 * decltype(jc)::value;
         float w0, w1;
         if constexpr (CAP) {
-          float f0, f1;
           if constexpr ((r & 3) == 0) lq = row_offsets(u, r >> 2);
-          bwd_weight<true>(sc[u][r], lq[r & 3], p, w0, f0);
-          bwd_weight<true>(sc[u][r + 1], lq[(r + 1) & 3], p, w1, f1);
-          const uint32_t b0 = __builtin_bit_cast(uint32_t, w0) & keep_bits(uc, IntC<r>{});
-          const uint32_t b1 = __builtin_bit_cast(uint32_t, w1) & keep_bits(uc, IntC<r + 1>{});
-          w0 = __builtin_bit_cast(float, b0);
-          w1 = __builtin_bit_cast(float, b1);
-          hb[u][r >> 3][(r & 7) >> 1] = pack2<BF16>(w0 * f0, w1 * f1);
+          const float r0 = capped_r(sc[u][r], p), r1 = capped_r(sc[u][r + 1], p), r04 = 4.f * r0, r14 = 4.f * r1;
+          w0 = __builtin_amdgcn_exp2f(__builtin_fmaf(r0, -2.f * p.cap_l2, lq[r & 3]));
+          w1 = __builtin_amdgcn_exp2f(__builtin_fmaf(r1, -2.f * p.cap_l2, lq[(r + 1) & 3]));
+          hb[u][r >> 3][(r & 7) >> 1] = pack2<BF16>(w0 * __builtin_fmaf(-r04, r0, r04), w1 * __builtin_fmaf(-r14, r1, r14));
         } else {  // the scores already carry their row's offset and the mask
           w0 = __builtin_amdgcn_exp2f(sc[u][r] * p.sl2);
           w1 = __builtin_amdgcn_exp2f(sc[u][r + 1] * p.sl2);
@@ -1029,6 +1082,13 @@ __device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
       if constexpr (((i + 1) * SPC) % 8 == 0) {  // four words are complete: to the partner
         constexpr int half = (i + 1) * SPC / 8 - 1;
         if constexpr (CAP) {
+          if (masked)
+            static_for<4>([&](auto jc) {
+              constexpr int j = decltype(jc)::value;
+              const uint32_t a = pb[u][half][j], b = hb[u][half][j];
+              pb[u][half][j] = keep_pair<8 * half + 2 * j>(a, kw[u]);
+              hb[u][half][j] = keep_pair<8 * half + 2 * j>(b, kw[u]);
+            });
           *(__attribute__((address_space(3))) u32x4_t*)(hand_at(par, u, half)) = hb[u][half];
         } else {
           *(__attribute__((address_space(3))) u32x4_t*)(hand_at(par, u, half)) = pb[u][half];
@@ -1134,18 +1194,43 @@ __device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
     if constexpr (PRIO) __builtin_amdgcn_s_setprio(0);
   };
 
-  // Bits of one partial tile for this lane's key: bit j = query row q_local0 + j of the tile
-  // attends the key.  Lane j of the wave fetches the 32 key bits of row j; the column of this
-  // lane's key is then collected from the 32 rows.
-  auto partial_column = [&](int pid, int q_local0) {
-    const int rl = lane & 31;
-    uint32_t roww;
-    if (p.partial_bits != nullptr) {
-      roww = p.partial_bits[(size_t(pid) * QB + q_local0 + rl) * (KB / 32) + kcol / 32];
+  // PARTIAL steps: the mask of a weight wave's 32 keys, as bytes or packed words, is requested with its rows,
+  // straight into LDS (writer and reader are the same wave).
+  const uint32_t lds_mask = lds_masks + uint32_t(kg) * (STEP * 32u);
+  auto request_mask = [&](const Step& st) {
+    const auto& pp = params_again();
+    int l = lane;  // (addresses are worked out here, not kept in registers over the walk)
+    asm volatile("" : "+v"(l));
+    const uint32_t first = uint32_t(st.row0 & (QB - 1));  // row of the tile
+    if (pp.partial_bits != nullptr) {
+      const uint32_t words = uint32_t(QB) * uint32_t(KB / 32);
+      const i32x4_t rM = make_buffer_resource(pp.partial_bits + size_t(st.info >> 2) * words, words * 4u);
+      if (l < STEP)
+        buffer_to_lds_b32(rM, uint32_t(l) * uint32_t(KB / 8), (first * uint32_t(KB / 32) + uint32_t(kcol / 32)) * 4u,
+                          lds_mask);
     } else {
-      const uint8_t* mp = p.partial_masks + (size_t(pid) * QB + q_local0 + rl) * KB + kcol;
-      roww = bwd_pack32(*reinterpret_cast<const u32x4_t*>(mp), *reinterpret_cast<const u32x4_t*>(mp + 16));
+      const i32x4_t rM = make_buffer_resource(pp.partial_masks + size_t(st.info >> 2) * size_t(QB * KB), uint32_t(QB * KB));
+#pragma unroll
+      for (int u = 0; u < NSUB; ++u)
+        buffer_to_lds_b128(rM, uint32_t(l / 2) * uint32_t(KB) + uint32_t(l % 2) * 16u,
+                           (first + 32 * u) * uint32_t(KB) + uint32_t(kcol), lds_mask + uint32_t(u) * 1024u);
     }
+  };
+  // Bits of half u for this lane's key: bit j = its row j attends the key.  Collected from the 32 rows, unless
+  // none of those inside the sequence leaves a key out (with a length that is no multiple of the block, all blocks
+  // of the last list are PARTIAL because of the rows beyond it).
+  auto mask_column = [&](int u, int row0) {
+    const auto& pp = params_again();
+    int l = lane & 31;
+    asm volatile("" : "+v"(l));
+    uint32_t roww;
+    if (pp.partial_bits != nullptr) {
+      roww = lds_u32_at(lds_mask + uint32_t(32 * u + l) * 4u);
+    } else {
+      const uint32_t at = lds_mask + uint32_t(32 * u + l) * 32u;
+      roww = pack_mask_bytes(lds_b128_at(at), lds_b128_at(at + 16u));
+    }
+    if (__builtin_amdgcn_ballot_w64(roww != 0xffffffffu && row0 + 32 * u + l < p.seqlen) == 0) return 0xffffffffu;
     uint32_t col = 0;
     static_for<32>([&](auto jc) {
       constexpr int j = decltype(jc)::value;
@@ -1180,21 +1265,25 @@ __device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
       i32x2_t coming = request(1);
       int s_prev = 2, s_cur = 0, s_nxt = 1;  // tile sets of steps j - 1, j, j + 1
       if (cur.valid) {
-        if constexpr (!GRAD) load_q(cur, 0); else load_do(cur, 0);
+        if constexpr (!GRAD) {
+          load_q(cur, 0);
+          if ((cur.info & 3) == kPartial) request_mask(cur);
+        } else {
+          load_do(cur, 0);
+        }
       }
       const int iterations = rounds > 0 ? rounds + 1 : 0;
       for (int j = 0; j < iterations; ++j) {
         const Step nxt = receive(coming, j + 1);
         coming = request(j + 2);
+        wait_loads();  // the tile (and mask) this wave loaded has landed
         // mask words of this lane's key: bit i of word u = query row row0 + 32 u + i attends it
         uint32_t kw[NSUB];
-#pragma unroll
-        for (int u = 0; u < NSUB; ++u) kw[u] = 0;
-        const int mode = cur.info & 3;
-        // (wave-uniform) a FULL step whose keys are all inside the sequence needs no mask
-        const bool masked = CAP || !(mode == kFull && key_wave_min + 32 <= p.seqlen);
+        bool masked = false;  // (wave-uniform) something is left out
         if constexpr (!GRAD) {
-          if (cur.valid && masked) {
+          const int mode = cur.info & 3;
+          if (__builtin_expect(cur.valid && !(mode == kFull && key_wave_min + 32 <= p.seqlen), 0)) {
+            uint32_t all = 0xffffffffu;
 #pragma unroll
             for (int u = 0; u < NSUB; ++u) {
               uint32_t m = key_live ? 0xffffffffu : 0u;
@@ -1202,16 +1291,21 @@ __device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
                 const int n = key - (cur.row0 + 32 * u);
                 m &= n <= 0 ? 0xffffffffu : (n >= 32 ? 0u : (0xffffffffu << (n & 31)));
               }
-              if (mode == kPartial) m &= partial_column(cur.info >> 2, (cur.row0 & (QB - 1)) + 32 * u);
+              if (mode == kPartial) m &= mask_column(u, cur.row0);
+              all &= m;
               kw[u] = m >> (4 * g);
             }
+            masked = __builtin_amdgcn_ballot_w64(all != 0xffffffffu) != 0;
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (read before the next request overwrites it)
           }
         }
-        wait_loads();  // the tile this wave loaded has landed
         __syncthreads();  // ... everybody's have; the hand-over of step j - 1 is written; the set
                           // about to be overwritten (step j - 2) is no longer read
         if constexpr (!GRAD) {
-          if (nxt.valid) load_q(nxt, s_nxt);
+          if (nxt.valid) {
+            load_q(nxt, s_nxt);
+            if (__builtin_expect((nxt.info & 3) == kPartial, 0)) request_mask(nxt);
+          }
           if (cur.valid) weight_step(s_cur, j & 1, kw, masked);
         } else {
           if (nxt.valid) load_do(nxt, s_nxt);
@@ -1231,11 +1325,11 @@ __device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
       if (window_done) {
         win_base = win_end;
         win_end = win_base + win_words < n_words ? win_base + win_words : n_words;
-        scan_window(IntC<1>{}, win_base, win_end);
+        scan_window(IntC<1>{}, params_again(), win_base, win_end);
       } else {
         __syncthreads();  // nobody reads the table any more
       }
-      n_steps = build_table(win_base, win_end, window_done);
+      n_steps = build_table(params_again(), win_base, win_end, window_done);
     }
     __syncthreads();
     if constexpr (G > 1) {

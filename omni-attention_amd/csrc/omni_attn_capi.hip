@@ -386,6 +386,7 @@ int backward(const void* q, const void* k, const void* v, const void* o, const v
   p.sl2 = float(1.4426950408889634 / std::sqrt(double(D)));
   p.softcap = softcap;
   p.cap_c2 = softcap > 0.f ? float(2.0 * 1.4426950408889634 / (std::sqrt(double(D)) * double(softcap))) : 0.f;
+  p.cap_l2 = float(1.4426950408889634 * double(softcap));
 
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool bf = dtype == OMNI_ATTN_DTYPE_BF16;

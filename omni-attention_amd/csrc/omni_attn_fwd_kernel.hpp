@@ -122,6 +122,25 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
   }
 }
 
+// 32 mask bytes -> 32 bits, byte i -> bit i; any non-zero byte means attend (attn_naive.cu:151).  Bit 7 of a
+// byte is brought to that, and the dot products of eight such bytes with 1, 2, 4 .. 128 are 128 times their bits:
+// 41 vector instructions (folding each byte onto its lowest bit and multiplying the nibbles out: 80).
+__device__ __forceinline__ uint32_t pack_mask_bytes(u32x4_t m0, u32x4_t m1) {
+  uint32_t part[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint32_t sum = 0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const uint32_t x = i < 2 ? m0[2 * i + h] : m1[2 * i + h - 4];
+      const uint32_t set = (((x & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x) & 0x80808080u;
+      sum = __builtin_amdgcn_udot4(set, h == 0 ? 0x08040201u : 0x80402010u, sum, false);
+    }
+    part[i] = sum;
+  }
+  return (part[0] >> 7) | (part[1] << 1) | (part[2] << 9) | (part[3] << 17);
+}
+
 // LDS tiles are [64 rows][D] 16-bit elements with no padding; 16-byte chunks are
 // XOR-swizzled inside a row so that the operand reads are bank-conflict free.
 // K is read with ds_read_b128 by 32 consecutive rows at one chunk column: the chunk
@@ -676,17 +695,7 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
     const uint8_t* mp = sMaskBytes + size_t(32 * w) * STEP + size_t(wi) * 32;
     const u32x4_t m0 = *reinterpret_cast<const u32x4_t*>(mp);
     const u32x4_t m1 = *reinterpret_cast<const u32x4_t*>(mp + 16);
-    uint32_t word = 0;  // byte i of the 32 (any non-zero value = attend, attn_naive.cu:151) -> bit i
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      uint32_t bytes = i < 4 ? m0[i] : m1[i - 4];
-      bytes |= bytes >> 4;  // fold each byte onto its lowest bit
-      bytes |= bytes >> 2;
-      bytes |= bytes >> 1;
-      const uint32_t nib = ((bytes & 0x01010101u) * 0x01020408u) >> 24;
-      word |= nib << (4 * i);
-    }
-    sBits[32 * w * NTL + wi] = word;
+    sBits[32 * w * NTL + wi] = pack_mask_bytes(m0, m1);
   };
 
   // Does this wave's 32 x STEP tile of the step need no mask at all?  (wave-uniform)
@@ -782,6 +791,12 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
     if (si.mode == kPartial) {
 #pragma unroll
       for (int t = 0; t < NTL; ++t) kw[t] = sBits[(32 * w + c) * NTL + t];
+      // A tile that leaves nothing out for these rows: with a length that is no multiple of the block, every
+      // block that the last query block lists is PARTIAL, because rows beyond the sequence attend nothing.
+      uint32_t all = kw[0];
+#pragma unroll
+      for (int t = 1; t < NTL; ++t) all &= kw[t];
+      if (si.row0 + STEP <= p.seqlen && __builtin_amdgcn_ballot_w64(all != 0xffffffffu && q_row < p.seqlen) == 0) return;
     }
     // the limit becomes part of the bit words: positions 0 .. lim_l - 32t of word t stay
     static_for<NTL>([&](auto tc) {
@@ -1026,7 +1041,7 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
     }
     l_run += sum;
     if (next_partial && !packed_tiles) {
-      wait_loads_but<LONE ? NL : 0>();  // (a lone wave has requested its tiles behind the bytes)
+      wait_loads_but<NL>();  // (the tile loads of the iteration were requested behind the bytes)
       stage_mask_bits();
     }
     const StepInfo n3 = step_info(it + 3);

@@ -377,3 +377,36 @@ def test_autograd_operator_matches_oracle_gradients(gpu_device):
         dense = prefix_mask(prefix[:, :S], S_pad)[..., :S].unsqueeze(1)
         ref = attention_dense_grads(q, k, v, dense, dout)
         check_grads((qd.grad, kd.grad, vd.grad), ref, torch.bfloat16, "autograd operator")
+
+
+@pytest.mark.parametrize("softcap", [0.0, 20.0])
+@pytest.mark.parametrize("D,QB,KB,H,S", [(64, 128, 128, 3, 384), (32, 64, 128, 40, 512), (128, 64, 64, 20, 512),
+                                         (128, 128, 128, 40, 1024), (64, 128, 64, 80, 1024)])
+def test_partial_tiles_that_leave_nothing_out_are_full(softcap, D, QB, KB, H, S, gpu_device):
+    """Tiles that allow every key to the rows inside the sequence (any non-zero byte) and none to the rows behind it,
+    as a mask builder stores them where the length is no multiple of the block: forward and backward
+    equal those of FULL blocks bit for bit, as bytes and as bits; one row that leaves out a key changes the result."""
+    gen = torch.Generator().manual_seed(D + QB + H)
+    dtype = torch.bfloat16 if D == 128 else torch.float16
+    q, k, v, dout = (torch.randn(1, H, S, D, generator=gen).to(dtype) for _ in range(4))
+    Tq, Tk, seqlen = S // QB, S // KB, S - 45
+    nb = torch.full((1, H, Tq), Tk, dtype=torch.int32)
+    idx = torch.arange(Tk, dtype=torch.int32).expand(1, H, Tq, Tk).contiguous()
+    full = torch.full((1, H, Tq, Tk), 2, dtype=torch.int32)
+    tys, pidx = full.clone(), torch.full_like(full, -1)
+    tys[:, :, -1], pidx[:, :, -1] = 3, 0  # the last query block; and one block of another
+    tys[:, :, 0, Tk // 2], pidx[:, :, 0, Tk // 2] = 3, 1
+    values = torch.tensor([1, 2, 0x40, 0x80, 0xff], dtype=torch.uint8)
+    tiles = values[torch.randint(0, 5, (3, QB, KB), generator=gen)]
+    tiles[0, QB - 45:] = 0
+    tiles[2] = tiles[1]
+    tiles[2, QB - 7, KB - 3] = 0
+    want = run_fwd_bwd(q, k, v, dout, nb, idx, full, QB, KB, seqlen, device=gpu_device, softcap=softcap)
+    for packed in (False, True):
+        got = run_fwd_bwd(q, k, v, dout, nb, idx, tys, QB, KB, seqlen, pidx, tiles, device=gpu_device, packed=packed,
+                          softcap=softcap)
+        for a, b in zip(got, want):
+            assert torch.equal(a, b)
+    pidx[pidx == 1] = 2
+    got = run_fwd_bwd(q, k, v, dout, nb, idx, tys, QB, KB, seqlen, pidx, tiles, device=gpu_device, softcap=softcap)
+    assert not torch.equal(got[1], want[1]) and torch.equal(got[3][:, :, QB:], want[3][:, :, QB:])

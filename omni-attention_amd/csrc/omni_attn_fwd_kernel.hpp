@@ -216,11 +216,9 @@ struct FwdShape {
   static constexpr int kTileElems = kStep * D;
   static constexpr bool kLone = QT == 32;  // a group is one wave: its steps need no barriers
   static constexpr int kSets = kLone ? 1 : 2;  // tiles of K, and of V
-  // per group: K tiles, V tiles, one mask word per row and 32 keys, one mask byte per row and key in
-  // transit
+  // per group: K tiles, V tiles, one mask byte per row and key in transit
   static constexpr size_t kTileBytes = size_t(kSets) * 2 * kTileElems * sizeof(uint16_t);
-  static constexpr size_t kGroupBytes = kTileBytes +
-                                        size_t(QT) * (kStep / 32) * sizeof(uint32_t) + size_t(QT) * kStep;
+  static constexpr size_t kGroupBytes = kTileBytes + size_t(QT) * kStep;
   static constexpr size_t kLdsBytes = kGroupBytes * KG;
 };
 
@@ -463,8 +461,7 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   constexpr int SETS = Shape::kSets;
   uint16_t* sK = reinterpret_cast<uint16_t*>(lds_raw + size_t(kg) * Shape::kGroupBytes);  // [SETS][TILE]
   uint16_t* sV = sK + SETS * TILE;                                  // [SETS][TILE]
-  uint32_t* sBits = reinterpret_cast<uint32_t*>(sV + SETS * TILE);  // [QT][NTL]
-  uint8_t* sMaskBytes = reinterpret_cast<uint8_t*>(sBits + QT * NTL);  // [QT][STEP]
+  uint8_t* sMaskBytes = reinterpret_cast<uint8_t*>(sV + SETS * TILE);  // [QT][STEP]
 
   // Workgroup -> (slab, query block).  Consecutive workgroup ids go round-robin over
   // the XCDs.  XCD x takes the slabs bh with bh % n_xcd == x (every batch element's heads
@@ -657,45 +654,59 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   };
   static_assert(!LONE || (NCH % 4 == 0 && 4 % KPER == 0), "loads of a lone wave come in fours");
 
-  // PARTIAL blocks, in two stages so that no load latency is exposed.  One iteration ahead
-  // each wave fetches the STEP mask bytes of its 32 rows for that step straight into LDS
-  // (buffer->LDS loads, no registers; the resource covers exactly the tile); at the end of
-  // that iteration a lane packs 32 of the bytes of a row to 32 bits and parks the word in LDS
-  // for the two lanes that own the row.  Writer and readers of both stages are the same wave,
-  // so no workgroup barrier is needed.
+  // PARTIAL blocks.  The mask of a step is one word per row and 32 keys; lane (g, c) of a wave has word g of row c
+  // (of its only word, with steps of 32 keys).  Packed tiles: the word is requested an iteration ahead.  Byte tiles:
+  // one iteration ahead each wave fetches the STEP mask bytes of its 32 rows for that step straight into LDS
+  // (buffer->LDS loads, no registers; the resource covers exactly the tile); at the end of that iteration a
+  // lane looks at the 32 bytes of its word, and packs them unless the tile leaves nothing out.  Writer and readers are
+  // the same wave, so no workgroup barrier is needed.
+  uint32_t mask_word = 0;
   constexpr int MCPR = STEP / 16;  // 16-byte chunks per row of mask bytes
   auto prefetch_mask_bytes = [&](int it, const StepInfo& si) {
+    int l = lane;  // (addresses are worked out here, not kept in registers over the walk)
+    asm volatile("" : "+v"(l));
     const int half = (KG == 1 ? it : it * KG + kg) & (SPB - 1);
     const i32x4_t rM = make_buffer_resource(p.partial_masks + size_t(si.pid) * size_t(QB * KB), uint32_t(QB * KB));
     const uint32_t dst = lds_offset_of(sMaskBytes) + uint32_t(w) * uint32_t(32 * STEP);
 #pragma unroll
     for (int i = 0; i < MCPR / 2; ++i) {  // 64 / MCPR rows per load
-      const uint32_t row = uint32_t(rb0 + 32 * w + i * (64 / MCPR)) + uint32_t(lane / MCPR);
-      buffer_to_lds_b128(rM, row * uint32_t(KB) + uint32_t(lane % MCPR) * 16u, uint32_t(half * STEP),
+      const uint32_t row = uint32_t(rb0 + 32 * w + i * (64 / MCPR)) + uint32_t(l / MCPR);
+      buffer_to_lds_b128(rM, row * uint32_t(KB) + uint32_t(l % MCPR) * 16u, uint32_t(half * STEP),
                          dst + uint32_t(i) * 1024u);
     }
   };
-  // Tiles that arrive already packed (one 32-bit word per row and 32 keys) need no second
-  // stage: one 4-byte buffer->LDS load per lane puts the step's words of the wave's 32 rows
-  // where the byte path parks the words it packs.
-  auto prefetch_mask_words = [&](int it, const StepInfo& si) {
-    const uint32_t TILE_WORDS = uint32_t(QB) * uint32_t(KB / 32);
+  auto prefetch_mask_word = [&](int it, const StepInfo& si) {
+    int l = lane;
+    asm volatile("" : "+v"(l));
     const int half = (KG == 1 ? it : it * KG + kg) & (SPB - 1);
-    const i32x4_t rM = make_buffer_resource(p.partial_bits + size_t(si.pid) * TILE_WORDS, TILE_WORDS * 4u);
-    if (lane < 32 * NTL) {
-      const uint32_t row = uint32_t(rb0 + 32 * w + lane / NTL);
-      buffer_to_lds_b32(rM, (row * uint32_t(KB / 32) + uint32_t(lane % NTL)) * 4u, uint32_t(half * NTL) * 4u,
-                        lds_offset_of(sBits) + uint32_t(32 * w * NTL) * 4u);
-    }
+    const uint32_t words = uint32_t(QB) * uint32_t(KB / 32);
+    auto rM = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(p.partial_bits) + size_t(si.pid) * words, 0,
+                                                words * 4u, 0x00020000);
+    mask_word = __builtin_amdgcn_raw_buffer_load_b32(
+        rM, (uint32_t(32 * w + l % 32) * uint32_t(KB / 32) + uint32_t(NTL == 2 ? l / 32 : 0)) * 4u,
+        (uint32_t(rb0) * uint32_t(KB / 32) + uint32_t(half * NTL)) * 4u, 0);
   };
-  auto stage_mask_bits = [&]() {  // (the bytes have landed)
-    // word NTL * row + h of the wave's 32 rows; with one word per row the upper half-wave
-    // repeats the lower one
-    const int wi = lane % (32 * NTL);
-    const uint8_t* mp = sMaskBytes + size_t(32 * w) * STEP + size_t(wi) * 32;
-    const u32x4_t m0 = *reinterpret_cast<const u32x4_t*>(mp);
-    const u32x4_t m1 = *reinterpret_cast<const u32x4_t*>(mp + 16);
-    sBits[32 * w * NTL + wi] = pack_mask_bytes(m0, m1);
+  // A tile that leaves nothing out for the rows of this wave that lie inside the sequence: with a length that is no
+  // multiple of the block, every block that the last query block lists is PARTIAL, because rows beyond the sequence
+  // attend nothing.
+  auto leaves_nothing_out = [&]() { return __builtin_amdgcn_ballot_w64(mask_word != 0xffffffffu && q_row < p.seqlen) == 0; };
+  // Returns whether the tile leaves nothing out: whether the lowest bit of every byte is set, as it is in a tensor of
+  // booleans (bytes of other values are packed, and looked at again).  (The bytes have landed.)
+  auto take_mask_bytes = [&]() {
+    int l = lane;
+    asm volatile("" : "+v"(l));
+    const uint8_t* wave_bytes = sMaskBytes + size_t(32 * w) * STEP;
+    bool whole = true;
+#pragma unroll
+    for (int i = 0; i < NTL; ++i) {  // 16 neighbouring bytes per lane: reads without bank conflicts
+      const u32x4_t m = *reinterpret_cast<const u32x4_t*>(wave_bytes + (64 * i + l) * 16);
+      whole &= ((m[0] & m[1] & m[2] & m[3] & 0x01010101u) == 0x01010101u) |
+               (q_wave_min + (64 * i + l) / MCPR >= p.seqlen);
+    }
+    if (__builtin_amdgcn_ballot_w64(!whole) == 0) return true;
+    const uint8_t* mp = wave_bytes + (l % 32) * STEP + (NTL == 2 ? l & 32 : 0);
+    mask_word = pack_mask_bytes(*reinterpret_cast<const u32x4_t*>(mp), *reinterpret_cast<const u32x4_t*>(mp + 16));
+    return false;
   };
 
   // Does this wave's 32 x STEP tile of the step need no mask at all?  (wave-uniform)
@@ -789,14 +800,14 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
 #pragma unroll
     for (int t = 0; t < NTL; ++t) kw[t] = 0xffffffffu;
     if (si.mode == kPartial) {
-#pragma unroll
-      for (int t = 0; t < NTL; ++t) kw[t] = sBits[(32 * w + c) * NTL + t];
-      // A tile that leaves nothing out for these rows: with a length that is no multiple of the block, every
-      // block that the last query block lists is PARTIAL, because rows beyond the sequence attend nothing.
-      uint32_t all = kw[0];
-#pragma unroll
-      for (int t = 1; t < NTL; ++t) all &= kw[t];
-      if (si.row0 + STEP <= p.seqlen && __builtin_amdgcn_ballot_w64(all != 0xffffffffu && q_row < p.seqlen) == 0) return;
+      if constexpr (NTL == 2) {
+        float w0, w1;
+        pair_split(__builtin_bit_cast(float, mask_word), w0, w1);
+        kw[0] = __builtin_bit_cast(uint32_t, w0);
+        kw[1] = __builtin_bit_cast(uint32_t, w1);
+      } else {
+        kw[0] = mask_word;
+      }
     }
     // the limit becomes part of the bit words: positions 0 .. lim_l - 32t of word t stay
     static_for<NTL>([&](auto tc) {
@@ -991,11 +1002,11 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
     }
     if (cur.mode == kPartial) {
       if (packed_tiles) {
-        prefetch_mask_words(0, cur);
+        prefetch_mask_word(0, cur);
       } else {
         prefetch_mask_bytes(0, cur);
         wait_loads();
-        stage_mask_bits();
+        if (take_mask_bytes()) cur.mode = kFull;
       }
     }
     step_barrier();
@@ -1016,19 +1027,22 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
     const bool next_partial = it + 1 < nsteps && nxt.mode == kPartial;
     const bool plain = (owed == 0) & !(p.softcap > 0.f) & unmasked(cur) & !next_partial;
     if (!plain) {
-      if (owed & kOwesRescale) {
+      if (cur.mode == kPartial && leaves_nothing_out()) cur.mode = kFull;
+      if ((owed != 0) | (p.softcap > 0.f) | !unmasked(cur)) {
+        if (owed & kOwesRescale) {
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
+          for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) ot[dt][r] *= alpha_pending;
-        owed &= ~kOwesRescale;
+            for (int r = 0; r < 16; ++r) ot[dt][r] *= alpha_pending;
+          owed &= ~kOwesRescale;
+        }
+        if (p.softcap > 0.f) apply_softcap(IntC<SET>{});
+        if (!unmasked(cur)) apply_mask(IntC<SET>{}, cur);
+        if (owed & kOwesLook) look(set_c);
       }
-      if (p.softcap > 0.f) apply_softcap(IntC<SET>{});
-      if (!unmasked(cur)) apply_mask(IntC<SET>{}, cur);
-      if (owed & kOwesLook) look(set_c);
       if (next_partial) {
         if (packed_tiles) {
-          prefetch_mask_words(it + 1, nxt);
+          prefetch_mask_word(it + 1, nxt);
         } else {
           prefetch_mask_bytes(it + 1, nxt);
         }
@@ -1040,9 +1054,9 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
       if (__builtin_amdgcn_ballot_w64(!(sum <= kRedo)) != 0) redo(set_c, sum);
     }
     l_run += sum;
-    if (next_partial && !packed_tiles) {
+    if (__builtin_expect(next_partial && !packed_tiles, 0)) {
       wait_loads_but<NL>();  // (the tile loads of the iteration were requested behind the bytes)
-      stage_mask_bits();
+      if (take_mask_bytes()) nxt.mode = kFull;
     }
     const StepInfo n3 = step_info(it + 3);
     cur = nxt;
@@ -1094,14 +1108,14 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   // rows: 64 lanes x 16 bytes = 64 / CPR complete rows per instruction.
   float l_tot = pair_sum(l_run);
   if constexpr (KG > 1) {
-    // Merge of the groups.  Row maxima and sums go where the mask words and bytes were (a wave
+    // Merge of the groups.  Row maxima and sums go where the mask bytes were (a wave
     // writes and has read its own rows only), the scaled O^T into the tiles once every group is
     // done with them; then each group adds up and stores its share of the columns.
     constexpr int UNITS = DT * 4;           // 4-register pieces of a lane's O^T
     constexpr int MINE = (UNITS + KG - 1) / KG;  // ... that a group stores
-    static_assert(QT * D * 4 <= Shape::kTileBytes && QT * STEP >= QT * 4, "merge layout");
+    static_assert(QT * D * 4 <= Shape::kTileBytes && QT * STEP >= QT * 8, "merge layout");
     auto group_at = [&](int i) { return lds_raw + size_t(i) * Shape::kGroupBytes; };
-    constexpr size_t kStatM = Shape::kTileBytes, kStatL = kStatM + size_t(QT) * NTL * 4;
+    constexpr size_t kStatM = Shape::kTileBytes, kStatL = kStatM + size_t(QT) * 4;
     const int row = 32 * w + c;
     if (g == 0) {
       reinterpret_cast<float*>(group_at(kg) + kStatM)[row] = m_run;

@@ -31,14 +31,17 @@ constexpr int fwd_split_rows(FwdSplit s, int QB) {
 //          kRows64x4   B H=16 S=1024 22-24 (-20 .. -23 %), S=1152 24 (-21, one layout +5); B H=12 S=2048 38-41
 //                      (-23 .. +3), B H=8 S=3072 54-58 (-21 .. -36); beyond: B H=20 S=1152 24 (-3 .. +24)
 //          kRows64x2   B H=20 S=1152 24 (0 .. -7), B H=24 S=1024 22-24 (-4 .. -10); beyond: B H=32 S=1237 30-35
-//                      (-6 .. -12), but S=1280 30 (-11 .. +11) and S=1408 32 (-6 .. +25)
+//                      (-6 .. -12), but S=1280 30 (-11 .. +11) and S=1408 32 (-6 .. +25); where an XCD has a few more blocks
+//                      than compute units: B H=26 S=1152 24 (-10 .. +1), B H=32 S=1100 24-29 (-8 .. -11), B H=48 S=700 19-22
+//                      (-3 .. -14), with as many: B H=32 S=1024 21-24 (-8 .. +3)
 //          kRows128x2  B H=20 S=1300 28-34 (-7 .. -17), B H=16 S=2048 38-42 (-8 .. -11), B H=14 S=2500 48-61 (-15
 //                      .. -23), B H=12 S=4096 79-85 (-18 .. 0), B H=8 S=8192 169-175 (-2 .. -14); beyond: B H=26
 //                      S=1152 26 (+10 .. +26; 39 workgroups for 32 compute units), B H=16 S=4096 89-96 (-9 .. +14)
 //   64-row blocks: kRows64x4  B H=16 S=1237 31-40 (-34 .. -40), B H=12 S=2048 48 (-20 .. -38); kRows64x2  B H=40
 //                      S=512 16 (-12), B H=24 S=1024 27 (-23), B H=20 S=2048 50-56 (-18 .. -26)
 //   D=64   kRows32x4   against kRows64x2: B H=16 S=1024 11 (-10), B H=8 S=2048 17 (-22), B H=4 S=4096 29 (-25);
-//                      beyond: B H=20 S=1024 12 (+31)
+//                      B H=8 S=2304 19-22 (-10 .. -15), B H=10 S=2000 18-22 (0 .. -17), B H=4 S=5000 35-46 (-25 .. -32);
+//                      beyond: B H=20 S=1024 12 (+31), B H=16 S=1237 13-16 (+3 .. +21), B H=6 S=4096 30-33 (-5 .. +8)
 //          kRows64x2   B H=64 S=512 11-13 (-11 .. +3), B H=32 S=1024 18-20 (-4 .. -21), S=1237 21-28 (-14 .. -27),
 //                      B H=20 S=2048 31-34 (-6 .. -24), B H=16 S=3072 45-49 (-8 .. -23), S=4096 60-65 (-8 .. +3);
 //                      beyond: B H=40 S=1024 18-20 (0 .. +19), B H=24 S=2048 32-34 (-10 .. +16)
@@ -47,7 +50,8 @@ constexpr int fwd_split_rows(FwdSplit s, int QB) {
 //          kRows64x2   B H=40 S=1024 16-18 (-3 .. -16), B H=32 S=1536 21-24 (-10 .. -21), S=2048 28-33 (-14 .. +1)
 inline FwdSplit fwd_choose_split(int D, int QB, long long rows32, int S, long long busiest, int cus) {
   const int one_round_32 = D == 128 ? 384 : (D == 64 ? 512 : 768);
-  if (rows32 <= one_round_32 || (D == 128 && rows32 <= 512 && S >= 2560)) return FwdSplit::kRows32x4;
+  if (rows32 <= one_round_32 || (D == 128 && rows32 <= 512 && S >= 2560) || (D == 64 && rows32 <= 672 && S >= 2000))
+    return FwdSplit::kRows32x4;
   const bool some = (rows32 <= 1024 && S >= 512) || (rows32 <= 1280 && S >= 2048) || (rows32 <= 2048 && S >= 2 * rows32);
   const bool lone = (rows32 <= 512 && S >= 512) || (rows32 <= 640 && S >= 1152) || (rows32 <= 768 && S >= 1536);
   if (QB != 128) {
@@ -64,7 +68,8 @@ inline FwdSplit fwd_choose_split(int D, int QB, long long rows32, int S, long lo
   const bool one_round = busiest <= cus || (S >= 1280 && 8 * busiest <= 9LL * cus);
   const bool long_lists = S >= 2048 && (rows32 <= 1152 || (rows32 <= 1280 && S >= 2 * rows32) ||
                                         (rows32 <= 2048 && 5LL * S >= 13 * rows32));
-  return (rows32 <= 1152 && S >= 1152 && one_round) || long_lists ? FwdSplit::kRows128x2 : FwdSplit::kNone;
+  if ((rows32 <= 1152 && S >= 1152 && one_round) || long_lists) return FwdSplit::kRows128x2;
+  return rows32 <= 1152 && S >= 640 && busiest > cus && 4 * busiest < 5LL * cus ? FwdSplit::kRows64x2 : FwdSplit::kNone;
 }
 
 // How the walk of a KV block is split over waves in the dK/dV kernel.

@@ -86,7 +86,9 @@ enum class DkdvSplit : int {
 //   D=128  B H=8  S=512 37.9 -> 29.5, S=1024 59.7 -> 41.0, S=2048 102.9 -> 71.7, S=4096 192.3 -> 154.9
 //   D=64   B H=8  S=512 29.4 -> 20.2, S=1024 46.2 -> 26.5, S=2048  79.7 -> 51.1, S=4096 146.9 -> 103.0
 // The operator's backward at the lines (causal, spans, images), whole blocks, us, and the split of that kernel:
-//   dQ     D=128  B H=20 S=1024 62 (-2 .. -10 %), B H=8 S=4096 177-217 (-12 .. +3); 64-row blocks: B H=16 S=2048
+//   dQ     D=128  B H=20 S=1024 62 (-2 .. -10 %), B H=8 S=4096 177-217 (-12 .. +3); with the forward, B H=8 S=3000 173-222
+//                 (-9 .. -14), B H=12 S=1700 112-125 (-12 .. -13), S=2048 131-152 (-1 .. -12), B H=16 S=1700 117-130 (-6
+//                 .. -8); beyond: B H=20 S=1408 104 (-5 .. +1), B H=28 S=1152 95-101 (-2 .. +5); 64-row blocks: B H=16 S=2048
 //                 107-140 (-7 .. +1), S=1024 beyond: B H=32 68-85 (+1 .. +5)
 //          D=64   B H=40 S=1024 52-59 (-3 .. +1), B H=32 S=1237 58-72 (-6 .. -12), B H=24 S=2048 87-106 (-7 .. +3), B H=16
 //                 S=4096 167-211 (-3 .. +2); 64-row blocks B H=32 S=1237 57-69 (-7 .. -13), B H=16 S=4096 172-225 (-8 .. 0)
@@ -99,7 +101,8 @@ inline FwdSplit bwd_choose_dq_split(int D, int QB, long long rows32, int S) {
   if (rows32 <= (D == 128 ? 256 : 512)) return FwdSplit::kRows32x4;
   bool two;
   if (D == 128) {
-    two = rows32 <= 640 || (rows32 <= 1024 && S >= (QB == 128 ? 4096 : 2048));
+    two = rows32 <= 640 || (rows32 <= 1024 && S >= (QB == 128 ? 4096 : 2048)) ||
+          (QB == 128 && ((rows32 <= 768 && S >= 1024) || (rows32 <= 896 && S >= 1536)));
   } else {
     two = (rows32 <= 1024 && S >= 512) || (rows32 <= 1536 && S >= 1024) || (rows32 <= 2048 && S >= 4096);
   }

@@ -183,12 +183,17 @@ int omni_attn_fwd_strided_gfx950(const void* q, const void* k, const void* v, om
  * omni_attn_mask_lists_gfx950 writes kv_num_blocks [B, H, Tq] and kv_indices, block_mask_types,
  * partial_idx [B, H, Tq, Tk] (Tq = ceil(q_len / QB), Tk = ceil(kv_len / KB); zeros, and -1 in
  * partial_idx, behind the lists), and the number of PARTIAL tiles to host_total[0] -- host
- * memory that the device can write (hipHostMalloc) -- and then `ticket` to host_total[1]: the caller
+ * memory that the device can write (hipHostMalloc) -- with or before `ticket` to host_total[1]: the caller
  * waits for the ticket (or for the stream), allocates the tiles and calls
  * omni_attn_mask_tiles_gfx950 with the same arguments and the same workspace
  * (omni_attn_mask_workspace_bytes), which writes partial_masks [P, QB, KB] bytes (16-byte
  * aligned) and, where asked for (KB a multiple of 32), the packed words of
  * omni_attn_pack_partial_masks_gfx950.  QB up to OMNI_ATTN_MASK_MAX_QB.
+ * In two launches instead of four: omni_attn_mask_classify_gfx950 writes, per (b, query block), the number of
+ * its PARTIAL tiles with `tag` (12 bits) in the upper bits to posted[b * Tq + block] -- host memory as above, any
+ * values there before but that tag -- and needs the workspace only, so that a caller can allocate the lists
+ * while it runs; the sum of the counts is the size of the tile arrays, and omni_attn_mask_finish_gfx950 writes
+ * lists and tiles.  Tk below 2^OMNI_ATTN_MASK_POSTED_COUNT_BITS.
  */
 #define OMNI_ATTN_MASK_MAX_QB 8192
 size_t omni_attn_mask_workspace_bytes(int B, int q_len, int kv_len, int QB, int KB);
@@ -196,6 +201,14 @@ int omni_attn_mask_lists_gfx950(const int64_t* spans_or_null, const int64_t* pre
                                 int32_t* kv_num_blocks, int32_t* kv_indices, int32_t* block_mask_types,
                                 int32_t* partial_idx, void* workspace, int32_t* host_total, int ticket,
                                 int B, int M, int H, int q_len, int kv_len, int QB, int KB, void* stream);
+#define OMNI_ATTN_MASK_POSTED_COUNT_BITS 20
+int omni_attn_mask_classify_gfx950(const int64_t* spans_or_null, const int64_t* prefix_or_null, void* workspace,
+                                   uint32_t* posted, int tag, int B, int M, int q_len, int kv_len, int QB, int KB,
+                                   void* stream);
+int omni_attn_mask_finish_gfx950(int32_t* kv_num_blocks, int32_t* kv_indices, int32_t* block_mask_types,
+                                 int32_t* partial_idx, void* workspace, uint8_t* partial_masks_or_null,
+                                 uint32_t* partial_bits_or_null, int num_partial, int B, int H, int q_len, int kv_len,
+                                 int QB, int KB, void* stream);
 int omni_attn_mask_tiles_gfx950(const int64_t* spans_or_null, const int64_t* prefix_or_null,
                                 void* workspace, uint8_t* partial_masks, uint32_t* partial_bits_or_null,
                                 int num_partial, int B, int M, int H, int q_len, int kv_len, int QB, int KB,

@@ -5,20 +5,25 @@
 // (type, offset, length) also lets every row from its offset on see its end).  What the operator needs
 // of it is the typed block list per (b, head, query block) and the tiles of the PARTIAL blocks, in
 // (b, query block, slot) order, shared by the heads.  As tensor algebra that is some 80 launches
-// over [B, S, S / KB] integers and two read-backs; here it is three kernels and one wait:
-//   classify   one wave per (b, query block): the rows' R from the spans, the type of every key
-//              block, the list compacted and written for all heads; the number of its PARTIAL tiles
-//   number     one wave per (b, query block): the tiles before it, numbers for its PARTIAL slots, a
-//              table of what each tile is; the total goes to the host (pinned memory), which waits
-//              for it -- the caller's tile arrays have that size
-//   tiles      one workgroup per tile: its bytes, and its bits where they are asked for
-// All three are bound by their launches and a chain of a few memory latencies; the bytes
+// over [B, S, S / KB] integers and two read-backs; here it is two kernels and one wait between them:
+//   classify   one workgroup per (b, query block): the rows' R from the spans; the blocks below the smallest are FULL,
+//              the blocks from the largest on are not listed, and the few between get their type from a look at
+//              the rows.  Each sends the number of its PARTIAL tiles to the host (one word of pinned memory), which
+//              adds them up -- the caller's tile arrays have that size -- while the lists are allocated
+//   write      one workgroup per (b, query block) and four heads, a head per wave, writes the list and the tile
+//              numbers (the tiles before the query block are a sum over the counts), and one per tile, which finds
+//              its query block by a scan of the counts, writes its bytes, and its bits where they are asked for
+// Both are bound by their launches and a chain of a few memory latencies; the bytes
 // (B=4 H=16 S=8192, 128x128 blocks: 3.1 MB of lists, 2.4 MB of tiles) take a microsecond.  That mask,
-// packed: 472 us as tensor algebra, 39 us so (kernels 8 + 4 + 5 us, the rest launches and the wait).
+// packed, in calls back to back: 472 us as tensor algebra; 38 us as three kernels (8.2, 3.9 and 5.0 us)
+// with the wait behind the second; 32 us so (4.9 and 5.8 us; 20 us of a call pass between the first launch and its last
+// count on the host).
 #include "../../include/omni_attn_gfx950.h"
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 namespace omni_attn {
 // Keeps the hipError_t behind an OMNI_ATTN_ERR_LAUNCH for omni_attn_last_hip_error() (defined
@@ -40,20 +45,54 @@ struct MaskParams {
   int32_t* types;         // [B, H, Tq, Tk]
   int32_t* pidx;          // [B, H, Tq, Tk]
   int32_t* counts;        // [B * Tq] PARTIAL tiles of a query block
-  int32_t* tile_src;      // [B * Tq * Tk] (b, query block, key block) of a tile, as one index
-  int32_t* host_total;    // pinned: [0] the number of tiles, [1] the ticket, written after it
+  int32_t* full;          // [B * Tq] leading FULL blocks of its list
+  int32_t* listed;        // [B * Tq] blocks of its list: 0, 1, ...
+  int32_t* open;          // [B * Tq * Tk] types of the blocks full .. listed - 1
+  int32_t* reach;         // [B * Tq * QB] keys that a row attends
+  uint32_t* posted;       // pinned, or null: [B * Tq] tag in the upper 12 bits, count in the lower 20
+  int32_t* host_total;    // pinned: [0] the number of tiles, [1] the ticket
   int ticket;
+  int num_partial;        // tiles that there is room for
+  int head_groups;        // workgroups per query block that write lists
   int B, M, H, Tq, Tk, QB, KB, q_len, kv_len;
 };
+
+constexpr int kPostedCountBits = OMNI_ATTN_MASK_POSTED_COUNT_BITS;
 
 // Spans of a batch element that are worked at a time: (offset, end) pairs in LDS.
 constexpr int kSpanChunk = 64;
 
-// Keys of batch element b that the rows first .. first + QB - 1 attend: a prefix each, its length to
-// reach[].  `spans`: 2 kSpanChunk words of LDS.  Called by all NT threads of the workgroup.
-template <int NT>
-__device__ __forceinline__ void row_reaches(const MaskParams& p, int b, int first, int32_t* reach, int64_t* spans) {
-  for (int r = threadIdx.x; r < p.QB; r += NT) {
+__device__ __forceinline__ int clamp_to(int x, int hi) { return x < 0 ? 0 : (x > hi ? hi : x); }
+
+// Smallest (or largest) x of a wave, for x >= 0: through the lanes of the vector pipe, without LDS.
+template <bool MAX>
+__device__ __forceinline__ int wave_extreme(int x) {
+  auto step = [&](auto ctrl) {
+    const int other = __builtin_amdgcn_update_dpp(x, x, decltype(ctrl)::value, 0xf, 0xf, false);
+    x = (MAX ? other > x : other < x) ? other : x;
+  };
+  step(std::integral_constant<int, 0x111>{});  // row_shr 1, 2, 4, 8
+  step(std::integral_constant<int, 0x112>{});
+  step(std::integral_constant<int, 0x114>{});
+  step(std::integral_constant<int, 0x118>{});
+  step(std::integral_constant<int, 0x142>{});  // row_bcast 15, 31
+  step(std::integral_constant<int, 0x143>{});
+  return __builtin_amdgcn_readlane(x, 63);
+}
+
+// One workgroup per (b, query block), a thread per row (and every 256th after it).
+__global__ void __launch_bounds__(256) mask_classify_kernel(const MaskParams p) {
+  __shared__ int2 spans[kSpanChunk];
+  __shared__ int lows[4], highs[4];
+  __shared__ uint64_t partials[4];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int row = blockIdx.x;  // (b, query block)
+  const int b = row / p.Tq, qb = row - b * p.Tq;
+  const int first = qb * p.QB;
+  int32_t* const reach = p.reach + size_t(row) * p.QB;  // (a thread reads what it has written itself)
+  int mine = 0;  // of the first of its rows
+  int lo = 0x7fffffff, hi = 0;
+  for (int r = threadIdx.x; r < p.QB; r += 256) {
     const int i = first + r;
     int64_t n = int64_t(i) + 1;
     if (i >= p.q_len) {
@@ -62,135 +101,114 @@ __device__ __forceinline__ void row_reaches(const MaskParams& p, int b, int firs
       n = p.prefix[size_t(b) * p.q_len + i];
       n = n < 0 ? 0 : n;
     }
-    reach[r] = int(n < p.kv_len ? n : p.kv_len);
+    const int own = int(n < p.kv_len ? n : p.kv_len);
+    if (r < 256) mine = own;
+    if (p.spans == nullptr || r >= 256) reach[r] = own;
   }
-  if (p.spans == nullptr) return;
-  const int64_t* sp = p.spans + size_t(b) * p.M * 3;
-  for (int m0 = 0; m0 < p.M; m0 += kSpanChunk) {
-    __syncthreads();
-    const int n_spans = p.M - m0 < kSpanChunk ? p.M - m0 : kSpanChunk;
-    if (threadIdx.x < n_spans) {
-      const int64_t off = sp[3 * (m0 + threadIdx.x) + 1], len = sp[3 * (m0 + threadIdx.x) + 2];
-      const int64_t end = len > 0 ? off + len : 0;
-      spans[2 * threadIdx.x] = off;
-      spans[2 * threadIdx.x + 1] = end < p.kv_len ? end : p.kv_len;
+  if (p.spans != nullptr) {
+    const int64_t* sp = p.spans + size_t(b) * p.M * 3;
+    for (int m0 = 0; m0 < p.M; m0 += kSpanChunk) {
+      if (m0 > 0) __syncthreads();
+      const int n_spans = p.M - m0 < kSpanChunk ? p.M - m0 : kSpanChunk;
+      if (threadIdx.x < n_spans) {
+        const int64_t off = sp[3 * (m0 + threadIdx.x) + 1], len = sp[3 * (m0 + threadIdx.x) + 2];
+        const int64_t end = len > 0 ? off + len : 0;
+        // (rows are below 2^31 - 1)
+        spans[threadIdx.x] = {int(off < 0 ? 0 : (off < 0x7fffffff ? off : 0x7fffffff)),
+                              int(end < 0 ? 0 : (end < p.kv_len ? end : p.kv_len))};
+      }
+      __syncthreads();
+      for (int r = threadIdx.x; r < p.QB; r += 256) {
+        const int i = first + r;
+        if (i >= p.q_len) continue;
+        int n = r < 256 ? mine : reach[r];
+#pragma unroll 4
+        for (int m = 0; m < n_spans; ++m) {
+          const int2 span = spans[m];
+          if (i >= span.x && span.y > n) n = span.y;
+        }
+        if (r < 256) mine = n; else reach[r] = n;
+      }
     }
-    __syncthreads();
-    for (int r = threadIdx.x; r < p.QB; r += NT) {
-      const int i = first + r;
-      if (i >= p.q_len) continue;
-      int64_t n = reach[r];
-      for (int m = 0; m < n_spans; ++m)
-        if (int64_t(i) >= spans[2 * m] && spans[2 * m + 1] > n) n = spans[2 * m + 1];
-      reach[r] = int(n);
-    }
+    if (threadIdx.x < p.QB) reach[threadIdx.x] = mine;
   }
-}
-
-__device__ __forceinline__ int clamp_to(int x, int hi) { return x < 0 ? 0 : (x > hi ? hi : x); }
-
-__global__ void __launch_bounds__(64) mask_classify_kernel(const MaskParams p) {
-  __shared__ int64_t spans[2 * kSpanChunk];
-  extern __shared__ int32_t reach[];  // [QB]
-  const int lane = threadIdx.x;
-  const int row = blockIdx.x;  // (b, query block)
-  const int b = row / p.Tq, qb = row - b * p.Tq;
-  row_reaches<64>(p, b, qb * p.QB, reach, spans);
-  __syncthreads();
-  int lo = 0x7fffffff, hi = 0;
-  for (int r = lane; r < p.QB; r += 64) {
-    const int v = reach[r];
+  for (int r = threadIdx.x; r < p.QB; r += 256) {
+    const int v = r < 256 ? mine : reach[r];
     lo = v < lo ? v : lo;
     hi = v > hi ? v : hi;
   }
-  for (int m = 32; m >= 1; m >>= 1) {
-    const int l2 = __shfl_xor(lo, m, 64), h2 = __shfl_xor(hi, m, 64);
-    lo = l2 < lo ? l2 : lo;
-    hi = h2 > hi ? h2 : hi;
+  lo = wave_extreme<false>(lo);
+  hi = wave_extreme<true>(hi);
+  if (lane == 0) {
+    lows[w] = lo;
+    highs[w] = hi;
   }
-  int listed = 0, partial = 0;
-  for (int kb0 = 0; kb0 < p.Tk; kb0 += 64) {
-    const int kb = kb0 + lane;
-    const int k0 = kb * p.KB;
-    const bool active = kb < p.Tk && hi > k0;
-    const bool full = active && lo >= k0 + p.KB;
-    // the few blocks that are neither: CAUSAL if every row's part of the block is what the causal
-    // pattern gives it.  A lane looks at rows here, one block at a time.
-    uint64_t open = __ballot(active && !full), causal = 0;
-    for (uint64_t left = open; left != 0; left &= left - 1) {
-      const int j = __builtin_ctzll(left);
-      const int kj = (kb0 + j) * p.KB;
-      bool same = true;
-      for (int r = lane; r < p.QB; r += 64)
-        same &= clamp_to(reach[r] - kj, p.KB) == clamp_to(qb * p.QB + r + 1 - kj, p.KB);
-      if (__ballot(!same) == 0) causal |= 1ull << j;
-    }
-    const int type = !active ? 0 : (full ? kFull : ((causal >> lane) & 1 ? kCausal : kPartial));
-    const uint64_t act = __ballot(active);
-    partial += __popcll(__ballot(type == kPartial));
-    const int slot = listed + __popcll(act & ((1ull << lane) - 1));
-    listed += __popcll(act);
-    if (active)
-      for (int h = 0; h < p.H; ++h) {
-        const size_t o = ((size_t(b) * p.H + h) * p.Tq + qb) * p.Tk + slot;
-        p.idx[o] = kb;
-        p.types[o] = type;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    lo = lows[i] < lo ? lows[i] : lo;
+    hi = highs[i] > hi ? highs[i] : hi;
+  }
+  const int full = lo / p.KB, listed = (hi + p.KB - 1) / p.KB;
+  // The few blocks that are neither FULL nor left out: CAUSAL if every row's part of the block is what the causal
+  // pattern gives it.  A row that attends R keys where causal is c differs from that in the blocks between the two.
+  int partial = 0;
+  for (int kb0 = full; kb0 < listed; kb0 += 64) {
+    const int n = listed - kb0 < 64 ? listed - kb0 : 64;
+    uint64_t differ = 0;  // (wave-uniform)
+    for (int r0 = 0; r0 < p.QB; r0 += 256) {
+      const int r = r0 + threadIdx.x;
+      int from = 0, to = 0;
+      if (r < p.QB) {
+        const int v = r < 256 ? mine : reach[r], c = first + r + 1;
+        const int a = v < c ? v : c, z = v < c ? c : v;
+        if (a != z) {
+          from = a / p.KB;
+          to = (z - 1) / p.KB + 1;
+        }
       }
-  }
-  for (int h = 0; h < p.H; ++h) {  // zeros behind the list
-    const size_t o = ((size_t(b) * p.H + h) * p.Tq + qb) * p.Tk;
-    for (int s = listed + lane; s < p.Tk; s += 64) {
-      p.idx[o + s] = 0;
-      p.types[o + s] = 0;
+      for (int i = 0; i < n; ++i)
+        if (__ballot(kb0 + i >= from && kb0 + i < to) != 0) differ |= 1ull << i;
     }
+    if (kb0 > full) __syncthreads();
+    if (lane == 0) partials[w] = differ;
+    __syncthreads();
+    differ = partials[0] | partials[1] | partials[2] | partials[3];
+    partial += __popcll(differ);
+    if (threadIdx.x < n) p.open[size_t(row) * p.Tk + kb0 + threadIdx.x] = (differ >> threadIdx.x) & 1 ? kPartial : kCausal;
   }
-  for (int h = lane; h < p.H; h += 64) p.nb[(size_t(b) * p.H + h) * p.Tq + qb] = listed;
-  if (lane == 0) p.counts[row] = partial;
+  if (threadIdx.x == 0) {
+    if (p.posted != nullptr)
+      __hip_atomic_store(p.posted + row, uint32_t(p.ticket) << kPostedCountBits | uint32_t(partial), __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
+    p.counts[row] = partial;
+    p.full[row] = full;
+    p.listed[row] = listed;
+  }
 }
 
-__global__ void __launch_bounds__(64) mask_number_kernel(const MaskParams p) {
-  const int lane = threadIdx.x;
-  const int row = blockIdx.x;
-  const int b = row / p.Tq, qb = row - b * p.Tq;
-  const int n = p.B * p.Tq;
-  int before = 0, all = 0;
-  for (int i = lane; i < n; i += 64) {
-    const int c = p.counts[i];
-    all += c;
-    before += i < row ? c : 0;
-  }
-  for (int m = 32; m >= 1; m >>= 1) {
-    before += __shfl_xor(before, m, 64);
-    all += __shfl_xor(all, m, 64);
-  }
-  if (row == 0 && lane == 0) {
+// Sum over a workgroup of four waves; `part`: 4 words of LDS.
+__device__ __forceinline__ int sum_of_256(int x, int32_t* part) {
+  for (int m = 32; m >= 1; m >>= 1) x += __shfl_xor(x, m, 64);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = x;
+  __syncthreads();
+  return part[0] + part[1] + part[2] + part[3];
+}
+
+// The number of tiles, to the host as one word (callers that take no counts).
+__global__ void __launch_bounds__(256) mask_total_kernel(const MaskParams p) {
+  __shared__ int32_t part[4];
+  int x = 0;
+  for (int i = threadIdx.x; i < p.B * p.Tq; i += 256) x += p.counts[i];
+  const int all = sum_of_256(x, part);
+  if (threadIdx.x == 0) {
     __hip_atomic_store(p.host_total, all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     __hip_atomic_store(p.host_total + 1, p.ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
-  const size_t o0 = (size_t(b) * p.H * p.Tq + qb) * p.Tk;  // head 0
-  for (int s0 = 0; s0 < p.Tk; s0 += 64) {
-    const int s = s0 + lane;
-    const bool is_p = s < p.Tk && p.types[o0 + s] == kPartial;
-    const uint64_t bits = __ballot(is_p);
-    const int pid = before + __popcll(bits & ((1ull << lane) - 1));
-    before += __popcll(bits);
-    if (is_p) p.tile_src[pid] = row * p.Tk + p.idx[o0 + s];
-    if (s < p.Tk)
-      for (int h = 0; h < p.H; ++h) p.pidx[o0 + size_t(h) * p.Tq * p.Tk + s] = is_p ? pid : -1;
-  }
 }
 
-__global__ void __launch_bounds__(256) mask_tiles_kernel(const MaskParams p, uint8_t* __restrict__ tiles,
-                                                         uint32_t* __restrict__ bits) {
-  __shared__ int64_t spans[2 * kSpanChunk];
-  extern __shared__ int32_t reach[];  // [QB]
-  const int src = p.tile_src[blockIdx.x];
-  const int row = src / p.Tk, kb = src - row * p.Tk;
-  const int b = row / p.Tq, qb = row - b * p.Tq;
-  row_reaches<256>(p, b, qb * p.QB, reach, spans);
-  __syncthreads();
-  const int k0 = kb * p.KB;
-  uint8_t* const tile = tiles + size_t(blockIdx.x) * p.QB * p.KB;
+// One tile: its bytes, and its bits.
+__device__ __forceinline__ void write_tile(const MaskParams& p, const int32_t* reach, int k0, uint8_t* tile, uint32_t* bits) {
   if (p.KB % 16 == 0) {
     const int per_row = p.KB / 16;
     for (int i = threadIdx.x; i < p.QB * per_row; i += 256) {
@@ -212,13 +230,90 @@ __global__ void __launch_bounds__(256) mask_tiles_kernel(const MaskParams p, uin
   }
   if (bits != nullptr) {
     const int words = p.KB / 32;
-    uint32_t* const out = bits + size_t(blockIdx.x) * p.QB * words;
     for (int i = threadIdx.x; i < p.QB * words; i += 256) {
       const int r = i / words;
       const int n = clamp_to(reach[r] - k0 - (i - r * words) * 32, 32);
-      out[i] = n == 32 ? 0xffffffffu : (1u << n) - 1u;
+      bits[i] = n == 32 ? 0xffffffffu : (1u << n) - 1u;
     }
   }
+}
+
+// The workgroups 0 .. num_partial - 1 write a tile each, the others the lists of four heads in a query block each.
+__global__ void __launch_bounds__(256) mask_write_kernel(const MaskParams p, uint8_t* __restrict__ tiles,
+                                                         uint32_t* __restrict__ bits) {
+  __shared__ int32_t part[4];
+  __shared__ int32_t found[2];  // query block of the tile, and which of its PARTIAL blocks
+  extern __shared__ int32_t reach[];  // [QB]
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int n_rows = p.B * p.Tq;
+  if (int(blockIdx.x) < p.num_partial) {
+    const int tile = blockIdx.x;
+    // a thread looks at `per` neighbouring query blocks
+    const int per = (n_rows + 255) / 256, r0 = threadIdx.x * per, r1 = r0 + per < n_rows ? r0 + per : n_rows;
+    int mine = 0;
+    for (int r = r0; r < r1; ++r) mine += p.counts[r];
+    int upto = mine;  // inclusive sum over the threads
+    for (int d = 1; d < 64; d <<= 1) {
+      const int other = __shfl_up(upto, d, 64);
+      upto += lane >= d ? other : 0;
+    }
+    if (lane == 63) part[w] = upto;
+    __syncthreads();
+    for (int i = 0; i < w; ++i) upto += part[i];
+    int left = tile - (upto - mine);
+    if (left >= 0 && left < mine) {
+      int r = r0;
+      for (int c = p.counts[r]; left >= c; c = p.counts[++r]) left -= c;
+      found[0] = r;
+      found[1] = left;
+    }
+    __syncthreads();
+    const int row = found[0];
+    left = found[1];
+    for (int r = threadIdx.x; r < p.QB; r += 256) reach[r] = p.reach[size_t(row) * p.QB + r];
+    const int listed = p.listed[row];
+    int kb = p.full[row];
+    for (;; kb += 64) {  // (the block is in the list)
+      const bool is = kb + lane < listed && p.open[size_t(row) * p.Tk + kb + lane] == kPartial;
+      uint64_t partials = __ballot(is);
+      const int n = __popcll(partials);
+      if (left < n) {
+        for (; left > 0; --left) partials &= partials - 1;
+        kb += __builtin_ctzll(partials);
+        break;
+      }
+      left -= n;
+      if (kb + 64 >= listed) return;
+    }
+    __syncthreads();
+    const size_t at = size_t(tile) * p.QB * p.KB;
+    write_tile(p, reach, kb * p.KB, tiles + at, bits != nullptr ? bits + at / 32 : nullptr);
+    return;
+  }
+  const int item = blockIdx.x - p.num_partial;
+  const int row = item / p.head_groups, group = item - row * p.head_groups;
+  const int b = row / p.Tq, qb = row - b * p.Tq;
+  const int full = p.full[row], listed = p.listed[row];
+  int x = 0;
+  for (int i = threadIdx.x; i < row; i += 256) x += p.counts[i];
+  int before = sum_of_256(x, part);  // tiles of the query blocks before this one
+  for (int s0 = 0; s0 < p.Tk; s0 += 64) {
+    const int s = s0 + lane;
+    int type = s < full ? kFull : 0;
+    if (s >= full && s < listed) type = p.open[size_t(row) * p.Tk + s];
+    const uint64_t partials = __ballot(type == kPartial);
+    const int pid = type == kPartial ? before + __popcll(partials & ((1ull << lane) - 1)) : -1;
+    before += __popcll(partials);
+    if (s >= p.Tk) continue;
+    for (int h = group * 4 + w; h < p.H; h += p.head_groups * 4) {
+      const size_t o = ((size_t(b) * p.H + h) * p.Tq + qb) * p.Tk + s;
+      p.idx[o] = s < listed ? s : 0;
+      p.types[o] = type;
+      p.pidx[o] = pid;
+    }
+  }
+  for (int h = group * 4 + w; h < p.H; h += p.head_groups * 4)
+    if (lane == 0) p.nb[(size_t(b) * p.H + h) * p.Tq + qb] = listed;
 }
 
 int bad_shape(int B, int M, int H, int q_len, int kv_len, int QB, int KB) {
@@ -244,8 +339,12 @@ MaskParams common(const int64_t* spans, const int64_t* prefix, void* workspace, 
   p.kv_len = kv_len;
   p.Tq = (q_len + QB - 1) / QB;
   p.Tk = (kv_len + KB - 1) / KB;
+  const size_t rows = size_t(B) * p.Tq;
   p.counts = static_cast<int32_t*>(workspace);
-  p.tile_src = p.counts + size_t(B) * p.Tq;
+  p.full = p.counts + rows;
+  p.listed = p.full + rows;
+  p.open = p.listed + rows;
+  p.reach = p.open + rows * p.Tk;
   return p;
 }
 
@@ -260,7 +359,64 @@ int launched(hipError_t e) {
 extern "C" size_t omni_attn_mask_workspace_bytes(int B, int q_len, int kv_len, int QB, int KB) {
   if (bad_shape(B, 0, 1, q_len, kv_len, QB, KB) != OMNI_ATTN_OK) return 0;
   const size_t Tq = size_t((q_len + QB - 1) / QB), Tk = size_t((kv_len + KB - 1) / KB);
-  return (size_t(B) * Tq + size_t(B) * Tq * Tk) * sizeof(int32_t);
+  return size_t(B) * Tq * (3 + Tk + QB) * sizeof(int32_t);
+}
+
+namespace {
+int launch_classify(const MaskParams& params, hipStream_t stream) {
+  MaskParams p = params;
+  void* args[] = {&p};
+  return launched(hipLaunchKernel(reinterpret_cast<const void*>(mask_classify_kernel), dim3(unsigned(p.B) * unsigned(p.Tq)),
+                                  dim3(256), args, 0, stream));
+}
+// Lists (where p.nb is given) and tiles (where there are any), in one launch.
+int launch_write(const MaskParams& params, uint8_t* tiles, uint32_t* bits, hipStream_t stream) {
+  MaskParams p = params;
+  const long long rows = (long long)p.B * p.Tq, room = 0x7fffffffLL - p.num_partial;
+  const long long by_four = (p.H + 3) / 4;
+  p.head_groups = p.nb == nullptr ? 0 : int(by_four * rows <= room ? by_four : (room / rows > 1 ? room / rows : 1));
+  const long long grid = p.num_partial + rows * p.head_groups;
+  if (grid > 0x7fffffffLL) return OMNI_ATTN_ERR_TOO_LARGE;
+  void* args[] = {&p, &tiles, &bits};
+  return launched(hipLaunchKernel(reinterpret_cast<const void*>(mask_write_kernel), dim3(unsigned(grid)), dim3(256), args,
+                                  p.num_partial > 0 ? size_t(p.QB) * sizeof(int32_t) : 0, stream));
+}
+int check_tiles(const uint8_t* partial_masks, const uint32_t* partial_bits_or_null, int num_partial, const MaskParams& p) {
+  if (num_partial < 0 || (partial_bits_or_null && p.KB % 32 != 0)) return OMNI_ATTN_ERR_BAD_SHAPE;
+  if ((reinterpret_cast<uintptr_t>(partial_masks) & 15) != 0 || (reinterpret_cast<uintptr_t>(partial_bits_or_null) & 3) != 0)
+    return OMNI_ATTN_ERR_MISALIGNED;
+  return (long long)num_partial > (long long)p.B * p.Tq * p.Tk ? OMNI_ATTN_ERR_BAD_SHAPE : OMNI_ATTN_OK;
+}
+}  // namespace
+
+extern "C" int omni_attn_mask_classify_gfx950(const int64_t* spans_or_null, const int64_t* prefix_or_null,
+                                              void* workspace, uint32_t* posted, int tag, int B, int M, int q_len,
+                                              int kv_len, int QB, int KB, void* stream) {
+  if ((!spans_or_null == !prefix_or_null) || !workspace || !posted) return OMNI_ATTN_ERR_NULL_POINTER;
+  if (const int rc = bad_shape(B, M, 1, q_len, kv_len, QB, KB)) return rc;
+  MaskParams p = common(spans_or_null, prefix_or_null, workspace, B, M, 1, q_len, kv_len, QB, KB);
+  if (p.Tk >> kPostedCountBits != 0 || tag < 0 || tag >> (32 - kPostedCountBits) != 0) return OMNI_ATTN_ERR_TOO_LARGE;
+  p.posted = posted;
+  p.ticket = tag;
+  return launch_classify(p, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int omni_attn_mask_finish_gfx950(int32_t* kv_num_blocks, int32_t* kv_indices, int32_t* block_mask_types,
+                                            int32_t* partial_idx, void* workspace, uint8_t* partial_masks_or_null,
+                                            uint32_t* partial_bits_or_null, int num_partial, int B, int H, int q_len,
+                                            int kv_len, int QB, int KB, void* stream) {
+  if (!kv_num_blocks || !kv_indices || !block_mask_types || !partial_idx || !workspace ||
+      (num_partial > 0 && !partial_masks_or_null))
+    return OMNI_ATTN_ERR_NULL_POINTER;
+  if (const int rc = bad_shape(B, 0, H, q_len, kv_len, QB, KB)) return rc;
+  MaskParams p = common(nullptr, nullptr, workspace, B, 0, H, q_len, kv_len, QB, KB);
+  if (const int rc = check_tiles(partial_masks_or_null, partial_bits_or_null, num_partial, p)) return rc;
+  p.nb = kv_num_blocks;
+  p.idx = kv_indices;
+  p.types = block_mask_types;
+  p.pidx = partial_idx;
+  p.num_partial = num_partial;
+  return launch_write(p, partial_masks_or_null, partial_bits_or_null, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int omni_attn_mask_lists_gfx950(const int64_t* spans_or_null, const int64_t* prefix_or_null,
@@ -278,14 +434,12 @@ extern "C" int omni_attn_mask_lists_gfx950(const int64_t* spans_or_null, const i
   p.pidx = partial_idx;
   p.host_total = host_total;
   p.ticket = ticket;
-  const dim3 grid(unsigned(B) * unsigned(p.Tq));
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  if (const int rc = launch_classify(p, s)) return rc;
   void* args[] = {&p};
-  hipError_t e = hipLaunchKernel(reinterpret_cast<const void*>(mask_classify_kernel), grid, dim3(64), args,
-                                 size_t(QB) * sizeof(int32_t), static_cast<hipStream_t>(stream));
-  if (e != hipSuccess) return launched(e);
-  e = hipLaunchKernel(reinterpret_cast<const void*>(mask_number_kernel), grid, dim3(64), args, 0,
-                      static_cast<hipStream_t>(stream));
-  return launched(e);
+  if (const int rc = launched(hipLaunchKernel(reinterpret_cast<const void*>(mask_total_kernel), dim3(1), dim3(256), args, 0, s)))
+    return rc;
+  return launch_write(p, nullptr, nullptr, s);
 }
 
 extern "C" int omni_attn_mask_tiles_gfx950(const int64_t* spans_or_null, const int64_t* prefix_or_null,
@@ -295,12 +449,8 @@ extern "C" int omni_attn_mask_tiles_gfx950(const int64_t* spans_or_null, const i
   if (num_partial == 0) return OMNI_ATTN_OK;
   if ((!spans_or_null == !prefix_or_null) || !workspace || !partial_masks) return OMNI_ATTN_ERR_NULL_POINTER;
   if (const int rc = bad_shape(B, M, H, q_len, kv_len, QB, KB)) return rc;
-  if (num_partial < 0 || (partial_bits_or_null && KB % 32 != 0)) return OMNI_ATTN_ERR_BAD_SHAPE;
-  if ((reinterpret_cast<uintptr_t>(partial_masks) & 15) != 0 || (reinterpret_cast<uintptr_t>(partial_bits_or_null) & 3) != 0)
-    return OMNI_ATTN_ERR_MISALIGNED;
   MaskParams p = common(spans_or_null, prefix_or_null, workspace, B, M, H, q_len, kv_len, QB, KB);
-  if ((long long)num_partial > (long long)B * p.Tq * p.Tk) return OMNI_ATTN_ERR_BAD_SHAPE;
-  void* args[] = {&p, &partial_masks, &partial_bits_or_null};
-  return launched(hipLaunchKernel(reinterpret_cast<const void*>(mask_tiles_kernel), dim3(unsigned(num_partial)),
-                                  dim3(256), args, size_t(QB) * sizeof(int32_t), static_cast<hipStream_t>(stream)));
+  if (const int rc = check_tiles(partial_masks, partial_bits_or_null, num_partial, p)) return rc;
+  p.num_partial = num_partial;
+  return launch_write(p, partial_masks, partial_bits_or_null, static_cast<hipStream_t>(stream));
 }

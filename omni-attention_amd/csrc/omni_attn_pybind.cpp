@@ -10,6 +10,7 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
+#include <cstring>
 #include <mutex>
 #include <stdexcept>
 #include <string>
@@ -297,69 +298,91 @@ void omni_attn_backward(torch::Tensor Q, torch::Tensor K, torch::Tensor V, torch
   }
 }
 
-// Where a kernel writes one number that the host waits for: pinned host memory, handed out per
-// call (so calls of several threads and streams do not meet) and taken back; at most kKeep of
-// them are kept between calls.
-class HostNumber {
+// Where the workgroups of a kernel write a count each that the host waits for, as words of a tag and the count:
+// pinned host memory, handed out per call (so calls of several threads and streams do not meet) and taken
+// back; at most kKeep pieces of kWords words are kept between calls.
+class HostCounts {
  public:
-  HostNumber() {
+  static constexpr int kWords = 4096;
+  HostCounts() {
     std::lock_guard<std::mutex> lock(mutex());
     if (!spare().empty()) {
-      slot_ = spare().back();
+      words_ = spare().back();
       spare().pop_back();
       return;
     }
     void* mem = nullptr;
-    // (portable: a word taken under one device is handed to calls on any)
-    const hipError_t e = hipHostMalloc(&mem, 64, hipHostMallocPortable | hipHostMallocMapped);
+    // (portable: memory taken under one device is handed to calls on any)
+    const hipError_t e = hipHostMalloc(&mem, size_t(kWords + 16) * 4, hipHostMallocPortable | hipHostMallocMapped);
     if (e != hipSuccess) throw std::runtime_error(std::string("omni_attn: hipHostMalloc: ") + hipGetErrorString(e));
-    slot_ = static_cast<int32_t*>(mem);
-    slot_[0] = slot_[1] = slot_[2] = 0;
+    words_ = static_cast<uint32_t*>(mem);
+    std::memset(words_, 0, size_t(kWords + 16) * 4);
   }
-  ~HostNumber() {
+  ~HostCounts() {
     if (!idle_) return;  // a kernel may still write it: the memory stays allocated
     std::lock_guard<std::mutex> lock(mutex());
     if (spare().size() < kKeep) {
-      spare().push_back(slot_);
+      spare().push_back(words_);
     } else {
-      (void)hipHostFree(slot_);
+      (void)hipHostFree(words_);
     }
   }
-  HostNumber(const HostNumber&) = delete;
-  HostNumber& operator=(const HostNumber&) = delete;
+  HostCounts(const HostCounts&) = delete;
+  HostCounts& operator=(const HostCounts&) = delete;
 
-  int32_t* memory() { return slot_; }
-  int next_ticket() {
+  uint32_t* memory() { return words_; }
+  // A tag that no word has: they are cleared where the tags begin again.
+  int next_tag() {
+    uint32_t& last = words_[kWords];
+    if (last == (1u << (32 - kCountBits)) - 1) {
+      std::memset(words_, 0, size_t(kWords) * 4);
+      last = 0;
+    }
     idle_ = false;
-    return ++slot_[2];
+    return int(++last);
   }
-  // The number, once the kernel that writes it has run.  Ends as well when the stream has
-  // nothing left to run or reports an error.
-  int wait(int ticket, hipStream_t stream) {
+  // The sum of the first n counts, once the kernel that writes them has run.
+  int64_t wait(int tag, int n, hipStream_t stream) {
+    int64_t sum = 0;
+    for (int i = 0; i < n; ++i) sum += wait_for(i, tag, stream) & ((1u << kCountBits) - 1);
+    idle_ = true;
+    return sum;
+  }
+  // A number of any size in word 0, written before the tag in word 1.
+  int32_t wait_total(int tag, hipStream_t stream) {
+    (void)wait_for(1, tag, stream);
+    idle_ = true;
+    const int32_t total = int32_t(words_[0]);
+    words_[0] = words_[1] = 0;
+    return total;
+  }
+  static int word_of(int tag) { return int(uint32_t(tag) << kCountBits); }
+
+ private:
+  // Ends as well when the stream has nothing left to run or reports an error.
+  uint32_t wait_for(int i, int tag, hipStream_t stream) {
     for (unsigned spins = 1;; ++spins) {
-      if (__atomic_load_n(slot_ + 1, __ATOMIC_ACQUIRE) == ticket) break;
+      const uint32_t x = __atomic_load_n(words_ + i, __ATOMIC_ACQUIRE);
+      if (int(x >> kCountBits) == tag) return x;
       if (spins % 8192 == 0) {
         const hipError_t e = hipStreamQuery(stream);
         if (e == hipErrorNotReady) continue;
-        if (e == hipSuccess && __atomic_load_n(slot_ + 1, __ATOMIC_ACQUIRE) == ticket) break;
+        if (e == hipSuccess && int(__atomic_load_n(words_ + i, __ATOMIC_ACQUIRE) >> kCountBits) == tag) continue;
         throw std::runtime_error(std::string("omni_attn: the mask was not built: ") + hipGetErrorString(e));
       }
     }
-    idle_ = true;
-    return slot_[0];
   }
-
- private:
+  static constexpr int kCountBits = OMNI_ATTN_MASK_POSTED_COUNT_BITS;
   static constexpr size_t kKeep = 16;
   static std::mutex& mutex() {
     static std::mutex* m = new std::mutex;
     return *m;
   }
-  static std::vector<int32_t*>& spare() {
-    static std::vector<int32_t*>* v = new std::vector<int32_t*>;
+  static std::vector<uint32_t*>& spare() {
+    static std::vector<uint32_t*>* v = new std::vector<uint32_t*>;
     return *v;
   }
-  int32_t* slot_ = nullptr;
+  uint32_t* words_ = nullptr;  // kWords counts; the last tag
   bool idle_ = true;
 };
 
@@ -606,35 +629,62 @@ pybind11::tuple omni_attn_build_prefix_mask(torch::Tensor source, bool spans, in
   if (ws_bytes == 0) throw std::runtime_error("omni_attn: the block mask's sizes are not positive or too large");
   const int64_t Tq = (q_len + QB - 1) / QB, Tk = (kv_len + KB - 1) / KB;
   const auto i32 = source.options().dtype(torch::kInt32);
-  torch::Tensor nb = torch::empty({B, H, Tq}, i32), idx = torch::empty({B, H, Tq, Tk}, i32),
-                types = torch::empty({B, H, Tq, Tk}, i32), pidx = torch::empty({B, H, Tq, Tk}, i32),
-                workspace = torch::empty({int64_t(ws_bytes / 4)}, i32);
+  torch::Tensor workspace = torch::empty({int64_t(ws_bytes / 4)}, i32);
   // (a span pointer of an empty [B, 0, 3] tensor may be null: any address, nothing is read through it)
   const int64_t* src = source.numel() > 0 ? source.data_ptr<int64_t>()
                                           : reinterpret_cast<const int64_t*>(workspace.data_ptr<int32_t>());
   const int64_t* sp = spans ? src : nullptr;
   const int64_t* prefix = spans ? nullptr : src;
-  int P = 0;
+  const auto refuse = [](int rc) {
+    if (rc != OMNI_ATTN_OK) throw std::runtime_error(std::string("omni_attn: ") + omni_attn_status_string(rc));
+  };
+  int* const ws = workspace.data_ptr<int32_t>();
+  torch::Tensor nb, idx, types, pidx, tiles, bits;
+  const auto allocate_lists = [&] {
+    nb = torch::empty({B, H, Tq}, i32);
+    idx = torch::empty({B, H, Tq, Tk}, i32);
+    types = torch::empty({B, H, Tq, Tk}, i32);
+    pidx = torch::empty({B, H, Tq, Tk}, i32);
+  };
+  const auto allocate_tiles = [&](int64_t P) {
+    if (P > 0x7fffffff) refuse(OMNI_ATTN_ERR_TOO_LARGE);
+    if (P == 0) return;
+    tiles = torch::empty({P, QB, KB}, source.options().dtype(torch::kBool));
+    if (pack) bits = torch::empty({P, QB, KB / 32}, i32);
+  };
+  const auto tile_bytes = [&] { return tiles.defined() ? static_cast<uint8_t*>(tiles.data_ptr()) : nullptr; };
+  const auto tile_words = [&] {
+    return bits.defined() ? reinterpret_cast<uint32_t*>(bits.data_ptr<int32_t>()) : nullptr;
+  };
+  void* const at = static_cast<void*>(stream);
   {
     py::gil_scoped_release release;
-    HostNumber total;
-    const int ticket = total.next_ticket();
-    const int rc = omni_attn_mask_lists_gfx950(
-        sp, prefix, nb.data_ptr<int32_t>(), idx.data_ptr<int32_t>(), types.data_ptr<int32_t>(),
-        pidx.data_ptr<int32_t>(), workspace.data_ptr<int32_t>(), total.memory(), ticket, int(B), int(M), int(H),
-        int(q_len), int(kv_len), int(QB), int(KB), static_cast<void*>(stream));
-    if (rc != OMNI_ATTN_OK) throw std::runtime_error(std::string("omni_attn: ") + omni_attn_status_string(rc));
-    P = total.wait(ticket, stream);
+    HostCounts counts;
+    const int tag = counts.next_tag();
+    if (B * Tq <= HostCounts::kWords && (Tk >> OMNI_ATTN_MASK_POSTED_COUNT_BITS) == 0) {
+      // The first kernel needs the workspace only, and sends its counts as they are known: the lists are allocated
+      // while it runs.
+      refuse(omni_attn_mask_classify_gfx950(sp, prefix, ws, counts.memory(), tag, int(B), int(M), int(q_len), int(kv_len),
+                                            int(QB), int(KB), at));
+      allocate_lists();
+      allocate_tiles(counts.wait(tag, int(B * Tq), stream));
+      refuse(omni_attn_mask_finish_gfx950(nb.data_ptr<int32_t>(), idx.data_ptr<int32_t>(), types.data_ptr<int32_t>(),
+                                          pidx.data_ptr<int32_t>(), ws, tile_bytes(), tile_words(),
+                                          tiles.defined() ? int(tiles.size(0)) : 0, int(B), int(H), int(q_len),
+                                          int(kv_len), int(QB), int(KB), at));
+    } else {
+      allocate_lists();
+      refuse(omni_attn_mask_lists_gfx950(sp, prefix, nb.data_ptr<int32_t>(), idx.data_ptr<int32_t>(),
+                                         types.data_ptr<int32_t>(), pidx.data_ptr<int32_t>(), ws,
+                                         reinterpret_cast<int32_t*>(counts.memory()), HostCounts::word_of(tag), int(B),
+                                         int(M), int(H), int(q_len), int(kv_len), int(QB), int(KB), at));
+      allocate_tiles(counts.wait_total(tag, stream));
+      if (tiles.defined())
+        refuse(omni_attn_mask_tiles_gfx950(sp, prefix, ws, tile_bytes(), tile_words(), int(tiles.size(0)), int(B), int(M),
+                                           int(H), int(q_len), int(kv_len), int(QB), int(KB), at));
+    }
   }
-  if (P == 0) return py::make_tuple(nb, idx, types, py::none(), py::none(), py::none());
-  torch::Tensor tiles = torch::empty({P, QB, KB}, source.options().dtype(torch::kBool));
-  torch::Tensor bits;
-  if (pack) bits = torch::empty({P, QB, KB / 32}, i32);
-  const int rc = omni_attn_mask_tiles_gfx950(
-      sp, prefix, workspace.data_ptr<int32_t>(), static_cast<uint8_t*>(tiles.data_ptr()),
-      pack ? reinterpret_cast<uint32_t*>(bits.data_ptr<int32_t>()) : nullptr, P, int(B), int(M), int(H), int(q_len),
-      int(kv_len), int(QB), int(KB), static_cast<void*>(stream));
-  if (rc != OMNI_ATTN_OK) throw std::runtime_error(std::string("omni_attn: ") + omni_attn_status_string(rc));
+  if (!tiles.defined()) return py::make_tuple(nb, idx, types, py::none(), py::none(), py::none());
   return py::make_tuple(nb, idx, types, pidx, tiles, pack ? py::cast(bits) : py::object(py::none()));
 }
 

@@ -25,6 +25,8 @@ EXPORTED_SYMBOLS = (
     "omni_attn_pack_partial_masks_gfx950",
     "omni_attn_mask_workspace_bytes",
     "omni_attn_mask_lists_gfx950",
+    "omni_attn_mask_classify_gfx950",
+    "omni_attn_mask_finish_gfx950",
     "omni_attn_mask_tiles_gfx950",
     "omni_attn_bwd_gfx950",
     "omni_attn_bwd_strided_gfx950",

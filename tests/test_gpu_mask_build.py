@@ -47,3 +47,29 @@ def test_packed_tiles_come_with_the_mask(gpu_device):
     m.partial_block_bits = None
     assert torch.equal(m.pack_partial_masks().partial_block_bits, bits)
     assert shim.create_transfusion_block_mask(mp.to(gpu_device), 2, 500, pack=False).partial_block_bits is None
+
+
+def test_more_query_blocks_than_counts_are_sent_for(gpu_device):
+    """9 x 512 query blocks: the number of tiles comes as one word instead of a count per query block."""
+    gen = torch.Generator().manual_seed(3)
+    spans = torch.zeros(9, 3, 3, dtype=torch.long)
+    cuts = torch.randint(0, 8000, (9, 3, 2), generator=gen)
+    spans[..., 1], spans[..., 2] = cuts.amin(-1), cuts.amax(-1) - cuts.amin(-1)
+    args = (spans, 9, 2, 8192, 8192, 16, 64)
+    want = oat.create_omni_block_mask_from_modality_positions(*args, device="cpu")
+    for _ in range(2):
+        same_mask(oat.create_omni_block_mask_from_modality_positions(*args, device=gpu_device), want)
+
+
+def test_many_masks_in_a_row(gpu_device):
+    """More calls than the counts have tags, of two sizes in turn, so that words of earlier calls are still there."""
+    small = torch.tensor([[[1, 37, 90], [1, 200, 141]]])
+    large = small.repeat(4, 1, 1)
+    sizes = [(small, 500), (large, 3000)]
+    want = [shim.create_transfusion_block_mask(mp, 2, S, 128, 128, pack=False).partial_block_masks.shape[0] for mp, S in sizes]
+    assert want[0] != want[1] > 0
+    sizes = [(mp.to(gpu_device), S) for mp, S in sizes]
+    for i in range(4200):
+        mp, S = sizes[i % 64 == 0]
+        m = shim.create_transfusion_block_mask(mp, 2, S, 128, 128, pack=False)
+        assert m.partial_block_masks.shape[0] == want[i % 64 == 0]

@@ -23,13 +23,15 @@
 // A key that a row may not attend to never reaches it, whatever its V row holds (0 * infinity would):
 // a wave whose sums end up infinite or NaN walks its list once more and leaves out the zero weights.
 //
-// Bound by the latency of a step (two matrix chains, the softmax and the split of the weights on the
-// vector pipe) times the steps of the longest list over the waves; from 192 columns on by LDS (a step
-// of 32 rows reads each K and V byte once for 32 query rows).  B=1 H=8 S=2048 D=96 fp16, causal in 32x32
-// blocks, launches back to back: 30 us (bf16 29), 38 where queries are four times as large (every row
-// peaked, a rest in most steps); D=95, rows at any alignment, 43.  Two parts per weight, cut off after 22 bits
-// and at 2^-32 of the reference: 28 us, but not the scalar kernel's sum.  One wave per row with vector
-// arithmetic: 1934 us.
+// Bound by the instructions of a step (softmax, split of the weights and bookkeeping on the vector pipe: about 3000
+// cycles of a wave against 770 of its products at D=96) times the steps of the longest list over the waves; from 192
+// columns on by LDS (a step of 32 rows reads each K and V byte once for 32 query rows).  So rows that go to LDS directly
+// have their offsets laid out once, their fragments are fetched in groups (K, and V under the weights), and a
+// weight's part is taken off without being converted first.  B=1 H=8 S=2048 D=96, causal in 32x32 blocks, launches back
+// to back: fp16 25.7 us, bf16 23.3 (28.7 and 26.9 without); S=1500 B=1 H=4, 64x64: D=160 30.9 (35.0), D=200 40.7
+// (46.1); D=95, rows at any alignment, 42.5.  33 us (37) at D=96 where queries are four times as large (every row peaked,
+// a rest in most steps).  Two parts per weight, cut off after 22 bits and at 2^-32 of the reference, gain 2 us, but are
+// not the scalar kernel's sum.  One wave per row with vector arithmetic: 1934 us.
 #include "../../include/omni_attn_gfx950.h"
 
 #include <hip/hip_runtime.h>
@@ -162,10 +164,11 @@ __device__ __forceinline__ uint32_t split_part(float& lo, float& hi) {
     return __builtin_amdgcn_perm(b, a, 0x07060302u);  // upper halves of both
   } else {
     const auto v = __builtin_amdgcn_cvt_pkrtz(lo, hi);
-    const f16x2_t h = __builtin_bit_cast(f16x2_t, v);
-    lo = __builtin_fmaf(float(h[0]), -1.f, lo);
-    hi = __builtin_fmaf(float(h[1]), -1.f, hi);
-    return __builtin_bit_cast(uint32_t, v);
+    const uint32_t h = __builtin_bit_cast(uint32_t, v);
+    // value - part, with the part's half read as it is (the compiler converts it first: two instructions more per part)
+    asm("v_fma_mix_f32 %0, %1, -1.0, %0 op_sel_hi:[1,0,0]" : "+v"(lo) : "v"(h));
+    asm("v_fma_mix_f32 %0, %1, -1.0, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(hi) : "v"(h));
+    return h;
   }
 }
 template <bool BF16>
@@ -189,8 +192,22 @@ __device__ __forceinline__ float to_float(uint32_t bits) {
   }
 }
 
-// The other half-wave's value (lane ^ 32).
-__device__ __forceinline__ float other_half(float x) { return __shfl_xor(x, 32, 64); }
+// x of this lane and of lane ^ 32, in any order.
+// (SWAP: without LDS.  The forms that read rows at any alignment have no register left for it.)
+template <bool SWAP>
+__device__ __forceinline__ void both_halves(float x, float& lo, float& hi) {
+  if constexpr (!SWAP) {
+    lo = x;
+    hi = __shfl_xor(x, 32, 64);
+    return;
+  }
+  typedef __attribute__((ext_vector_type(2))) unsigned u2;
+  const unsigned a = __builtin_bit_cast(unsigned, x);
+  const u2 r = __builtin_amdgcn_permlane32_swap(a, a, false, false);
+  const unsigned r0 = r[0], r1 = r[1];
+  lo = __builtin_bit_cast(float, r0);
+  hi = __builtin_bit_cast(float, r1);
+}
 
 // DT: 32-column tiles of the head dimension; NW: waves.
 template <int DT, int NW>
@@ -283,22 +300,46 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
   u32x4_t qf[Traits::kQInLds ? 1 : KS];
   {
     const uint16_t* qrow = q_slab + int64_t(q_live ? q_idx : 0) * p.q_at.row;
+    if constexpr (R == Rows::kDirect) {  // (16-byte chunks of D % 8 == 0 columns: none has columns of the one before)
+      constexpr int NQ = Traits::kQInLds ? (KS + NW - 1) / NW : KS;  // chunks of this wave
+      u32x4_t x[NQ];  // all in flight together, and cleared below: one under a condition is waited for
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      if (Traits::kQInLds && s % NW != w) continue;
-      const int d0 = 16 * s + 8 * g;
-      u32x4_t x = load8<R == Rows::kDirect ? Rows::kWide : R>(qrow, d0, p.D);
-      if (!q_live || d0 >= p.D) x = u32x4_t{0u, 0u, 0u, 0u};
-      if (R != Rows::kSmall && d0 < p.D) {
-        const int repeats = d0 - chunk_start(d0, p.D);  // leading columns that the chunk before has
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          x[i] &= (2 * i >= repeats ? 0xffffu : 0u) | (2 * i + 1 >= repeats ? 0xffff0000u : 0u);
+      for (int n = 0; n < NQ; ++n) {
+        const int d0 = 16 * (Traits::kQInLds ? n * NW + w : n) + 8 * g;
+        x[n] = load8<Rows::kWide>(qrow, d0 < p.D ? d0 : 0, p.D);
       }
-      if constexpr (Traits::kQInLds) {
-        *reinterpret_cast<u32x4_t*>(sQ + tile_at(c, 2 * s + g)) = x;
-      } else {
-        qf[s] = x;
+      if constexpr (NQ > 1) {
+#pragma unroll
+        for (int n = 0; n < NQ; ++n) asm volatile("" : "+v"(x[n]));
+      }
+#pragma unroll
+      for (int n = 0; n < NQ; ++n) {
+        const int s = Traits::kQInLds ? n * NW + w : n;
+        if (!q_live || 16 * s + 8 * g >= p.D) x[n] = u32x4_t{0u, 0u, 0u, 0u};
+        if constexpr (Traits::kQInLds) {
+          if (s < KS) *reinterpret_cast<u32x4_t*>(sQ + tile_at(c, 2 * s + g)) = x[n];
+        } else {
+          qf[s] = x[n];
+        }
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        if (Traits::kQInLds && s % NW != w) continue;
+        const int d0 = 16 * s + 8 * g;
+        u32x4_t x = load8<R>(qrow, d0, p.D);
+        if (!q_live || d0 >= p.D) x = u32x4_t{0u, 0u, 0u, 0u};
+        if (R != Rows::kSmall && d0 < p.D) {
+          const int repeats = d0 - chunk_start(d0, p.D);  // leading columns that the chunk before has
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            x[i] &= (2 * i >= repeats ? 0xffffu : 0u) | (2 * i + 1 >= repeats ? 0xffff0000u : 0u);
+        }
+        if constexpr (Traits::kQInLds) {
+          *reinterpret_cast<u32x4_t*>(sQ + tile_at(c, 2 * s + g)) = x;
+        } else {
+          qf[s] = x;
+        }
       }
     }
     if (Traits::kQInLds) __syncthreads();
@@ -401,16 +442,29 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
     const int id = i * 64 + lane;
     cols[i] = uint32_t(chunk_start(((id % C) ^ swizzle(id / C)) * 8, p.D)) * 2u;
   }
-  auto load_tile = [&](auto again, const uint16_t* slab, const i32x4_t& rsrc, int64_t pitch, uint8_t* dst) {
+  // ... and of its chunks in a whole step, K and V
+  constexpr int NAT = R == Rows::kDirect ? NLD : 1;
+  uint32_t k_at[NAT], v_at[NAT];
+#pragma unroll
+  for (int i = 0; i < NAT; ++i) {
+    k_at[i] = uint32_t(from[i]) * uint32_t(p.k_at.row * 2) + cols[i];
+    v_at[i] = uint32_t(from[i]) * uint32_t(p.v_at.row * 2) + cols[i];
+  }
+  auto load_tile = [&](auto again, bool is_k, const uint16_t* slab, const i32x4_t& rsrc, int64_t pitch, uint8_t* dst) {
     if constexpr (R == Rows::kDirect) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the tile has been read
       const uint32_t to = uint32_t(size_t((__attribute__((address_space(3))) void*)dst));
       const uint32_t pitch2 = uint32_t(pitch * 2);
+      if (p.whole) {
+        const uint32_t first = uint32_t(base) * pitch2;
 #pragma unroll
-      for (int i = 0; i < NLD; ++i) {
-        uint32_t at = uint32_t(from[i]) * pitch2 + cols[i];
-        if (!p.whole) at = from[i] < 0 ? 0xffffffffu : at;
-        buffer_to_lds(rsrc, at, uint32_t(base) * pitch2, to + uint32_t(i) * 1024u);
+        for (int i = 0; i < NLD; ++i) buffer_to_lds(rsrc, is_k ? k_at[i] : v_at[i], first, to + uint32_t(i) * 1024u);
+      } else {
+#pragma unroll
+        for (int i = 0; i < NLD; ++i) {
+          const uint32_t at = uint32_t(from[i]) * pitch2 + cols[i];
+          buffer_to_lds(rsrc, from[i] < 0 ? 0xffffffffu : at, 0u, to + uint32_t(i) * 1024u);
+        }
       }
     } else {
       int l = lane;
@@ -451,8 +505,8 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
   };
   auto first_rows = [&](auto again) {
     advance();
-    load_tile(again, k_slab, rK, p.k_at.row, sK);
-    load_tile(again, v_slab, rV, p.v_at.row, sV);
+    load_tile(again, true, k_slab, rK, p.k_at.row, sK);
+    load_tile(again, false, v_slab, rV, p.v_at.row, sV);
   };
   const int q_first = qb * p.QB + row0;  // first row of the workgroup
   // `again`: the second walk of a wave whose first met an infinity or a NaN in V (or overflowed); rare, so
@@ -534,15 +588,25 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
       }
       if constexpr (R == Rows::kDirect) wait_but<NLD>();  // K is there (V was requested after it)
       f32x16_t st = zero16;
+      // (fragments are fetched in groups, so that a group waits for LDS once)
+      constexpr int AHEAD = R == Rows::kDirect ? (KS < 8 ? KS : 8) : 1;
 #pragma unroll
-      for (int s = 0; s < KS; ++s)
-        st = mfma<BF16>(*reinterpret_cast<const u32x4_t*>(sK + tile_at(c, 2 * s + g)), q_frag(s), st);
+      for (int s0 = 0; s0 < KS; s0 += AHEAD) {
+        u32x4_t kf[AHEAD];
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i)
+          if (s0 + i < KS) kf[i] = *reinterpret_cast<const u32x4_t*>(sK + tile_at(c, 2 * (s0 + i) + g));
+        if constexpr (AHEAD > 1) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i)
+          if (s0 + i < KS) st = mfma<BF16>(kf[i], q_frag(s0 + i), st);
+      }
       asm volatile("" : "+v"(keep));  // (the mask's own loads are waited for here, not behind the next request)
       // K has been read: the rows of the wave's next step
       go = more();
       if (go) {
         advance();
-        load_tile(again, k_slab, rK, p.k_at.row, sK);
+        load_tile(again, true, k_slab, rK, p.k_at.row, sK);
       }
       if (p.softcap > 0.f) {
 #pragma unroll
@@ -564,7 +628,11 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
 #pragma unroll
       for (int r = 0; r < 16; ++r) mx = fmaxf(mx, st[r]);
       mx *= p.sl2;
-      mx = fmaxf(mx, other_half(mx));
+      {
+        float lower, upper;
+        both_halves<R == Rows::kDirect>(mx, lower, upper);
+        mx = fmaxf(lower, upper);
+      }
       if (__builtin_amdgcn_ballot_w64(mx > m_run + kSlack) != 0) {
         const float m_new = fmaxf(m_run, mx);
         const float m_ref = m_new == -INFINITY ? 0.f : m_new;
@@ -577,6 +645,34 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
         m_run = m_new;
       }
       const float m_ref = m_run == -INFINITY ? 0.f : m_run;
+      if constexpr (R == Rows::kDirect) {  // V is there (the next K was requested after it)
+        if (go) {
+          wait_but<NLD>();
+        } else {
+          wait_but<0>();
+        }
+      }
+      // O^T += V^T.P^T: k-slot e of lane group g in 16-key half ts is key 16 ts + 8 (e / 4) + 4 g + e % 4
+      const int i16 = c & 15, j16 = c >> 4;
+      auto v_frag = [&](const uint8_t* tile, int ts, int dt) {
+        const int chunk = 2 * (2 * dt + j16) + ((i16 & 3) >> 1);
+        const int r0 = 16 * ts + 4 * g + (i16 >> 2), r1 = r0 + 8;
+        const uint8_t* a0 = tile + tile_at(r0, chunk) + (i16 & 1) * 8;
+        const uint8_t* a1 = tile + tile_at(r1, chunk) + (i16 & 1) * 8;
+        const u32x2_t lo = __builtin_bit_cast(
+            u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(a0)));
+        const u32x2_t hi = __builtin_bit_cast(
+            u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(a1)));
+        return u32x4_t{lo[0], lo[1], hi[0], hi[1]};
+      };
+      // (the fragments of the first half are fetched under the weights)
+      constexpr bool FETCHED = R == Rows::kDirect && DT <= 4 && !decltype(again)::value;
+      u32x4_t vf[DT];
+      if constexpr (FETCHED) {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) vf[dt] = v_frag(sV, 0, dt);
+        __builtin_amdgcn_sched_barrier(0);
+      }
       // The weights, in place of the scores, and their parts.
       u32x4_t pb[PARTS][2];
       auto split = [&](int r) {
@@ -593,15 +689,6 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
         if (!decltype(again)::value && (r & 1)) split(r - 1);
       }
       l_run += sum;
-      if constexpr (R == Rows::kDirect) {  // V is there (the next K was requested after it)
-        if (go) {
-          wait_but<NLD>();
-        } else {
-          wait_but<0>();
-        }
-      }
-      // O^T += V^T.P^T: k-slot e of lane group g in 16-key half ts is key 16 ts + 8 (e / 4) + 4 g + e % 4
-      const int i16 = c & 15, j16 = c >> 4;
       if constexpr (decltype(again)::value) {
         // one key after the other, without those of weight zero
 #pragma unroll 1
@@ -632,24 +719,14 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
         }
       }
       if constexpr (!decltype(again)::value) {
-        auto v_frag = [&](const uint8_t* tile, int ts, int dt) {
-          const int chunk = 2 * (2 * dt + j16) + ((i16 & 3) >> 1);
-          const int r0 = 16 * ts + 4 * g + (i16 >> 2), r1 = r0 + 8;
-          const uint8_t* a0 = tile + tile_at(r0, chunk) + (i16 & 1) * 8;
-          const uint8_t* a1 = tile + tile_at(r1, chunk) + (i16 & 1) * 8;
-          const u32x2_t lo = __builtin_bit_cast(
-              u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(a0)));
-          const u32x2_t hi = __builtin_bit_cast(
-              u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(a1)));
-          return u32x4_t{lo[0], lo[1], hi[0], hi[1]};
-        };
 #pragma unroll
         for (int ts = 0; ts < 2; ++ts) {
 #pragma unroll
           for (int dt = 0; dt < DT; ++dt) {
-            const u32x4_t a = v_frag(sV, ts, dt);
+            const u32x4_t a = FETCHED ? vf[dt] : v_frag(sV, ts, dt);
 #pragma unroll
             for (int n = 0; n < PARTS; ++n) ot[dt] = mfma<BF16>(a, pb[n][ts], ot[dt]);
+            if constexpr (FETCHED) if (ts == 0) vf[dt] = v_frag(sV, 1, dt);
           }
         }
         // Weights below 1/2 (2^-(1 + kShift) of the reference) may have bits below 2^-24, where fp16 ends: that rest,
@@ -689,7 +766,7 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
           __builtin_amdgcn_sched_barrier(0);
         }
       }
-      if (go) load_tile(again, v_slab, rV, p.v_at.row, sV);
+      if (go) load_tile(again, false, v_slab, rV, p.v_at.row, sV);
     }
   };
   if (go) {
@@ -715,7 +792,11 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
 
   // Merge: row maxima and sums of the waves, then the O^T tiles, kGroup at a time: every wave
   // writes its tiles, wave i adds up and stores tile i of the group.
-  l_run += other_half(l_run);
+  {
+    float lower, upper;
+    both_halves<R == Rows::kDirect>(l_run, lower, upper);
+    l_run = lower + upper;
+  }
   if (g == 0) {
     sStat[w * 32 + c] = m_run;
     sStat[(NW + w) * 32 + c] = l_run;

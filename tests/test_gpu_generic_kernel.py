@@ -164,3 +164,22 @@ def test_small_weights_reach_the_result(dtype, D, gpu_device):
         o, _ = run_generic(q, k, v, nb, idx, torch.full_like(idx, kind), blk, blk, S, None, None, gpu_device)
         ref = torch.softmax(scores.masked_fill(~allow, float("-inf")), -1) @ v.double()
         assert bool(((o.double().cpu() - ref).abs() <= ref * (ulp + 2.0 ** -16) + least).all()), kind
+
+
+@pytest.mark.parametrize("blk", [32, 64, 48], ids=lambda b: f"{b}x{b}")  # 48: steps that cross blocks
+@pytest.mark.parametrize("D", [8, 40, 96, 136, 168, 256])
+def test_rows_of_keys_and_values_lie_differently(D, blk, gpu_device):
+    """Rows read straight to LDS keep an offset per lane for K and for V: another distance between rows of one, the
+    other, or both gives the same bits."""
+    import omni_attn_torch as oat
+    from omni_attn_torch import create_causal_omni_block_mask
+    gen = torch.Generator().manual_seed(D + blk)
+    S = 3 * 64 - 5  # (the last block is ragged)
+    q, k, v = (torch.randn(1, 2, S, D, generator=gen).to(torch.float16).to(gpu_device) for _ in range(3))
+    mask = create_causal_omni_block_mask(1, 2, S, S, blk, blk, device=gpu_device)
+    rows_apart = lambda t: t.transpose(1, 2).contiguous().transpose(1, 2)
+    out = oat.omni_attention_simple(q, k, v, mask)
+    ref, _ = attention_dense_fp32(q.cpu(), k.cpu(), v.cpu(), torch.tril(torch.ones(S, S, dtype=torch.bool)))
+    assert (out.float().cpu() - ref).abs().max().item() <= 2e-3
+    for kk, vv in ((rows_apart(k), v), (k, rows_apart(v)), (rows_apart(k), rows_apart(v))):
+        assert torch.equal(oat.omni_attention_simple(q, kk, vv, mask), out)

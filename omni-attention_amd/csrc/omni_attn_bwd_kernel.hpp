@@ -81,6 +81,7 @@ struct BwdParams {
   int slab_group;  // slabs of one XCD that are walked together (>= 1)
   int flat_first;  // (at most 64 slabs per XCD) slabs without short lists go first
   int n_xcd;      // XCDs (L2 domains) of the device; workgroup ids go round-robin over them
+  DealPlan deal;
   float sl2;      // log2(e) / sqrt(D)
   float scale;    // 1 / sqrt(D)
   float softcap;  // > 0: the forward replaced x = s / sqrt(D) by softcap * tanh(x / softcap)
@@ -327,13 +328,13 @@ __device__ __forceinline__ void bwd_dq_walk(const BwdParams& p) {
   // K/V rows of a few slabs and share them through that XCD's L2.
   // (A slab may be dealt in parts, see the forward.)
   const int tiles = KG == 1 ? p.Tq : p.Tq * (QB / QT);
-  const Dealt deal = deal_slab(p, tiles, p.slab_group, p.flat_first != 0);
+  const Dealt deal = deal_slab(p, p.slab_group, p.flat_first != 0);
   if (deal.slab < 0) return;
-  const int bh = deal.slab / p.parts;
+  const int bh = deal.slab >> p.deal.part_shift;
   const int qt = tiles - 1 - (deal.rank * p.parts + deal.slab - bh * p.parts);
   const int q0 = qt * QT;  // first row of this workgroup
   if (qt < 0 || (KG > 1 && q0 >= p.S)) return;
-  const int qb = KG == 1 ? qt : q0 / QB;
+  const int qb = KG == 1 ? qt : q0 >> (QB == 128 ? 7 : 6);
   const int tid = KG == 1 ? threadIdx.x : threadIdx.x - kg * NT;  // thread of the group
   const int lane = tid & 63;
   const int g = lane >> 5, c = lane & 31;
@@ -343,8 +344,8 @@ __device__ __forceinline__ void bwd_dq_walk(const BwdParams& p) {
   // caller left in the padding.
   const size_t slab = size_t(bh) * size_t(p.S) * D;  // of the contiguous ones
   const uint32_t k_pitch = p.k_at.row * 2u, v_pitch = p.v_at.row * 2u;  // bytes from row to row
-  const i32x4_t rK = row_resource<D>(p.k, p.k_at, bh, p.H, p.seqlen);
-  const i32x4_t rV = row_resource<D>(p.v, p.v_at, bh, p.H, p.seqlen);
+  const i32x4_t rK = row_resource<D>(p.k, p.k_at, bh, p.H, p.deal.heads, p.seqlen);
+  const i32x4_t rV = row_resource<D>(p.v, p.v_at, bh, p.H, p.deal.heads, p.seqlen);
   const int q_row = q0 + 32 * w + c;
   const int q_wave_min = q0 + 32 * w;
   const int qr = q_row < p.S ? q_row : p.S - 1;
@@ -373,8 +374,8 @@ __device__ __forceinline__ void bwd_dq_walk(const BwdParams& p) {
   float dsum = 0.f;
   {
     const int ql = q_row < p.seqlen ? q_row : 0;
-    const uint16_t* qp = row_base(p.q, p.q_at, bh, p.H) + size_t(ql) * p.q_at.row + 8 * g;
-    const uint16_t* dop = row_base(p.dout, p.dout_at, bh, p.H) + size_t(ql) * p.dout_at.row + 8 * g;
+    const uint16_t* qp = row_base(p.q, p.q_at, bh, p.H, p.deal.heads) + size_t(ql) * p.q_at.row + 8 * g;
+    const uint16_t* dop = row_base(p.dout, p.dout_at, bh, p.H, p.deal.heads) + size_t(ql) * p.dout_at.row + 8 * g;
     const uint16_t* op = p.o + slab + size_t(qr) * D + 8 * g;
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
@@ -832,13 +833,13 @@ __device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
   // blocks (the longest walks of a causal mask) first, so the workgroups that run together on an XCD
   // read the Q and dO rows of a few slabs and share them through that XCD's L2.
   const int tiles = G == 1 ? p.Tk : p.Tk * (KB / KT);
-  const Dealt deal = deal_slab(p, tiles, p.slab_group, p.flat_first != 0);
+  const Dealt deal = deal_slab(p, p.slab_group, p.flat_first != 0);
   if (deal.slab < 0) return;
-  const int bh = deal.slab / p.parts;
+  const int bh = deal.slab >> p.deal.part_shift;
   const int kt = deal.rank * p.parts + deal.slab - bh * p.parts;
   const int key0 = kt * KT;  // first key of this workgroup
   if (kt >= tiles || (G > 1 && key0 >= p.S)) return;
-  const int kvb = G == 1 ? kt : key0 / KB;
+  const int kvb = G == 1 ? kt : key0 >> (KB == 128 ? 7 : 6);
   const int tid = G == 1 ? threadIdx.x : threadIdx.x - group * Traits::kGroupThreads;  // thread of the group
   const int lane = tid & 63;
   const bool grad_role = w >= NKG;        // wave-uniform
@@ -850,8 +851,8 @@ __device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
   // those rows arrive as zeros whatever the caller left in them.
   const size_t slab = size_t(bh) * size_t(p.S) * D;
   const uint32_t q_pitch = p.q_at.row * 2u, do_pitch = p.dout_at.row * 2u;  // bytes from row to row
-  const i32x4_t rQ = row_resource<D>(p.q, p.q_at, bh, p.H, p.seqlen);
-  const i32x4_t rD = row_resource<D>(p.dout, p.dout_at, bh, p.H, p.seqlen);
+  const i32x4_t rQ = row_resource<D>(p.q, p.q_at, bh, p.H, p.deal.heads, p.seqlen);
+  const i32x4_t rD = row_resource<D>(p.dout, p.dout_at, bh, p.H, p.deal.heads, p.seqlen);
   const i32x4_t rNd = make_buffer_resource(p.ws + size_t(bh) * p.S, uint32_t(p.S) * 4u);
   const i32x4_t rL2 = make_buffer_resource(p.ws + size_t(p.n_slabs) * p.S + size_t(bh) * p.S, uint32_t(p.S) * 4u);
   const int key_wave_min = key0 + 32 * kg;
@@ -872,8 +873,8 @@ __device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
   // beyond the sequence).
   u32x4_t bop[KS];
   {
-    const uint16_t* src = (grad_role ? row_base(p.v, p.v_at, bh, p.H) + size_t(key_live ? key : 0) * p.v_at.row
-                                     : row_base(p.k, p.k_at, bh, p.H) + size_t(key_live ? key : 0) * p.k_at.row) + 8 * g;
+    const uint16_t* src = (grad_role ? row_base(p.v, p.v_at, bh, p.H, p.deal.heads) + size_t(key_live ? key : 0) * p.v_at.row
+                                     : row_base(p.k, p.k_at, bh, p.H, p.deal.heads) + size_t(key_live ? key : 0) * p.k_at.row) + 8 * g;
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
       bop[s] = key_live ? *reinterpret_cast<const u32x4_t*>(src + 16 * s) : u32x4_t{0u, 0u, 0u, 0u};
@@ -1379,6 +1380,7 @@ int launch_bwd_kernel(const BwdParams& p, int tiles, int threads, size_t lds, si
   const unsigned slabs_per_xcd = unsigned(p.n_slabs * p.parts + p.n_xcd - 1) / unsigned(p.n_xcd);
   const dim3 grid(unsigned(p.n_xcd) * slabs_per_xcd * (unsigned(tiles + p.parts - 1) / unsigned(p.parts)));
   BwdParams params = p;
+  params.deal = plan_deal(p.n_slabs, p.parts, p.n_xcd, p.slab_group, tiles, p.H);
   void* args[] = {&params};
   return int(hipLaunchKernel(reinterpret_cast<const void*>(Kernel), grid, dim3(threads), args, lds, stream));
 }

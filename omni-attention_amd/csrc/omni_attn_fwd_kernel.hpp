@@ -39,6 +39,7 @@
 #include <atomic>
 #include <utility>
 
+#include "omni_attn_deal.hpp"
 #include "omni_attn_split_rules.hpp"
 
 namespace omni_attn {
@@ -91,6 +92,7 @@ struct FwdParams {
   int tiles;       // workgroups per slab (query blocks, or parts of them)
   int parts;       // parts a slab is dealt to the XCDs in
   int n_slabs;     // B*H
+  DealPlan deal;
   int n_xcd;       // XCDs (L2 domains) of the device; workgroup ids go round-robin over them
   int slab_group;  // slabs of one XCD that are walked together (>= 1)
   int flat_first;  // (at most 64 slabs per XCD) slabs without short lists go first
@@ -261,14 +263,17 @@ __device__ __forceinline__ i32x4_t make_buffer_resource(const void* base, uint32
 }
 // First row of slab bh of an operand, and a buffer resource that ends with its last live row (so rows
 // at or beyond the sequence read as zeros).
-__device__ __forceinline__ const uint16_t* row_base(const uint16_t* base, const RowStrides& at, int bh, int H) {
-  const int b = bh / H;
+// `heads`: DealPlan's division by H.
+__device__ __forceinline__ const uint16_t* row_base(const uint16_t* base, const RowStrides& at, int bh, int H,
+                                                    const FastDiv& heads) {
+  const int b = int(divide(bh, heads));
   return base + int64_t(b) * at.b + int64_t(bh - b * H) * at.h;
 }
 template <int D>
-__device__ __forceinline__ i32x4_t row_resource(const uint16_t* base, const RowStrides& at, int bh, int H, int live) {
+__device__ __forceinline__ i32x4_t row_resource(const uint16_t* base, const RowStrides& at, int bh, int H,
+                                                const FastDiv& heads, int live) {
   const uint32_t bytes = live > 0 ? uint32_t(live - 1) * at.row * 2u + uint32_t(D * 2) : 0u;
-  return make_buffer_resource(row_base(base, at, bh, H), bytes);
+  return make_buffer_resource(row_base(base, at, bh, H, heads), bytes);
 }
 // 16 bytes per lane from a buffer straight into LDS: the wave's 64 chunks land at
 // lds_base + 16 * lane.  The source offset is a wave-uniform part plus a per-lane part.
@@ -384,18 +389,18 @@ __device__ __forceinline__ void static_for(F&& f) {
 }
 
 // Which slab (or part of one) a workgroup has, and which of its tiles, longest first; slab -1: none.
-// `tiles` per slab, `group` slabs are walked together (the kernels say why); Params: of the forward or the
-// backward.
+// `group` slabs are walked together (the kernels say why); Params: of the forward or the backward.
 struct Dealt {
   int slab, rank;
 };
 template <class Params>
-__device__ __forceinline__ Dealt deal_slab(const Params& p, int tiles, int group, bool flat_first) {
+__device__ __forceinline__ Dealt deal_slab(const Params& p, int group, bool flat_first) {
   const int wg = blockIdx.x;
-  const int slot = wg / p.n_xcd;
+  const int slot = int(divide(wg, p.deal.xcd));
   const int xcd = wg - slot * p.n_xcd;
-  const int slabs_here = (p.n_slabs * p.parts - xcd + p.n_xcd - 1) / p.n_xcd;
-  const int part_tiles = (tiles + p.parts - 1) / p.parts;
+  const bool one_more = xcd < p.deal.one_more;
+  const int slabs_here = p.deal.slabs + int(one_more);
+  const int part_tiles = p.deal.part_tiles;
   if (slot >= slabs_here * part_tiles) return {-1, 0};
   // Batch elements may have different masks.  Slabs whose first query block lists more than half of the
   // KV blocks (nothing is masked, say: all their lists are long) go first, so that the launch ends with
@@ -408,7 +413,7 @@ __device__ __forceinline__ Dealt deal_slab(const Params& p, int tiles, int group
     const int i = threadIdx.x & 63;
     bool flat = false;
     if (i < slabs_here)
-      flat = 2 * p.kv_num_blocks[size_t((xcd + p.n_xcd * i) / p.parts) * size_t(p.Tq)] > p.Tk;
+      flat = 2 * p.kv_num_blocks[size_t((xcd + p.n_xcd * i) >> p.deal.part_shift) * size_t(p.Tq)] > p.Tk;
     const uint64_t flats = __builtin_amdgcn_ballot_w64(flat);
     const int n = __builtin_popcountll(flats);
     if (n != 0 && n != slabs_here) {
@@ -419,11 +424,18 @@ __device__ __forceinline__ Dealt deal_slab(const Params& p, int tiles, int group
     }
   }
   const int per_group = group * part_tiles;
-  const int gi = at / per_group;
+  const int gi = int(divide(at, p.deal.per_group));
   const int in_group = at - gi * per_group;
   const int g_left = slabs_kind - gi * group;
   const int g_eff = g_left < group ? g_left : group;
-  const int qrank = in_group / g_eff;
+  int qrank;
+  if (g_left >= group) {
+    qrank = int(divide(in_group, p.deal.group));
+  } else if (kind == 0) {
+    qrank = int(divide(in_group, one_more ? p.deal.last[1] : p.deal.last[0]));
+  } else {
+    qrank = in_group / g_eff;
+  }
   int pick = gi * group + (in_group - qrank * g_eff);  // which slab of its kind
   if (kind != 0) {
     const int i = threadIdx.x & 63;
@@ -475,13 +487,13 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   // (Launches of few rounds walk all slabs of an XCD as one group.)
   // Where there are too few slabs to go round, a slab is dealt in p.parts parts (part i has the
   // query tiles i, i + parts, ... from the end): "slab" in the lines below is a part then.
-  const Dealt deal = deal_slab(p, p.tiles, p.slab_group, p.flat_first != 0);
+  const Dealt deal = deal_slab(p, p.slab_group, p.flat_first != 0);
   if (deal.slab < 0) return;
-  const int bh = deal.slab / p.parts;
+  const int bh = deal.slab >> p.deal.part_shift;
   const int qt = p.tiles - 1 - (deal.rank * p.parts + deal.slab - bh * p.parts);  // query tile
   const int q0 = qt * QT;  // first row of this workgroup
   if (qt < 0 || (KG > 1 && q0 >= p.S)) return;
-  const int qb = KG == 1 ? qt : q0 / QB;
+  const int qb = KG == 1 ? qt : q0 >> (QB == 128 ? 7 : 6);
   const int rb0 = KG == 1 ? 0 : q0 - qb * QB;  // ... inside its query block
 
   const int tid = KG == 1 ? threadIdx.x : threadIdx.x - kg * NT;  // thread of the group
@@ -494,8 +506,8 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   // left in the padding.
   const size_t slab = size_t(bh) * size_t(p.S) * D;  // of o
   const uint32_t pitch = p.k_at.row * 2u;  // bytes from row to row of K, and of V
-  const i32x4_t rK = row_resource<D>(p.k, p.k_at, bh, p.H, p.seqlen);
-  const i32x4_t rV = row_resource<D>(p.v, p.v_at, bh, p.H, p.seqlen);
+  const i32x4_t rK = row_resource<D>(p.k, p.k_at, bh, p.H, p.deal.heads, p.seqlen);
+  const i32x4_t rV = row_resource<D>(p.v, p.v_at, bh, p.H, p.deal.heads, p.seqlen);
 
   const int q_row = q0 + 32 * w + c;  // this lane's query row inside the slab
   const int q_wave_min = q0 + 32 * w;
@@ -575,7 +587,7 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   // Q as the B operand of S^T = K.Q^T: lane holds Q[q_row][16s + 8g .. +7].
   u32x4_t qf[KS];
   {
-    const uint16_t* qp = row_base(p.q, p.q_at, bh, p.H) + size_t(q_row < p.seqlen ? q_row : 0) * p.q_at.row + 8 * g;
+    const uint16_t* qp = row_base(p.q, p.q_at, bh, p.H, p.deal.heads) + size_t(q_row < p.seqlen ? q_row : 0) * p.q_at.row + 8 * g;
 #pragma unroll
     for (int s = 0; s < KS; ++s)
       qf[s] = q_row < p.seqlen ? *reinterpret_cast<const u32x4_t*>(qp + 16 * s) : u32x4_t{0u, 0u, 0u, 0u};
@@ -1224,6 +1236,7 @@ int launch_fwd_shape(const FwdParams& p, hipStream_t stream) {
   const unsigned slabs_per_xcd = unsigned(p.n_slabs * p.parts + p.n_xcd - 1) / unsigned(p.n_xcd);
   const dim3 grid(unsigned(p.n_xcd) * slabs_per_xcd * (unsigned(p.tiles + p.parts - 1) / unsigned(p.parts)));
   FwdParams params = p;
+  params.deal = plan_deal(p.n_slabs, p.parts, p.n_xcd, p.slab_group, p.tiles, p.H);
   void* args[] = {&params};
   return int(hipLaunchKernel(reinterpret_cast<const void*>(Kernel), grid, dim3(Shape::kThreads), args,
                              Shape::kLdsBytes, stream));

@@ -275,6 +275,16 @@ __device__ __forceinline__ i32x4_t row_resource(const uint16_t* base, const RowS
   const uint32_t bytes = live > 0 ? uint32_t(live - 1) * at.row * 2u + uint32_t(D * 2) : 0u;
   return make_buffer_resource(row_base(base, at, bh, H, heads), bytes);
 }
+// 16 bytes per lane from a buffer of rows into registers, at a lane offset and a constant inside the row.  A lane at
+// kNoRow gets zeros: no buffer of rows that 32-bit offsets reach ends behind it, and no constant leads past 2^32.  (The
+// constant goes with the lane's offset, where the check of the range sees the sum.)
+template <int D>
+constexpr uint32_t kNoRow = 0u - 2u * uint32_t(D);
+__device__ __forceinline__ u32x4_t buffer_load_b128(const i32x4_t& r, uint32_t lane_off, int constant) {
+  const uint64_t base = uint64_t(uint32_t(r[0])) | uint64_t(uint32_t(r[1])) << 32;
+  auto rsrc = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(base), 0, r[2], r[3]);
+  return __builtin_amdgcn_raw_buffer_load_b128(rsrc, int(lane_off) + constant, 0, 0);
+}
 // 16 bytes per lane from a buffer straight into LDS: the wave's 64 chunks land at
 // lds_base + 16 * lane.  The source offset is a wave-uniform part plus a per-lane part.
 // Written as inline asm so that the compiler does not order later LDS reads of *other*
@@ -490,25 +500,19 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   const Dealt deal = deal_slab(p, p.slab_group, p.flat_first != 0);
   if (deal.slab < 0) return;
   const int bh = deal.slab >> p.deal.part_shift;
-  const int qt = p.tiles - 1 - (deal.rank * p.parts + deal.slab - bh * p.parts);  // query tile
+  const int qt = p.tiles - 1 - ((deal.rank << p.deal.part_shift) + deal.slab - (bh << p.deal.part_shift));  // query tile
   const int q0 = qt * QT;  // first row of this workgroup
   if (qt < 0 || (KG > 1 && q0 >= p.S)) return;
   const int qb = KG == 1 ? qt : q0 >> (QB == 128 ? 7 : 6);
   const int rb0 = KG == 1 ? 0 : q0 - qb * QB;  // ... inside its query block
 
-  const int tid = KG == 1 ? threadIdx.x : threadIdx.x - kg * NT;  // thread of the group
+  static_assert((NT & (NT - 1)) == 0, "threads of a group");
+  const int tid = threadIdx.x & (NT - 1);  // thread of the group
   const int lane = tid & 63;
   const int g = lane >> 5;
   const int c = lane & 31;
 
-  // Rows at or beyond the sequence are never used: the resources of K and V end there (those
-  // rows arrive as zeros) and the query rows beyond it are replaced by zeros, whatever the caller
-  // left in the padding.
   const size_t slab = size_t(bh) * size_t(p.S) * D;  // of o
-  const uint32_t pitch = p.k_at.row * 2u;  // bytes from row to row of K, and of V
-  const i32x4_t rK = row_resource<D>(p.k, p.k_at, bh, p.H, p.deal.heads, p.seqlen);
-  const i32x4_t rV = row_resource<D>(p.v, p.v_at, bh, p.H, p.deal.heads, p.seqlen);
-
   const int q_row = q0 + 32 * w + c;  // this lane's query row inside the slab
   const int q_wave_min = q0 + 32 * w;
 
@@ -523,21 +527,47 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   // the count and Q are all in flight together at the start of the kernel.
   const bool packed_tiles = p.partial_bits != nullptr;
   int32_t mv_row0 = 0, mv_mode = kMasked, mv_pid = -1;
-  auto load_chunk = [&](int chunk) {
+  struct Raw {
+    int32_t kvb, ty, pid;
+  };
+  auto request_chunk = [&](int chunk) {
     const int j = chunk * 64 + lane;
     const size_t o = meta_off + size_t(j < p.max_blocks ? j : 0);
-    const int32_t kvb_raw = p.kv_indices[o];
-    const int32_t ty = p.types[o];
-    const int32_t pid = p.partial_idx[o];
-    const int32_t kvb = kvb_raw < 0 ? 0 : (kvb_raw >= p.Tk ? p.Tk - 1 : kvb_raw);
-    int32_t mode = (ty == kCausal || ty == kFull || ty == kPartial) ? ty : int32_t(kMasked);
-    if (ty == kPartial && (pid < 0 || pid >= p.num_partial)) mode = kMasked;
+    return Raw{p.kv_indices[o], p.types[o], p.partial_idx[o]};
+  };
+  auto take_chunk = [&](const Raw& raw) {
+    const int32_t kvb = raw.kvb < 0 ? 0 : (raw.kvb >= p.Tk ? p.Tk - 1 : raw.kvb);
+    int32_t mode = (raw.ty == kCausal || raw.ty == kFull || raw.ty == kPartial) ? raw.ty : int32_t(kMasked);
+    if (raw.ty == kPartial && (raw.pid < 0 || raw.pid >= p.num_partial)) mode = kMasked;
     mv_row0 = kvb * KB;
     mv_mode = mode;
-    mv_pid = pid;
+    mv_pid = raw.pid;
   };
-  load_chunk(0);
+  auto load_chunk = [&](int chunk) { take_chunk(request_chunk(chunk)); };
+  // The list and its length are requested as soon as their addresses are known; what else depends on the slab is
+  // worked out meanwhile.  (The length was requested behind the list's arrival, and Q with a branch per load:
+  // B=2 H=16 S=1237 D=128 unaligned spans 29.3 -> 28.75 us without.)
   int nb = load_uniform(p.kv_num_blocks + meta_row);
+  const Raw first_chunk = request_chunk(0);
+  __builtin_amdgcn_sched_barrier(0);
+  // Rows at or beyond the sequence are never used: the resources of K and V end there (those
+  // rows arrive as zeros) and the query rows beyond it are replaced by zeros, whatever the caller
+  // left in the padding.
+  const uint32_t pitch = p.k_at.row * 2u;  // bytes from row to row of K, and of V
+  const i32x4_t rK = row_resource<D>(p.k, p.k_at, bh, p.H, p.deal.heads, p.seqlen);
+  const i32x4_t rV = row_resource<D>(p.v, p.v_at, bh, p.H, p.deal.heads, p.seqlen);
+  const i32x4_t rQ = row_resource<D>(p.q, p.q_at, bh, p.H, p.deal.heads, p.seqlen);
+  // Q as the B operand of S^T = K.Q^T: lane holds Q[q_row][16s + 8g .. +7].  Lone waves ask for it while
+  // the list is on its way (B=1 H=8 S=512 D=128 6.33 -> 6.08 us), others when it is there: their waves share the
+  // way to memory, and the list and K come first (B=1 H=8 S=2048 in 64-row blocks 12.2 us, 12.3 the other way).
+  u32x4_t qf[KS];
+  auto request_q = [&]() {
+    const uint32_t at = q_row < p.seqlen ? uint32_t(q_row) * (p.q_at.row * 2u) + 16u * uint32_t(g) : kNoRow<D>;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) qf[s] = buffer_load_b128(rQ, at, 32 * s);
+  };
+  if constexpr (LONE) request_q();
+  take_chunk(first_chunk);
   nb = nb < 0 ? 0 : (nb > p.max_blocks ? p.max_blocks : nb);
   int all_steps = nb * SPB;
   // Groups share the steps of the live slots only (those that allow something), so a list and the same
@@ -584,14 +614,7 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   }
   const int nsteps = KG == 1 ? all_steps : (all_steps + KG - 1) / KG;  // iterations of every group
 
-  // Q as the B operand of S^T = K.Q^T: lane holds Q[q_row][16s + 8g .. +7].
-  u32x4_t qf[KS];
-  {
-    const uint16_t* qp = row_base(p.q, p.q_at, bh, p.H, p.deal.heads) + size_t(q_row < p.seqlen ? q_row : 0) * p.q_at.row + 8 * g;
-#pragma unroll
-    for (int s = 0; s < KS; ++s)
-      qf[s] = q_row < p.seqlen ? *reinterpret_cast<const u32x4_t*>(qp + 16 * s) : u32x4_t{0u, 0u, 0u, 0u};
-  }
+  if constexpr (!LONE) request_q();
   // Step `it` (clamped to the last step of the walk; steps past the end are only ever
   // used as the address of a tile load whose data nobody reads).
   auto step_info = [&](int i) {

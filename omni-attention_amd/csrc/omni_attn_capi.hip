@@ -189,7 +189,9 @@ int forward(const void* q, const void* k, const void* v, const omni_attn_strides
   const int slots_per_xcd = topo.cus_per_xcd * (QB == 128 ? 2 : 4);
   p.parts = slab_parts(p.n_slabs, X);
   const long long busiest = ((long long)p.n_slabs * p.parts + X - 1) / X * ((Tq * QB / 128 + p.parts - 1) / p.parts);
-  p.split = fwd_choose_split(D, QB, (long long)B * H * Tq * (QB / 32), Tq * QB, busiest, topo.cus_per_xcd);
+  const long long rows32 = (long long)B * H * Tq * (QB / 32);
+  const bool even = 100 * 4 * busiest * X <= 106 * rows32;
+  p.split = fwd_choose_split(D, QB, rows32, Tq * QB, busiest, topo.cus_per_xcd, p.seqlen % QB != 0, even, B > 1);
   p.tiles = Tq * (QB / fwd_split_rows(p.split, QB));
   const int part_tiles = (p.tiles + p.parts - 1) / p.parts;
   const int fill = slots_per_xcd / part_tiles > 1 ? slots_per_xcd / part_tiles : 1;
@@ -363,7 +365,7 @@ int backward(const void* q, const void* k, const void* v, const void* o, const v
   p.QB = QB;
   p.KB = KB;
   const long long rows32 = (long long)B * H * Tq * (QB / 32);
-  p.dq_split = bwd_choose_dq_split(D, QB, rows32, Tq * QB);
+  p.dq_split = bwd_choose_dq_split(D, QB, rows32, Tq * QB, p.seqlen % QB != 0, B > 1);
   p.dkdv_split = bwd_choose_dkdv_split(D, softcap > 0.f, rows32, Tq * QB);
   DeviceTopology topo;
   if (const int e = query_topology(&topo)) {

@@ -48,7 +48,49 @@ constexpr int fwd_split_rows(FwdSplit s, int QB) {
 //   D=32   kRows32x4   against kRows64x2: B H=16 S=1237 11-16 (-17 .. -29), B H=6 S=4096 25-27 (-17 .. -26); beyond: B H=8
 //                      S=4096 25-27 (-3 .. +7)
 //          kRows64x2   B H=40 S=1024 16-18 (-3 .. -16), B H=32 S=1536 21-24 (-10 .. -21), S=2048 28-33 (-14 .. +1)
-inline FwdSplit fwd_choose_split(int D, int QB, long long rows32, int S, long long busiest, int cus) {
+// `ragged`: the sequence ends inside a query block.  With PARTIAL tiles every block of that list is one then (its last
+// rows attend nothing): the longest list of a slab also has the slowest steps, and sharing it gains in larger
+// launches.  `even`: no XCD has more than 6 % above the mean.  `batched`: more than one batch element; one in three may
+// attend everything, and a launch of many long lists is bound by K/V loads.  Whole blocks, us, and the split against
+// them, causal, two layouts of spans and images, then "mixed" (such a batch):
+//   D=128  one batch element
+//          kRows64x2   B H=32 S=1153 25-30 (-17 .. +3 %), S=1237 25-30 (-8 .. -10); beyond: S=1400 28-34 (-10 .. +16),
+//                      B H=40 S=1000 22-26 (-15 .. +20), uneven B H=36 S=1100 24-29 (-9 .. +13)
+//          kRows128x2  B H=24 S=1600 31-38 (-1 .. -19), S=1900 37-43 (-2 .. -17), B H=20 S=2100 39-48 (-8 .. -18), B H=16
+//                      S=2600 47-58 (-11 .. -23), S=3700 70-89 (-18 .. +1); beyond: B H=24 S=2100 42-50 (-5 .. +10), B H=16
+//                      S=4200 83-103 (-13 .. +4), uneven B H=22 S=1800 36-46 (-9 .. +15)
+//          batched
+//          kRows64x2   B H=24 S=1600 31-38 (-5 .. -14), mixed 41-43 (-15 .. +1), B H=20 S=2000 37-45 (-5 .. -13), mixed
+//                      49 (-5); kRows128x2 there: mixed +10; beyond: B H=24 S=1750 mixed 45 (+13), B H=20 S=2100 39-48
+//                      (-14 .. +7), B H=32 S=1153 mixed 34 (+20)
+//   D=64   kRows64x2   B H=32 S=1500 22-29 (-4 .. -25), mixed 30 (-5), B H=24 S=1900 26-34 (-15 .. -33), mixed 36 (-21);
+//                      one batch element: B H=24 S=2700 38-52 (-3 .. -21), B H=16 S=4500 60-80 (-5 .. -18), B H=12 S=6000
+//                      76-103 (-6 .. -21); beyond: B H=32 S=2000 mixed 39 (+11), B H=24 S=2000 mixed 38 (+8), B H=32 S=2300
+//                      33-43 (-5 .. +10), B H=40 S=1237 19-25 (-13 .. +8), B H=20 S=4000 55-78 (-8 .. +8)
+//   D=32   kRows64x2   B H=48 S=1237 16-23 (-5 .. -18), mixed 23 (-16), B H=40 S=1700 22-31 (-8 .. -27), B H=32 S=2300 27-37
+//                      (-17 .. -24), S=3000 38-50 (-3 .. -18), mixed 57 (-1 .. -5), B H=16 S=6000 68-93 (-7 .. -28); beyond:
+//                      B H=48 S=1500 20-27 (-18 .. +3)
+inline FwdSplit fwd_ragged_split(int D, long long rows32, int S, bool even, bool batched) {
+  bool two;
+  if (D == 128) {
+    if (!even) return FwdSplit::kNone;
+    if (batched) {
+      two = rows32 <= 1280 && S >= 1600;
+    } else {
+      if ((rows32 <= 1440 && S >= 1600) || (rows32 <= 1856 && S >= 2 * rows32)) return FwdSplit::kRows128x2;
+      two = rows32 <= 1280 && S >= 1152;
+    }
+  } else if (D == 64) {
+    if (S < 1408 || S < rows32) return FwdSplit::kNone;
+    two = batched ? (rows32 <= 1440 && 4 * rows32 >= 3LL * S) || (rows32 <= 1792 && rows32 >= S)
+                  : rows32 <= 2112 || (rows32 <= 2304 && S >= 2 * rows32);
+  } else {
+    two = (rows32 <= 1920 && S >= 1280) || (rows32 <= 2304 && S >= 1792) || (rows32 <= 3072 && S >= rows32);
+  }
+  return two ? FwdSplit::kRows64x2 : FwdSplit::kNone;
+}
+inline FwdSplit fwd_choose_split(int D, int QB, long long rows32, int S, long long busiest, int cus,
+                                 bool ragged = false, bool even = true, bool batched = true) {
   const int one_round_32 = D == 128 ? 384 : (D == 64 ? 512 : 768);
   if (rows32 <= one_round_32 || (D == 128 && rows32 <= 512 && S >= 2560) || (D == 64 && rows32 <= 672 && S >= 2000))
     return FwdSplit::kRows32x4;
@@ -61,7 +103,8 @@ inline FwdSplit fwd_choose_split(int D, int QB, long long rows32, int S, long lo
   if (D != 128) {
     const bool more = D == 64 ? rows32 <= 1280 && S >= 1152
                               : (rows32 <= 1280 && S >= 1024) || (rows32 <= 1536 && S >= 1536) || (rows32 <= 2048 && S >= 2048);
-    return some || more ? FwdSplit::kRows64x2 : FwdSplit::kNone;
+    if (some || more) return FwdSplit::kRows64x2;
+    return ragged ? fwd_ragged_split(D, rows32, S, even, batched) : FwdSplit::kNone;
   }
   if (lone) return FwdSplit::kRows64x4;
   if (rows32 <= 768 && S >= 1024) return FwdSplit::kRows64x2;
@@ -69,7 +112,8 @@ inline FwdSplit fwd_choose_split(int D, int QB, long long rows32, int S, long lo
   const bool long_lists = S >= 2048 && (rows32 <= 1152 || (rows32 <= 1280 && S >= 2 * rows32) ||
                                         (rows32 <= 2048 && 5LL * S >= 13 * rows32));
   if ((rows32 <= 1152 && S >= 1152 && one_round) || long_lists) return FwdSplit::kRows128x2;
-  return rows32 <= 1152 && S >= 640 && busiest > cus && 4 * busiest < 5LL * cus ? FwdSplit::kRows64x2 : FwdSplit::kNone;
+  if (rows32 <= 1152 && S >= 640 && busiest > cus && 4 * busiest < 5LL * cus) return FwdSplit::kRows64x2;
+  return ragged ? fwd_ragged_split(D, rows32, S, even, batched) : FwdSplit::kNone;
 }
 
 // How the walk of a KV block is split over waves in the dK/dV kernel.
@@ -97,14 +141,18 @@ enum class DkdvSplit : int {
 //          D=64   B H=16 S=1237 51-60 (-4 .. -15), soft-capped 68-77 (-10), B H=12 S=2048 71-81 (-4 .. -17), B H=20 S=2048
 //                 75-95 (0 .. -13); 64-key blocks 73-90 (-3 .. +9); beyond: B H=24 S=2048 78-106 (-2 .. +9), B H=12
 //                 S=4096 136-170 (-7 .. +6)
-inline FwdSplit bwd_choose_dq_split(int D, int QB, long long rows32, int S) {
+//   dQ, D=64, lengths that end inside a block, where the forward is split for that: B H=24 S=2300 127-172 (-2 .. -5), B H=16
+//          S=4500 248-317 (0 .. -5), soft-capped 437 (-10); beyond: B H=40 S=1700 107-134 (-3 .. +4); D=128 gains
+//          nowhere: B H=32 S=1237 101-130 (0 .. +4), B H=24 S=1700 128-171 (-2 .. +4)
+inline FwdSplit bwd_choose_dq_split(int D, int QB, long long rows32, int S, bool ragged = false, bool batched = true) {
   if (rows32 <= (D == 128 ? 256 : 512)) return FwdSplit::kRows32x4;
   bool two;
   if (D == 128) {
     two = rows32 <= 640 || (rows32 <= 1024 && S >= (QB == 128 ? 4096 : 2048)) ||
           (QB == 128 && ((rows32 <= 768 && S >= 1024) || (rows32 <= 896 && S >= 1536)));
   } else {
-    two = (rows32 <= 1024 && S >= 512) || (rows32 <= 1536 && S >= 1024) || (rows32 <= 2048 && S >= 4096);
+    two = (rows32 <= 1024 && S >= 512) || (rows32 <= 1536 && S >= 1024) || (rows32 <= 2048 && S >= 4096) ||
+          (D == 64 && QB == 128 && ragged && fwd_ragged_split(D, rows32, S, true, batched) != FwdSplit::kNone);
   }
   return two ? FwdSplit::kRows64x2 : FwdSplit::kNone;
 }

@@ -144,3 +144,29 @@ def test_backward_of_slabs_walked_together_with_different_masks(H, S, gpu_device
     got = torch.autograd.grad(omni_attention(*leaves, m), leaves, dout.to(gpu_device))
     allow = (torch.arange(S).view(1, 1, S) < prefix.unsqueeze(-1)).unsqueeze(1).expand(B, H, S, S)
     check_grads(got, attention_dense_grads(q, k, v, allow, dout), torch.float16, f"H={H} S={S}")
+
+
+@pytest.mark.parametrize("D,B,H,S,copies", [
+    (128, 1, 2, 1160, 16), (128, 1, 2, 1610, 12), (128, 1, 1, 2700, 16), (128, 3, 1, 1630, 8), (64, 2, 1, 1500, 16),
+    (64, 1, 1, 4400, 16), (32, 2, 1, 1300, 24), (32, 1, 1, 2950, 32)])
+def test_lengths_that_end_inside_a_block(D, B, H, S, copies, gpu_device):
+    """Launches that are split because of such a length: 64- and 128-row groups, dQ in 64-row groups at head_dim 64.
+    The slabs of a batch element are repeated; the first ones against the oracle, the copies bit for bit."""
+    from test_gpu_backward import check_grads, run_fwd_bwd
+    from oracle.dense_oracle import attention_dense_grads
+    gen = torch.Generator().manual_seed(D + S)
+    QB = KB = 128
+    n = -(-S // QB) * QB
+    q, k, v, dout = (torch.randn(B, H, n, D, generator=gen).to(torch.bfloat16) for _ in range(4))
+    nb, idx, tys, pidx, pm = random_block_metadata(gen, B, H, n // QB, n // KB, QB, KB, p_empty=0.5, shuffle=True)
+    many = lambda t: t.to(gpu_device).repeat(1, copies, *[1] * (t.dim() - 2)).contiguous()
+    got = run_fwd_bwd(*(many(t) for t in (q, k, v, dout)), many(nb), many(idx), many(tys), QB, KB, S, many(pidx), pm,
+                      device=gpu_device, softcap=0.0, packed=True)
+    for t in got:
+        assert torch.equal(t, t[:, :H].repeat(1, copies, *[1] * (t.dim() - 2)))
+        assert t.dim() < 4 or (t[:, :, S:] == 0).all()
+    dq, dk, dv, o, lse = (t[:, :H] for t in got[:5])
+    dense = dense_mask_from_blocks(nb, idx, tys, QB, KB, n, n, pidx, pm, seqlen_orig=S)
+    ro, rl = attention_dense_fp32(q, k, v, dense)
+    compare_with_oracle(o, lse, ro, rl, torch.bfloat16, f"S={S}")
+    check_grads((dq, dk, dv), attention_dense_grads(q, k, v, dense, dout), torch.bfloat16, f"S={S}")

@@ -59,3 +59,33 @@ def test_fewer_rows_and_longer_lists_stay_split(rules, kind):
             assert shortest is None or upto >= shortest, (D, block, S, "length")
             shortest = upto
         assert 0 < upto < len(bits)  # (with the longest lists: some, and not all)
+
+
+def test_lengths_that_end_inside_a_block(tmp_path):
+    """What is split for a length that fills its blocks is split the same way for one that does not; beyond that, fewer
+    rows of the same length are split too, and so are one batch element's where a batch's are."""
+    source, program = tmp_path / "ragged.cpp", tmp_path / "ragged"
+    source.write_text(r"""
+#include "omni_attn_split_rules.hpp"
+using namespace omni_attn;
+int main() {
+  for (int D = 32; D <= 128; D *= 2)
+    for (int S = 128; S <= 16384; S += 128)
+      for (int batched = 0; batched < 2; ++batched) {
+        bool all = false;  // from many rows to few: once split, always
+        for (long long rows = 4096; rows >= 16; rows -= 16) {
+          const long long busiest = (rows / 4 + 7) / 8;
+          const FwdSplit plain = fwd_choose_split(D, 128, rows, S, busiest, 32);
+          const FwdSplit ragged = fwd_choose_split(D, 128, rows, S, busiest, 32, true, true, batched);
+          if (plain != FwdSplit::kNone && plain != ragged) return 1;
+          if (batched && ragged != FwdSplit::kNone && fwd_choose_split(D, 128, rows, S, busiest, 32, true, true, false) == FwdSplit::kNone) return 2;
+          if (ragged != FwdSplit::kNone) all = true;
+          else if (all && !batched && S >= 1152) return 3;
+          if (bwd_choose_dq_split(D, 128, rows, S) != FwdSplit::kNone &&
+              bwd_choose_dq_split(D, 128, rows, S) != bwd_choose_dq_split(D, 128, rows, S, true, batched)) return 4;
+        }
+      }
+}
+""")
+    subprocess.run(["g++", "-std=c++17", "-I", CSRC, str(source), "-o", str(program)], check=True)
+    assert subprocess.run([str(program)]).returncode == 0

@@ -14,6 +14,12 @@ enum class FwdSplit : int {
 constexpr int fwd_split_rows(FwdSplit s, int QB) {
   return s == FwdSplit::kNone ? QB : (s == FwdSplit::kRows32x4 ? 32 : (s == FwdSplit::kRows128x2 ? 128 : 64));
 }
+// Workgroups that an XCD has room for: eight waves per compute unit, and 160 KiB of LDS (four lone waves have
+// 136 KiB of tiles at head_dim 128).
+constexpr int fwd_places(FwdSplit s, int D, int QB, int cus) {
+  const bool whole = s == FwdSplit::kRows64x4 || s == FwdSplit::kRows128x2 || (s == FwdSplit::kRows32x4 && D == 128);
+  return whole ? cus : (s == FwdSplit::kNone && QB == 64 ? 4 * cus : 2 * cus);
+}
 
 // Which split?  `rows32`: 32-row tiles of the whole launch, S: rows per slab; `busiest`: 128-row tiles dealt
 // to the XCD that has most, `cus`: compute units of an XCD.  A wave walks a list of up
@@ -62,7 +68,7 @@ constexpr int fwd_split_rows(FwdSplit s, int QB) {
 //          batched
 //          kRows64x2   B H=24 S=1600 31-38 (-5 .. -14), mixed 41-43 (-15 .. +1), B H=20 S=2000 37-45 (-5 .. -13), mixed
 //                      49 (-5); kRows128x2 there: mixed +10; beyond: B H=24 S=1750 mixed 45 (+13), B H=20 S=2100 39-48
-//                      (-14 .. +7), B H=32 S=1153 mixed 34 (+20)
+//                      (-14 .. +7), B H=32 S=1237, four elements' spans 31 (+13)
 //   D=64   kRows64x2   B H=32 S=1500 22-29 (-4 .. -25), mixed 30 (-5), B H=24 S=1900 26-34 (-15 .. -33), mixed 36 (-21);
 //                      one batch element: B H=24 S=2700 38-52 (-3 .. -21), B H=16 S=4500 60-80 (-5 .. -18), B H=12 S=6000
 //                      76-103 (-6 .. -21); beyond: B H=32 S=2000 mixed 39 (+11), B H=24 S=2000 mixed 38 (+8), B H=32 S=2300
@@ -74,12 +80,8 @@ inline FwdSplit fwd_ragged_split(int D, long long rows32, int S, bool even, bool
   bool two;
   if (D == 128) {
     if (!even) return FwdSplit::kNone;
-    if (batched) {
-      two = rows32 <= 1280 && S >= 1600;
-    } else {
-      if ((rows32 <= 1440 && S >= 1600) || (rows32 <= 1856 && S >= 2 * rows32)) return FwdSplit::kRows128x2;
-      two = rows32 <= 1280 && S >= 1152;
-    }
+    if (!batched && ((rows32 <= 1440 && S >= 1600) || (rows32 <= 1856 && S >= 2 * rows32))) return FwdSplit::kRows128x2;
+    two = rows32 <= 1280 && S >= (batched ? 1600 : 1152);
   } else if (D == 64) {
     if (S < 1408 || S < rows32) return FwdSplit::kNone;
     two = batched ? (rows32 <= 1440 && 4 * rows32 >= 3LL * S) || (rows32 <= 1792 && rows32 >= S)

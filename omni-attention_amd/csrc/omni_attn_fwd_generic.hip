@@ -42,6 +42,8 @@
 #include <type_traits>
 #include <utility>
 
+#include "omni_attn_deal.hpp"
+
 namespace omni_attn {
 // Keeps the hipError_t behind an OMNI_ATTN_ERR_LAUNCH for omni_attn_last_hip_error() (defined
 // beside that function).
@@ -85,6 +87,7 @@ struct GenericParams {
   int mask_words;     // four keys of a tile row may be read as one 32-bit word
   int whole;          // a step never crosses a block (blocks of 32 n keys, mask_words)
   unsigned n_slabs;   // B * H
+  omni_attn::FastDiv by_slabs, by_tiles, by_heads;  // by n_slabs, q_tiles, H
   float scale, sl2, softcap;
 };
 
@@ -240,10 +243,10 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
 
   const unsigned wg = blockIdx.x;
-  const unsigned rank = wg / p.n_slabs;
-  const size_t bh = wg - rank * p.n_slabs;
+  const unsigned rank = omni_attn::divide(wg, p.by_slabs);
+  const unsigned bh = wg - rank * p.n_slabs;
   const unsigned tile = unsigned(p.Tq) * unsigned(p.q_tiles) - 1 - rank;  // longest lists of a causal mask first
-  const int qb = int(tile / unsigned(p.q_tiles));
+  const int qb = int(omni_attn::divide(tile, p.by_tiles));
   const int row0 = int(tile - unsigned(qb) * unsigned(p.q_tiles)) * 32;  // first row inside the block
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -261,11 +264,11 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
   int32_t* const sPid = sKey + 64;
   float* const sStat = reinterpret_cast<float*>(lds + Traits::kTiles + Traits::kQBytes + NW * 384);  // [2][NW][32]
 
-  const int64_t b = int64_t(bh) / p.H, h = int64_t(bh) - b * p.H;
+  const int64_t b = omni_attn::divide(bh, p.by_heads), h = bh - unsigned(b) * unsigned(p.H);
   const uint16_t* const q_slab = p.q + b * p.q_at.batch + h * p.q_at.head;
   const uint16_t* const k_slab = p.k + b * p.k_at.batch + h * p.k_at.head;
   const uint16_t* const v_slab = p.v + b * p.v_at.batch + h * p.v_at.head;
-  const size_t mrow = bh * p.Tq + qb;
+  const size_t mrow = size_t(bh) * p.Tq + qb;
   const size_t moff = mrow * p.max_blocks;
   const bool has_partial = p.partial_idx != nullptr && p.partial_masks != nullptr;
 
@@ -815,7 +818,7 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
   const float inv = some ? 1.f / l_all : 0.f;  // :283-288; rows without a key: zeros (:177-183)
   const float mine = __builtin_amdgcn_exp2f(m_run - m_fin) * inv;
   if (w == 0 && g == 0 && q_here && p.lse)
-    p.lse[bh * p.S + q_idx] = some ? (m_fin + __builtin_amdgcn_logf(l_all) - kShift) * 0.6931471805599453f : -INFINITY;
+    p.lse[size_t(bh) * p.S + q_idx] = some ? (m_fin + __builtin_amdgcn_logf(l_all) - kShift) * 0.6931471805599453f : -INFINITY;
   float* const stage = reinterpret_cast<float*>(lds);
   constexpr int G = Traits::kGroup;
 #pragma unroll
@@ -843,7 +846,7 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
         x += *reinterpret_cast<const f32x4_t*>(stage + ((size_t(j) * G + i) * 4 + r4) * 256 + lane * 4);
       if (empty) x = f32x4_t{0.f, 0.f, 0.f, 0.f};
       const int d = 32 * (d0 + i) + 8 * r4 + 4 * g;
-      uint16_t* orow = p.o + (bh * p.S + q_idx) * p.D;
+      uint16_t* orow = p.o + (size_t(bh) * p.S + q_idx) * p.D;
       uint16_t hv[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) hv[j] = from_float<BF16>(x[j]);
@@ -888,6 +891,9 @@ int launch(const GenericParams& p, unsigned grid, hipStream_t stream) {
   GenericParams params = p;
   params.adv_slot = 32 * NW / p.kb_eff;
   params.adv_off = 32 * NW % p.kb_eff;
+  params.by_slabs = omni_attn::fast_div(p.n_slabs);
+  params.by_tiles = omni_attn::fast_div(uint32_t(p.q_tiles));
+  params.by_heads = omni_attn::fast_div(uint32_t(p.H));
   void* args[] = {&params};
   return int(hipLaunchKernel(fn, dim3(grid), dim3(64 * NW), args, lds, stream));
 }

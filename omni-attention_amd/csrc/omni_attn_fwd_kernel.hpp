@@ -1030,10 +1030,9 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
       for (int i = 0; i < NCH / 4; ++i) issue_four(false, i, nxt.row0, lds_v0);
     } else {
 #pragma unroll
-      for (int i = 0; i < NCH; ++i) {
-        issue_load(NCH + i, 0, cur.row0, 0);
-        issue_load(NCH + i, 1, nxt.row0, 0);
-      }
+      for (int i = 0; i < NCH; ++i) issue_load(NCH + i, 0, cur.row0, 0);
+#pragma unroll
+      for (int i = 0; i < NCH; ++i) issue_load(NCH + i, 1, nxt.row0, 0);
     }
     if (cur.mode == kPartial) {
       if (packed_tiles) {
@@ -1044,7 +1043,8 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
         if (take_mask_bytes()) cur.mode = kFull;
       }
     }
-    step_barrier();
+    wait_loads_but<NCH>();  // K(1) may be under way
+    if constexpr (!LONE) __syncthreads();
 #pragma unroll
     for (int s = 0; s < KS; ++s)
 #pragma unroll

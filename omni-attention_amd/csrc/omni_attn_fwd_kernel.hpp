@@ -10,9 +10,9 @@
 //   O^T[d,  q] = V^T[d, kv] . P^T[kv, q]  A = V^T (LDS transpose read), B = P^T
 // With v_mfma_f32_32x32x16 the accumulator of S^T puts query row (lane % 32) in a
 // lane and 16 kv positions in its registers, which is exactly the B-operand layout
-// the second product needs: P never leaves registers, row max / row sum are in-lane
-// reductions plus one exchange with lane ^ 32, and the online-softmax rescale is a
-// per-lane scalar.
+// the second product needs: P never leaves registers, row sums (and maxima, in the few steps
+// that look at them) are in-lane reductions plus one exchange with lane ^ 32, and the
+// online-softmax rescale is a per-lane scalar.
 //
 // A wave owns 32 query rows; a workgroup has QB/32 waves.  KV blocks are consumed in
 // steps of 64 keys (a 128-key block is two steps; 32 keys for 64-row query blocks).  K and

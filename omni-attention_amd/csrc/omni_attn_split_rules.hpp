@@ -76,6 +76,22 @@ constexpr int fwd_places(FwdSplit s, int D, int QB, int cus) {
 //   D=32   kRows64x2   B H=48 S=1237 16-23 (-5 .. -18), mixed 23 (-16), B H=40 S=1700 22-31 (-8 .. -27), B H=32 S=2300 27-37
 //                      (-17 .. -24), S=3000 38-50 (-3 .. -18), mixed 57 (-1 .. -5), B H=16 S=6000 68-93 (-7 .. -28); beyond:
 //                      B H=48 S=1500 20-27 (-18 .. +3)
+//   64-row blocks (every head_dim: half the waves per workgroup, so half of the device stands by longer)
+//          kRows64x2   D=128 B H=32 S=1237 30-38 (-16 .. -31), B H=24 S=1500 35-44 (-28 .. -33), B H=20 S=2300 50-64 (-15 ..
+//                      -32); D=64 B H=32 S=1700 25-32 (-5 .. -26), B H=16 S=5000 72-91 (-2 .. -20), B H=12 S=6000 81-104 (-10 ..
+//                      -26); batched B H=24 S=1500 22-29 (-12 .. -34), S=1700 24-32 (-4 .. -30), B H=16 S=5000 72-104
+//                      (-2 .. -12); D=32 B H=32 S=2000 24-31 (-7 .. -32), batched B H=40 S=1300 17-22 (-2 .. -28); beyond:
+//                      batched, D=64 B H=32 S=1700 mixed 33 (+15), S=1237 mixed 25 (+3)
+inline FwdSplit fwd_ragged_split_64(int D, long long rows32, int S, bool even, bool batched) {
+  if (!even || S < 1152) return FwdSplit::kNone;
+  bool two;
+  if (batched) {
+    two = rows32 <= 1344 && (D == 32 || 5 * rows32 <= 4LL * S);
+  } else {
+    two = rows32 <= (D == 128 ? 1440 : (D == 64 ? 1792 : 2048));
+  }
+  return two || (D != 128 && rows32 <= 2560 && S >= 2 * rows32) ? FwdSplit::kRows64x2 : FwdSplit::kNone;
+}
 inline FwdSplit fwd_ragged_split(int D, long long rows32, int S, bool even, bool batched) {
   bool two;
   if (D == 128) {
@@ -100,7 +116,8 @@ inline FwdSplit fwd_choose_split(int D, int QB, long long rows32, int S, long lo
   const bool lone = (rows32 <= 512 && S >= 512) || (rows32 <= 640 && S >= 1152) || (rows32 <= 768 && S >= 1536);
   if (QB != 128) {
     if (D == 128 && (lone || (rows32 <= 768 && S >= 1152))) return FwdSplit::kRows64x4;
-    return some ? FwdSplit::kRows64x2 : FwdSplit::kNone;
+    if (some) return FwdSplit::kRows64x2;
+    return ragged ? fwd_ragged_split_64(D, rows32, S, even, batched) : FwdSplit::kNone;
   }
   if (D != 128) {
     const bool more = D == 64 ? rows32 <= 1280 && S >= 1152

@@ -146,16 +146,17 @@ def test_backward_of_slabs_walked_together_with_different_masks(H, S, gpu_device
     check_grads(got, attention_dense_grads(q, k, v, allow, dout), torch.float16, f"H={H} S={S}")
 
 
-@pytest.mark.parametrize("D,B,H,S,copies", [
-    (128, 1, 2, 1160, 16), (128, 1, 2, 1610, 12), (128, 1, 1, 2700, 16), (128, 3, 1, 1630, 8), (64, 2, 1, 1500, 16),
-    (64, 1, 1, 4400, 16), (32, 2, 1, 1300, 24), (32, 1, 1, 2950, 32)])
-def test_lengths_that_end_inside_a_block(D, B, H, S, copies, gpu_device):
+@pytest.mark.parametrize("D,B,H,S,copies,QB", [
+    (128, 1, 2, 1160, 16, 128), (128, 1, 2, 1610, 12, 128), (128, 1, 1, 2700, 16, 128), (128, 3, 1, 1630, 8, 128),
+    (64, 2, 1, 1500, 16, 128), (64, 1, 1, 4400, 16, 128), (32, 2, 1, 1300, 24, 128), (32, 1, 1, 2950, 32, 128),
+    (128, 1, 2, 1170, 16, 64), (128, 2, 1, 1500, 12, 64), (64, 2, 1, 1500, 12, 64), (32, 1, 2, 1900, 16, 64)])
+def test_lengths_that_end_inside_a_block(D, B, H, S, copies, QB, gpu_device):
     """Launches that are split because of such a length: 64- and 128-row groups, dQ in 64-row groups at head_dim 64.
     The slabs of a batch element are repeated; the first ones against the oracle, the copies bit for bit."""
     from test_gpu_backward import check_grads, run_fwd_bwd
     from oracle.dense_oracle import attention_dense_grads
     gen = torch.Generator().manual_seed(D + S)
-    QB = KB = 128
+    KB = QB
     n = -(-S // QB) * QB
     q, k, v, dout = (torch.randn(B, H, n, D, generator=gen).to(torch.bfloat16) for _ in range(4))
     nb, idx, tys, pidx, pm = random_block_metadata(gen, B, H, n // QB, n // KB, QB, KB, p_empty=0.5, shuffle=True)

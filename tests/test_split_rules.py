@@ -78,6 +78,8 @@ int main() {
           const FwdSplit plain = fwd_choose_split(D, 128, rows, S, busiest, 32);
           const FwdSplit ragged = fwd_choose_split(D, 128, rows, S, busiest, 32, true, true, batched);
           if (plain != FwdSplit::kNone && plain != ragged) return 1;
+          const FwdSplit plain64 = fwd_choose_split(D, 64, rows, S, busiest, 32);
+          if (plain64 != FwdSplit::kNone && plain64 != fwd_choose_split(D, 64, rows, S, busiest, 32, true, true, batched)) return 5;
           if (batched && ragged != FwdSplit::kNone && fwd_choose_split(D, 128, rows, S, busiest, 32, true, true, false) == FwdSplit::kNone) return 2;
           if (ragged != FwdSplit::kNone) all = true;
           else if (all && !batched && S >= 1152) return 3;

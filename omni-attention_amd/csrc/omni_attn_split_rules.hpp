@@ -161,7 +161,8 @@ enum class DkdvSplit : int {
 //                 75-95 (0 .. -13); 64-key blocks 73-90 (-3 .. +9); beyond: B H=24 S=2048 78-106 (-2 .. +9), B H=12
 //                 S=4096 136-170 (-7 .. +6)
 //   dQ, D=64, lengths that end inside a block, where the forward is split for that: B H=24 S=2300 127-172 (-2 .. -5), B H=16
-//          S=4500 248-317 (0 .. -5), soft-capped 437 (-10); beyond: B H=40 S=1700 107-134 (-3 .. +4); D=128 gains
+//          S=4500 248-317 (0 .. -5), soft-capped 437 (-10), 64-row blocks B H=32 S=1700 97-117 (-3 .. -13), B H=24 S=2300
+//          123-158 (-6 .. -10), B H=16 S=4500 258-327 (-3 .. -5); beyond: B H=40 S=1700 107-134 (-3 .. +4); D=128 gains
 //          nowhere: B H=32 S=1237 101-130 (0 .. +4), B H=24 S=1700 128-171 (-2 .. +4)
 inline FwdSplit bwd_choose_dq_split(int D, int QB, long long rows32, int S, bool ragged = false, bool batched = true) {
   if (rows32 <= (D == 128 ? 256 : 512)) return FwdSplit::kRows32x4;
@@ -171,7 +172,9 @@ inline FwdSplit bwd_choose_dq_split(int D, int QB, long long rows32, int S, bool
           (QB == 128 && ((rows32 <= 768 && S >= 1024) || (rows32 <= 896 && S >= 1536)));
   } else {
     two = (rows32 <= 1024 && S >= 512) || (rows32 <= 1536 && S >= 1024) || (rows32 <= 2048 && S >= 4096) ||
-          (D == 64 && QB == 128 && ragged && fwd_ragged_split(D, rows32, S, true, batched) != FwdSplit::kNone);
+          (D == 64 && ragged &&
+           (QB == 128 ? fwd_ragged_split(D, rows32, S, true, batched)
+                      : fwd_ragged_split_64(D, rows32, S, true, batched)) != FwdSplit::kNone);
   }
   return two ? FwdSplit::kRows64x2 : FwdSplit::kNone;
 }

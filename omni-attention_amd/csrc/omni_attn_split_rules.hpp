@@ -164,7 +164,12 @@ enum class DkdvSplit : int {
 //          S=4500 248-317 (0 .. -5), soft-capped 437 (-10), 64-row blocks B H=32 S=1700 97-117 (-3 .. -13), B H=24 S=2300
 //          123-158 (-6 .. -10), B H=16 S=4500 258-327 (-3 .. -5); beyond: B H=40 S=1700 107-134 (-3 .. +4); D=128 gains
 //          nowhere: B H=32 S=1237 101-130 (0 .. +4), B H=24 S=1700 128-171 (-2 .. +4)
-inline FwdSplit bwd_choose_dq_split(int D, int QB, long long rows32, int S, bool ragged = false, bool batched = true) {
+//   dQ, D=64, soft-capped (three exponentials and a reciprocal per score: twice the vector work against a list's
+//          loads), lengths that end inside a block: B H=32 S=2300 188-237 (-1 .. -9), S=2500 212-366 (-1 .. -5), B H=24 S=3000
+//          242-356 (-2 .. -7), B H=20 S=4000 322-388 (-1 .. -9); beyond: S=3000 279-455 (0 .. -2), whole blocks B H=32
+//          S=2048 161-230 (-5 .. +5), S=3072 286-406 (0 .. +2); D=128 B H=32 S=1500 148-208 (+3 .. +6)
+inline FwdSplit bwd_choose_dq_split(int D, int QB, long long rows32, int S, bool ragged = false, bool batched = true,
+                                    bool capped = false) {
   if (rows32 <= (D == 128 ? 256 : 512)) return FwdSplit::kRows32x4;
   bool two;
   if (D == 128) {
@@ -172,6 +177,7 @@ inline FwdSplit bwd_choose_dq_split(int D, int QB, long long rows32, int S, bool
           (QB == 128 && ((rows32 <= 768 && S >= 1024) || (rows32 <= 896 && S >= 1536)));
   } else {
     two = (rows32 <= 1024 && S >= 512) || (rows32 <= 1536 && S >= 1024) || (rows32 <= 2048 && S >= 4096) ||
+          (D == 64 && capped && ragged && QB == 128 && rows32 <= 2688 && S >= 2048 && S >= rows32) ||
           (D == 64 && ragged &&
            (QB == 128 ? fwd_ragged_split(D, rows32, S, true, batched)
                       : fwd_ragged_split_64(D, rows32, S, true, batched)) != FwdSplit::kNone);

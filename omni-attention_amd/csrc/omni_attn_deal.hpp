@@ -15,7 +15,7 @@ namespace omni_attn {
 // Division of n < 2^31 by a number that the host knows: three scalar instructions, where a division by a kernel
 // argument is 25 - 30 with a trip to the vector unit and back.  A workgroup made seven of them, 150 of the 400
 // instructions before it could ask for its list, one after the other (a lone wave issues one in about five cycles).
-// Without them: B=1 H=8 S=512 D=128 causal 6.55 -> 6.31 us, B=1 H=16 S=1024 D=64 10.2 -> 9.5, unaligned spans of
+// Without them: B=1 H=8 S=512 D=64 causal 6.55 -> 6.31 us, B=1 H=16 S=1024 D=64 10.2 -> 9.5, unaligned spans of
 // 1237 rows 29.8 -> 29.3.
 // mul = floor(2^(31 + shift) / d) + 1 with 2^shift >= d exceeds 2^(31 + shift) / d by less than 2^shift / d, so
 // n * mul / 2^(31 + shift) exceeds n / d by less than 1 / d: the floors are the same.

@@ -558,8 +558,8 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   const i32x4_t rV = row_resource<D>(p.v, p.v_at, bh, p.H, p.deal.heads, p.seqlen);
   const i32x4_t rQ = row_resource<D>(p.q, p.q_at, bh, p.H, p.deal.heads, p.seqlen);
   // Q as the B operand of S^T = K.Q^T: lane holds Q[q_row][16s + 8g .. +7].  Lone waves ask for it while
-  // the list is on its way (B=1 H=8 S=512 D=128 6.33 -> 6.08 us), others when it is there: their waves share the
-  // way to memory, and the list and K come first (B=1 H=8 S=2048 in 64-row blocks 12.2 us, 12.3 the other way).
+  // the list is on its way (D=64 B H=8 S=512 6.33 -> 6.08 us, 64-row blocks S=2048 12.17 -> 12.28), others when it is
+  // there (no difference at B H=32 S=1237 D=128).
   u32x4_t qf[KS];
   auto request_q = [&]() {
     const uint32_t at = q_row < p.seqlen ? uint32_t(q_row) * (p.q_at.row * 2u) + 16u * uint32_t(g) : kNoRow<D>;

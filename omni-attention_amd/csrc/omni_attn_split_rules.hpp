@@ -168,6 +168,10 @@ enum class DkdvSplit : int {
 //          loads), lengths that end inside a block: B H=32 S=2300 188-237 (-1 .. -9), S=2500 212-366 (-1 .. -5), B H=24 S=3000
 //          242-356 (-2 .. -7), B H=20 S=4000 322-388 (-1 .. -9); beyond: S=3000 279-455 (0 .. -2), whole blocks B H=32
 //          S=2048 161-230 (-5 .. +5), S=3072 286-406 (0 .. +2); D=128 B H=32 S=1500 148-208 (+3 .. +6)
+//   dQ, D=32, lengths that end inside a block: B H=32 S=1700 76-125 (-7 .. -10), S=3000 152-267 (-1 .. -9), B H=40 S=2000 98-181 (0 ..
+//          -8), B H=16 S=4500 184-234 (-6 .. -16), S=6000 274-354 (-2 .. -17), soft-capped B H=32 S=2000 135-211 (-4 .. -7),
+//          64-row blocks B H=40 S=1700 83-148 (-3 .. -5), B H=16 S=4500 200-384 (-10 .. -14); beyond: B H=48 S=1237 67-96
+//          (-8 .. +3); whole blocks B H=32 S=2048 90-129 (-7 .. +6), S=3072 157-215 (-1 .. +1)
 inline FwdSplit bwd_choose_dq_split(int D, int QB, long long rows32, int S, bool ragged = false, bool batched = true,
                                     bool capped = false) {
   if (rows32 <= (D == 128 ? 256 : 512)) return FwdSplit::kRows32x4;
@@ -177,6 +181,7 @@ inline FwdSplit bwd_choose_dq_split(int D, int QB, long long rows32, int S, bool
           (QB == 128 && ((rows32 <= 768 && S >= 1024) || (rows32 <= 896 && S >= 1536)));
   } else {
     two = (rows32 <= 1024 && S >= 512) || (rows32 <= 1536 && S >= 1024) || (rows32 <= 2048 && S >= 4096) ||
+          (D == 32 && ragged && ((rows32 <= 2560 && S >= 1664) || (rows32 <= 3072 && S >= rows32))) ||
           (D == 64 && capped && ragged && QB == 128 && rows32 <= 2688 && S >= 2048 && S >= rows32) ||
           (D == 64 && ragged &&
            (QB == 128 ? fwd_ragged_split(D, rows32, S, true, batched)

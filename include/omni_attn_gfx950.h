@@ -194,6 +194,8 @@ int omni_attn_fwd_strided_gfx950(const void* q, const void* k, const void* v, om
  * values there before but that tag -- and needs the workspace only, so that a caller can allocate the lists
  * while it runs; the sum of the counts is the size of the tile arrays, and omni_attn_mask_finish_gfx950 writes
  * lists and tiles.  Tk below 2^OMNI_ATTN_MASK_POSTED_COUNT_BITS.
+ * num_partial is the number of tiles that there is room for: with more room than tiles the rest stays as it is, with
+ * less the tiles beyond are not written (their numbers are in partial_idx all the same).
  */
 #define OMNI_ATTN_MASK_MAX_QB 8192
 size_t omni_attn_mask_workspace_bytes(int B, int q_len, int kv_len, int QB, int KB);

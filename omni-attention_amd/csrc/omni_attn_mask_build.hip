@@ -258,6 +258,7 @@ __global__ void __launch_bounds__(256) mask_write_kernel(const MaskParams p, uin
       upto += lane >= d ? other : 0;
     }
     if (lane == 63) part[w] = upto;
+    if (threadIdx.x == 0) found[0] = -1;
     __syncthreads();
     for (int i = 0; i < w; ++i) upto += part[i];
     int left = tile - (upto - mine);
@@ -269,6 +270,7 @@ __global__ void __launch_bounds__(256) mask_write_kernel(const MaskParams p, uin
     }
     __syncthreads();
     const int row = found[0];
+    if (row < 0) return;  // there is room for more tiles than the mask has
     left = found[1];
     for (int r = threadIdx.x; r < p.QB; r += 256) reach[r] = p.reach[size_t(row) * p.QB + r];
     const int listed = p.listed[row];

@@ -73,3 +73,47 @@ def test_many_masks_in_a_row(gpu_device):
         mp, S = sizes[i % 64 == 0]
         m = shim.create_transfusion_block_mask(mp, 2, S, 128, 128, pack=False)
         assert m.partial_block_masks.shape[0] == want[i % 64 == 0]
+
+
+@pytest.mark.parametrize("two_launches", [True, False])
+@pytest.mark.parametrize("room", [-2, 0, 3, 1000])
+def test_room_for_another_number_of_tiles(two_launches, room, gpu_device):
+    """The C calls with a tile store of a fixed size: what it has room for is written, the rest of it is left alone."""
+    import ctypes
+    import omni_attn_capi as capi
+    lib = capi.load_library()
+    lib.omni_attn_mask_workspace_bytes.restype = ctypes.c_size_t
+    B, H, S, QB, KB = 2, 3, 3000, 128, 64
+    spans = torch.tensor([[[1, 37, 90], [1, 200, 1041]], [[1, 700, 1500], [0, 0, 0]]])
+    want = oat.create_omni_block_mask_from_modality_positions(spans, B, H, S, S, QB, KB, device="cpu")
+    n = want.partial_block_masks.shape[0]
+    Tq, Tk = want.kv_indices.shape[2:]
+    sp = spans.to(gpu_device)
+    i32 = lambda *shape: torch.empty(*shape, dtype=torch.int32, device=gpu_device)
+    nb, idx, tys, pidx = i32(B, H, Tq), i32(B, H, Tq, Tk), i32(B, H, Tq, Tk), i32(B, H, Tq, Tk)
+    ws = i32(lib.omni_attn_mask_workspace_bytes(B, S, S, QB, KB) // 4)
+    posted = torch.zeros(B * Tq, dtype=torch.int32, pin_memory=True)
+    tiles = torch.full((n + 1000, QB, KB), 7, dtype=torch.uint8, device=gpu_device)
+    bits = torch.full((n + 1000, QB, KB // 32), 7, dtype=torch.int32, device=gpu_device)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    lists = (ptr(nb), ptr(idx), ptr(tys), ptr(pidx))
+    if two_launches:
+        assert lib.omni_attn_mask_classify_gfx950(ptr(sp), None, ptr(ws), ptr(posted), 5, B, 2, S, S, QB, KB, stream) == 0
+        torch.cuda.synchronize()
+        assert bool((posted >> 20 == 5).all()) and int((posted & 0xfffff).sum()) == n
+        assert lib.omni_attn_mask_finish_gfx950(*lists, ptr(ws), ptr(tiles), ptr(bits), n + room, B, H, S, S, QB, KB,
+                                                stream) == 0
+    else:
+        assert lib.omni_attn_mask_lists_gfx950(ptr(sp), None, *lists, ptr(ws), ptr(posted), 9, B, 2, H, S, S, QB, KB,
+                                               stream) == 0
+        torch.cuda.synchronize()
+        assert posted[:2].tolist() == [n, 9]
+        assert lib.omni_attn_mask_tiles_gfx950(ptr(sp), None, ptr(ws), ptr(tiles), ptr(bits), n + room, B, 2, H, S, S, QB,
+                                               KB, stream) == 0
+    same_mask(oat.OmniBlockMask(nb, idx, tys, Tq * QB, Tk * KB, QB, KB, pidx, tiles[:n].view(torch.bool) if room >= 0 else
+                                want.partial_block_masks.to(gpu_device)), want)
+    written = min(n + room, n)
+    assert torch.equal(tiles[:written].cpu(), want.partial_block_masks[:written].to(torch.uint8))
+    assert torch.equal(bits[:written], capi.pack_partial_masks(tiles[:written]))
+    assert bool((tiles[written:] == 7).all()) and bool((bits[written:] == 7).all())

@@ -189,7 +189,7 @@ int omni_attn_fwd_strided_gfx950(const void* q, const void* k, const void* v, om
  * (omni_attn_mask_workspace_bytes), which writes partial_masks [P, QB, KB] bytes (16-byte
  * aligned) and, where asked for (KB a multiple of 32), the packed words of
  * omni_attn_pack_partial_masks_gfx950.  QB up to OMNI_ATTN_MASK_MAX_QB.
- * In two launches instead of four: omni_attn_mask_classify_gfx950 writes, per (b, query block), the number of
+ * In two launches instead of four (three beyond 1024 query blocks): omni_attn_mask_classify_gfx950 writes, per (b, query block), the number of
  * its PARTIAL tiles with `tag` (12 bits) in the upper bits to posted[b * Tq + block] -- host memory as above, any
  * values there before but that tag -- and needs the workspace only, so that a caller can allocate the lists
  * while it runs; the sum of the counts is the size of the tile arrays, and omni_attn_mask_finish_gfx950 writes

@@ -13,6 +13,9 @@
 //   write      one workgroup per (b, query block) and four heads, a head per wave, writes the list and the tile
 //              numbers (the tiles before the query block are a sum over the counts), and one per tile, which finds
 //              its query block by a scan of the counts, writes its bytes, and its bits where they are asked for
+// With many query blocks a sum and a scan per workgroup, and a word per query block over the bus, are what a call takes;
+// there a kernel of one workgroup sums up the counts once (and sends their total): a call, us, B=32 H=16 S=65536
+// 1097 -> 415, B=64 H=4 S=65536 3739 -> 416, B=64 H=16 S=8192 127 -> 54 (the host's share of that: a word instead of 4096).
 // Both are bound by their launches and a chain of a few memory latencies; the bytes
 // (B=4 H=16 S=8192, 128x128 blocks: 3.1 MB of lists, 2.4 MB of tiles) take a microsecond.  That mask,
 // packed, in calls back to back: 472 us as tensor algebra; 38 us as three kernels (8.2, 3.9 and 5.0 us)
@@ -47,10 +50,11 @@ struct MaskParams {
   int32_t* counts;        // [B * Tq] PARTIAL tiles of a query block
   int32_t* full;          // [B * Tq] leading FULL blocks of its list
   int32_t* listed;        // [B * Tq] blocks of its list: 0, 1, ...
+  int32_t* before;        // [B * Tq] PARTIAL tiles of the query blocks before it; null: summed up where needed
   int32_t* open;          // [B * Tq * Tk] types of the blocks full .. listed - 1
   int32_t* reach;         // [B * Tq * QB] keys that a row attends
   uint32_t* posted;       // pinned, or null: [B * Tq] tag in the upper 12 bits, count in the lower 20
-  int32_t* host_total;    // pinned: [0] the number of tiles, [1] the ticket
+  int32_t* host_total;    // pinned, or null: [0] the number of tiles, [1] the ticket
   int ticket;
   int num_partial;        // tiles that there is room for
   int head_groups;        // workgroups per query block that write lists
@@ -58,6 +62,10 @@ struct MaskParams {
 };
 
 constexpr int kPostedCountBits = OMNI_ATTN_MASK_POSTED_COUNT_BITS;
+// Query blocks up to which the lists and tiles sum the counts up where they need them: every workgroup reads the counts
+// before its own, and another launch costs 3 us.  In calls back to back, us, with and without that launch: 1024 query
+// blocks (B=16 H=16 S=8192) 40.9 / 37.6, 2048 (S=16384) 62.0 / 65.7, 4096 (B=64 S=8192) 98 / 129.
+constexpr int kSumRows = 1024;
 
 // Spans of a batch element that are worked at a time: (offset, end) pairs in LDS.
 constexpr int kSpanChunk = 64;
@@ -195,13 +203,36 @@ __device__ __forceinline__ int sum_of_256(int x, int32_t* part) {
   return part[0] + part[1] + part[2] + part[3];
 }
 
-// The number of tiles, to the host as one word (callers that take no counts).
-__global__ void __launch_bounds__(256) mask_total_kernel(const MaskParams p) {
-  __shared__ int32_t part[4];
-  int x = 0;
-  for (int i = threadIdx.x; i < p.B * p.Tq; i += 256) x += p.counts[i];
-  const int all = sum_of_256(x, part);
-  if (threadIdx.x == 0) {
+// The tiles before each query block, by one workgroup, a wave per run of query blocks; their number goes to the host as
+// one word where that is asked for.
+__global__ void __launch_bounds__(1024) mask_number_kernel(const MaskParams p) {
+  __shared__ int32_t part[16];
+  const unsigned lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const unsigned n = unsigned(p.B) * unsigned(p.Tq);
+  const unsigned run = ((n + 63) / 64 + 15) / 16 * 64;  // query blocks of a wave
+  const unsigned first = w * run, last = first + run < n ? first + run : n;
+  int sum = 0;
+  for (unsigned i = first + lane; i < last; i += 64) sum += p.counts[i];
+  for (int m = 32; m >= 1; m >>= 1) sum += __shfl_xor(sum, m, 64);
+  if (lane == 0) part[w] = sum;
+  __syncthreads();
+  int upto = 0, all = 0;
+  for (unsigned i = 0; i < 16; ++i) {
+    upto += i < w ? part[i] : 0;
+    all += part[i];
+  }
+  for (unsigned i0 = first; i0 < last; i0 += 64) {
+    const unsigned i = i0 + lane;
+    const int own = i < last ? p.counts[i] : 0;
+    int here = own;  // inclusive sum over the lanes
+    for (unsigned d = 1; d < 64; d <<= 1) {
+      const int other = __shfl_up(here, d, 64);
+      here += lane >= d ? other : 0;
+    }
+    if (i < last) p.before[i] = upto + here - own;
+    upto += __shfl(here, 63, 64);
+  }
+  if (threadIdx.x == 0 && p.host_total != nullptr) {
     __hip_atomic_store(p.host_total, all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     __hip_atomic_store(p.host_total + 1, p.ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
@@ -248,30 +279,42 @@ __global__ void __launch_bounds__(256) mask_write_kernel(const MaskParams p, uin
   const int n_rows = p.B * p.Tq;
   if (int(blockIdx.x) < p.num_partial) {
     const int tile = blockIdx.x;
-    // a thread looks at `per` neighbouring query blocks
-    const int per = (n_rows + 255) / 256, r0 = threadIdx.x * per, r1 = r0 + per < n_rows ? r0 + per : n_rows;
-    int mine = 0;
-    for (int r = r0; r < r1; ++r) mine += p.counts[r];
-    int upto = mine;  // inclusive sum over the threads
-    for (int d = 1; d < 64; d <<= 1) {
-      const int other = __shfl_up(upto, d, 64);
-      upto += lane >= d ? other : 0;
+    int row = 0, left;
+    if (p.before != nullptr) {
+      for (int n = n_rows; n > 1;) {  // it is one of the query blocks row .. row + n - 1: 256 looks at a time
+        const int step = (n + 255) / 256, at = int(threadIdx.x) * step;
+        const int c = __syncthreads_count(at < n && p.before[row + at] <= tile) - 1;
+        row += c * step;
+        n = n - c * step < step ? n - c * step : step;
+      }
+      left = tile - p.before[row];
+      if (left >= p.counts[row]) return;  // there is room for more tiles than the mask has
+    } else {
+      // a thread looks at `per` neighbouring query blocks
+      const int per = (n_rows + 255) / 256, r0 = threadIdx.x * per, r1 = r0 + per < n_rows ? r0 + per : n_rows;
+      int mine = 0;
+      for (int r = r0; r < r1; ++r) mine += p.counts[r];
+      int upto = mine;  // inclusive sum over the threads
+      for (int d = 1; d < 64; d <<= 1) {
+        const int other = __shfl_up(upto, d, 64);
+        upto += lane >= d ? other : 0;
+      }
+      if (lane == 63) part[w] = upto;
+      if (threadIdx.x == 0) found[0] = -1;
+      __syncthreads();
+      for (int i = 0; i < w; ++i) upto += part[i];
+      left = tile - (upto - mine);
+      if (left >= 0 && left < mine) {
+        int r = r0;
+        for (int c = p.counts[r]; left >= c; c = p.counts[++r]) left -= c;
+        found[0] = r;
+        found[1] = left;
+      }
+      __syncthreads();
+      row = found[0];
+      if (row < 0) return;  // (as above)
+      left = found[1];
     }
-    if (lane == 63) part[w] = upto;
-    if (threadIdx.x == 0) found[0] = -1;
-    __syncthreads();
-    for (int i = 0; i < w; ++i) upto += part[i];
-    int left = tile - (upto - mine);
-    if (left >= 0 && left < mine) {
-      int r = r0;
-      for (int c = p.counts[r]; left >= c; c = p.counts[++r]) left -= c;
-      found[0] = r;
-      found[1] = left;
-    }
-    __syncthreads();
-    const int row = found[0];
-    if (row < 0) return;  // there is room for more tiles than the mask has
-    left = found[1];
     for (int r = threadIdx.x; r < p.QB; r += 256) reach[r] = p.reach[size_t(row) * p.QB + r];
     const int listed = p.listed[row];
     int kb = p.full[row];
@@ -296,9 +339,14 @@ __global__ void __launch_bounds__(256) mask_write_kernel(const MaskParams p, uin
   const int row = item / p.head_groups, group = item - row * p.head_groups;
   const int b = row / p.Tq, qb = row - b * p.Tq;
   const int full = p.full[row], listed = p.listed[row];
-  int x = 0;
-  for (int i = threadIdx.x; i < row; i += 256) x += p.counts[i];
-  int before = sum_of_256(x, part);  // tiles of the query blocks before this one
+  int before;  // tiles of the query blocks before this one
+  if (p.before != nullptr) {
+    before = p.before[row];
+  } else {
+    int x = 0;
+    for (int i = threadIdx.x; i < row; i += 256) x += p.counts[i];
+    before = sum_of_256(x, part);
+  }
   for (int s0 = 0; s0 < p.Tk; s0 += 64) {
     const int s = s0 + lane;
     int type = s < full ? kFull : 0;
@@ -345,7 +393,8 @@ MaskParams common(const int64_t* spans, const int64_t* prefix, void* workspace, 
   p.counts = static_cast<int32_t*>(workspace);
   p.full = p.counts + rows;
   p.listed = p.full + rows;
-  p.open = p.listed + rows;
+  p.before = p.listed + rows;
+  p.open = p.before + rows;
   p.reach = p.open + rows * p.Tk;
   return p;
 }
@@ -361,7 +410,7 @@ int launched(hipError_t e) {
 extern "C" size_t omni_attn_mask_workspace_bytes(int B, int q_len, int kv_len, int QB, int KB) {
   if (bad_shape(B, 0, 1, q_len, kv_len, QB, KB) != OMNI_ATTN_OK) return 0;
   const size_t Tq = size_t((q_len + QB - 1) / QB), Tk = size_t((kv_len + KB - 1) / KB);
-  return size_t(B) * Tq * (3 + Tk + QB) * sizeof(int32_t);
+  return size_t(B) * Tq * (4 + Tk + QB) * sizeof(int32_t);
 }
 
 namespace {
@@ -370,6 +419,11 @@ int launch_classify(const MaskParams& params, hipStream_t stream) {
   void* args[] = {&p};
   return launched(hipLaunchKernel(reinterpret_cast<const void*>(mask_classify_kernel), dim3(unsigned(p.B) * unsigned(p.Tq)),
                                   dim3(256), args, 0, stream));
+}
+int launch_number(const MaskParams& params, hipStream_t stream) {
+  MaskParams p = params;
+  void* args[] = {&p};
+  return launched(hipLaunchKernel(reinterpret_cast<const void*>(mask_number_kernel), dim3(1), dim3(1024), args, 0, stream));
 }
 // Lists (where p.nb is given) and tiles (where there are any), in one launch.
 int launch_write(const MaskParams& params, uint8_t* tiles, uint32_t* bits, hipStream_t stream) {
@@ -418,7 +472,13 @@ extern "C" int omni_attn_mask_finish_gfx950(int32_t* kv_num_blocks, int32_t* kv_
   p.types = block_mask_types;
   p.pidx = partial_idx;
   p.num_partial = num_partial;
-  return launch_write(p, partial_masks_or_null, partial_bits_or_null, static_cast<hipStream_t>(stream));
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  if (p.B * p.Tq <= kSumRows) {
+    p.before = nullptr;
+  } else if (const int rc = launch_number(p, s)) {
+    return rc;
+  }
+  return launch_write(p, partial_masks_or_null, partial_bits_or_null, s);
 }
 
 extern "C" int omni_attn_mask_lists_gfx950(const int64_t* spans_or_null, const int64_t* prefix_or_null,
@@ -438,9 +498,7 @@ extern "C" int omni_attn_mask_lists_gfx950(const int64_t* spans_or_null, const i
   p.ticket = ticket;
   const hipStream_t s = static_cast<hipStream_t>(stream);
   if (const int rc = launch_classify(p, s)) return rc;
-  void* args[] = {&p};
-  if (const int rc = launched(hipLaunchKernel(reinterpret_cast<const void*>(mask_total_kernel), dim3(1), dim3(256), args, 0, s)))
-    return rc;
+  if (const int rc = launch_number(p, s)) return rc;
   return launch_write(p, nullptr, nullptr, s);
 }
 

@@ -406,7 +406,7 @@ _NATIVE_MASK_MAX_QB = 8192
 def _native_prefix_mask(source: Tensor, spans: bool, nheads: int, q_len: int, kv_len: int, QB: int, KB: int,
                         pack: bool) -> Optional[OmniBlockMask]:
     """Block mask of ``source`` ([B, M, 3] spans or [B, q_len] prefix lengths, on a GPU), built there by
-    two kernels; None for sizes outside their range (the tensor algebra below takes those)."""
+    two kernels (four where there are many query blocks); None for sizes outside their range (the tensor algebra below takes those)."""
     B, Tq, Tk = source.shape[0], -(-q_len // QB), -(-kv_len // KB)
     if min(B, nheads, q_len, kv_len) <= 0 or QB > _NATIVE_MASK_MAX_QB or B * Tq * Tk > 0x7fffffff:
         return None

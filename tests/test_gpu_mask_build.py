@@ -117,3 +117,64 @@ def test_room_for_another_number_of_tiles(two_launches, room, gpu_device):
     assert torch.equal(tiles[:written].cpu(), want.partial_block_masks[:written].to(torch.uint8))
     assert torch.equal(bits[:written], capi.pack_partial_masks(tiles[:written]))
     assert bool((tiles[written:] == 7).all()) and bool((bits[written:] == 7).all())
+
+
+@pytest.mark.parametrize("two_launches", [True, False])
+@pytest.mark.parametrize("B,S,QB", [(1, 100, 128), (1, 65 * 16, 16), (3, 16 * 341 - 3, 16), (16, 1024, 16), (9, 8191, 16)],
+                         ids=["1", "65", "1023", "1024", "4608"])
+def test_tiles_are_numbered_over_query_blocks(two_launches, B, S, QB, gpu_device):
+    """The C calls at numbers of query blocks on both sides of those that are summed up in place, with runs of query
+    blocks that have no tile, and room for a few tiles more than there are."""
+    import ctypes
+    import omni_attn_capi as capi
+    lib = capi.load_library()
+    lib.omni_attn_mask_workspace_bytes.restype = ctypes.c_size_t
+    H, KB = 2, 64
+    gen = torch.Generator().manual_seed(S)
+    spans = torch.zeros(B, 2, 3, dtype=torch.long)
+    cuts = torch.randint(0, S, (B, 2, 2), generator=gen)
+    spans[..., 1], spans[..., 2] = cuts.amin(-1), cuts.amax(-1) - cuts.amin(-1)
+    spans[::3] = 0
+    want = oat.create_omni_block_mask_from_modality_positions(spans, B, H, S, S, QB, KB, device="cpu")
+    tiles_wanted = want.partial_block_masks
+    n = 0 if tiles_wanted is None else tiles_wanted.shape[0]
+    Tq, Tk = want.kv_indices.shape[2:]
+    sp = spans.to(gpu_device)
+    i32 = lambda *shape: torch.empty(*shape, dtype=torch.int32, device=gpu_device)
+    nb, idx, tys, pidx = i32(B, H, Tq), i32(B, H, Tq, Tk), i32(B, H, Tq, Tk), i32(B, H, Tq, Tk)
+    ws = i32(lib.omni_attn_mask_workspace_bytes(B, S, S, QB, KB) // 4)
+    posted = torch.zeros(max(2, B * Tq), dtype=torch.int32, pin_memory=True)
+    room = min(n + 3, B * Tq * Tk)
+    tiles = torch.full((room, QB, KB), 7, dtype=torch.uint8, device=gpu_device)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    lists = (ptr(nb), ptr(idx), ptr(tys), ptr(pidx))
+    if two_launches:
+        assert lib.omni_attn_mask_classify_gfx950(ptr(sp), None, ptr(ws), ptr(posted), 5, B, 2, S, S, QB, KB, stream) == 0
+        assert lib.omni_attn_mask_finish_gfx950(*lists, ptr(ws), ptr(tiles), None, room, B, H, S, S, QB, KB, stream) == 0
+        torch.cuda.synchronize()
+        assert int((posted[:B * Tq] & 0xfffff).sum()) == n
+    else:
+        assert lib.omni_attn_mask_lists_gfx950(ptr(sp), None, *lists, ptr(ws), ptr(posted), 9, B, 2, H, S, S, QB, KB,
+                                               stream) == 0
+        assert lib.omni_attn_mask_tiles_gfx950(ptr(sp), None, ptr(ws), ptr(tiles), None, room, B, 2, H, S, S, QB, KB,
+                                               stream) == 0
+        torch.cuda.synchronize()
+        assert posted[:2].tolist() == [n, 9]
+    for got, ref in ((nb, want.kv_num_blocks), (idx, want.kv_indices), (tys, want.block_mask_types)):
+        assert torch.equal(got.cpu(), ref.to(torch.int32))
+    if n:
+        assert torch.equal(pidx.cpu(), want.partial_block_mask_indices)
+        assert torch.equal(tiles[:n].cpu(), tiles_wanted.to(torch.uint8))
+    else:
+        assert bool((pidx == -1).all())
+    assert bool((tiles[n:] == 7).all())
+
+
+@pytest.mark.parametrize("blocks", [512, 513])
+def test_counts_and_their_sum(blocks, gpu_device):
+    """As many query blocks as send a count each, and one more."""
+    spans = torch.tensor([[[1, 37, 900], [1, 2000, 1141], [1, 8000, 100]]])
+    args = (spans, 1, 3, blocks * 16, blocks * 16, 16, 128)
+    want = oat.create_omni_block_mask_from_modality_positions(*args, device="cpu")
+    same_mask(oat.create_omni_block_mask_from_modality_positions(*args, device=gpu_device), want)

@@ -216,10 +216,10 @@ int forward(const void* q, const void* k, const void* v, const omni_attn_strides
     p.slab_group = int(slabs);
     p.flat_first = p.n_slabs > H;  // batch elements may have masks of their own
   }
-  // One group anyway: where not all its workgroups start at once, and their lists are long against the load.
+  // One group anyway: where workgroups wait for a place or share one, and their lists are long against the load.
   // B=2 H=8 S=2500 D=128, one element unmasked, 75 -> 52 us; causal 38.65 -> 38.85.
   if (p.slab_group >= slabs && slabs > 1 && slabs <= 64 && p.n_slabs > H && S_pad >= 2048 &&
-      slabs * part_tiles > fwd_places(p.split, D, QB, topo.cus_per_xcd))
+      slabs * part_tiles > fwd_order_line(p.split, D, QB, topo.cus_per_xcd))
     p.flat_first = 1;
   p.softcap = softcap;
   p.cap_c2 = softcap > 0.f ? float(2.0 * 1.4426950408889634 / (std::sqrt(double(D)) * double(softcap))) : 0.f;

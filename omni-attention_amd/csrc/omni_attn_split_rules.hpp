@@ -14,11 +14,19 @@ enum class FwdSplit : int {
 constexpr int fwd_split_rows(FwdSplit s, int QB) {
   return s == FwdSplit::kNone ? QB : (s == FwdSplit::kRows32x4 ? 32 : (s == FwdSplit::kRows128x2 ? 128 : 64));
 }
-// Workgroups that an XCD has room for: eight waves per compute unit, and 160 KiB of LDS (four lone waves have
-// 136 KiB of tiles at head_dim 128).
-constexpr int fwd_places(FwdSplit s, int D, int QB, int cus) {
-  const bool whole = s == FwdSplit::kRows64x4 || s == FwdSplit::kRows128x2 || (s == FwdSplit::kRows32x4 && D == 128);
-  return whole ? cus : (s == FwdSplit::kNone && QB == 64 ? 4 * cus : 2 * cus);
+// Workgroups of an XCD from which on the longest lists of a batch's slabs go first (the caller says why).  With two waves
+// on every SIMD, the others wait for a place (head_dim 32 has registers for three; the second and the third share
+// the vector pipe all the same: B=3 H=5 S=2500, 64-row blocks, one element of three unmasked, 25.6 -> 26.2 us from the third).
+// Four lone waves at head_dim 128 take longest over a list, and one such workgroup beside another is what
+// a launch ends with: from the second workgroup of a compute unit (of two that fit), B=3 H=2 S=2048, one of
+// three unmasked, 22.8 -> 20.4 us, causal 19.04 -> 19.20, spans 19.26 -> 19.45.  Elsewhere that costs nearly as often: head_dim 64,
+// B=3 H=2 S=2304, 15.5 -> 13.8, causal 12.7 -> 12.95, spans 15.9 -> 16.1; B=3 H=4 S=2500 27.9 -> 27.9, 21.1 -> 21.4, 27.5 -> 27.7.
+constexpr int fwd_waves(FwdSplit s, int QB) {
+  const int groups = s == FwdSplit::kNone ? 1 : (s == FwdSplit::kRows32x4 || s == FwdSplit::kRows64x4 ? 4 : 2);
+  return fwd_split_rows(s, QB) / 32 * groups;
+}
+constexpr int fwd_order_line(FwdSplit s, int D, int QB, int cus) {
+  return s == FwdSplit::kRows32x4 && D == 128 ? cus : cus * (8 / fwd_waves(s, QB));
 }
 
 // Which split?  `rows32`: 32-row tiles of the whole launch, S: rows per slab; `busiest`: 128-row tiles dealt

@@ -91,3 +91,30 @@ int main() {
 """)
     subprocess.run(["g++", "-std=c++17", "-I", CSRC, str(source), "-o", str(program)], check=True)
     assert subprocess.run([str(program)]).returncode == 0
+
+
+def test_order_line_of_a_form(tmp_path):
+    """Workgroups from which on long lists go first: what two waves per SIMD make (one workgroup per compute unit for lone
+    waves at head_dim 128), and never more than the LDS holds: per group K and V rows of a step, twice unless the group
+    is one wave, and a mask byte per row and key."""
+    source, program = tmp_path / "line.cpp", tmp_path / "line"
+    source.write_text(r"""
+#include "omni_attn_split_rules.hpp"
+#include <cstdio>
+using namespace omni_attn;
+int main() {
+  for (int s = 0; s < 5; ++s)
+    for (int D = 32; D <= 128; D *= 2)
+      for (int QB = 64; QB <= 128; QB += 64) printf("%d %d %d %d\n", s, D, QB, fwd_order_line(FwdSplit(s), D, QB, 32));
+}
+""")
+    subprocess.run(["g++", "-std=c++17", "-I", CSRC, str(source), "-o", str(program)], check=True)
+    out = subprocess.run([str(program)], check=True, capture_output=True, text=True).stdout
+    for line in out.splitlines():
+        split, D, QB, workgroups = map(int, line.split())
+        rows, groups = [(QB, 1), (32, 4), (64, 2), (64, 4), (128, 2)][split]
+        step = 32 if D == 128 and rows != 128 else 64
+        tiles = groups * ((1 if rows == 32 else 2) * 2 * step * D * 2 + rows * step)
+        by_waves = 8 // (groups * rows // 32)
+        assert by_waves * tiles <= 160 * 1024, (split, D, QB)
+        assert workgroups == 32 * (1 if (split, D) == (1, 128) else by_waves), (split, D, QB)

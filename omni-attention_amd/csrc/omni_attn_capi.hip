@@ -86,18 +86,6 @@ int query_topology(DeviceTopology* out) {
 }  // namespace
 
 namespace {
-// Slabs are dealt to the XCDs round-robin.  Where their number leaves some XCDs with more than 6 % less
-// than others (4 slabs on 8 XCDs: half the device idle), each is dealt in parts of its tiles instead.
-int slab_parts(int n_slabs, int n_xcd) {
-  int parts = 1;
-  while (parts < n_xcd) {
-    const long long n = (long long)n_slabs * parts, most = (n + n_xcd - 1) / n_xcd;
-    if (most * n_xcd * 100 <= n * 106) break;
-    parts *= 2;
-  }
-  return parts;
-}
-
 // [B, H, S, D] contiguous.
 omni_attn_strides contiguous(int H, int S, int D) {
   return {int64_t(H) * S * D, int64_t(S) * D, D};
@@ -187,11 +175,11 @@ int forward(const void* q, const void* k, const void* v, const omni_attn_strides
   // than have their K and V in the XCD's L2 (4 MiB on MI355X) together, when at least two
   // do: a bigger group was 2 % faster still on 4096-token slabs and doubled the L2 misses.
   const int slots_per_xcd = topo.cus_per_xcd * (QB == 128 ? 2 : 4);
-  p.parts = slab_parts(p.n_slabs, X);
-  const long long busiest = ((long long)p.n_slabs * p.parts + X - 1) / X * ((Tq * QB / 128 + p.parts - 1) / p.parts);
+  const Dealing dealing = fwd_dealing(p.n_slabs, Tq * QB, X);
+  p.parts = dealing.parts;
   const long long rows32 = (long long)B * H * Tq * (QB / 32);
-  const bool even = 100 * 4 * busiest * X <= 106 * rows32;
-  p.split = fwd_choose_split(D, QB, rows32, Tq * QB, busiest, topo.cus_per_xcd, p.seqlen % QB != 0, even, B > 1);
+  p.split = fwd_choose_split(D, QB, rows32, Tq * QB, dealing.busiest, topo.cus_per_xcd, p.seqlen % QB != 0, dealing.even,
+                             B > 1);
   p.tiles = Tq * (QB / fwd_split_rows(p.split, QB));
   const int part_tiles = (p.tiles + p.parts - 1) / p.parts;
   const int fill = slots_per_xcd / part_tiles > 1 ? slots_per_xcd / part_tiles : 1;

@@ -3,6 +3,30 @@
 
 namespace omni_attn {
 
+// Slabs are dealt to the XCDs round-robin.  Where their number leaves some XCDs with more than 6 % less
+// than others (4 slabs on 8 XCDs: half the device idle), each is dealt in parts of its tiles instead.
+inline int slab_parts(int n_slabs, int n_xcd) {
+  int parts = 1;
+  while (parts < n_xcd) {
+    const long long n = (long long)n_slabs * parts, most = (n + n_xcd - 1) / n_xcd;
+    if (most * n_xcd * 100 <= n * 106) break;
+    parts *= 2;
+  }
+  return parts;
+}
+// ... and what that makes of slabs of S rows (a multiple of 64): the 128-row tiles of the XCD that has most, and
+// whether none has more than 6 % above the mean.
+struct Dealing {
+  int parts;
+  long long busiest;
+  bool even;
+};
+inline Dealing fwd_dealing(int n_slabs, int S, int n_xcd) {
+  const int parts = slab_parts(n_slabs, n_xcd);
+  const long long busiest = ((long long)n_slabs * parts + n_xcd - 1) / n_xcd * ((S / 128 + parts - 1) / parts);
+  return {parts, busiest, 100 * 4 * busiest * n_xcd <= 106 * ((long long)n_slabs * (S / 32))};
+}
+
 // How the walk of a query block is split over waves (FwdShape says what the numbers are).
 enum class FwdSplit : int {
   kNone,       // one workgroup per query block
@@ -168,10 +192,12 @@ enum class DkdvSplit : int {
 //          D=64   B H=16 S=1237 51-60 (-4 .. -15), soft-capped 68-77 (-10), B H=12 S=2048 71-81 (-4 .. -17), B H=20 S=2048
 //                 75-95 (0 .. -13); 64-key blocks 73-90 (-3 .. +9); beyond: B H=24 S=2048 78-106 (-2 .. +9), B H=12
 //                 S=4096 136-170 (-7 .. +6)
-//   dQ, D=64, lengths that end inside a block, where the forward is split for that: B H=24 S=2300 127-172 (-2 .. -5), B H=16
+//   dQ, D=64, lengths that end inside a block, where the forward is split for that if dealt evenly: B H=24 S=2300 127-172 (-2 .. -5), B H=16
 //          S=4500 248-317 (0 .. -5), soft-capped 437 (-10), 64-row blocks B H=32 S=1700 97-117 (-3 .. -13), B H=24 S=2300
 //          123-158 (-6 .. -10), B H=16 S=4500 258-327 (-3 .. -5); beyond: B H=40 S=1700 107-134 (-3 .. +4); D=128 gains
-//          nowhere: B H=32 S=1237 101-130 (0 .. +4), B H=24 S=1700 128-171 (-2 .. +4)
+//          nowhere: B H=32 S=1237 101-130 (0 .. +4), B H=24 S=1700 128-171 (-2 .. +4).  However the slabs
+//          are dealt, where the forward with 64-row blocks looks at that too: 64-row blocks with 7 - 17 % more on one XCD,
+//          B H=37 S=1300 90-111 (0 .. -4, one layout +1), B H=35 S=1400 83-102 (-4 .. -8), B H=28 S=1900 105-131 (-6 .. -11)
 //   dQ, D=64, soft-capped (three exponentials and a reciprocal per score: twice the vector work against a list's
 //          loads), lengths that end inside a block: B H=32 S=2300 188-237 (-1 .. -9), S=2500 212-366 (-1 .. -5), B H=24 S=3000
 //          242-356 (-2 .. -7), B H=20 S=4000 322-388 (-1 .. -9); beyond: S=3000 279-455 (0 .. -2), whole blocks B H=32

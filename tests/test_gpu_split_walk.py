@@ -149,9 +149,11 @@ def test_backward_of_slabs_walked_together_with_different_masks(H, S, gpu_device
 @pytest.mark.parametrize("D,B,H,S,copies,QB", [
     (128, 1, 2, 1160, 16, 128), (128, 1, 2, 1610, 12, 128), (128, 1, 1, 2700, 16, 128), (128, 3, 1, 1630, 8, 128),
     (64, 2, 1, 1500, 16, 128), (64, 1, 1, 4400, 16, 128), (32, 2, 1, 1300, 24, 128), (32, 1, 1, 2950, 32, 128),
-    (128, 1, 2, 1170, 16, 64), (128, 2, 1, 1500, 12, 64), (64, 2, 1, 1500, 12, 64), (32, 1, 2, 1900, 16, 64)])
+    (128, 1, 2, 1170, 16, 64), (128, 2, 1, 1500, 12, 64), (64, 2, 1, 1500, 12, 64), (32, 1, 2, 1900, 16, 64),
+    (32, 2, 1, 1300, 20, 128), (64, 1, 1, 1300, 37, 64)])
 def test_lengths_that_end_inside_a_block(D, B, H, S, copies, QB, gpu_device):
-    """Launches that are split because of such a length: 64- and 128-row groups, dQ in 64-row groups at head_dim 64.
+    """Launches that are split because of such a length: 64- and 128-row groups, dQ in 64-row groups at head_dim 32 and 64
+    (the test of the rules holds which is which).
     The slabs of a batch element are repeated; the first ones against the oracle, the copies bit for bit."""
     from test_gpu_backward import check_grads, run_fwd_bwd
     from oracle.dense_oracle import attention_dense_grads

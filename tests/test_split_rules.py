@@ -118,3 +118,66 @@ int main() {
         by_waves = 8 // (groups * rows // 32)
         assert by_waves * tiles <= 160 * 1024, (split, D, QB)
         assert workgroups == 32 * (1 if (split, D) == (1, 128) else by_waves), (split, D, QB)
+
+
+# The launches of tests/test_gpu_split_walk.py's test of lengths that end inside a block: D, B, slabs per element, S, block,
+# and the splits that it runs: of the forward, and of dQ (0 none, 2 and 4: 64- and 128-row groups).  The launch without
+# any is one that the rule leaves whole.
+RAGGED_LAUNCHES = [
+    (128, 1, 32, 1160, 128, 2, 0), (128, 1, 24, 1610, 128, 4, 0), (128, 1, 16, 2700, 128, 4, 0),
+    (128, 3, 8, 1630, 128, 2, 0), (64, 2, 16, 1500, 128, 2, 2), (64, 1, 16, 4400, 128, 2, 2), (32, 2, 24, 1300, 128, 0, 0),
+    (32, 2, 20, 1300, 128, 2, 0), (64, 1, 37, 1300, 64, 0, 2), (32, 1, 32, 2950, 128, 2, 2), (128, 1, 32, 1170, 64, 2, 0),
+    (128, 2, 12, 1500, 64, 2, 0), (64, 2, 12, 1500, 64, 2, 2), (32, 1, 32, 1900, 64, 2, 2)]
+
+
+def test_dealing_and_the_rules_that_look_at_it(tmp_path):
+    """Uneven launches and soft-capped ones: what is split for a length that fills its blocks stays split; with 64-row
+    blocks the forward is split for a length inside a block in even launches only, dQ in both (and where the even forward is);
+    soft-capped dQ wherever the plain one is.  And the launches that a GPU test runs for their split have it."""
+    source, program = tmp_path / "dealing.cpp", tmp_path / "dealing"
+    launches = ",".join("{%s}" % ",".join(map(str, l)) for l in RAGGED_LAUNCHES)
+    source.write_text(r"""
+#include "omni_attn_split_rules.hpp"
+#include <cstdio>
+using namespace omni_attn;
+int main() {
+  const FwdSplit none = FwdSplit::kNone;
+  bool uneven_dq = false;
+  for (int D = 32; D <= 128; D *= 2)
+    for (int QB = 64; QB <= 128; QB += 64)
+      for (int S = QB; S <= 8192; S += QB)
+        for (int slabs = 1; slabs <= 96; ++slabs)
+          for (int batched = 0; batched < 2; ++batched) {
+            const Dealing d = fwd_dealing(slabs, S, 8);
+            const long long rows = (long long)slabs * (S / 32);
+            const FwdSplit whole = fwd_choose_split(D, QB, rows, S, d.busiest, 32, false, d.even, batched);
+            const FwdSplit ragged = fwd_choose_split(D, QB, rows, S, d.busiest, 32, true, d.even, batched);
+            const FwdSplit if_even = fwd_choose_split(D, QB, rows, S, d.busiest, 32, true, true, batched);
+            if (whole != none && whole != ragged) return 1;
+            if (QB == 64 && !d.even && ragged != whole) return 2;
+            const FwdSplit dq = bwd_choose_dq_split(D, QB, rows, S, true, batched, false);
+            if (bwd_choose_dq_split(D, QB, rows, S) != none && dq == none) return 3;
+            if (D == 64 && if_even != none && whole == none && dq != FwdSplit::kRows64x2) return 4;
+            if (dq != none && bwd_choose_dq_split(D, QB, rows, S, true, batched, true) == none) return 5;
+            if (D == 64 && QB == 64 && !d.even && ragged == none && dq != none && bwd_choose_dq_split(D, QB, rows, S) == none)
+              uneven_dq = true;
+          }
+  if (!uneven_dq) return 6;
+  const int launches[][7] = {""" + launches + r"""};
+  for (const auto& l : launches) {
+    const int D = l[0], slabs = l[1] * l[2], QB = l[4], S = (l[3] + QB - 1) / QB * QB;
+    const Dealing d = fwd_dealing(slabs, S, 8);
+    const long long rows = (long long)slabs * (S / 32);
+    const int f = int(fwd_choose_split(D, QB, rows, S, d.busiest, 32, true, d.even, l[1] > 1));
+    const int q = int(bwd_choose_dq_split(D, QB, rows, S, true, l[1] > 1));
+    const int f0 = int(fwd_choose_split(D, QB, rows, S, d.busiest, 32, false, d.even, l[1] > 1));
+    if (f != l[5] || q != l[6] || f0 != 0) {
+      printf("D=%d slabs=%d S=%d: %d %d, without the length %d\n", D, slabs, l[3], f, q, f0);
+      return 7;
+    }
+  }
+}
+""")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I", CSRC, str(source), "-o", str(program)], check=True)
+    run = subprocess.run([str(program)], capture_output=True, text=True)
+    assert run.returncode == 0, (run.returncode, run.stdout)

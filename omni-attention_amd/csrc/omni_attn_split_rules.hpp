@@ -92,7 +92,8 @@ constexpr int fwd_order_line(FwdSplit s, int D, int QB, int cus) {
 // attend everything, and a launch of many long lists is bound by K/V loads.  Whole blocks, us, and the split against
 // them, causal, two layouts of spans and images, then "mixed" (such a batch):
 //   D=128  one batch element
-//          kRows64x2   B H=32 S=1153 25-30 (-17 .. +3 %), S=1237 25-30 (-8 .. -10); beyond: S=1400 28-34 (-10 .. +16),
+//          kRows64x2   B H=32 S=1153 22-32 (-10 .. -15 %; the layouts with most work, one in four, +5), S=1237 and
+//                      S=1270 28-32 (-3 .. -9; one in four, +4); beyond: S=1400 28-34 (-10 .. +16),
 //                      B H=40 S=1000 22-26 (-15 .. +20), uneven B H=36 S=1100 24-29 (-9 .. +13)
 //          kRows128x2  B H=24 S=1600 31-38 (-1 .. -19), S=1900 37-43 (-2 .. -17), B H=20 S=2100 39-48 (-8 .. -18), B H=16
 //                      S=2600 47-58 (-11 .. -23), S=3700 70-89 (-18 .. +1); beyond: B H=24 S=2100 42-50 (-5 .. +10), B H=16

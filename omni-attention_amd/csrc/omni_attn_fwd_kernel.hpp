@@ -921,6 +921,9 @@ __device__ __forceinline__ void fwd_walk(const FwdParams& p) {
   auto look_again = [&]() { return __builtin_amdgcn_ballot_w64(m_run == -INFINITY) != 0 ? kOwesLook : 0u; };
   auto look = [&](auto set_c) {
     const float m_cand = step_max(set_c);
+    // (a step that allows nothing, a MASKED slot say, leaves the look to the next one and changes no bits; groups that
+    // share a list have no such slots)
+    if (KG == 1 && __builtin_amdgcn_ballot_w64(m_cand != -INFINITY) == 0) return;
     owed = 0;
     if (__builtin_amdgcn_ballot_w64(m_cand > m_run + kSlack) != 0) {
       alpha_pending = set_reference(vmax(m_run, m_cand));

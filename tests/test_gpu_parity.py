@@ -349,6 +349,32 @@ def test_scores_that_outgrow_the_reference(dtype, D, QB, KB, H, S, gpu_device):
     assert ((l32 - rl)[live].abs() / rl[live].abs().clamp(min=1.0)).max().item() <= TOL_LSE
 
 
+@pytest.mark.parametrize("D,QB,KB", [(32, 128, 128), (64, 64, 128), (64, 128, 128), (128, 64, 64), (128, 128, 64)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+def test_masked_slots_change_no_bits(dtype, D, QB, KB, gpu_device):
+    """One workgroup per query block, scores that grow from step to step: a list and the same list with MASKED slots
+    between its blocks give the same bits, also where a slot follows a step whose weights have outgrown their reference."""
+    H, S = 70, 1024
+    gen = torch.Generator().manual_seed(D + QB)
+    q = (1.0 + 0.05 * torch.randn(1, H, S, D, generator=gen)).to(dtype)
+    k = 0.2 * torch.randn(1, H, S, D, generator=gen)
+    # (log2 of the weights, a level per 64 keys: one that grows past 2^6, then little more, is what a look moves)
+    jumps = torch.tensor([0.4, 0.8, 5.5, 6.3, 7.0, 9.0, -0.5])
+    level = jumps[torch.randint(len(jumps), (H, S // 64), generator=gen)].cumsum(1)
+    k = (k + (level.repeat_interleave(64, 1) / (1.4427 * D ** 0.5)).view(1, H, S, 1)).to(dtype)
+    v = torch.randn(1, H, S, D, generator=gen).to(dtype)
+    Tq, Tk = S // QB, S // KB
+    nb = torch.full((1, H, Tq), Tk, dtype=torch.int32)
+    idx = torch.arange(Tk, dtype=torch.int32).expand(1, H, Tq, Tk).contiguous()
+    tys = torch.full((1, H, Tq, Tk), 2, dtype=torch.int32)
+    want = run_kernel(q, k, v, nb, idx, tys, QB, KB, S - 13, device=gpu_device)
+    between = torch.zeros_like(tys)
+    idx2 = torch.stack((idx, torch.randint(Tk, idx.shape, generator=gen, dtype=torch.int32)), -1).flatten(-2)
+    tys2 = torch.stack((tys, between), -1).flatten(-2)
+    got = run_kernel(q, k, v, 2 * nb, idx2, tys2, QB, KB, S - 13, device=gpu_device)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
 def sparse_rows_bf16_case():
     """B=2 H=9 S=1152 D=128 128/128 bf16, standard-normal operands, 80 % of the blocks left out
     and shuffled lists: many rows attend one, two or a handful of keys, so outputs are single V

@@ -10,13 +10,12 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
-#include <cstring>
-#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <vector>
 
 #include "omni_attn_gfx950.h"
+#include "omni_attn_host_counts.hpp"
 
 namespace {
 
@@ -298,95 +297,29 @@ void omni_attn_backward(torch::Tensor Q, torch::Tensor K, torch::Tensor V, torch
   }
 }
 
-// Where the workgroups of a kernel write a count each that the host waits for, as words of a tag and the count:
-// pinned host memory, handed out per call (so calls of several threads and streams do not meet) and taken
-// back; at most kKeep pieces of kWords words are kept between calls.
-class HostCounts {
- public:
-  // (a word per query block costs the host 10 ns and more; their sum costs two launches more.  A call, us, with words /
-  // with their sum: 512 query blocks 33 / 31, 1024 35 / 34, 2048 62 / 41, 4096 98 / 54)
-  static constexpr int kWords = 512;
-  HostCounts() {
-    std::lock_guard<std::mutex> lock(mutex());
-    if (!spare().empty()) {
-      words_ = spare().back();
-      spare().pop_back();
-      return;
-    }
+struct PinnedWords {
+  typedef hipStream_t Stream;
+  static void* allocate(size_t bytes) {
     void* mem = nullptr;
     // (portable: memory taken under one device is handed to calls on any)
-    const hipError_t e = hipHostMalloc(&mem, size_t(kWords + 16) * 4, hipHostMallocPortable | hipHostMallocMapped);
+    const hipError_t e = hipHostMalloc(&mem, bytes, hipHostMallocPortable | hipHostMallocMapped);
     if (e != hipSuccess) throw std::runtime_error(std::string("omni_attn: hipHostMalloc: ") + hipGetErrorString(e));
-    words_ = static_cast<uint32_t*>(mem);
-    std::memset(words_, 0, size_t(kWords + 16) * 4);
+    return mem;
   }
-  ~HostCounts() {
-    if (!idle_) return;  // a kernel may still write it: the memory stays allocated
-    std::lock_guard<std::mutex> lock(mutex());
-    if (spare().size() < kKeep) {
-      spare().push_back(words_);
-    } else {
-      (void)hipHostFree(words_);
-    }
+  static void release(void* memory) { (void)hipHostFree(memory); }
+  static bool running(hipStream_t stream) {
+    const hipError_t e = hipStreamQuery(stream);
+    if (e != hipSuccess && e != hipErrorNotReady)
+      throw std::runtime_error(std::string("omni_attn: the mask was not built: ") + hipGetErrorString(e));
+    return e == hipErrorNotReady;
   }
-  HostCounts(const HostCounts&) = delete;
-  HostCounts& operator=(const HostCounts&) = delete;
-
-  uint32_t* memory() { return words_; }
-  // A tag that no word has: they are cleared where the tags begin again.
-  int next_tag() {
-    uint32_t& last = words_[kWords];
-    if (last == (1u << (32 - kCountBits)) - 1) {
-      std::memset(words_, 0, size_t(kWords) * 4);
-      last = 0;
-    }
-    idle_ = false;
-    return int(++last);
+  static bool drain(hipStream_t stream) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone &&
+           hipStreamSynchronize(stream) == hipSuccess;
   }
-  // The sum of the first n counts, once the kernel that writes them has run.
-  int64_t wait(int tag, int n, hipStream_t stream) {
-    int64_t sum = 0;
-    for (int i = 0; i < n; ++i) sum += wait_for(i, tag, stream) & ((1u << kCountBits) - 1);
-    idle_ = true;
-    return sum;
-  }
-  // A number of any size in word 0, written before the tag in word 1.
-  int32_t wait_total(int tag, hipStream_t stream) {
-    (void)wait_for(1, tag, stream);
-    idle_ = true;
-    const int32_t total = int32_t(words_[0]);
-    words_[0] = words_[1] = 0;
-    return total;
-  }
-  static int word_of(int tag) { return int(uint32_t(tag) << kCountBits); }
-
- private:
-  // Ends as well when the stream has nothing left to run or reports an error.
-  uint32_t wait_for(int i, int tag, hipStream_t stream) {
-    for (unsigned spins = 1;; ++spins) {
-      const uint32_t x = __atomic_load_n(words_ + i, __ATOMIC_ACQUIRE);
-      if (int(x >> kCountBits) == tag) return x;
-      if (spins % 8192 == 0) {
-        const hipError_t e = hipStreamQuery(stream);
-        if (e == hipErrorNotReady) continue;
-        if (e == hipSuccess && int(__atomic_load_n(words_ + i, __ATOMIC_ACQUIRE) >> kCountBits) == tag) continue;
-        throw std::runtime_error(std::string("omni_attn: the mask was not built: ") + hipGetErrorString(e));
-      }
-    }
-  }
-  static constexpr int kCountBits = OMNI_ATTN_MASK_POSTED_COUNT_BITS;
-  static constexpr size_t kKeep = 16;
-  static std::mutex& mutex() {
-    static std::mutex* m = new std::mutex;
-    return *m;
-  }
-  static std::vector<uint32_t*>& spare() {
-    static std::vector<uint32_t*>* v = new std::vector<uint32_t*>;
-    return *v;
-  }
-  uint32_t* words_ = nullptr;  // kWords counts; the last tag
-  bool idle_ = true;
 };
+typedef omni_attn::HostCounts<PinnedWords, OMNI_ATTN_MASK_POSTED_COUNT_BITS> HostCounts;
 
 // ---- the operator as one call -----------------------------------------------------------------
 // What the wrappers of omni_attn_torch.py do per call, in one native call: look the operands and the
@@ -662,14 +595,14 @@ pybind11::tuple omni_attn_build_prefix_mask(torch::Tensor source, bool spans, in
   {
     py::gil_scoped_release release;
     HostCounts counts;
-    const int tag = counts.next_tag();
+    const int tag = counts.next_tag(stream);
     if (B * Tq <= HostCounts::kWords && (Tk >> OMNI_ATTN_MASK_POSTED_COUNT_BITS) == 0) {
       // The first kernel needs the workspace only, and sends its counts as they are known: the lists are allocated
       // while it runs.
       refuse(omni_attn_mask_classify_gfx950(sp, prefix, ws, counts.memory(), tag, int(B), int(M), int(q_len), int(kv_len),
                                             int(QB), int(KB), at));
       allocate_lists();
-      allocate_tiles(counts.wait(tag, int(B * Tq), stream));
+      allocate_tiles(counts.wait(tag, int(B * Tq)));
       refuse(omni_attn_mask_finish_gfx950(nb.data_ptr<int32_t>(), idx.data_ptr<int32_t>(), types.data_ptr<int32_t>(),
                                           pidx.data_ptr<int32_t>(), ws, tile_bytes(), tile_words(),
                                           tiles.defined() ? int(tiles.size(0)) : 0, int(B), int(H), int(q_len),
@@ -680,7 +613,7 @@ pybind11::tuple omni_attn_build_prefix_mask(torch::Tensor source, bool spans, in
                                          types.data_ptr<int32_t>(), pidx.data_ptr<int32_t>(), ws,
                                          reinterpret_cast<int32_t*>(counts.memory()), HostCounts::word_of(tag), int(B),
                                          int(M), int(H), int(q_len), int(kv_len), int(QB), int(KB), at));
-      allocate_tiles(counts.wait_total(tag, stream));
+      allocate_tiles(counts.wait_total(tag));
       if (tiles.defined())
         refuse(omni_attn_mask_tiles_gfx950(sp, prefix, ws, tile_bytes(), tile_words(), int(tiles.size(0)), int(B), int(M),
                                            int(H), int(q_len), int(kv_len), int(QB), int(KB), at));

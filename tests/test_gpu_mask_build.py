@@ -178,3 +178,14 @@ def test_counts_and_their_sum(blocks, gpu_device):
     args = (spans, 1, 3, blocks * 16, blocks * 16, 16, 128)
     want = oat.create_omni_block_mask_from_modality_positions(*args, device="cpu")
     same_mask(oat.create_omni_block_mask_from_modality_positions(*args, device=gpu_device), want)
+
+
+def test_lists_that_do_not_fit(gpu_device):
+    """A call that finds no memory for its lists, while its first kernel runs, ends with torch's own error, and the next ones
+    are whole."""
+    spans = torch.tensor([[[1, 37, 900], [1, 2000, 1141]]])
+    want = oat.create_omni_block_mask_from_modality_positions(spans, 1, 2, 8192, 8192, 128, 128, device="cpu")
+    for _ in range(3):
+        with pytest.raises(torch.OutOfMemoryError):
+            oat.create_omni_block_mask_from_modality_positions(spans, 1, 20_000_000, 8192, 8192, 128, 128, device=gpu_device)
+        same_mask(oat.create_omni_block_mask_from_modality_positions(spans, 1, 2, 8192, 8192, 128, 128, device=gpu_device), want)

@@ -37,13 +37,14 @@
 // for the rows inside the sequence runs as an unmasked one: where the length is no multiple of the block, every block of
 // the last list is PARTIAL.  (Requested by the step that uses them, a memory latency each, and always applied:
 // forward and backward, us, before -> now, B=1 H=8 S=3000 D=128 images 230 -> 196, B=4 H=8 S=1157 D=64 85 -> 72,
-// soft-capped 95 -> 86, of which 4 from two vector instructions less per capped weight and masks only where needed.)
+// soft-capped 95 -> 86.)
 // Workgroups are dealt to the XCDs by slab, so the workgroups that run together on an XCD share
 // their operands through its L2.
 #pragma once
 
 #include "omni_attn_bwd_plan.hpp"
 #include "omni_attn_fwd_kernel.hpp"
+#include "omni_attn_softcap.hpp"
 
 namespace omni_attn {
 
@@ -63,7 +64,7 @@ struct BwdParams {
   // workspace [2][B,H,S], written by the dQ kernel and read by the dK/dV kernel: plane 0 is
   // -delta = -rowsum(dO . O); plane 1 the offset of the row's scores, -LSE * sqrt(D), -inf for a
   // row without any allowed key or beyond the sequence (every weight of such a row becomes 0) --
-  // or, in the soft-capped instances, the exponent offset (cap - LSE) * log2(e), -inf for such a row
+  // or, in the soft-capped instances, the exponent offset -LSE * log2(e), -inf for such a row
   float* ws;
   const int32_t* kv_num_blocks;
   const int32_t* kv_indices;
@@ -103,11 +104,6 @@ __device__ __forceinline__ const __attribute__((address_space(4))) BwdParams& pa
   return *at;
 }
 
-// Soft-capped scores: with r = 1 / (exp(2 s / sqrt(D) / cap) + 1) the capped score is cap (1 - 2 r), its
-// derivative 4 r (1 - r).  A weight is exp2(off - 2 cap log2(e) r), off = cap log2(e) - lse log2(e).
-__device__ __forceinline__ float capped_r(float s, const BwdParams& p) {
-  return __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(s * p.cap_c2) + 1.f);
-}
 // Pair of 16-bit values of registers r, r + 1, zero where the mask word (shifted by 4 g) forbids them.
 template <int R>
 __device__ __forceinline__ uint32_t keep_pair(uint32_t pair, uint32_t kw) {
@@ -429,7 +425,7 @@ __device__ __forceinline__ void bwd_dq_walk(const BwdParams& p) {
   // The dK/dV kernel, too, starts the accumulator of a row's scores at -LSE * sqrt(D), so that the
   // exponent of a weight is the score times log2(e) / sqrt(D) and nothing else.  A soft-capped score is not
   // linear in the product: there it is the offset of the exponent itself.
-  const float row_start = !row_live ? -INFINITY : (CAP ? __builtin_fmaf(lse, -1.4426950408889634f, p.cap_l2) : -lse * SqrtOf<D>::value);
+  const float row_start = !row_live ? -INFINITY : (CAP ? lse * -1.4426950408889634f : -lse * SqrtOf<D>::value);
   if (q_row < p.S && g == 0 && kg == 0) {
     p.ws[size_t(bh) * p.S + q_row] = -delta;
     p.ws[size_t(p.n_slabs) * p.S + size_t(bh) * p.S + q_row] = row_start;
@@ -501,8 +497,6 @@ __device__ __forceinline__ void bwd_dq_walk(const BwdParams& p) {
   constexpr int NTR = 2 * DT;                    // last products of a half
   constexpr int NS = NSUB * (2 * KS + NTR);      // slots of a step
   constexpr int PF = D == 128 ? 2 : 3;           // operand fetch distance in slots (registers are tight at 128)
-  // (capped: the derivative's factor 4 comes with the exponent)
-  const float row_off = CAP ? row_start + 2.f : row_start;
   const float neg_delta = -delta;
   auto compute = [&](int set, const uint32_t (&kw)[NTL], bool masked) {
     const uint32_t base = lds_tiles + uint32_t(set) * (2u * TILE * 2u);
@@ -529,9 +523,9 @@ __device__ __forceinline__ void bwd_dq_walk(const BwdParams& p) {
       constexpr int u = decltype(uc)::value, r = decltype(rc)::value;
       float w0, w1;
       if constexpr (CAP) {
-        const float r0 = capped_r(st[u][r], p), r1 = capped_r(st[u][r + 1], p);
-        w0 = __builtin_amdgcn_exp2f(__builtin_fmaf(r0, -2.f * p.cap_l2, row_off)) * __builtin_fmaf(-r0, r0, r0);
-        w1 = __builtin_amdgcn_exp2f(__builtin_fmaf(r1, -2.f * p.cap_l2, row_off)) * __builtin_fmaf(-r1, r1, r1);
+        const float d0 = capped_d(st[u][r], p.cap_c2), d1 = capped_d(st[u][r + 1], p.cap_c2), t0 = 1.f - d0, t1 = 1.f - d1;
+        w0 = __builtin_amdgcn_exp2f(capped_exponent(t0, p.cap_l2, row_start)) * capped_slope(d0, t0);
+        w1 = __builtin_amdgcn_exp2f(capped_exponent(t1, p.cap_l2, row_start)) * capped_slope(d1, t1);
       } else {
         w0 = __builtin_amdgcn_exp2f(st[u][r] * p.sl2);
         w1 = __builtin_amdgcn_exp2f(st[u][r + 1] * p.sl2);
@@ -552,7 +546,7 @@ __device__ __forceinline__ void bwd_dq_walk(const BwdParams& p) {
         if constexpr (sl == 0) {
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            st[ch][r] = CAP ? 0.f : row_off;
+            st[ch][r] = CAP ? 0.f : row_start;
             dp[ch][r] = neg_delta;
           }
           if constexpr (!CAP) {
@@ -1085,10 +1079,10 @@ __device__ __forceinline__ void bwd_dkdv_walk(const BwdParams& p) {
         float w0, w1;
         if constexpr (CAP) {
           if constexpr ((r & 3) == 0) lq = row_offsets(u, r >> 2);
-          const float r0 = capped_r(sc[u][r], p), r1 = capped_r(sc[u][r + 1], p), r04 = 4.f * r0, r14 = 4.f * r1;
-          w0 = __builtin_amdgcn_exp2f(__builtin_fmaf(r0, -2.f * p.cap_l2, lq[r & 3]));
-          w1 = __builtin_amdgcn_exp2f(__builtin_fmaf(r1, -2.f * p.cap_l2, lq[(r + 1) & 3]));
-          hb[u][r >> 3][(r & 7) >> 1] = pack2<BF16>(w0 * __builtin_fmaf(-r04, r0, r04), w1 * __builtin_fmaf(-r14, r1, r14));
+          const float d0 = capped_d(sc[u][r], p.cap_c2), d1 = capped_d(sc[u][r + 1], p.cap_c2), t0 = 1.f - d0, t1 = 1.f - d1;
+          w0 = __builtin_amdgcn_exp2f(capped_exponent(t0, p.cap_l2, lq[r & 3]));
+          w1 = __builtin_amdgcn_exp2f(capped_exponent(t1, p.cap_l2, lq[(r + 1) & 3]));
+          hb[u][r >> 3][(r & 7) >> 1] = pack2<BF16>(w0 * capped_slope(d0, t0), w1 * capped_slope(d1, t1));
         } else {  // the scores already carry their row's offset and the mask
           w0 = __builtin_amdgcn_exp2f(sc[u][r] * p.sl2);
           w1 = __builtin_amdgcn_exp2f(sc[u][r + 1] * p.sl2);

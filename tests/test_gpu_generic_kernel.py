@@ -73,7 +73,8 @@ def test_simple_wrapper_takes_shapes_the_other_wrappers_refuse(gpu_device):
 
 
 @pytest.mark.parametrize("QB,KB,D", [(16, 16, 5), (48, 48, 8), (33, 7, 13), (32, 32, 31), (40, 40, 33), (64, 48, 100),
-                                     (16, 32, 129), (128, 128, 161), (32, 64, 224), (48, 16, 250)])
+                                     (16, 32, 129), (128, 128, 161), (32, 64, 224), (48, 16, 250), (16, 16, 193),
+                                     (32, 64, 217)])
 def test_generic_kernel_edges_of_tiles_and_chunks(QB, KB, D, gpu_device):
     """Head dimensions around the 8-column chunks and 32-column tiles, key blocks that do not fill or
     that straddle a 32-key step, query blocks of a fraction of a 32-row tile.  Tighter than the bars:

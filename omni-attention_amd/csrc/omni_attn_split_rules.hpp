@@ -84,7 +84,8 @@ constexpr int fwd_order_line(FwdSplit s, int D, int QB, int cus) {
 //                      B H=20 S=2048 31-34 (-6 .. -24), B H=16 S=3072 45-49 (-8 .. -23), S=4096 60-65 (-8 .. +3);
 //                      beyond: B H=40 S=1024 18-20 (0 .. +19), B H=24 S=2048 32-34 (-10 .. +16)
 //   D=32   kRows32x4   against kRows64x2: B H=16 S=1237 11-16 (-17 .. -29), B H=6 S=4096 25-27 (-17 .. -26); beyond: B H=8
-//                      S=4096 25-27 (-3 .. +7)
+//                      S=4096 25-27 (-3 .. +7).  (Sparse lists of a single block each take longer so: B H=16 S=1152
+//                      5.7 -> 6.2, of half the blocks 9.6 -> 7.8.)
 //          kRows64x2   B H=40 S=1024 16-18 (-3 .. -16), B H=32 S=1536 21-24 (-10 .. -21), S=2048 28-33 (-14 .. +1)
 // `ragged`: the sequence ends inside a query block.  With PARTIAL tiles every block of that list is one then (its last
 // rows attend nothing): the longest list of a slab also has the slowest steps, and sharing it gains in larger

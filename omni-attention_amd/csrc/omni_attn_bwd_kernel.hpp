@@ -709,9 +709,17 @@ __device__ __forceinline__ void bwd_dq_walk(const BwdParams& p) {
   bwd_store_rows<BF16, D>(dq, p.scale, stage, p.dq + slab, q_wave_min, p.S, lane_out);
 }
 
+// One workgroup per query block, all steps in one group.  A 64-row block is two waves.  At head_dim 128 its tiles of 64 keys
+// take 68 KiB of LDS: two workgroups, four waves, on a compute unit, one wave per SIMD.  With 32 keys four workgroups
+// fit, and the second wave of a SIMD is worth more than halves that overlap inside one: both backward kernels,
+// us, 64 -> 32 keys, causal B H=128 S=4096 fp16 2351 -> 2089, spans bf16 2744 -> 2446, interleaved B H=64 128-key
+// blocks soft-capped 1485 -> 1288, images B H=48 S=2000 272 -> 262.  (The sums are formed in the same order: the same bits.)
+template <bool BF16, bool CAP, int D, int QB, int KB>
+using BwdDqBlockShape = BwdDqShape<BF16, CAP, D, QB, KB, QB, 1, (QB == 64 && D == 128) ? 32 : 64>;
+
 template <bool BF16, bool CAP, int D, int QB, int KB>
 __global__ void __launch_bounds__(QB * 2, 2) bwd_dq_kernel(const BwdParams p) {
-  bwd_dq_walk<BwdDqShape<BF16, CAP, D, QB, KB, QB, 1, 64>>(p);
+  bwd_dq_walk<BwdDqBlockShape<BF16, CAP, D, QB, KB>>(p);
 }
 // The steps of a list shared by the groups of a workgroup (fwd_choose_split says when).
 template <bool BF16, bool CAP, int D, int QT, int KG, int STEP>
@@ -1396,7 +1404,7 @@ int launch_bwd_kernel(const BwdParams& p, int tiles, int threads, size_t lds, si
 
 template <bool BF16, bool CAP, int D, int QB, int KB>
 int launch_dq(const BwdParams& p, hipStream_t stream) {
-  using Shape = BwdDqShape<BF16, CAP, D, QB, KB, QB, 1, 64>;
+  using Shape = BwdDqBlockShape<BF16, CAP, D, QB, KB>;
   return launch_bwd_kernel<bwd_dq_kernel<BF16, CAP, D, QB, KB>>(p, p.Tq, Shape::kThreads, Shape::kLdsBytes,
                                                                 Shape::kLdsBytes, stream);
 }

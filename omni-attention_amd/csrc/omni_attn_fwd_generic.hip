@@ -24,13 +24,13 @@
 // a wave whose sums end up infinite or NaN walks its list once more and leaves out the zero weights.
 //
 // Bound by the instructions of a step (softmax, split of the weights and bookkeeping on the vector pipe: about 3000
-// cycles of a wave against 770 of its products at D=96) times the steps of the longest list over the waves; from 192
-// columns on by LDS (a step of 32 rows reads each K and V byte once for 32 query rows).  So rows that go to LDS directly
-// have their offsets laid out once, their fragments are fetched in groups (K, and V under the weights), and a
-// weight's part is taken off without being converted first.  B=1 H=8 S=2048 D=96, causal in 32x32 blocks, launches back
-// to back: fp16 25.7 us, bf16 23.3 (28.7 and 26.9 without); S=1500 B=1 H=4, 64x64: D=160 30.9 (35.0), D=200 40.7
-// (46.1); D=95, rows at any alignment, 42.5.  33 us (37) at D=96 where queries are four times as large (every row peaked,
-// a rest in most steps).  Two parts per weight, cut off after 22 bits and at 2^-32 of the reference, gain 2 us, but are
+// cycles of a wave against 770 of its products at D=96) times the steps of the longest list over the waves.  So rows
+// that go to LDS directly have their offsets laid out once, their fragments are fetched in groups (K, and V under the
+// weights; three ahead beyond 128 columns), and a weight's part is taken off without being converted first.  B=1 H=8
+// S=2048 D=96, causal in 32x32 blocks, launches back to back: fp16 24.4 us, bf16 23.0 (28.7 and 26.9 without); spans in
+// 64x64 blocks at B=1 H=4 S=1500: D=136 21.6, D=208 26.3, D=256 29.6; rows at any alignment, D=101 34.7, D=165 40.3.
+// 33 us (37) at D=96 where queries are four times as large (every row peaked, a rest in most steps).  Two parts per
+// weight, cut off after 22 bits and at 2^-32 of the reference, gain 2 us, but are
 // not the scalar kernel's sum.  One wave per row with vector arithmetic: 1934 us.
 #include "../../include/omni_attn_gfx950.h"
 
@@ -99,7 +99,12 @@ __device__ __forceinline__ int chunk_start(int d0, int D) { return d0 + 8 <= D ?
 
 // How rows are read: straight to LDS (rows of k and v on 16-byte boundaries, D a multiple of 8), by
 // 16-byte loads at any alignment, or element by element (head dimensions below 8).
-enum class Rows : int { kDirect, kWide, kSmall };
+// A step straight to LDS is two halves of 16 keys.  kWhole (blocks of 32 n keys) has both in one block, kHalves (16 n keys)
+// each in one: what a step needs to know (first key row, mode, tile) is one or two sets of scalars, and the offsets of
+// 16 rows are laid out once.  kKeys takes other block sizes: every key is followed by a lane of its own.  B=1 H=8, us,
+// 16 n keys by key -> in halves: S=715 48x48 spans D=40 11.3 -> 10.0, D=96 14.1 -> 11.4; S=2048 causal D=96 48x48
+// 37.0 -> 33.4, 16x16 49.7 -> 45.3; 32x32, one kernel for all -> kWhole, bf16 23.5 -> 23.0, fp16 24.5 -> 24.4.
+enum class Rows : int { kWhole, kWide, kSmall, kHalves, kKeys };
 
 // The chunk of `row` at column d0 (kSmall: zeros behind the row).
 template <Rows R>
@@ -217,20 +222,32 @@ template <int DT, int NW>
 struct GenericTraits {
   static constexpr int kRowBytes = 64 * DT;
   static constexpr int kTileBytes = 32 * kRowBytes;
-  static constexpr int kGroup = DT < NW ? DT : NW;  // output tiles merged per pass
+  // Beyond 128 columns LDS has room for K and V of four waves, one to a SIMD, or for one tile of eight, where V takes
+  // the place of K as soon as that is read.  The loads of a wave then run under its softmax and the other wave of the SIMD
+  // only, but a list has half the steps per wave and a SIMD two waves to issue from.  (A lone wave took 7000 cycles for a
+  // step of 1800 cycles of products at D=208.)  What eight waves have no registers for is worked out anew in each step
+  // (addresses of fragments) or lies in LDS (Q, offsets of rows).  B=1 H=8, bf16, us, four waves -> eight: S=1024 causal 32x32
+  // D=136 20.0 -> 15.5, D=208 29.8 -> 19.4, D=256 29.7 -> 21.9; S=64 D=208 10.5 -> 8.5; S=715 rows at any alignment D=165
+  // 43.8 -> 23.5, D=250 51.3 -> 30.8; blocks of 40 keys D=256 34.1 -> 23.8.  Twelve waves up to 96 columns: 4 % slower.
+  static constexpr bool kShared = DT > 4 && NW == 8;
+  static constexpr size_t kWaveBytes = size_t(kShared ? 1 : 2) * kTileBytes;
+  static constexpr int kGroup = DT < 4 ? DT : 4;  // output tiles merged per pass
   static constexpr size_t kMergeBytes = size_t(NW) * kGroup * 4096;
   // K and V of every wave; the merge overlaps them
-  static constexpr size_t kTiles = size_t(NW) * 2 * kTileBytes > kMergeBytes ? size_t(NW) * 2 * kTileBytes : kMergeBytes;
-  // With 97 - 128 columns (eight waves, 256 registers each) and from 193 on Q lives in LDS, shared by the waves.
-  static constexpr bool kQInLds = DT == 4 || DT >= 7;
+  static constexpr size_t kTiles = NW * kWaveBytes > kMergeBytes ? NW * kWaveBytes : kMergeBytes;
+  // With 97 - 128 columns (eight waves, 256 registers each) and from 161 on Q lives in LDS, shared by the waves.
+  static constexpr bool kQInLds = DT == 4 || DT >= 6;
   static constexpr size_t kQBytes = kQInLds ? size_t(kTileBytes) : 0;
-  // behind the tiles: Q; per wave, compare key, offset inside the block and tile of 32 keys; and
+  // ... and there the byte offsets of a lane's chunks of 16 rows, K and V, which eight waves have no registers for
+  static constexpr bool kOffsetsInLds = kShared && DT >= 7;
+  static constexpr size_t kOffsetBytes = kOffsetsInLds ? size_t(2 * DT * 64 * 4) : 0;
+  // behind the tiles: Q; per wave, compare key, offset inside the block, tile and row of 32 keys; and
   // the maximum and sum of 32 rows
-  static constexpr size_t kLdsBytes = kTiles + kQBytes + NW * (32 * 12 + 32 * 8);
+  static constexpr size_t kLdsBytes = kTiles + kQBytes + NW * (32 * 16 + 32 * 8) + kOffsetBytes;
 };
 
 template <bool BF16, int DT, int NW, Rows R>
-__global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2 : 1)) fwd_generic_kernel(const GenericParams p) {
+__device__ __forceinline__ void generic_walk(const GenericParams& p) {
   using Traits = GenericTraits<DT, NW>;
   constexpr int KS = 2 * DT;
   constexpr int C = 4 * DT;     // 16-byte chunks of a tile row
@@ -256,13 +273,18 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
   const bool q_here = q_local < p.QB && q_idx < p.S;  // a row of this tile
   const bool q_live = q_here && q_idx < p.seqlen;
 
-  uint8_t* const sK = lds + size_t(w) * 2 * Traits::kTileBytes;
-  uint8_t* const sV = sK + Traits::kTileBytes;
+  constexpr bool SHARED = Traits::kShared;
+  uint8_t* const sK = lds + size_t(w) * Traits::kWaveBytes;
+  uint8_t* const sV = SHARED ? sK : sK + Traits::kTileBytes;
   uint8_t* const sQ = lds + Traits::kTiles;
-  int32_t* const sKey = reinterpret_cast<int32_t*>(lds + Traits::kTiles + Traits::kQBytes) + w * 96;
+  int32_t* const sKey = reinterpret_cast<int32_t*>(lds + Traits::kTiles + Traits::kQBytes) + w * 128;
   int32_t* const sOff = sKey + 32;
   int32_t* const sPid = sKey + 64;
-  float* const sStat = reinterpret_cast<float*>(lds + Traits::kTiles + Traits::kQBytes + NW * 384);  // [2][NW][32]
+  int32_t* const sRow = sKey + 96;  // (rows at any alignment, eight waves) -1: zeros
+  constexpr bool ROWS_IN_LDS = SHARED && R == Rows::kWide;
+  float* const sStat = reinterpret_cast<float*>(lds + Traits::kTiles + Traits::kQBytes + NW * 512);  // [2][NW][32]
+
+  uint32_t* const sAt = reinterpret_cast<uint32_t*>(sStat + 2 * NW * 32);  // [2][DT][64], K and V
 
   const int64_t b = omni_attn::divide(bh, p.by_heads), h = bh - unsigned(b) * unsigned(p.H);
   const uint16_t* const q_slab = p.q + b * p.q_at.batch + h * p.q_at.head;
@@ -299,11 +321,22 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
     return DT % 2 == 1 ? low : (DT % 4 == 2 ? (low | ((r >> 1) & 1) << 2) : (low | (r & 3) << 2));
   };
   auto tile_at = [&](int r, int ch) { return r * Traits::kRowBytes + (ch ^ swizzle(r)) * 16; };
+  constexpr bool WHOLE = R == Rows::kWhole, HALVES = WHOLE || R == Rows::kHalves, DIRECT = HALVES || R == Rows::kKeys;
+  // Byte offset of a lane's chunk id of a tile inside its row.
+  auto col_at = [&](int id) { return uint32_t(chunk_start(((id % C) ^ swizzle(id / C)) * 8, p.D)) * 2u; };
+  if constexpr (Traits::kOffsetsInLds) {  // (read behind the barrier that Q has)
+    static_assert(Traits::kQInLds, "a barrier");
+    for (int i = w; i < DT; i += NW) {
+      const int id = i * 64 + lane;
+      sAt[id] = uint32_t(id / C) * uint32_t(p.k_at.row * 2) + col_at(id);
+      sAt[DT * 64 + id] = uint32_t(id / C) * uint32_t(p.v_at.row * 2) + col_at(id);
+    }
+  }
   // Q as B operand: lane holds Q[row][16 s + 8 g .. +7]
   u32x4_t qf[Traits::kQInLds ? 1 : KS];
   {
     const uint16_t* qrow = q_slab + int64_t(q_live ? q_idx : 0) * p.q_at.row;
-    if constexpr (R == Rows::kDirect) {  // (16-byte chunks of D % 8 == 0 columns: none has columns of the one before)
+    if constexpr (DIRECT) {  // (16-byte chunks of D % 8 == 0 columns: none has columns of the one before)
       constexpr int NQ = Traits::kQInLds ? (KS + NW - 1) / NW : KS;  // chunks of this wave
       u32x4_t x[NQ];  // all in flight together, and cleared below: one under a condition is waited for
 #pragma unroll
@@ -355,13 +388,15 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
     }
   };
 
-  // Position of this lane's key (lanes c and c + 32 follow the same key) in the wave's next step.
+  // Position of this lane's key (lanes c and c + 32 follow the same key) in the wave's next step; with steps in halves,
+  // of its first key.
   int slot, off;
-  {
-    const int pos = 32 * w + c;
+  auto first_step = [&]() {
+    const int pos = 32 * w + (HALVES ? 0 : c);
     slot = pos / p.kb_eff;
     off = pos - slot * p.kb_eff;
-  }
+  };
+  first_step();
   // The key of this lane.  `cmp`: the key is allowed for the query rows >= cmp (all of them for FULL and
   // PARTIAL, none for a key that does not exist, lies beyond the sequence or belongs to a skipped slot).
   struct Key {
@@ -418,9 +453,42 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
     return k;
   };
 
+  // A step in halves of 16 keys, each inside one block.
+  Block half[2] = {{0, kMasked, 0, 0}, {0, kMasked, 0, 0}};
+  auto block_at = [&](int s, int at) {
+    if ((s >> 6) != chunk_at) load_chunk(s >> 6);
+    const int idx = __builtin_amdgcn_readlane(mv_idx, s & 63), info = __builtin_amdgcn_readlane(mv_info, s & 63);
+    const int kvb = idx < 0 ? 0 : (idx >= p.Tk ? p.Tk - 1 : idx);
+    const long long row0 = (long long)kvb * p.KB + at;
+    Block k;
+    k.mode = row0 < p.seqlen && (WHOLE || s < nb) ? info & 3 : int(kMasked);
+    k.row0 = k.mode != kMasked ? int(row0) : 0;
+    k.pid = info >> 2;
+    k.off = at;
+    return k;
+  };
+  auto next_halves = [&]() {
+    slot = __builtin_amdgcn_readfirstlane(slot);
+    off = __builtin_amdgcn_readfirstlane(off);
+    half[0] = block_at(slot, off);
+    if constexpr (WHOLE) {  // the second half follows the first (rows beyond the sequence are masked)
+      half[1] = {half[0].row0 + 16, half[0].mode, half[0].pid, off + 16};
+    } else {
+      const bool next = off + 16 >= p.kb_eff;
+      half[1] = block_at(slot + int(next), next ? 0 : off + 16);
+    }
+    slot += p.adv_slot;
+    off += p.adv_off;
+    if (off >= p.kb_eff) {
+      off -= p.kb_eff;
+      ++slot;
+    }
+  };
+
   // Rows of a step into a tile: lane l takes the chunks l, l + 64, ... of the tile, in the order they
   // lie in LDS.  from[i]: row of the operand that chunk i of this lane comes from, -1 for zeros; of a
-  // whole step only the first row matters (base) and from[i] counts from there.
+  // whole step only the first row matters (base) and from[i] counts from there.  (The chunks of 16 rows are DT per
+  // lane, so chunk i + DT is chunk i of the second half: the swizzle repeats after 16 rows.)
   int from[NLD], base = 0;
   auto take_rows = [&](const Key& k) {
 #pragma unroll
@@ -442,30 +510,38 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
   uint32_t cols[NLD];
 #pragma unroll
   for (int i = 0; i < NLD; ++i) {
-    const int id = i * 64 + lane;
-    cols[i] = uint32_t(chunk_start(((id % C) ^ swizzle(id / C)) * 8, p.D)) * 2u;
+    cols[i] = col_at(i * 64 + lane);
   }
-  // ... and of its chunks in a whole step, K and V
-  constexpr int NAT = R == Rows::kDirect ? NLD : 1;
+  // ... and of its chunks in half a step, K and V
+  constexpr int NAT = HALVES && !Traits::kOffsetsInLds ? DT : 1;
   uint32_t k_at[NAT], v_at[NAT];
 #pragma unroll
   for (int i = 0; i < NAT; ++i) {
     k_at[i] = uint32_t(from[i]) * uint32_t(p.k_at.row * 2) + cols[i];
     v_at[i] = uint32_t(from[i]) * uint32_t(p.v_at.row * 2) + cols[i];
   }
-  // `first`: a tile of the walk's first step.  Its loads belong in flight together, nothing else hides them.  The compiler
-  // does that by itself but with seven 32-column tiles, where it asked for one chunk after the other: B=2 H=4 S=81 D=194
-  // 15.1 -> 13.2 us.  (Forced on the other forms: D=165 13.3 -> 13.8, D=225 15.1 -> 15.3.)
-  constexpr bool TOGETHER = DT == 7;
-  auto load_tile = [&](auto again, auto first, bool is_k, const uint16_t* slab, const i32x4_t& rsrc, int64_t pitch, uint8_t* dst) {
-    if constexpr (R == Rows::kDirect) {
+  auto load_tile = [&](auto again, bool is_k, const uint16_t* slab, const i32x4_t& rsrc, int64_t pitch, uint8_t* dst) {
+    if constexpr (DIRECT) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the tile has been read
       const uint32_t to = uint32_t(size_t((__attribute__((address_space(3))) void*)dst));
       const uint32_t pitch2 = uint32_t(pitch * 2);
-      if (p.whole) {
-        const uint32_t row0_at = uint32_t(base) * pitch2;
+      if constexpr (HALVES) {
+        uint32_t at[DT];
 #pragma unroll
-        for (int i = 0; i < NLD; ++i) buffer_to_lds(rsrc, is_k ? k_at[i] : v_at[i], row0_at, to + uint32_t(i) * 1024u);
+        for (int i = 0; i < DT; ++i) {
+          if constexpr (Traits::kOffsetsInLds) {
+            at[i] = sAt[((is_k ? 0 : DT) + i) * 64 + lane];
+          } else {
+            at[i] = is_k ? k_at[i] : v_at[i];
+          }
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const uint32_t row0_at =
+              WHOLE ? uint32_t(half[0].row0) * pitch2 + (h == 0 ? 0u : 16u * pitch2) : uint32_t(half[h].row0) * pitch2;
+#pragma unroll
+          for (int i = 0; i < DT; ++i) buffer_to_lds(rsrc, at[i], row0_at, to + uint32_t(h * DT + i) * 1024u);
+        }
       } else {
 #pragma unroll
         for (int i = 0; i < NLD; ++i) {
@@ -473,11 +549,27 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
           buffer_to_lds(rsrc, from[i] < 0 ? 0xffffffffu : at, 0u, to + uint32_t(i) * 1024u);
         }
       }
+    } else if constexpr (SHARED) {
+      int l = lane;  // (addresses are worked out anew: eight waves have no registers to keep them in)
+      asm volatile("" : "+v"(l));
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {  // 16 rows in flight together
+        u32x4_t x[DT];
+#pragma unroll
+        for (int i = 0; i < DT; ++i) {
+          const int id = i * 64 + l, row = sRow[16 * h + id / C];
+          x[i] = load8<R>(slab + int64_t(row < 0 ? 0 : row) * pitch, ((id % C) ^ swizzle(id / C)) * 8, p.D);
+          if (row < 0) x[i] = u32x4_t{0u, 0u, 0u, 0u};
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < DT; ++i) *reinterpret_cast<u32x4_t*>(dst + size_t((h * DT + i) * 64 + l) * 16) = x[i];
+        __builtin_amdgcn_sched_barrier(0);
+      }
     } else {
       int l = lane;
-      // (addresses worked out anew: kept over the walk they cost it registers, which the fp16 form has none left of)
-      if constexpr (decltype(again)::value || (DT == 8 && !BF16)) asm volatile("" : "+v"(l));
-      u32x4_t ahead[NLD];
+      // (addresses worked out anew: kept over the walk they cost it registers)
+      if constexpr (decltype(again)::value) asm volatile("" : "+v"(l));
 #pragma unroll
       for (int i = 0; i < NLD; ++i) {
         if constexpr (decltype(again)::value) __builtin_amdgcn_sched_barrier(0);
@@ -485,21 +577,8 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
         const int row = from[i] + base;  // (base is 0 unless the step is whole)
         const bool none = from[i] < 0 || row >= p.seqlen;
         u32x4_t x = load8<R>(slab + int64_t(none ? 0 : row) * pitch, ((id % C) ^ swizzle(id / C)) * 8, p.D);
-        if constexpr (TOGETHER && decltype(first)::value && !decltype(again)::value) {
-          ahead[i] = x;
-          continue;
-        }
         if (none) x = u32x4_t{0u, 0u, 0u, 0u};
         *reinterpret_cast<u32x4_t*>(dst + size_t(id) * 16) = x;
-      }
-      if constexpr (TOGETHER && decltype(first)::value && !decltype(again)::value) {
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < NLD; ++i) {
-          const int row = from[i] + base;
-          if (from[i] < 0 || row >= p.seqlen) ahead[i] = u32x4_t{0u, 0u, 0u, 0u};
-          *reinterpret_cast<u32x4_t*>(dst + size_t(i * 64 + l) * 16) = ahead[i];
-        }
       }
     }
   };
@@ -516,18 +595,27 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
   Key cur = {-1, 0x7fffffff, 0, -1};
   Block blk = {0, kMasked, 0, 0};
   auto advance = [&]() {
-    if (p.whole) {
+    if constexpr (HALVES) {
+      next_halves();
+    } else if (!DIRECT && p.whole) {
       blk = next_block();
       base = blk.row0;
+      if constexpr (ROWS_IN_LDS) {
+        if (g == 0) sRow[c] = base + c < p.seqlen ? base + c : -1;
+      }
     } else {
       cur = next_key();
-      take_rows(cur);
+      if constexpr (ROWS_IN_LDS) {
+        if (g == 0) sRow[c] = cur.row;
+      } else {
+        take_rows(cur);
+      }
     }
   };
   auto first_rows = [&](auto again) {
     advance();
-    load_tile(again, std::true_type{}, true, k_slab, rK, p.k_at.row, sK);
-    load_tile(again, std::true_type{}, false, v_slab, rV, p.v_at.row, sV);
+    load_tile(again, true, k_slab, rK, p.k_at.row, sK);
+    if constexpr (!SHARED) load_tile(again, false, v_slab, rV, p.v_at.row, sV);
   };
   const int q_first = qb * p.QB + row0;  // first row of the workgroup
   // `again`: the second walk of a wave whose first met an infinity or a NaN in V (or overflowed); rare, so
@@ -537,7 +625,22 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
       // Allowed keys of this step as bits: register r (key 8 (r / 4) + 4 g + r % 4) is bit r.
       uint32_t keep = 0xffffu;
       bool masked;  // (uniform) some of them are not allowed
-      if (p.whole) {
+      uint32_t word[2][2];
+      if constexpr (HALVES) {
+        constexpr int BLOCKS = WHOLE ? 1 : 2, KEYS = 32 / BLOCKS;
+        masked = false;
+#pragma unroll
+        for (int h = 0; h < BLOCKS; ++h) {
+          const Block& k = half[h];
+          masked |= !(k.row0 + KEYS <= p.seqlen && (k.mode == kFull || (k.mode == kCausal && k.row0 + KEYS - 1 <= q_first)));
+          // PARTIAL (attn_naive.cu:143-154): the tile's bytes are asked for here and looked at behind the products
+          if (k.mode == kPartial) {
+            const uint8_t* t = p.partial_masks + (size_t(k.pid) * p.QB + (q_here ? q_local : 0)) * p.KB + k.off + 4 * g;
+#pragma unroll
+            for (int i = 0; i < KEYS / 8; ++i) word[h + i / 2][i % 2] = *reinterpret_cast<const uint32_t*>(t + 8 * i);
+          }
+        }
+      } else if (!DIRECT && p.whole) {
         masked = !(blk.row0 + 32 <= p.seqlen && (blk.mode == kFull || (blk.mode == kCausal && blk.row0 + 31 <= q_first)));
         if (masked) {
           if (blk.mode == kPartial) {  // attn_naive.cu:143-154: any non-zero byte of the tile = attend
@@ -607,27 +710,79 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
           }
         }
       }
-      if constexpr (R == Rows::kDirect) wait_but<NLD>();  // K is there (V was requested after it)
+      if constexpr (SHARED && DIRECT) {
+        wait_but<0>();  // K is there
+      } else if constexpr (DIRECT) {
+        wait_but<NLD>();  // ... (V was requested after it)
+      }
       f32x16_t st = zero16;
+      // (SHARED: the addresses of the fragments are worked out anew in every step, from one register that the compiler
+      // knows nothing about: kept over the walk they are what the eight waves have no registers for)
+      uint32_t k_turn = uint32_t(g ^ swizzle(c)) * 16u;
+      if constexpr (SHARED) asm volatile("" : "+v"(k_turn));
+      auto k_frag = [&](int s) {
+        if constexpr (SHARED) {
+          return *reinterpret_cast<const u32x4_t*>(sK + c * Traits::kRowBytes + ((32u * s) ^ k_turn));
+        } else {
+          return *reinterpret_cast<const u32x4_t*>(sK + tile_at(c, 2 * s + g));
+        }
+      };
+      auto q_operand = [&](int s) {
+        if constexpr (SHARED && Traits::kQInLds) {
+          return *reinterpret_cast<const u32x4_t*>(sQ + c * Traits::kRowBytes + ((32u * s) ^ k_turn));
+        } else {
+          return q_frag(s);
+        }
+      };
       // (fragments are fetched in groups, so that a group waits for LDS once)
-      constexpr int AHEAD = R == Rows::kDirect ? (KS < 8 ? KS : 8) : 1;
+      constexpr int AHEAD = SHARED ? 4 : (DIRECT ? (KS < 8 ? KS : 8) : 1);
 #pragma unroll
       for (int s0 = 0; s0 < KS; s0 += AHEAD) {
         u32x4_t kf[AHEAD];
 #pragma unroll
         for (int i = 0; i < AHEAD; ++i)
-          if (s0 + i < KS) kf[i] = *reinterpret_cast<const u32x4_t*>(sK + tile_at(c, 2 * (s0 + i) + g));
+          if (s0 + i < KS) kf[i] = k_frag(s0 + i);
         if constexpr (AHEAD > 1) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < AHEAD; ++i)
-          if (s0 + i < KS) st = mfma<BF16>(kf[i], q_frag(s0 + i), st);
+          if (s0 + i < KS) st = mfma<BF16>(kf[i], q_operand(s0 + i), st);
+      }
+      if constexpr (HALVES) {
+        if (masked) {
+          keep = 0;
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const Block& k = half[h];
+            int limit = p.seqlen - 1;
+            if (k.mode == kCausal) limit = limit < q_idx ? limit : q_idx;
+            if (k.mode == kMasked) limit = -1;
+            const int n = limit - k.row0 - 4 * g + 1;  // leading keys of this half-wave's pattern that are allowed
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+              const int m = n - 8 * i;
+              uint32_t four = m >= 4 ? 15u : (m <= 0 ? 0u : (1u << m) - 1u);
+              if (k.mode == kPartial) {  // any non-zero byte of the tile = attend
+                uint32_t x = word[h][i];
+                x |= x >> 4;
+                x |= x >> 2;
+                x |= x >> 1;
+                four &= ((x & 0x01010101u) * 0x01020408u) >> 24;
+              }
+              keep |= four << (4 * (2 * h + i));
+            }
+          }
+        }
       }
       asm volatile("" : "+v"(keep));  // (the mask's own loads are waited for here, not behind the next request)
-      // K has been read: the rows of the wave's next step
-      go = more();
-      if (go) {
-        advance();
-        load_tile(again, std::false_type{}, true, k_slab, rK, p.k_at.row, sK);
+      // K has been read: the rows of the wave's next step, or V into its place
+      if constexpr (SHARED) {
+        load_tile(again, false, v_slab, rV, p.v_at.row, sV);
+      } else {
+        go = more();
+        if (go) {
+          advance();
+          load_tile(again, true, k_slab, rK, p.k_at.row, sK);
+        }
       }
       if (p.softcap > 0.f) {
 #pragma unroll
@@ -651,7 +806,7 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
       mx *= p.sl2;
       {
         float lower, upper;
-        both_halves<R == Rows::kDirect>(mx, lower, upper);
+        both_halves<DIRECT>(mx, lower, upper);
         mx = fmaxf(lower, upper);
       }
       if (__builtin_amdgcn_ballot_w64(mx > m_run + kSlack) != 0) {
@@ -666,7 +821,9 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
         m_run = m_new;
       }
       const float m_ref = m_run == -INFINITY ? 0.f : m_run;
-      if constexpr (R == Rows::kDirect) {  // V is there (the next K was requested after it)
+      if constexpr (SHARED && DIRECT) {  // V is there
+        wait_but<0>();
+      } else if constexpr (DIRECT) {  // ... (the next K was requested after it)
         if (go) {
           wait_but<NLD>();
         } else {
@@ -675,7 +832,20 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
       }
       // O^T += V^T.P^T: k-slot e of lane group g in 16-key half ts is key 16 ts + 8 (e / 4) + 4 g + e % 4
       const int i16 = c & 15, j16 = c >> 4;
+      // (row r0 + 8 has the swizzle of r0 with bit 1 flipped)
+      uint32_t v_turn = uint32_t((2 * j16 + ((i16 & 3) >> 1)) ^ swizzle(4 * g + (i16 >> 2))) * 16u;
+      if constexpr (SHARED) asm volatile("" : "+v"(v_turn));
       auto v_frag = [&](const uint8_t* tile, int ts, int dt) {
+        if constexpr (SHARED) {
+          const uint8_t* row = tile + (16 * ts + 4 * g + (i16 >> 2)) * Traits::kRowBytes + (i16 & 1) * 8;
+          const uint8_t* a0 = row + ((64u * dt) ^ v_turn);
+          const uint8_t* a1 = row + 8 * Traits::kRowBytes + ((64u * dt) ^ v_turn ^ 32u);
+          const u32x2_t lo = __builtin_bit_cast(
+              u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(a0)));
+          const u32x2_t hi = __builtin_bit_cast(
+              u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(a1)));
+          return u32x4_t{lo[0], lo[1], hi[0], hi[1]};
+        }
         const int chunk = 2 * (2 * dt + j16) + ((i16 & 3) >> 1);
         const int r0 = 16 * ts + 4 * g + (i16 >> 2), r1 = r0 + 8;
         const uint8_t* a0 = tile + tile_at(r0, chunk) + (i16 & 1) * 8;
@@ -687,7 +857,7 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
         return u32x4_t{lo[0], lo[1], hi[0], hi[1]};
       };
       // (the fragments of the first half are fetched under the weights)
-      constexpr bool FETCHED = R == Rows::kDirect && DT <= 4 && !decltype(again)::value;
+      constexpr bool FETCHED = DIRECT && DT <= 4 && !decltype(again)::value;
       u32x4_t vf[DT];
       if constexpr (FETCHED) {
 #pragma unroll
@@ -739,9 +909,22 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
           }
         }
       }
+      if constexpr (!decltype(again)::value && SHARED) {
+        constexpr int FAR = 3;  // fragments in flight
+        u32x4_t a[FAR];
+#pragma unroll
+        for (int j = 0; j < FAR; ++j) a[j] = v_frag(sV, j / DT, j % DT);
+#pragma unroll
+        for (int j = 0; j < 2 * DT; ++j) {
+#pragma unroll
+          for (int n = 0; n < PARTS; ++n) ot[j % DT] = mfma<BF16>(a[j % FAR], pb[n][j / DT], ot[j % DT]);
+          if (j + FAR < 2 * DT) a[j % FAR] = v_frag(sV, (j + FAR) / DT, (j + FAR) % DT);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
       if constexpr (!decltype(again)::value) {
 #pragma unroll
-        for (int ts = 0; ts < 2; ++ts) {
+        for (int ts = 0; ts < (SHARED ? 0 : 2); ++ts) {
 #pragma unroll
           for (int dt = 0; dt < DT; ++dt) {
             const u32x4_t a = FETCHED ? vf[dt] : v_frag(sV, ts, dt);
@@ -787,7 +970,15 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
           __builtin_amdgcn_sched_barrier(0);
         }
       }
-      if (go) load_tile(again, std::false_type{}, false, v_slab, rV, p.v_at.row, sV);
+      if constexpr (SHARED) {
+        go = more();
+        if (go) {
+          advance();
+          load_tile(again, true, k_slab, rK, p.k_at.row, sK);
+        }
+      } else {
+        if (go) load_tile(again, false, v_slab, rV, p.v_at.row, sV);
+      }
     }
   };
   if (go) {
@@ -803,8 +994,7 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
       for (int dt = 0; dt < DT; ++dt) ot[dt] = zero16;
       l_run = 0.f;
       m_run += kSlack;  // no score is beyond this: weights stay below 2^kShift, nothing is rescaled
-      slot = (32 * w + c) / p.kb_eff;
-      off = 32 * w + c - slot * p.kb_eff;
+      first_step();
       go = true;
       first_rows(std::true_type{});
       walk(std::true_type{});
@@ -815,7 +1005,7 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
   // writes its tiles, wave i adds up and stores tile i of the group.
   {
     float lower, upper;
-    both_halves<R == Rows::kDirect>(l_run, lower, upper);
+    both_halves<DIRECT>(l_run, lower, upper);
     l_run = lower + upper;
   }
   if (g == 0) {
@@ -886,12 +1076,26 @@ __global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : (DT <= 4 ? 2
   }
 }
 
+template <bool BF16, int DT, int NW, Rows R>
+__global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : 2) fwd_generic_kernel(const GenericParams p) {
+  generic_walk<BF16, DT, NW, R>(p);
+}
+// Steps that may cross a block.
+template <bool BF16, int DT, int NW, Rows R>
+__global__ void __launch_bounds__(64 * NW, DT == 1 && NW == 8 ? 4 : 2) fwd_generic_steps_kernel(const GenericParams p) {
+  generic_walk<BF16, DT, NW, R>(p);
+}
+
 constexpr int kMaxDevices = 64;
 
 template <bool BF16, int DT, int NW, Rows R>
 int launch(const GenericParams& p, unsigned grid, hipStream_t stream) {
-  auto kern = fwd_generic_kernel<BF16, DT, NW, R>;
-  const void* fn = reinterpret_cast<const void*>(kern);
+  const void* fn;
+  if constexpr (R == Rows::kHalves || R == Rows::kKeys) {
+    fn = reinterpret_cast<const void*>(fwd_generic_steps_kernel<BF16, DT, NW, R>);
+  } else {
+    fn = reinterpret_cast<const void*>(fwd_generic_kernel<BF16, DT, NW, R>);
+  }
   constexpr int lds = int(GenericTraits<DT, NW>::kLdsBytes);
   static_assert(lds <= 160 * 1024, "LDS of a compute unit");
   if (lds > 48 * 1024) {  // the dynamic-LDS limit of an instance is raised once per device
@@ -918,9 +1122,10 @@ int launch(const GenericParams& p, unsigned grid, hipStream_t stream) {
 
 template <bool BF16, int DT>
 int launch_rows(const GenericParams& p, Rows rows, unsigned grid, hipStream_t s) {
-  constexpr int NW = DT <= 4 ? 8 : 4;  // what the tiles leave room for in LDS
-  return rows == Rows::kDirect ? launch<BF16, DT, NW, Rows::kDirect>(p, grid, s)
-                               : launch<BF16, DT, NW, Rows::kWide>(p, grid, s);
+  return rows == Rows::kWhole    ? launch<BF16, DT, 8, Rows::kWhole>(p, grid, s)
+         : rows == Rows::kHalves ? launch<BF16, DT, 8, Rows::kHalves>(p, grid, s)
+         : rows == Rows::kKeys   ? launch<BF16, DT, 8, Rows::kKeys>(p, grid, s)
+                                 : launch<BF16, DT, 8, Rows::kWide>(p, grid, s);
 }
 
 template <bool BF16, int... I>
@@ -986,7 +1191,6 @@ int forward_generic(const void* q, const void* k, const void* v, const omni_attn
   p.q_tiles = ((QB < S_pad ? QB : S_pad) + 31) / 32;
   p.mask_words = KB % 4 == 0 && p.kb_eff % 4 == 0 && !misaligned(partial_masks_or_null, 4);
   p.whole = KB % 32 == 0 && !misaligned(partial_masks_or_null, 4);
-  if (p.whole) p.kb_eff = KB;  // (the keys of a block behind the sequence are masked like any others)
   p.n_slabs = unsigned(B) * unsigned(H);
   p.scale = float(1.0 / std::sqrt(double(D)));
   p.softcap = softcap;
@@ -999,8 +1203,15 @@ int forward_generic(const void* q, const void* k, const void* v, const omni_attn
     return !misaligned(ptr, 16) && at.batch % 8 == 0 && at.head % 8 == 0 && at.row % 8 == 0 && at.row >= D &&
            ((long long)p.seqlen + 31) * at.row * 2 < 0xffffff00LL;  // (a step may run 31 rows past the sequence)
   };
-  const Rows reads = D < 8 ? Rows::kSmall
-                           : (D % 8 == 0 && direct(k, k_at) && direct(v, v_at) ? Rows::kDirect : Rows::kWide);
+  const bool halves = KB % 16 == 0 && !misaligned(partial_masks_or_null, 4);  // half a step never crosses a block
+  const Rows reads = D < 8                                                         ? Rows::kSmall
+                     : !(D % 8 == 0 && direct(k, k_at) && direct(v, v_at))         ? Rows::kWide
+                     : p.whole                                                     ? Rows::kWhole
+                     : halves                                                      ? Rows::kHalves
+                                                                                   : Rows::kKeys;
+  // (the keys of such a block behind the sequence are masked like any others, up to the end of a step)
+  const int end = p.whole ? (S_pad + 31) / 32 * 32 : (S_pad + 15) / 16 * 16;
+  if (p.whole || reads == Rows::kHalves) p.kb_eff = KB < end ? KB : end;
   const auto tiles = std::make_integer_sequence<int, kMaxD / 32>{};
   const int e = dtype == OMNI_ATTN_DTYPE_BF16
                     ? launch_tiles<true>(p, reads, unsigned(grid), static_cast<hipStream_t>(stream), tiles)

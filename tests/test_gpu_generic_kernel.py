@@ -184,3 +184,25 @@ def test_rows_of_keys_and_values_lie_differently(D, blk, gpu_device):
     assert (out.float().cpu() - ref).abs().max().item() <= 2e-3
     for kk, vv in ((rows_apart(k), v), (k, rows_apart(v)), (rows_apart(k), rows_apart(v))):
         assert torch.equal(oat.omni_attention_simple(q, kk, vv, mask), out)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+@pytest.mark.parametrize("QB,KB,D,S", [(16, 16, 136, 69 * 16), (48, 48, 168, 70 * 48), (32, 80, 200, 480), (32, 32, 256, 66 * 32),
+                                       (64, 112, 224, 448), (16, 144, 64, 96), (32, 256, 160, 96), (24, 24, 144, 72 * 24),
+                                       (40, 40, 256, 200), (16, 16, 165, 69 * 16), (64, 32, 131, 192), (20, 36, 250, 180)])
+def test_steps_in_halves_and_tiles_that_keys_and_values_take_in_turn(dtype, QB, KB, D, S, gpu_device):
+    """Steps whose halves lie in one block, in two, or in two chunks of a list (more than 64 slots); blocks longer than the
+    sequence; eight waves with one tile each, whose rows go to LDS directly, key by key or through registers; peaked rows
+    (the rests of fp16 weights).  The result's error is its rounding (half an ulp of |o| < 4) and fp32 sums."""
+    gen = torch.Generator().manual_seed(QB * 1000 + KB * 10 + D)
+    q, k, v = (torch.randn(1, 1, S, D, generator=gen).to(dtype) for _ in range(3))
+    nb, idx, tys, pidx, pm = random_block_metadata(gen, 1, 1, -(-S // QB), -(-S // KB), QB, KB, p_empty=0.1, shuffle=True)
+    for seqlen, query in ((S, q), (S - 11, 3 * q)):
+        o, lse = run_generic(query, k, v, nb, idx, tys, QB, KB, seqlen, pidx, pm, gpu_device)
+        wo, wl = attention_block_walk(query, k, v, nb, idx, tys, QB, KB, seqlen, pidx, pm)
+        assert torch.equal(torch.isinf(lse.cpu()), torch.isinf(wl))
+        ulp = 2.0 ** -10 if dtype == torch.float16 else 2.0 ** -7
+        # (exponents of up to 128 in fp32, in either sum: 2 * 2^-17 of a weight, times |v| < 5)
+        assert (o.float().cpu() - wo).abs().max().item() <= ulp + 2.0 ** -13, (QB, KB, D, seqlen)
+        live = ~torch.isinf(wl)
+        assert (lse.cpu()[live] - wl[live]).abs().max().item() <= 5e-5

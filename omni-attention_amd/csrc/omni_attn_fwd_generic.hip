@@ -27,7 +27,7 @@
 // cycles of a wave against 770 of its products at D=96) times the steps of the longest list over the waves.  So rows
 // that go to LDS directly have their offsets laid out once, their fragments are fetched in groups (K, and V under the
 // weights; three ahead beyond 128 columns), and a weight's part is taken off without being converted first.  B=1 H=8
-// S=2048 D=96, causal in 32x32 blocks, launches back to back: fp16 24.4 us, bf16 23.0 (28.7 and 26.9 without); spans in
+// S=2048 D=96, causal in 32x32 blocks, launches back to back: fp16 23.8 us, bf16 23.0 (28.7 and 26.9 without); spans in
 // 64x64 blocks at B=1 H=4 S=1500: D=136 21.6, D=208 26.3, D=256 29.6; rows at any alignment, D=101 34.7, D=165 40.3.
 // 33 us (37) at D=96 where queries are four times as large (every row peaked, a rest in most steps).  Two parts per
 // weight, cut off after 22 bits and at 2^-32 of the reference, gain 2 us, but are
@@ -142,6 +142,56 @@ __device__ __forceinline__ void buffer_to_lds(i32x4_t rsrc, uint32_t lane_off, u
         "s"(__builtin_amdgcn_readfirstlane(uniform_off))
       : "memory", "m0");
 }
+// N such loads from one uniform offset, 1 KiB of LDS apart.  (The offset in the instruction counts for both addresses, and
+// is taken off the uniform one again, which is at least kBack: the check of the range does not take a negative one.  A load by
+// itself takes three scalar instructions more.  With scores that are masked in place and weights that are split without
+// copies, fp16 B=1 H=8 S=2048 causal 32x32 D=96 24.3 -> 23.8 us, D=120 29.3 -> 28.8, D=256 S=1024 21.9 -> 21.3.)
+constexpr uint32_t kBack = 3072;
+template <int N>
+__device__ __forceinline__ void buffer_to_lds_in_a_row(i32x4_t rsrc, const uint32_t* lane_off, uint32_t uniform_off,
+                                                       uint32_t lds_base) {
+  static_assert(N >= 1 && N <= 4, "twelve bits of offset");
+  i32x4_t r;
+  r[0] = __builtin_amdgcn_readfirstlane(rsrc[0]);
+  r[1] = __builtin_amdgcn_readfirstlane(rsrc[1]);
+  r[2] = __builtin_amdgcn_readfirstlane(rsrc[2]);
+  r[3] = __builtin_amdgcn_readfirstlane(rsrc[3]);
+  const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds_base), u = __builtin_amdgcn_readfirstlane(uniform_off);
+  if constexpr (N == 1) {
+    buffer_to_lds(r, lane_off[0], u, m0);
+  } else if constexpr (N == 2) {
+    asm volatile(
+        "s_mov_b32 m0, %0\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %1, %3, %4 offen lds\n\t"
+        "buffer_load_dwordx4 %2, %3, %5 offen offset:1024 lds"
+        :
+        : "s"(m0), "v"(lane_off[0]), "v"(lane_off[1]), "s"(r), "s"(u), "s"(u - 1024u)
+        : "memory", "m0");
+  } else if constexpr (N == 3) {
+    asm volatile(
+        "s_mov_b32 m0, %0\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %1, %4, %5 offen lds\n\t"
+        "buffer_load_dwordx4 %2, %4, %6 offen offset:1024 lds\n\t"
+        "buffer_load_dwordx4 %3, %4, %7 offen offset:2048 lds"
+        :
+        : "s"(m0), "v"(lane_off[0]), "v"(lane_off[1]), "v"(lane_off[2]), "s"(r), "s"(u), "s"(u - 1024u), "s"(u - 2048u)
+        : "memory", "m0");
+  } else {
+    asm volatile(
+        "s_mov_b32 m0, %0\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %1, %5, %6 offen lds\n\t"
+        "buffer_load_dwordx4 %2, %5, %7 offen offset:1024 lds\n\t"
+        "buffer_load_dwordx4 %3, %5, %8 offen offset:2048 lds\n\t"
+        "buffer_load_dwordx4 %4, %5, %9 offen offset:3072 lds"
+        :
+        : "s"(m0), "v"(lane_off[0]), "v"(lane_off[1]), "v"(lane_off[2]), "v"(lane_off[3]), "s"(r), "s"(u), "s"(u - 1024u),
+          "s"(u - 2048u), "s"(u - 3072u)
+        : "memory", "m0");
+  }
+}
 // At most N vector-memory operations of this wave are outstanding.
 template <int N>
 __device__ __forceinline__ void wait_but() {
@@ -174,8 +224,11 @@ __device__ __forceinline__ uint32_t split_part(float& lo, float& hi) {
     const auto v = __builtin_amdgcn_cvt_pkrtz(lo, hi);
     const uint32_t h = __builtin_bit_cast(uint32_t, v);
     // value - part, with the part's half read as it is (the compiler converts it first: two instructions more per part)
-    asm("v_fma_mix_f32 %0, %1, -1.0, %0 op_sel_hi:[1,0,0]" : "+v"(lo) : "v"(h));
-    asm("v_fma_mix_f32 %0, %1, -1.0, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(hi) : "v"(h));
+    float a, b;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(a) : "v"(h), "v"(lo));
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(b) : "v"(h), "v"(hi));
+    lo = a;
+    hi = b;
     return h;
   }
 }
@@ -496,12 +549,14 @@ __device__ __forceinline__ void generic_walk(const GenericParams& p) {
   };
 #pragma unroll
   for (int i = 0; i < NLD; ++i) from[i] = (i * 64 + lane) / C;
+  // (with steps in halves the buffer begins kBack bytes before the slab; nothing is read there)
   auto resource = [&](const uint16_t* slab, int64_t pitch) {
-    const uint64_t a = reinterpret_cast<uint64_t>(slab);
+    constexpr uint32_t back = HALVES ? kBack : 0u;
+    const uint64_t a = reinterpret_cast<uint64_t>(slab) - back;
     i32x4_t r;
     r[0] = __builtin_amdgcn_readfirstlane(int32_t(uint32_t(a)));
     r[1] = __builtin_amdgcn_readfirstlane(int32_t(uint32_t(a >> 32) & 0xffffu));
-    r[2] = __builtin_amdgcn_readfirstlane(int32_t(uint32_t((int64_t(p.seqlen) - 1) * pitch + p.D) * 2u));
+    r[2] = __builtin_amdgcn_readfirstlane(int32_t(uint32_t((int64_t(p.seqlen) - 1) * pitch + p.D) * 2u + back));
     r[3] = 0x00020000;
     return r;
   };
@@ -538,9 +593,9 @@ __device__ __forceinline__ void generic_walk(const GenericParams& p) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const uint32_t row0_at =
-              WHOLE ? uint32_t(half[0].row0) * pitch2 + (h == 0 ? 0u : 16u * pitch2) : uint32_t(half[h].row0) * pitch2;
-#pragma unroll
-          for (int i = 0; i < DT; ++i) buffer_to_lds(rsrc, at[i], row0_at, to + uint32_t(h * DT + i) * 1024u);
+              kBack + (WHOLE ? uint32_t(half[0].row0) * pitch2 + (h == 0 ? 0u : 16u * pitch2) : uint32_t(half[h].row0) * pitch2);
+          buffer_to_lds_in_a_row<(DT < 4 ? DT : 4)>(rsrc, at, row0_at, to + uint32_t(h * DT) * 1024u);
+          if constexpr (DT > 4) buffer_to_lds_in_a_row<DT - 4>(rsrc, at + 4, row0_at, to + uint32_t(h * DT + 4) * 1024u);
         }
       } else {
 #pragma unroll
@@ -788,17 +843,16 @@ __device__ __forceinline__ void generic_walk(const GenericParams& p) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) st[r] = tanhf(st[r] * p.scale / p.softcap) * p.softcap;
       }
-      float mn = INFINITY;  // the lowest allowed score of this lane (fp16, for the rests of the weights)
-      if (masked) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const bool kept = (keep >> r) & 1u;
-          if constexpr (!BF16) mn = fminf(mn, kept ? st[r] : INFINITY);
-          st[r] = kept ? st[r] : -INFINITY;
-        }
-      } else if constexpr (!BF16) {
+      // the lowest score of this lane (fp16, for the rests of the weights; allowed or not: a step that looks for rests in
+      // vain costs less than a selection per score)
+      float mn = INFINITY;
+      if constexpr (!BF16) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) mn = fminf(mn, st[r]);
+      }
+      if (masked) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) st[r] = (keep >> r) & 1u ? st[r] : -INFINITY;
       }
       float mx = -INFINITY;
 #pragma unroll
@@ -1201,7 +1255,7 @@ int forward_generic(const void* q, const void* k, const void* v, const omni_attn
   if (grid > 0x7fffffffLL) return OMNI_ATTN_ERR_TOO_LARGE;
   const auto direct = [&](const void* ptr, const omni_attn_strides& at) {  // 32-bit offsets inside a slab
     return !misaligned(ptr, 16) && at.batch % 8 == 0 && at.head % 8 == 0 && at.row % 8 == 0 && at.row >= D &&
-           ((long long)p.seqlen + 31) * at.row * 2 < 0xffffff00LL;  // (a step may run 31 rows past the sequence)
+           ((long long)p.seqlen + 31) * at.row * 2 < 0xffffff00LL - kBack;  // (a step may run 31 rows past the sequence)
   };
   const bool halves = KB % 16 == 0 && !misaligned(partial_masks_or_null, 4);  // half a step never crosses a block
   const Rows reads = D < 8                                                         ? Rows::kSmall

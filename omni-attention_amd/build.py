@@ -57,14 +57,13 @@ MIN_WAVES_PER_SIMD = {"fwd_kernel": 2, "fwd_ksplit": 2, "bwd_dq_kernel": 2, "bwd
 SGPR_SPILLS_ALLOWED = ("bwd_dq_", "bwd_dkdv_", "fwd_ksplit", "fwd_generic_")
 # For the generic kernel scratch memory is what counts.  Forms that read rows at any alignment (E1E) have some: up to 32 columns
 # and 97 - 128 in fp16 (two registers' worth; at B=1 H=8 S=2048 D=125 48.5 us, 52.9 without, where the addresses of the
-# loads are worked out anew in every step), 129 - 160 and 193 - 224 in fp16 (the same), and 225 - 256 (half a tile's rows in
-# flight in registers; with four waves, which have twice as many, B=1 H=4 S=1500 D=250 took 97.6 us, 54.2 so); and blocks of any
-# number of keys (E4E) at 193 - 256 columns in fp16.
+# loads are worked out anew in every step) and 225 - 256 (half a tile's rows in flight in registers; with four waves, which
+# have twice as many, B=1 H=4 S=1500 D=250 took 97.6 us, 54.2 so); and blocks of any number of keys (E4E) at 225 - 256
+# columns in fp16.
 VGPR_SPILLS_ALLOWED = ("fwd_generic_",)
 SCRATCH_ALLOWED = {"fwd_generic_kernelILb0ELi1ELi8ELNS_4RowsE1E": 8, "fwd_generic_kernelILb0ELi4ELi8ELNS_4RowsE1E": 8,
-                   "fwd_generic_kernelILb0ELi5ELi8ELNS_4RowsE1E": 8, "fwd_generic_kernelILb0ELi7ELi8ELNS_4RowsE1E": 8,
                    "fwd_generic_kernelILb0ELi8ELi8ELNS_4RowsE1E": 64, "fwd_generic_kernelILb1ELi8ELi8ELNS_4RowsE1E": 64,
-                   "fwd_generic_steps_kernelILb0ELi7ELi8ELNS_4RowsE4E": 12, "fwd_generic_steps_kernelILb0ELi8ELi8ELNS_4RowsE4E": 16}
+                   "fwd_generic_steps_kernelILb0ELi8ELi8ELNS_4RowsE4E": 16}
 
 INSTANCES = [(bf, d) for bf in (0, 1) for d in (32, 64, 128)]
 LIB_NAME = "libomni_attn_gfx950.so"

@@ -849,6 +849,8 @@ __device__ __forceinline__ void generic_walk(const GenericParams& p) {
       if constexpr (!BF16) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) mn = fminf(mn, st[r]);
+        // (here, before the scores change: one register less in most forms, eleven more in this one)
+        if constexpr (R != Rows::kWide || DT != 4) asm volatile("" : "+v"(mn));
       }
       if (masked) {
 #pragma unroll

@@ -43,6 +43,7 @@
 #include <utility>
 
 #include "omni_attn_deal.hpp"
+#include "omni_attn_generic_rows.hpp"
 
 namespace omni_attn {
 // Keeps the hipError_t behind an OMNI_ATTN_ERR_LAUNCH for omni_attn_last_hip_error() (defined
@@ -143,18 +144,18 @@ __device__ __forceinline__ void buffer_to_lds(i32x4_t rsrc, uint32_t lane_off, u
       : "memory", "m0");
 }
 // N such loads from one uniform offset, 1 KiB of LDS apart.  (The offset in the instruction counts for both addresses, and
-// is taken off the uniform one again, which is at least kBack: the check of the range does not take a negative one.  A load by
-// itself takes three scalar instructions more.  With scores that are masked in place and weights that are split without
+// is taken off the uniform one again, which is at least kBack: the check of the range does not take a negative one.  size: of
+// the buffer, for these loads.  A load by itself takes three scalar instructions more.  With scores that are masked in place and weights that are split without
 // copies, fp16 B=1 H=8 S=2048 causal 32x32 D=96 24.3 -> 23.8 us, D=120 29.3 -> 28.8, D=256 S=1024 21.9 -> 21.3.)
-constexpr uint32_t kBack = 3072;
+using omni_attn::kBack;
 template <int N>
-__device__ __forceinline__ void buffer_to_lds_in_a_row(i32x4_t rsrc, const uint32_t* lane_off, uint32_t uniform_off,
-                                                       uint32_t lds_base) {
-  static_assert(N >= 1 && N <= 4, "twelve bits of offset");
+__device__ __forceinline__ void buffer_to_lds_in_a_row(i32x4_t rsrc, uint32_t size, const uint32_t* lane_off,
+                                                       uint32_t uniform_off, uint32_t lds_base) {
+  static_assert(N >= 1 && (N - 1) * 1024 <= int(kBack), "offsets in the instruction");
   i32x4_t r;
   r[0] = __builtin_amdgcn_readfirstlane(rsrc[0]);
   r[1] = __builtin_amdgcn_readfirstlane(rsrc[1]);
-  r[2] = __builtin_amdgcn_readfirstlane(rsrc[2]);
+  r[2] = __builtin_amdgcn_readfirstlane(int32_t(size));
   r[3] = __builtin_amdgcn_readfirstlane(rsrc[3]);
   const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds_base), u = __builtin_amdgcn_readfirstlane(uniform_off);
   if constexpr (N == 1) {
@@ -565,7 +566,7 @@ __device__ __forceinline__ void generic_walk(const GenericParams& p) {
     i32x4_t r;
     r[0] = __builtin_amdgcn_readfirstlane(int32_t(uint32_t(a)));
     r[1] = __builtin_amdgcn_readfirstlane(int32_t(uint32_t(a >> 32) & 0xffffu));
-    r[2] = __builtin_amdgcn_readfirstlane(int32_t(uint32_t((int64_t(p.seqlen) - 1) * pitch + p.D) * 2u + back));
+    r[2] = __builtin_amdgcn_readfirstlane(int32_t(omni_attn::rows_end(p.seqlen, pitch, p.D, back)));
     r[3] = 0x00020000;
     return r;
   };
@@ -601,10 +602,12 @@ __device__ __forceinline__ void generic_walk(const GenericParams& p) {
         }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          const uint32_t row0_at =
-              kBack + (WHOLE ? uint32_t(half[0].row0) * pitch2 + (h == 0 ? 0u : 16u * pitch2) : uint32_t(half[h].row0) * pitch2);
-          buffer_to_lds_in_a_row<(DT < 4 ? DT : 4)>(rsrc, at, row0_at, to + uint32_t(h * DT) * 1024u);
-          if constexpr (DT > 4) buffer_to_lds_in_a_row<DT - 4>(rsrc, at + 4, row0_at, to + uint32_t(h * DT + 4) * 1024u);
+          const int row0 = WHOLE ? half[0].row0 + 16 * h : half[h].row0;
+          // (of a block that ends with the step, the second half may begin behind the sequence)
+          const omni_attn::HalfAt from = omni_attn::half_at(row0 < p.seqlen, row0, pitch2, uint32_t(rsrc[2]));
+          buffer_to_lds_in_a_row<(DT < 4 ? DT : 4)>(rsrc, from.size, at, from.offset, to + uint32_t(h * DT) * 1024u);
+          if constexpr (DT > 4)
+            buffer_to_lds_in_a_row<DT - 4>(rsrc, from.size, at + 4, from.offset, to + uint32_t(h * DT + 4) * 1024u);
         }
       } else {
 #pragma unroll

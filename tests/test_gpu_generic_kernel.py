@@ -206,3 +206,28 @@ def test_steps_in_halves_and_tiles_that_keys_and_values_take_in_turn(dtype, QB, 
         assert (o.float().cpu() - wo).abs().max().item() <= ulp + 2.0 ** -13, (QB, KB, D, seqlen)
         live = ~torch.isinf(wl)
         assert (lse.cpu()[live] - wl[live]).abs().max().item() <= 5e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+@pytest.mark.parametrize("blk,D", [(32, 40), (64, 96), (32, 120), (64, 136), (32, 168), (64, 208), (32, 256), (48, 40), (16, 208)])
+def test_nothing_behind_the_sequence_is_read(dtype, blk, D, gpu_device):
+    """Sequences that end in the first or the second half of a step, or between them: NaNs behind them change no bit."""
+    from omni_attn_torch import create_causal_omni_block_mask
+    gen = torch.Generator().manual_seed(D + blk)
+    S = 4 * blk
+    q, k, v = (torch.randn(1, 2, S, D, generator=gen).to(dtype) for _ in range(3))
+    m = create_causal_omni_block_mask(1, 2, S, S, blk, blk, device="cpu")
+    for seqlen in (S, S - 1, S - blk // 2, S - 16, S - 17, 16, 1):
+        args = (m.kv_num_blocks, m.kv_indices, m.block_mask_types, blk, blk, seqlen, None, None, gpu_device)
+        behind = [t.clone() for t in (k, v)]
+        zeros = [t.clone() for t in (k, v)]
+        for t in behind:
+            t[:, :, seqlen:] = float("nan")
+        for t in zeros:
+            t[:, :, seqlen:] = 0
+        o, lse = run_generic(q, *behind, *args)
+        wo, wl = run_generic(q, *zeros, *args)
+        assert torch.equal(o, wo) and torch.equal(lse, wl), seqlen
+        ref, _ = attention_dense_fp32(q[:, :, :seqlen], k[:, :, :seqlen], v[:, :, :seqlen],
+                                      torch.tril(torch.ones(seqlen, seqlen, dtype=torch.bool)))
+        assert (o[:, :, :seqlen].float().cpu() - ref).abs().max().item() <= (2e-3 if dtype == torch.float16 else 1e-2), seqlen

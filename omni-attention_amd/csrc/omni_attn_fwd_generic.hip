@@ -525,7 +525,9 @@ __device__ __forceinline__ void generic_walk(const GenericParams& p) {
     const long long row0 = (long long)kvb * p.KB + at;
     Block k;
     k.mode = row0 < p.seqlen && (WHOLE || s < nb) ? info & 3 : int(kMasked);
-    k.row0 = k.mode != kMasked ? int(row0) : 0;
+    // (no rows are read from the end of the sequence on: those of a half that no row attends to would not count, but an
+    // infinity in them would send the wave through its list again)
+    k.row0 = k.mode != kMasked ? int(row0) : p.seqlen;
     k.pid = info >> 2;
     k.off = at;
     return k;
@@ -603,7 +605,7 @@ __device__ __forceinline__ void generic_walk(const GenericParams& p) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const int row0 = WHOLE ? half[0].row0 + 16 * h : half[h].row0;
-          // (of a block that ends with the step, the second half may begin behind the sequence)
+          // (not so where no row attends to the half, and a second half may begin behind the sequence)
           const omni_attn::HalfAt from = omni_attn::half_at(row0 < p.seqlen, row0, pitch2, uint32_t(rsrc[2]));
           buffer_to_lds_in_a_row<(DT < 4 ? DT : 4)>(rsrc, from.size, at, from.offset, to + uint32_t(h * DT) * 1024u);
           if constexpr (DT > 4)

@@ -21,8 +21,9 @@ OMNI_ATTN_ROWS_HOST_DEVICE uint32_t rows_end(int seqlen, int64_t pitch, int D, u
 }
 
 // Uniform offset and size of the buffer for half a step.  A load is checked as lane offset + offset in the instruction against
-// size - uniform offset, and that difference must not be negative: a half that begins behind the sequence has a buffer that
-// ends where the half begins, all of its lanes are outside, write zeros and touch no memory.
+// size - uniform offset, and that difference must not be negative: a half that is not `live` (it begins behind the sequence, or
+// no row attends to it) has a buffer that ends where the half begins, all of its lanes are outside, write zeros and touch no
+// memory.
 struct HalfAt {
   uint32_t offset, size;
 };

@@ -231,3 +231,29 @@ def test_nothing_behind_the_sequence_is_read(dtype, blk, D, gpu_device):
         ref, _ = attention_dense_fp32(q[:, :, :seqlen], k[:, :, :seqlen], v[:, :, :seqlen],
                                       torch.tril(torch.ones(seqlen, seqlen, dtype=torch.bool)))
         assert (o[:, :, :seqlen].float().cpu() - ref).abs().max().item() <= (2e-3 if dtype == torch.float16 else 1e-2), seqlen
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+@pytest.mark.parametrize("blk,D", [(16, 40), (48, 96), (80, 120), (16, 136), (48, 208), (16, 256), (32, 96), (32, 208), (24, 96),
+                                   (24, 208)])
+def test_keys_that_no_slot_names_are_not_read(dtype, blk, D, gpu_device):
+    """Lists of an odd number of slots, MASKED ones among them and block 0 in none but those: infinities and NaNs in block 0
+    and behind the sequence change no bit (a wave that meets one adds up its list again, in another order)."""
+    gen = torch.Generator().manual_seed(D + blk)
+    T, H = 9, 2
+    S = T * blk
+    q, k, v = (torch.randn(1, H, S, D, generator=gen).to(dtype) for _ in range(3))
+    nb = torch.full((1, H, T), 7, dtype=torch.int32)
+    idx = torch.zeros(1, H, T, T, dtype=torch.int32)
+    idx[..., :7] = torch.tensor([1, 0, 3, 4, 5, 6, 8])
+    tys = torch.zeros_like(idx)
+    tys[..., :7] = torch.tensor([2, 0, 2, 2, 0, 2, 2])
+    for seqlen in (S, S - 9):
+        args = (nb, idx, tys, blk, blk, seqlen, None, None, gpu_device)
+        clean, lse0 = run_generic(q, k, v, *args)
+        bad = v.clone()
+        bad[:, :, 0:blk, ::3] = float("inf")
+        bad[:, :, 0:blk, 1::3] = float("nan")
+        bad[:, :, seqlen:] = float("nan")
+        o, lse = run_generic(q, k, bad, *args)
+        assert torch.isfinite(o).all() and torch.equal(o, clean) and torch.equal(lse, lse0), seqlen

@@ -454,6 +454,7 @@ __device__ __forceinline__ void generic_walk(const GenericParams& p) {
   // Position of this lane's key (lanes c and c + 32 follow the same key) in the wave's next step; with steps in halves,
   // of its first key.
   int slot, off;
+  using Key32 = std::conditional_t<R == Rows::kSmall, uint32_t, int>;
   auto first_step = [&]() {
     const int pos = 32 * w + (HALVES ? 0 : c);
     slot = pos / p.kb_eff;
@@ -483,12 +484,7 @@ __device__ __forceinline__ void generic_walk(const GenericParams& p) {
     k.cmp = !live ? 0x7fffffff : (mode == kCausal ? int(row) : -1);
     k.pid = (live && mode == kPartial) ? info >> 2 : -1;
     k.off = off;
-    slot += p.adv_slot;
-    off += p.adv_off;
-    if (off >= p.kb_eff) {
-      off -= p.kb_eff;
-      ++slot;
-    }
+    omni_attn::move_on<Key32>(slot, off, p.adv_slot, p.adv_off, p.kb_eff);
     return k;
   };
 
@@ -507,12 +503,7 @@ __device__ __forceinline__ void generic_walk(const GenericParams& p) {
     k.row0 = k.mode != kMasked ? int(row0) : 0;
     k.pid = info >> 2;
     k.off = at;
-    slot += p.adv_slot;
-    off += p.adv_off;
-    if (off >= p.kb_eff) {
-      off -= p.kb_eff;
-      ++slot;
-    }
+    omni_attn::move_on<Key32>(slot, off, p.adv_slot, p.adv_off, p.kb_eff);
     return k;
   };
 
@@ -542,12 +533,7 @@ __device__ __forceinline__ void generic_walk(const GenericParams& p) {
       const bool next = off + 16 >= p.kb_eff;
       half[1] = block_at(slot + int(next), next ? 0 : off + 16);
     }
-    slot += p.adv_slot;
-    off += p.adv_off;
-    if (off >= p.kb_eff) {
-      off -= p.kb_eff;
-      ++slot;
-    }
+    omni_attn::move_on<Key32>(slot, off, p.adv_slot, p.adv_off, p.kb_eff);
   };
 
   // Rows of a step into a tile: lane l takes the chunks l, l + 64, ... of the tile, in the order they
@@ -710,7 +696,7 @@ __device__ __forceinline__ void generic_walk(const GenericParams& p) {
           }
         }
       } else if (!DIRECT && p.whole) {
-        masked = !(blk.row0 + 32 <= p.seqlen && (blk.mode == kFull || (blk.mode == kCausal && blk.row0 + 31 <= q_first)));
+        masked = !(p.seqlen - blk.row0 >= 32 && (blk.mode == kFull || (blk.mode == kCausal && blk.row0 + 31 <= q_first)));
         if (masked) {
           if (blk.mode == kPartial) {  // attn_naive.cu:143-154: any non-zero byte of the tile = attend
             const uint8_t* t = p.partial_masks + (size_t(blk.pid) * p.QB + (q_here ? q_local : 0)) * p.KB + blk.off + 4 * g;
@@ -1234,7 +1220,7 @@ int forward_generic(const void* q, const void* k, const void* v, const omni_attn
   if (B <= 0 || H <= 0 || S_pad <= 0 || Tq <= 0 || max_blocks <= 0 || seqlen_orig < 0 || num_partial < 0 ||
       !(softcap >= 0.f) || std::isinf(softcap))
     return OMNI_ATTN_ERR_BAD_SHAPE;
-  if (Tq != (S_pad + QB - 1) / QB) return OMNI_ATTN_ERR_BAD_SHAPE;
+  if (Tq != omni_attn::blocks_of(S_pad, QB)) return OMNI_ATTN_ERR_BAD_SHAPE;
   const long long rows = (long long)B * H * S_pad;
   if ((long long)S_pad * D > 0x7fffffffLL || rows > (1LL << 33) || (long long)B * H * Tq * max_blocks > (1LL << 40))
     return OMNI_ATTN_ERR_TOO_LARGE;
@@ -1258,13 +1244,13 @@ int forward_generic(const void* q, const void* k, const void* v, const omni_attn
   p.D = D;
   p.H = H;
   p.Tq = Tq;
-  p.Tk = (S_pad + KB - 1) / KB;
+  p.Tk = omni_attn::blocks_of(S_pad, KB);
   p.max_blocks = max_blocks;
   p.QB = QB;
   p.KB = KB;
   p.seqlen = seqlen_orig < S_pad ? seqlen_orig : S_pad;
-  p.kb_eff = KB < S_pad ? KB : S_pad;
-  p.q_tiles = ((QB < S_pad ? QB : S_pad) + 31) / 32;
+  p.kb_eff = omni_attn::walked_keys(KB, S_pad, 1);
+  p.q_tiles = omni_attn::blocks_of(QB < S_pad ? QB : S_pad, 32);
   p.mask_words = KB % 4 == 0 && p.kb_eff % 4 == 0 && !misaligned(partial_masks_or_null, 4);
   p.whole = KB % 32 == 0 && !misaligned(partial_masks_or_null, 4);
   p.n_slabs = unsigned(B) * unsigned(H);
@@ -1286,8 +1272,7 @@ int forward_generic(const void* q, const void* k, const void* v, const omni_attn
                      : halves                                                      ? Rows::kHalves
                                                                                    : Rows::kKeys;
   // (the keys of such a block behind the sequence are masked like any others, up to the end of a step)
-  const int end = p.whole ? (S_pad + 31) / 32 * 32 : (S_pad + 15) / 16 * 16;
-  if (p.whole || reads == Rows::kHalves) p.kb_eff = KB < end ? KB : end;
+  if (p.whole || reads == Rows::kHalves) p.kb_eff = omni_attn::walked_keys(KB, S_pad, p.whole ? 32 : 16);
   const auto tiles = std::make_integer_sequence<int, kMaxD / 32>{};
   const int e = dtype == OMNI_ATTN_DTYPE_BF16
                     ? launch_tiles<true>(p, reads, unsigned(grid), static_cast<hipStream_t>(stream), tiles)

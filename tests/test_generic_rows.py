@@ -41,3 +41,36 @@ int main() {
         }
 }
 """)
+
+
+def test_positions_in_lists_of_the_largest_blocks(tmp_path):
+    """One column passes the check of sizes with as many rows as an int holds: nothing wraps around, and a walk ends."""
+    run_program(tmp_path, r"""
+int main() {
+  const int most = 0x7fffffff;
+  for (int S : {1, 15, 16, 17, 31, 32, 33, 4096, most - 33, most - 32, most - 31, most - 30, most - 16, most - 15, most - 1, most})
+    for (int unit : {1, 16, 32})
+      for (int KB : {1, 16, 31, 32, 48, 4096, most / 8, most - 257, most - 31, most - 1, most}) {
+        const long long end = (S + (unit - 1LL)) / unit * unit;
+        const int keys = walked_keys(KB, S, unit);
+        CHECK(keys > 0 && keys == (KB < end ? KB : end));
+        CHECK(blocks_of(S, KB) == (S + (KB - 1LL)) / KB);
+        for (int step : {128, 256}) {  // the first and the last positions of a walk over two blocks
+          const int adv_slot = step / keys, adv_off = step % keys;
+          for (long long pos : {0LL, 31LL, keys - 1LL, keys - 32LL, keys - 256LL, 2LL * keys - 1}) {
+            if (pos < 0) continue;
+            int slot = int(pos / keys), off = int(pos % keys);
+            for (int n = 1; n < 4; ++n) {
+              int slot_of_int = slot, off_of_int = off;
+              move_on<uint32_t>(slot, off, adv_slot, adv_off, keys);
+              const long long to = pos + (long long)n * step;
+              CHECK(slot == to / keys && off == to % keys);
+              if (keys > most - 257) continue;
+              move_on<int>(slot_of_int, off_of_int, adv_slot, adv_off, keys);
+              CHECK(slot == slot_of_int && off == off_of_int);
+            }
+          }
+        }
+      }
+}
+""")

@@ -295,8 +295,10 @@ struct GenericTraits {
   static constexpr size_t kMergeBytes = size_t(NW) * kGroup * 4096;
   // K and V of every wave; the merge overlaps them
   static constexpr size_t kTiles = NW * kWaveBytes > kMergeBytes ? NW * kWaveBytes : kMergeBytes;
-  // With 97 - 128 columns (eight waves, 256 registers each) and from 161 on Q lives in LDS, shared by the waves.
-  static constexpr bool kQInLds = DT == 4 || DT >= 6;
+  // From 97 columns on Q lives in LDS, shared by the waves.  (With 129 - 160 in the registers of each of eight waves, rows
+  // at any alignment read one chunk after the other: B=1 H=8 S=64 D=131 bf16 12.6 us, 9.7 so, 11.0 with four waves; S=1024 27.3,
+  // 24.9, 42.5; rows straight to LDS, D=136 S=64 7.6, 7.4, 8.5.)
+  static constexpr bool kQInLds = DT >= 4;
   static constexpr size_t kQBytes = kQInLds ? size_t(kTileBytes) : 0;
   // ... and there the byte offsets of a lane's chunks of 16 rows, K and V, which eight waves have no registers for
   static constexpr bool kOffsetsInLds = kShared && DT >= 7;

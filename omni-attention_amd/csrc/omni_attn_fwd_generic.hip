@@ -1093,18 +1093,25 @@ __device__ __forceinline__ void generic_walk(const GenericParams& p) {
     p.lse[size_t(bh) * p.S + q_idx] = some ? (m_fin + __builtin_amdgcn_logf(l_all) - kShift) * 0.6931471805599453f : -INFINITY;
   float* const stage = reinterpret_cast<float*>(lds);
   constexpr int G = Traits::kGroup;
+  // A list of no more steps than half of the waves leaves the others nothing to add.  (Rows at any alignment beyond 128
+  // columns, where eight waves took longer over such lists than four: B=1 H=8 S=128 bf16, four waves -> eight -> so, D=131 11.4
+  // -> 10.2 -> 9.6 us, D=165 13.5 -> 11.6 -> 10.9, D=225 14.7 -> 15.1 -> 14.2; B=8 H=32 D=225 63.5 -> 65.1 -> 62.7.
+  // Elsewhere eight waves take no longer, and the question costs long lists 0.1 us.)
+  const bool half_full = ROWS_IN_LDS && (long long)nb * p.kb_eff <= 32 * (NW / 2);
 #pragma unroll
   for (int d0 = 0; d0 < DT; d0 += G) {
     if (d0 > 0) __syncthreads();  // the previous group has been read
+    if (!half_full || w < NW / 2) {
 #pragma unroll
-    for (int i = 0; i < G; ++i) {
-      if (d0 + i >= DT) continue;
+      for (int i = 0; i < G; ++i) {
+        if (d0 + i >= DT) continue;
 #pragma unroll
-      for (int r4 = 0; r4 < 4; ++r4) {
-        f32x4_t x;
+        for (int r4 = 0; r4 < 4; ++r4) {
+          f32x4_t x;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) x[j] = ot[d0 + i][4 * r4 + j] * mine;
-        *reinterpret_cast<f32x4_t*>(stage + ((size_t(w) * G + i) * 4 + r4) * 256 + lane * 4) = x;
+          for (int j = 0; j < 4; ++j) x[j] = ot[d0 + i][4 * r4 + j] * mine;
+          *reinterpret_cast<f32x4_t*>(stage + ((size_t(w) * G + i) * 4 + r4) * 256 + lane * 4) = x;
+        }
       }
     }
     __syncthreads();
@@ -1113,9 +1120,14 @@ __device__ __forceinline__ void generic_walk(const GenericParams& p) {
       const int i = u >> 2, r4 = u & 3;
       if (d0 + i >= DT) break;
       f32x4_t x = {0.f, 0.f, 0.f, 0.f};
+      auto add = [&](int j) { x += *reinterpret_cast<const f32x4_t*>(stage + ((size_t(j) * G + i) * 4 + r4) * 256 + lane * 4); };
+      if (half_full) {
 #pragma unroll
-      for (int j = 0; j < NW; ++j)
-        x += *reinterpret_cast<const f32x4_t*>(stage + ((size_t(j) * G + i) * 4 + r4) * 256 + lane * 4);
+        for (int j = 0; j < NW / 2; ++j) add(j);
+      } else {
+#pragma unroll
+        for (int j = 0; j < NW; ++j) add(j);
+      }
       if (empty) x = f32x4_t{0.f, 0.f, 0.f, 0.f};
       const int d = 32 * (d0 + i) + 8 * r4 + 4 * g;
       uint16_t* orow = p.o + (size_t(bh) * p.S + q_idx) * p.D;

@@ -257,3 +257,23 @@ def test_keys_that_no_slot_names_are_not_read(dtype, blk, D, gpu_device):
         bad[:, :, seqlen:] = float("nan")
         o, lse = run_generic(q, k, bad, *args)
         assert torch.isfinite(o).all() and torch.equal(o, clean) and torch.equal(lse, lse0), seqlen
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+@pytest.mark.parametrize("blk,D", [(32, 131), (32, 250), (16, 165), (48, 225), (64, 194), (20, 161)])
+def test_lists_of_as_many_steps_as_half_of_the_waves(dtype, blk, D, gpu_device):
+    """Rows at any alignment beyond 128 columns: up to 128 listed keys leave half of the waves out of the sum at the end.
+    Query block i lists i blocks, so that lists end before, at and behind that line.  The result's error is its rounding
+    (half an ulp of |o| < 4) and fp32 sums."""
+    gen = torch.Generator().manual_seed(D)
+    T = 256 // blk
+    S = T * blk
+    q, k, v = (torch.randn(1, 1, S, D, generator=gen).to(dtype) for _ in range(3))
+    nb = torch.arange(T, dtype=torch.int32).view(1, 1, T)
+    idx = torch.arange(T, dtype=torch.int32).repeat(T, 1).view(1, 1, T, T)
+    tys = torch.full_like(idx, 2)
+    o, lse = run_generic(q, k, v, nb, idx, tys, blk, blk, S, None, None, gpu_device)
+    wo, wl = attention_block_walk(q, k, v, nb, idx, tys, blk, blk, S, None, None)
+    assert torch.equal(torch.isinf(lse.cpu()), torch.isinf(wl))
+    assert (o.float().cpu() - wo).abs().max().item() <= (2.0 ** -10 if dtype == torch.float16 else 2.0 ** -7) + 2.0 ** -16
+    assert (lse.cpu()[..., blk:] - wl[..., blk:]).abs().max().item() <= 2e-5

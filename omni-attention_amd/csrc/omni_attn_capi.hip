@@ -359,6 +359,7 @@ int backward(const void* q, const void* k, const void* v, const void* o, const v
   p.KB = KB;
   const long long rows32 = (long long)B * H * Tq * (QB / 32);
   p.dq_split = bwd_choose_dq_split(D, QB, rows32, Tq * QB, p.seqlen % QB != 0, B > 1, softcap > 0.f);
+  p.dq_step = bwd_dq_step(D, QB, rows32, Tq * QB, p.seqlen % QB != 0);
   p.dkdv_split = bwd_choose_dkdv_split(D, softcap > 0.f, rows32, Tq * QB);
   DeviceTopology topo;
   if (const int e = query_topology(&topo)) {

@@ -185,8 +185,8 @@ enum class DkdvSplit : int {
 // The operator's backward at the lines (causal, spans, images), whole blocks, us, and the split of that kernel:
 //   dQ     D=128  B H=20 S=1024 62 (-2 .. -10 %), B H=8 S=4096 177-217 (-12 .. +3); with the forward, B H=8 S=3000 173-222
 //                 (-9 .. -14), B H=12 S=1700 112-125 (-12 .. -13), S=2048 131-152 (-1 .. -12), B H=16 S=1700 117-130 (-6
-//                 .. -8); beyond: B H=20 S=1408 104 (-5 .. +1), B H=28 S=1152 95-101 (-2 .. +5); 64-row blocks: B H=16 S=2048
-//                 107-140 (-7 .. +1), S=1024 beyond: B H=32 68-85 (+1 .. +5)
+//                 .. -8); beyond: B H=20 S=1408 104 (-5 .. +1), B H=28 S=1152 95-101 (-2 .. +5); 64-row blocks (against
+//                 steps of 64 keys, bwd_dq_step): B H=16 S=2048 107-140 (-7 .. +1), S=1024 beyond: B H=32 68-85 (+1 .. +5)
 //          D=64   B H=40 S=1024 52-59 (-3 .. +1), B H=32 S=1237 58-72 (-6 .. -12), B H=24 S=2048 87-106 (-7 .. +3), B H=16
 //                 S=4096 167-211 (-3 .. +2); 64-row blocks B H=32 S=1237 57-69 (-7 .. -13), B H=16 S=4096 172-225 (-8 .. 0)
 //   dK/dV  D=128  B H=16 S=1237 62-73 (-1 .. -13), B H=8 S=4096 176-216 (-10 .. +2); 64-key blocks B H=12 S=1237 62-71
@@ -224,6 +224,27 @@ inline FwdSplit bwd_choose_dq_split(int D, int QB, long long rows32, int S, bool
                       : fwd_ragged_split_64(D, rows32, S, true, batched)) != FwdSplit::kNone);
   }
   return two ? FwdSplit::kRows64x2 : FwdSplit::kNone;
+}
+// Keys per step of a dQ launch without a split.  A 64-row block is two waves, and at head_dim 128 its tiles of 64 keys leave room
+// for two workgroups on a compute unit, one wave per SIMD; with 32 keys four fit, but a step's halves no longer overlap inside
+// a wave, and barriers come twice as often.  The second wave of a SIMD is worth more than that where the launch is bound by its
+// total work; where the longest lists are its time, they take longer with 32 keys.  That changes at nearly two rounds of
+// 512 workgroups; later for a length that ends inside a block, whose last list has the slowest steps, and where the
+// rows belong to few slabs, with lists that differ more.  Both backward kernels, causal, spans, images (and `mixed` batches), us
+// with 64 keys (and what 32 change):
+//   lengths of whole blocks: B H=28 S=2048 150-255 (-6 .. +1 %), B H=64 S=896 81-121 (-3 .. +3), B H=32 S=1792 129-196 (-1 ..
+//          +4), from 1920 row tiles B H=32 S=1920 144-239 (-2 .. -8), batched 145-265 (-2 .. -11), B H=24 S=2560 184-294 (-4 .. +8),
+//          batched 185-370 (-12 .. +4), B H=40 S=1536 124-184 (-3 .. +5), B H=120 S=512 65-97 (-2 .. -8), B H=32 S=2048 162-261
+//          (-8 .. +1), B H=16 S=4096 288-452 (-2 .. -4); below: B H=32 S=1024 65-92 (+5 .. +8), B H=48 S=1024 80-120 (+1 .. +7)
+//   others: B H=20 S=1100 69-101 (+4 .. +11), B H=32 S=1400 95 (+6 .. +13), B H=24 S=2600 192-296 (-2 .. +10), B H=48 S=1400 126-190
+//          (-3 .. +6); from 2208 row tiles B H=24 S=2900 229-365 (0 .. -3), B H=32 S=2500 230-364 (-6 .. +3), B H=64 S=1237
+//          139-236 (-3 .. -9), B H=24 S=3700 346-559 (-6 .. +1); fewer than 20 slabs B H=16 S=5000 432-644 (-4 .. +3), B H=8
+//          S=9000 711-1010 (-2 .. +11), S=12000 1184-1598 (-7 .. +3), from 3072 B H=8 S=14000 1671-2193 (0 .. -9), B H=16
+//          S=7000 797-1101 (-4 .. -10)
+inline int bwd_dq_step(int D, int QB, long long rows32, int S, bool ragged) {
+  if (D != 128 || QB != 64) return 64;
+  const long long from = !ragged ? 1920 : (5LL * S <= 8 * rows32 ? 2208 : 3072);
+  return rows32 >= from ? 32 : 64;
 }
 inline DkdvSplit bwd_choose_dkdv_split(int D, bool capped, long long rows32, int S) {
   if (D != 128 && rows32 <= 256) return DkdvSplit::kKeys32x4;

@@ -126,14 +126,17 @@ def test_operands_are_read_where_they_lie(S, QB, KB, D, gpu_device):
         assert torch.equal(a, b[:, :, :S]), name
 
 
+WHOLE_64_ROW_COPIES = (60, 140)  # of two slabs of 256 rows: 960 and 2240 row tiles
+
+
 @pytest.mark.parametrize("KB", [64, 128])
 @pytest.mark.parametrize("seqlen", [129, 159, 160, 161, 191, 192, 193, 255])
 def test_gradients_of_64_row_blocks_at_the_edges_of_their_steps(seqlen, KB, gpu_device):
-    """64-row query blocks at head_dim 128 walk their lists by 32 keys: sequences that end around a step and around a
-    block, every slot kind, NaN behind the sequence."""
+    """64-row query blocks at head_dim 128 walk their lists by 32 keys in large launches and by 64 in others: sequences that
+    end around a step and around a block, every slot kind, NaN behind the sequence.  Two launches, on either side of the
+    lines of bwd_dq_step (csrc/omni_attn_split_rules.hpp; tests/test_split_rules.py) and not split."""
     gen = torch.Generator().manual_seed(seqlen + KB)
-    H, S, D, QB, copies = 2, 256, 128, 64, 130
-    assert H * copies * S // 32 > 2048
+    H, S, D, QB = 2, 256, 128, 64
     q, k, v, dout = (torch.randn(1, H, S, D, generator=gen).to(torch.bfloat16) for _ in range(4))
     nb, idx, tys, pidx, pm = random_block_metadata(gen, 1, H, S // QB, S // KB, QB, KB, p_empty=0.2, shuffle=True)
     many = lambda t: t.to(gpu_device).repeat(1, copies, *[1] * (t.dim() - 2)).contiguous()
@@ -142,9 +145,10 @@ def test_gradients_of_64_row_blocks_at_the_edges_of_their_steps(seqlen, KB, gpu_
         t[:, :, seqlen:] = float("nan")
     dense = dense_mask_from_blocks(nb, idx, tys, QB, KB, S, S, pidx, pm, seqlen_orig=seqlen)
     zeroed = [torch.where(torch.isnan(t), torch.zeros_like(t), t) for t in operands]
-    got = run_fwd_bwd(*(many(t) for t in operands), many(nb), many(idx), many(tys), QB, KB, seqlen, many(pidx), pm,
-                      device=gpu_device, softcap=0.0, packed=seqlen % 2 == 0)
-    for t in got:
-        assert torch.equal(t, t[:, :H].repeat(1, copies, *[1] * (t.dim() - 2)))
-    check_grads([t[:, :H] for t in got[:3]], attention_dense_grads(*zeroed[:3], dense, zeroed[3]), torch.bfloat16,
-                f"seqlen={seqlen}")
+    wanted = attention_dense_grads(*zeroed[:3], dense, zeroed[3])
+    for copies in WHOLE_64_ROW_COPIES:
+        got = run_fwd_bwd(*(many(t) for t in operands), many(nb), many(idx), many(tys), QB, KB, seqlen, many(pidx), pm,
+                          device=gpu_device, softcap=0.0, packed=seqlen % 2 == 0)
+        for t in got:
+            assert torch.equal(t, t[:, :H].repeat(1, copies, *[1] * (t.dim() - 2)))
+        check_grads([t[:, :H] for t in got[:3]], wanted, torch.bfloat16, f"seqlen={seqlen}, copies={copies}")

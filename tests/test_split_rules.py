@@ -130,6 +130,38 @@ RAGGED_LAUNCHES = [
     (128, 2, 12, 1500, 64, 2, 0), (64, 2, 12, 1500, 64, 2, 2), (32, 1, 32, 1900, 64, 2, 2)]
 
 
+def test_keys_per_step_of_dq(tmp_path):
+    """32 keys for 64-row blocks at head_dim 128 alone, in launches of many rows: more rows of the same length keep them, and so
+    does a length that fills its blocks.  And the launches that a GPU test runs for their steps have them."""
+    source, program = tmp_path / "step.cpp", tmp_path / "step"
+    source.write_text(r"""
+#include "omni_attn_split_rules.hpp"
+using namespace omni_attn;
+int main() {
+  for (int S = 64; S <= 32768; S += 64) {
+    int before[2] = {64, 64};
+    for (long long rows = 16; rows <= 8192; rows += 16) {
+      for (int ragged = 0; ragged < 2; ++ragged) {
+        const int step = bwd_dq_step(128, 64, rows, S, ragged);
+        if (step != 64 && step != 32) return 1;
+        if (step > before[ragged]) return 2;
+        before[ragged] = step;
+        if (ragged && step == 32 && bwd_dq_step(128, 64, rows, S, false) != 32) return 3;
+        if (bwd_dq_step(128, 128, rows, S, ragged) != 64 || bwd_dq_step(64, 64, rows, S, ragged) != 64) return 4;
+        if (rows <= 1536 && step != 64) return 5;  // (two workgroups on a compute unit, and half as many again)
+      }
+    }
+    if (before[0] != 32 || before[1] != 32) return 6;
+  }
+  for (int ragged = 0; ragged < 2; ++ragged)  // tests/test_gpu_whole_blocks.py
+    if (bwd_dq_step(128, 64, 960, 256, ragged) != 64 || bwd_dq_step(128, 64, 2240, 256, ragged) != 32 ||
+        bwd_choose_dq_split(128, 64, 960, 256, ragged, false) != FwdSplit::kNone) return 7;
+}
+""")
+    subprocess.run(["g++", "-std=c++17", "-I", CSRC, str(source), "-o", str(program)], check=True)
+    assert subprocess.run([str(program)]).returncode == 0
+
+
 def test_dealing_and_the_rules_that_look_at_it(tmp_path):
     """Uneven launches and soft-capped ones: what is split for a length that fills its blocks stays split; with 64-row
     blocks the forward is split for a length inside a block in even launches only, dQ in both (and where the even forward is);

@@ -98,7 +98,9 @@ def test_generic_kernel_edges_of_tiles_and_chunks(QB, KB, D, gpu_device):
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
 @pytest.mark.parametrize("QB,KB,D,S", [(16, 16, 5, 80), (32, 32, 64, 160), (48, 48, 96, 144), (128, 128, 161, 256),
-                                       (64, 32, 256, 192), (32, 32, 250, 96)])
+                                       (64, 32, 256, 192), (32, 32, 250, 96), (24, 24, 40, 120), (40, 40, 256, 200),
+                                       (24, 24, 144, 144), (48, 48, 168, 144), (16, 16, 136, 80), (64, 64, 208, 576),
+                                       (48, 48, 131, 336), (20, 20, 194, 100)])
 def test_values_of_keys_that_are_not_allowed_never_reach_a_row(dtype, QB, KB, D, S, gpu_device):
     """Infinities, NaNs and large values in V: rows that may not attend to those keys get what
     they get without them, rows that may get the infinity, the NaN or the (finite) average.  A query row
@@ -277,3 +279,20 @@ def test_lists_of_as_many_steps_as_half_of_the_waves(dtype, blk, D, gpu_device):
     assert torch.equal(torch.isinf(lse.cpu()), torch.isinf(wl))
     assert (o.float().cpu() - wo).abs().max().item() <= (2.0 ** -10 if dtype == torch.float16 else 2.0 ** -7) + 2.0 ** -16
     assert (lse.cpu()[..., blk:] - wl[..., blk:]).abs().max().item() <= 2e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+@pytest.mark.parametrize("QB,KB,D", [(32, 32, 96), (48, 48, 120), (24, 24, 40), (32, 32, 101), (32, 32, 136), (64, 32, 256), (48, 48, 168),
+                                     (16, 16, 208), (40, 40, 256), (24, 24, 144), (32, 32, 131), (48, 48, 165), (64, 64, 250)])
+def test_soft_capped_scores_in_every_form(dtype, QB, KB, D, gpu_device):
+    """Rows straight to LDS in steps of one block, of halves and by key, and rows at any alignment, up to 128 columns and
+    beyond, with scores that reach the cap: the result's error is its rounding and the hyperbolic tangent's."""
+    gen = torch.Generator().manual_seed(QB + D)
+    S = 7 * max(QB, KB)
+    q, k, v = (torch.randn(1, 2, S, D, generator=gen).to(dtype) for _ in range(3))
+    nb, idx, tys, pidx, pm = random_block_metadata(gen, 1, 2, S // QB, S // KB, QB, KB, p_empty=0.2, shuffle=True)
+    for seqlen in (S, S - 13):
+        o, lse = run_generic(q, k, v, nb, idx, tys, QB, KB, seqlen, pidx, pm, gpu_device, softcap=1.5)
+        dense = dense_mask_from_blocks(nb, idx, tys, QB, KB, S, S, pidx, pm, seqlen_orig=seqlen)
+        ro, rl = attention_dense_fp32(q, k, v, dense, softcap=1.5)
+        compare_with_oracle(o, lse, ro, rl, dtype, f"soft-capped, seqlen={seqlen}")

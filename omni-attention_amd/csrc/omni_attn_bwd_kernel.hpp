@@ -710,12 +710,17 @@ __device__ __forceinline__ void bwd_dq_walk(const BwdParams& p) {
   bwd_store_rows<BF16, D>(dq, p.scale, stage, p.dq + slab, q_wave_min, p.S, lane_out);
 }
 
-// One workgroup per query block, all steps in one group.  STEP: keys per step, 64, or 32 for 64-row blocks at head_dim 128 in
-// large launches (bwd_dq_step says why and where the line lies): both backward kernels, us, 64 -> 32 keys, causal B H=128
-// S=4096 bf16 2273 -> 2016, spans 2744 -> 2456, images 2613 -> 2325.  (The sums are formed in the same order: the same bits.)
-template <bool BF16, bool CAP, int D, int QB, int KB, int STEP>
+// One workgroup per query block, all steps in one group.
+template <bool BF16, bool CAP, int D, int QB, int KB>
 __global__ void __launch_bounds__(QB * 2, 2) bwd_dq_kernel(const BwdParams p) {
-  bwd_dq_walk<BwdDqShape<BF16, CAP, D, QB, KB, QB, 1, STEP>>(p);
+  bwd_dq_walk<BwdDqShape<BF16, CAP, D, QB, KB, QB, 1, 64>>(p);
+}
+// With 32 keys per step: 64-row blocks at head_dim 128 in large launches (bwd_dq_step says why and where the line lies).  Both
+// backward kernels, us, 64 -> 32 keys, causal B H=128 S=4096 bf16 2273 -> 2016, spans 2744 -> 2456, images 2613 -> 2325.  (The
+// sums are formed in the same order: the same bits.)
+template <bool BF16, bool CAP, int D, int QB, int KB>
+__global__ void __launch_bounds__(QB * 2, 2) bwd_dq_short(const BwdParams p) {
+  bwd_dq_walk<BwdDqShape<BF16, CAP, D, QB, KB, QB, 1, 32>>(p);
 }
 // The steps of a list shared by the groups of a workgroup (fwd_choose_split says when).
 template <bool BF16, bool CAP, int D, int QT, int KG, int STEP>
@@ -1398,18 +1403,18 @@ int launch_bwd_kernel(const BwdParams& p, int tiles, int threads, size_t lds, si
   return int(hipLaunchKernel(reinterpret_cast<const void*>(Kernel), grid, dim3(threads), args, lds, stream));
 }
 
-template <bool BF16, bool CAP, int D, int QB, int KB, int STEP>
-int launch_dq(const BwdParams& p, hipStream_t stream) {
-  using Shape = BwdDqShape<BF16, CAP, D, QB, KB, QB, 1, STEP>;
-  return launch_bwd_kernel<bwd_dq_kernel<BF16, CAP, D, QB, KB, STEP>>(p, p.Tq, Shape::kThreads, Shape::kLdsBytes,
-                                                                      Shape::kLdsBytes, stream);
-}
 template <bool BF16, bool CAP, int D, int QB, int KB>
-int launch_dq_blocks(const BwdParams& p, hipStream_t stream) {
+int launch_dq(const BwdParams& p, hipStream_t stream) {
   if constexpr (QB == 64 && D == 128) {
-    if (p.dq_step == 32) return launch_dq<BF16, CAP, D, QB, KB, 32>(p, stream);
+    if (p.dq_step == 32) {
+      using Shape = BwdDqShape<BF16, CAP, D, QB, KB, QB, 1, 32>;
+      return launch_bwd_kernel<bwd_dq_short<BF16, CAP, D, QB, KB>>(p, p.Tq, Shape::kThreads, Shape::kLdsBytes,
+                                                                   Shape::kLdsBytes, stream);
+    }
   }
-  return launch_dq<BF16, CAP, D, QB, KB, 64>(p, stream);
+  using Shape = BwdDqShape<BF16, CAP, D, QB, KB, QB, 1, 64>;
+  return launch_bwd_kernel<bwd_dq_kernel<BF16, CAP, D, QB, KB>>(p, p.Tq, Shape::kThreads, Shape::kLdsBytes,
+                                                                Shape::kLdsBytes, stream);
 }
 template <bool BF16, bool CAP, int D, int QT, int KG, int STEP>
 int launch_dq_ksplit(const BwdParams& p, hipStream_t stream) {
@@ -1444,7 +1449,7 @@ int launch_bwd_cap(const BwdParams& p, hipStream_t stream) {
   switch (p.dq_split) {
     case FwdSplit::kRows32x4: e = launch_dq_ksplit<BF16, CAP, D, 32, 4, 32>(p, stream); break;
     case FwdSplit::kRows64x2: e = launch_dq_ksplit<BF16, CAP, D, 64, 2, 64>(p, stream); break;
-    default: e = launch_dq_blocks<BF16, CAP, D, QB, KB>(p, stream); break;
+    default: e = launch_dq<BF16, CAP, D, QB, KB>(p, stream); break;
   }
   if (e != 0) return e;
   if constexpr (D != 128) {

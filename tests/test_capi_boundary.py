@@ -120,6 +120,10 @@ def test_kernel_resources_of_the_built_library():
         assert len(inst) == 48
         for name, r in inst.items():
             assert r["scratch_bytes"] == 0 and r["waves_per_simd"] >= 2, (name, r)
+    short = {k: v for k, v in kernels.items() if "bwd_dq_short" in k}  # 64-row blocks at head_dim 128
+    assert len(short) == 8
+    for name, r in short.items():
+        assert r["scratch_bytes"] == 0 and r["waves_per_simd"] >= 2, (name, r)
     low_bwd = {"k_bwd_dkdv_kernel_x": {"scratch_bytes": 0, "vgpr_spills": 0, "sgpr_spills": 0, "waves_per_simd": 1}}
     with pytest.raises(RuntimeError, match="waves per SIMD"):
         build.check_resources(low_bwd)

@@ -52,14 +52,14 @@ RESOURCES_JSON = os.path.join(OBJ, "kernel_resources.json")
 # The backward kernels and the forward with split lists keep scalar values in spare vector lanes here
 # and there (SGPR spills, no memory behind them): for them only scratch memory and spilled vector registers fail the build.
 MIN_WAVES_PER_SIMD = {"fwd_kernel": 2, "fwd_ksplit": 2, "bwd_dq_kernel": 2, "bwd_dq_short": 2, "bwd_dq_ksplit": 2,
-                      "bwd_dkdv_kernel": 2, "bwd_dkdv_split": 2, "fwd_generic_kernel": 1,
-                      "ELi8ELNS_4Rows": 2}  # (its forms of eight waves)
+                      "bwd_dkdv_kernel": 2, "bwd_dkdv_split": 2, "fwd_generic_": 2}
 SGPR_SPILLS_ALLOWED = ("bwd_dq_", "bwd_dkdv_", "fwd_ksplit", "fwd_generic_")
 # For the generic kernel scratch memory is what counts.  Forms that read rows at any alignment (E1E) have some: up to 32 columns
 # and 97 - 128 in fp16 (two registers' worth; at B=1 H=8 S=2048 D=125 48.5 us, 52.9 without, where the addresses of the
 # loads are worked out anew in every step) and 225 - 256 (half a tile's rows in flight in registers; with four waves, which
-# have twice as many, B=1 H=4 S=1500 D=250 took 97.6 us, 54.2 so); and blocks of any number of keys (E4E) at 225 - 256
-# columns in fp16.
+# have twice as many, B=1 H=4 S=1500 D=250 took 97 us in bf16 and 112 in fp16, 56 and 57 so); and blocks of any number of
+# keys (E4E) at 225 - 256 columns in fp16 (three registers' worth; B=1 H=8 24x24 D=256 S=512 27.2 us with four waves, 16.7 so,
+# S=720 32.7 and 20.0).
 VGPR_SPILLS_ALLOWED = ("fwd_generic_",)
 SCRATCH_ALLOWED = {"fwd_generic_kernelILb0ELi1ELi8ELNS_4RowsE1E": 8, "fwd_generic_kernelILb0ELi4ELi8ELNS_4RowsE1E": 8,
                    "fwd_generic_kernelILb0ELi8ELi8ELNS_4RowsE1E": 64, "fwd_generic_kernelILb1ELi8ELi8ELNS_4RowsE1E": 64,

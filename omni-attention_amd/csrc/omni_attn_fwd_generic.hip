@@ -15,10 +15,11 @@
 //
 // S^T = K.Q^T and O^T = V^T.P^T with v_mfma_f32_32x32x16 as in the tuned forward: a lane owns a query
 // row; the K and V rows of a step go to tiles of the wave in LDS, straight from global memory where rows
-// lie on 16-byte boundaries (the rows of the next step are requested as soon as the products have read
-// a tile).  A weight is a sum of three 16-bit parts with one product each.  fp16 has few exponents: weights
-// are scaled by 2^11 first, and those below 2^-12 of the reference (scores of a peaked row) leave a rest
-// that goes through two more products of the steps that have any.
+// lie on 16-byte boundaries.  Up to 128 columns a wave has a tile for each, and the rows of the next step are
+// requested as soon as the products have read it; beyond, it has one tile, which V takes over from K and the next step's
+// K from V, and the other wave of its SIMD works meanwhile.  A weight is a sum of three 16-bit parts with one
+// product each.  fp16 has few exponents: weights are scaled by 2^11 first, and those below 2^-12 of the
+// reference (scores of a peaked row) leave a rest that goes through two more products of the steps that have any.
 //
 // A key that a row may not attend to never reaches it, whatever its V row holds (0 * infinity would):
 // a wave whose sums end up infinite or NaN walks its list once more and leaves out the zero weights.
@@ -28,7 +29,7 @@
 // that go to LDS directly have their offsets laid out once, their fragments are fetched in groups (K, and V under the
 // weights; three ahead beyond 128 columns), and a weight's part is taken off without being converted first.  B=1 H=8
 // S=2048 D=96, causal in 32x32 blocks, launches back to back: fp16 23.8 us, bf16 23.0 (28.7 and 26.9 without); spans in
-// 64x64 blocks at B=1 H=4 S=1500: D=136 21.6, D=208 26.3, D=256 29.6; rows at any alignment, D=101 34.7, D=165 40.3.
+// 64x64 blocks at B=1 H=4 S=1500 bf16: D=136 22.4, D=208 26.9, D=256 29.2; rows at any alignment, D=101 35.3, D=131 37.0, D=165 41.9.
 // 33 us (37) at D=96 where queries are four times as large (every row peaked, a rest in most steps).  Two parts per
 // weight, cut off after 22 bits and at 2^-32 of the reference, gain 2 us, but are
 // not the scalar kernel's sum.  One wave per row with vector arithmetic: 1934 us.
@@ -284,10 +285,10 @@ struct GenericTraits {
   static constexpr int kTileBytes = 32 * kRowBytes;
   // Beyond 128 columns LDS has room for K and V of four waves, one to a SIMD, or for one tile of eight, where V takes
   // the place of K as soon as that is read.  The loads of a wave then run under its softmax and the other wave of the SIMD
-  // only, but a list has half the steps per wave and a SIMD two waves to issue from.  (A lone wave took 7000 cycles for a
-  // step of 1800 cycles of products at D=208.)  What eight waves have no registers for is worked out anew in each step
-  // (addresses of fragments) or lies in LDS (Q, offsets of rows).  B=1 H=8, bf16, us, four waves -> eight: S=1024 causal 32x32
-  // D=136 20.0 -> 15.5, D=208 29.8 -> 19.4, D=256 29.7 -> 21.9; S=64 D=208 10.5 -> 8.5; S=715 rows at any alignment D=165
+  // only, but a list has half the steps per wave and a SIMD two waves to issue from.  (At S=1024 D=208 a lone wave took
+  // 29.8 us over eight steps of 1800 cycles of products.)  What eight waves have no registers for is worked out anew in each
+  // step (addresses of fragments) or lies in LDS (Q, offsets of rows).  B=1 H=8, bf16, us, four waves -> eight: S=1024 causal 32x32
+  // D=136 20.0 -> 15.2, D=208 29.8 -> 19.4, D=256 29.7 -> 21.9; S=64 D=208 10.5 -> 8.5; S=715 rows at any alignment D=165
   // 43.8 -> 23.5, D=250 51.3 -> 30.8; blocks of 40 keys D=256 34.1 -> 23.8.  Twelve waves up to 96 columns: 4 % slower.
   static constexpr bool kShared = DT > 4 && NW == 8;
   static constexpr size_t kWaveBytes = size_t(kShared ? 1 : 2) * kTileBytes;

@@ -29,8 +29,8 @@
 // that go to LDS directly have their offsets laid out once, their fragments are fetched in groups (K, and V under the
 // weights; three ahead beyond 128 columns), and a weight's part is taken off without being converted first.  B=1 H=8
 // S=2048 D=96, causal in 32x32 blocks, launches back to back: fp16 23.8 us, bf16 23.0 (28.7 and 26.9 without); spans in
-// 64x64 blocks at B=1 H=4 S=1500 bf16: D=136 22.4, D=208 26.9, D=256 29.2; rows at any alignment, D=101 35.3, D=131 37.0, D=165 41.9.
-// 33 us (37) at D=96 where queries are four times as large (every row peaked, a rest in most steps).  Two parts per
+// 64x64 blocks at B=1 H=4 S=1500 bf16: D=136 22.4, D=208 26.9, D=256 29.2; rows at any alignment, D=101 35.3, D=131 37.0,
+// D=165 41.9.  33 us (37) at D=96 where queries are four times as large (every row peaked, a rest in most steps).  Two parts per
 // weight, cut off after 22 bits and at 2^-32 of the reference, gain 2 us, but are
 // not the scalar kernel's sum.  One wave per row with vector arithmetic: 1934 us.
 #include "../../include/omni_attn_gfx950.h"
@@ -145,18 +145,18 @@ __device__ __forceinline__ void buffer_to_lds(i32x4_t rsrc, uint32_t lane_off, u
       : "memory", "m0");
 }
 // N such loads from one uniform offset, 1 KiB of LDS apart.  (The offset in the instruction counts for both addresses, and
-// is taken off the uniform one again, which is at least kBack: the check of the range does not take a negative one.  size: of
-// the buffer, for these loads.  A load by itself takes three scalar instructions more.  With scores that are masked in place and weights that are split without
+// is taken off the uniform one again, which is at least kBack: the check of the range does not take a negative one.  A load by
+// itself takes three scalar instructions more.  With scores that are masked in place and weights that are split without
 // copies, fp16 B=1 H=8 S=2048 causal 32x32 D=96 24.3 -> 23.8 us, D=120 29.3 -> 28.8, D=256 S=1024 21.9 -> 21.3.)
-using omni_attn::kBack;
+constexpr uint32_t kBack = 3072;
 template <int N>
-__device__ __forceinline__ void buffer_to_lds_in_a_row(i32x4_t rsrc, uint32_t size, const uint32_t* lane_off,
-                                                       uint32_t uniform_off, uint32_t lds_base) {
-  static_assert(N >= 1 && (N - 1) * 1024 <= int(kBack), "offsets in the instruction");
+__device__ __forceinline__ void buffer_to_lds_in_a_row(i32x4_t rsrc, const uint32_t* lane_off, uint32_t uniform_off,
+                                                       uint32_t lds_base) {
+  static_assert(N >= 1 && N <= 4, "twelve bits of offset");
   i32x4_t r;
   r[0] = __builtin_amdgcn_readfirstlane(rsrc[0]);
   r[1] = __builtin_amdgcn_readfirstlane(rsrc[1]);
-  r[2] = __builtin_amdgcn_readfirstlane(int32_t(size));
+  r[2] = __builtin_amdgcn_readfirstlane(rsrc[2]);
   r[3] = __builtin_amdgcn_readfirstlane(rsrc[3]);
   const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds_base), u = __builtin_amdgcn_readfirstlane(uniform_off);
   if constexpr (N == 1) {
@@ -557,7 +557,7 @@ __device__ __forceinline__ void generic_walk(const GenericParams& p) {
     i32x4_t r;
     r[0] = __builtin_amdgcn_readfirstlane(int32_t(uint32_t(a)));
     r[1] = __builtin_amdgcn_readfirstlane(int32_t(uint32_t(a >> 32) & 0xffffu));
-    r[2] = __builtin_amdgcn_readfirstlane(int32_t(omni_attn::rows_end(p.seqlen, pitch, p.D, back)));
+    r[2] = __builtin_amdgcn_readfirstlane(int32_t(uint32_t((int64_t(p.seqlen) - 1) * pitch + p.D) * 2u + back));
     r[3] = 0x00020000;
     return r;
   };
@@ -593,12 +593,11 @@ __device__ __forceinline__ void generic_walk(const GenericParams& p) {
         }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          const int row0 = WHOLE ? half[0].row0 + 16 * h : half[h].row0;
-          // (not so where no row attends to the half, and a second half may begin behind the sequence)
-          const omni_attn::HalfAt from = omni_attn::half_at(row0 < p.seqlen, row0, pitch2, uint32_t(rsrc[2]));
-          buffer_to_lds_in_a_row<(DT < 4 ? DT : 4)>(rsrc, from.size, at, from.offset, to + uint32_t(h * DT) * 1024u);
-          if constexpr (DT > 4)
-            buffer_to_lds_in_a_row<DT - 4>(rsrc, from.size, at + 4, from.offset, to + uint32_t(h * DT + 4) * 1024u);
+          // (of a half that begins at the end of the sequence or behind it every lane is outside the buffer)
+          const uint32_t row0_at =
+              kBack + (WHOLE ? uint32_t(half[0].row0) * pitch2 + (h == 0 ? 0u : 16u * pitch2) : uint32_t(half[h].row0) * pitch2);
+          buffer_to_lds_in_a_row<(DT < 4 ? DT : 4)>(rsrc, at, row0_at, to + uint32_t(h * DT) * 1024u);
+          if constexpr (DT > 4) buffer_to_lds_in_a_row<DT - 4>(rsrc, at + 4, row0_at, to + uint32_t(h * DT + 4) * 1024u);
         }
       } else {
 #pragma unroll
@@ -1278,7 +1277,7 @@ int forward_generic(const void* q, const void* k, const void* v, const omni_attn
   if (grid > 0x7fffffffLL) return OMNI_ATTN_ERR_TOO_LARGE;
   const auto direct = [&](const void* ptr, const omni_attn_strides& at) {  // 32-bit offsets inside a slab
     return !misaligned(ptr, 16) && at.batch % 8 == 0 && at.head % 8 == 0 && at.row % 8 == 0 && at.row >= D &&
-           ((long long)p.seqlen + 31) * at.row * 2 < 0xffffff00LL - kBack;  // (a step may run 31 rows past the sequence)
+           ((long long)p.seqlen + 32) * at.row * 2 < 0xffffff00LL - kBack;  // (a step that is not read begins behind the sequence)
   };
   const bool halves = KB % 16 == 0 && !misaligned(partial_masks_or_null, 4);  // half a step never crosses a block
   const Rows reads = D < 8                                                         ? Rows::kSmall

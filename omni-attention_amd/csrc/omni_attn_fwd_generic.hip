@@ -1234,7 +1234,8 @@ int forward_generic(const void* q, const void* k, const void* v, const omni_attn
   if (B <= 0 || H <= 0 || S_pad <= 0 || Tq <= 0 || max_blocks <= 0 || seqlen_orig < 0 || num_partial < 0 ||
       !(softcap >= 0.f) || std::isinf(softcap))
     return OMNI_ATTN_ERR_BAD_SHAPE;
-  if (Tq != omni_attn::blocks_of(S_pad, QB)) return OMNI_ATTN_ERR_BAD_SHAPE;
+  // (rows of the last query block are ints, also those behind the sequence)
+  if ((long long)S_pad + QB - 1 > 0x7fffffffLL || Tq != omni_attn::blocks_of(S_pad, QB)) return OMNI_ATTN_ERR_BAD_SHAPE;
   const long long rows = (long long)B * H * S_pad;
   if ((long long)S_pad * D > 0x7fffffffLL || rows > (1LL << 33) || (long long)B * H * Tq * max_blocks > (1LL << 40))
     return OMNI_ATTN_ERR_TOO_LARGE;

@@ -2,6 +2,8 @@
 import os
 import subprocess
 
+import omni_attn_capi
+
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "omni-attention_amd", "csrc")
 
 
@@ -46,3 +48,16 @@ int main() {
       }
 }
 """)
+
+
+def test_query_blocks_beyond_the_largest_int_are_refused():
+    """Rows are ints, also those of the last query block that lie behind the sequence."""
+    lib = omni_attn_capi.load_library()
+    one = 4096  # any non-null value: validation fails before it would be dereferenced
+    def call(S, QB, KB=32, D=1):
+        return lib.omni_attn_fwd_generic_gfx950(one, one, one, one, 0, one, one, one, 0, 0, 1, 1, S, D, -(-S // QB), 1, QB, KB,
+                                                0, 0, 0, 0.0, 0)
+    most = 2 ** 31 - 1
+    for S, QB in ((most, 2), (most, 64), (most, most), (most - 30, 32), (100, most), (most - 46, 48)):
+        assert call(S, QB) == 2, (S, QB)
+    assert call(most - 1, 1, D=2) == 7  # too large, not a bad shape
